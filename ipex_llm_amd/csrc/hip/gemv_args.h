@@ -1,5 +1,5 @@
 // Host/device-shared argument block and enums of the low-bit GEMV
-// (lowbit_gemv.cuh).  No device code: included by the torch op wrappers.
+// (lowbit_gemv5.cuh, lowbit_skinny.cuh).  No device code: included by the torch op wrappers.
 #pragma once
 #include <stdint.h>
 

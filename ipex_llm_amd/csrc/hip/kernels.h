@@ -12,10 +12,7 @@ namespace illm {
 #include "gemv_args.h"
 namespace illm {
 
-// ---- low-bit GEMV / skinny GEMM (lowbit_gemv.cuh) -------------------------
-// dk = decoder kind (fmt_to_dk), mt = ceil(M/16) in {1,2,4}
-template <int DK>
-void launch_gemv_dk(bool bf16, int mt, int epi, dim3 grid, const GemvArgs& a, hipStream_t st);
+// ---- low-bit GEMV (17 rows and up: kernels_skinny.h) -----------------------
 // v5 (M <= 16, lowbit_gemv5.cuh): workgroup = 4 waves = (4 / kw) tile groups
 // x kw k-parts; grid = (ceil(groups / (4 / kw)), ksplit[, experts]),
 // shmem = gemv5_shmem(rows, chunks per split) <= 159 KiB

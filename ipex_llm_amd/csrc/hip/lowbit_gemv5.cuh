@@ -34,96 +34,9 @@
 #include "../common/quant_block.h"
 #include "gemv_args.h"
 #include "illm_device.h"
+#include "lowbit_raw.h"
 
 namespace illm {
-
-// packed-pair nibble extract (x & m) | c as ONE v_and_or_b32: hipcc splits
-// the pattern into v_and + v_or (gfx9 VOP3 takes no literal and one
-// constant-bus read), so the mask is an SGPR and the magic a VGPR operand
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t m_s, uint32_t c_v) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(m_s), "v"(c_v));
-  return r;
-}
-
-template <typename C> struct Raw;
-template <> struct Raw<BF16> {
-  static constexpr uint32_t k4 = 0x43004300u;   // bf16(128 + q)
-  static constexpr float off4 = 128.f;
-};
-template <> struct Raw<F16> {
-  static constexpr uint32_t k4 = 0x64006400u;   // f16(1024 + q)
-  static constexpr float off4 = 1024.f;
-};
-
-// raw value offset per decoder: value = code_raw - OFF (before scale)
-template <int DK, typename C>
-__host__ __device__ constexpr float raw_off() {
-  return DK == DK_INT4S ? Raw<C>::off4 + 8.f
-       : DK == DK_INT4A ? Raw<C>::off4
-       : DK == DK_INT8S ? 128.f
-       : 0.f;
-}
-
-template <int DK, typename C>
-__device__ __forceinline__ uint4 raw_a4(uint32_t u, uint32_t mask_s, uint32_t magic_v, const uint32_t* lut2) {
-  uint4 r;
-  if constexpr (DK == DK_INT4S || DK == DK_INT4A) {
-    r.x = and_or(u, mask_s, magic_v);
-    r.y = and_or(u >> 4, mask_s, magic_v);
-    r.z = and_or(u >> 8, mask_s, magic_v);
-    r.w = and_or(u >> 12, mask_s, magic_v);
-  } else if constexpr (DK == DK_FP4) {
-    if constexpr (std::is_same<C, BF16>::value) {
-      r.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(u, 1.0f, 0));
-      r.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(u, 1.0f, 1));
-      r.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(u, 1.0f, 2));
-      r.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(u, 1.0f, 3));
-    } else {
-      r.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(u, 1.0f, 0));
-      r.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(u, 1.0f, 1));
-      r.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(u, 1.0f, 2));
-      r.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(u, 1.0f, 3));
-    }
-  } else {  // DK_LUT4 (C = F16 pair table)
-    r.x = lut2[u & 0xff];
-    r.y = lut2[(u >> 8) & 0xff];
-    r.z = lut2[(u >> 16) & 0xff];
-    r.w = lut2[u >> 24];
-  }
-  return r;
-}
-
-template <int DK, typename C>
-__device__ __forceinline__ uint32_t raw_pair8(uint32_t u, bool hi) {
-  if constexpr (DK == DK_FP8E4) {
-    if constexpr (std::is_same<C, BF16>::value)
-      return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u, 1.0f, true)
-                                             : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u, 1.0f, false));
-    else
-      return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u, 1.0f, true)
-                                             : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u, 1.0f, false));
-  } else if constexpr (DK == DK_FP8E5) {
-    if constexpr (std::is_same<C, BF16>::value)
-      return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(u, 1.0f, true)
-                                             : __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(u, 1.0f, false));
-    else
-      return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_f16_bf8(u, 1.0f, true)
-                                             : __builtin_amdgcn_cvt_scalef32_pk_f16_bf8(u, 1.0f, false));
-  } else {
-    // integer bytes through the exact small-integer float conversion;
-    // signed codes are biased by 128 (raw_off = 128)
-    if constexpr (DK == DK_INT8S) u ^= 0x80808080u;
-    const int sh = hi ? 16 : 0;
-    return pack2<C>((float)((u >> sh) & 0xff), (float)((u >> (sh + 8)) & 0xff));
-  }
-}
-
-template <int DK, typename C>
-__device__ __forceinline__ uint4 raw_a8(uint32_t lo, uint32_t hi) {
-  return make_uint4(raw_pair8<DK, C>(lo, false), raw_pair8<DK, C>(lo, true), raw_pair8<DK, C>(hi, false),
-                    raw_pair8<DK, C>(hi, true));
-}
 
 // LDS plan of one workgroup (bytes): x slice [rows][kw + 8] in C, then per
 // (row, chunk) float4 {-OFF*sx0, -OFF*sx1, sx0, sx1}, then the KW reduction

@@ -10,6 +10,7 @@
 
 #include "../common/formats.h"
 #include "../hip/kernels.h"
+#include "../hip/kernels_skinny.h"
 #include "../hip/gemv_args.h"
 
 using at::Tensor;
@@ -75,9 +76,50 @@ Tensor dequantize_device(const Tensor& blob, int64_t fmt, int64_t n, int64_t k, 
     default: TORCH_CHECK(false, "gemv: unsupported fmt ", fmt);              \
   }
 
-void launch_gemv_any(int fmt, bool bf16, int mt, int epi, dim3 grid, const illm::GemvArgs& a) {
+// geometry of lowbit_skinny.cuh: workgroups of nw tiles x 16 mt rows x cpk chunks
+struct SkinnyPlan {
+  int mt, nw, cpk;
+  dim3 grid;
+};
+// The split with the least estimated time.  A CU runs one 8-wave or two 4-wave workgroups at a time; a
+// round of them takes 3 us (launch, first loads, epilogue) and 0.5 / 0.6 / 0.8 us per 128-k chunk at
+// 2 / 3 / 4 row tiles (MI355X: gate/up of Llama-3-8B, 32 chunks in one round, 21 / 25 / 30 us; two 4-wave
+// groups 24 / 30 / 36, one alone on its CU about 0.65 of that: Qwen2.5-7B's 296 column blocks as 592 of
+// half the size 36 instead of 40 us, a [2048, 1024] gate/up 5.7 instead of 6.7); slabs cost their write
+// and read (4.5 TB/s) and the reduction.  ks_req > 0: that many slabs as asked.
+SkinnyPlan skinny_plan(int64_t M, int64_t NT, int64_t KC, bool can_split, int64_t ks_req = 0) {
+  SkinnyPlan best{};
+  const int64_t MB = (M + 63) / 64;
+  const int mt = std::max<int>(2, (int)(((M + MB - 1) / MB + 15) / 16));
+  const double chunk = mt == 2 ? 0.5 : mt == 3 ? 0.6 : 0.8;
+  const int64_t kmax = !can_split ? 1 : ks_req > 0 ? ks_req : (KC + 3) / 4;
+  double cost = 1e30;
+  for (int nw = 8; nw >= 4; nw -= 4) {
+    const int64_t NB = (NT + nw - 1) / nw, slots = 256 * 8 / nw;
+    int64_t last = 0;
+    for (int64_t k = ks_req > 0 && can_split ? kmax : 1; k <= kmax && k <= 64; k++) {
+      int64_t ks = k, cpk = (KC + k - 1) / k;
+      if (ks_req > 0 && can_split) cpk = (cpk + 1) / 2 * 2;
+      else cpk = (cpk + 3) / 4 * 4, ks = (KC + cpk - 1) / cpk;     // the kernel's two steps of two chunks
+      if (cpk == last) continue;
+      last = cpk;
+      const int64_t wg = NB * MB * ks, rest = wg % slots;
+      const double rounds = wg / slots + (rest == 0 ? 0. : nw == 4 && rest <= 256 ? 0.65 : 1.);
+      const double c = rounds * (nw == 8 ? 3. + cpk * chunk : 2.5 + 1.15 * cpk * chunk) + (ks > 1 ? 2.5 + ks * M * NT * 16 * 8 / 4.5e6 : 0.);
+      if (c < cost) {
+        cost = c;
+        best = SkinnyPlan{mt, nw, (int)cpk, dim3((unsigned)(MB == 1 ? NB : (NB + 7) / 8 * 8 * MB), (unsigned)ks)};
+      }
+    }
+  }
+  return best;
+}
+void launch_skinny_any(int fmt, bool bf16, const SkinnyPlan& p, int epi, const illm::GemvArgs& a0) {
   hipStream_t st = cur_stream();
-  ILLM_DK_SWITCH(fmt, illm::launch_gemv_dk<DKV>(bf16, mt, epi, grid, a, st));
+  illm::GemvArgs a = a0;
+  a.cpk = p.cpk;
+  TORCH_CHECK((int64_t)a.M * a.ldx * 2 < ((int64_t)1 << 32), "gemv: x of 4 GB or more");
+  ILLM_DK_SWITCH(fmt, illm::launch_skinny_dk<DKV>(bf16, p.mt, p.nw, epi, p.grid, a, st));
 }
 int* kernel_err(const c10::Device& dev);
 void launch_gemv5_any(int fmt, bool bf16, int kw, int epi, dim3 grid, size_t shmem, const illm::GemvArgs& a0) {
@@ -94,13 +136,6 @@ void launch_gemv5_any(int fmt, bool bf16, int kw, int epi, dim3 grid, size_t shm
 }
 
 constexpr size_t kMaxLds = 159 * 1024;
-
-// v1 (M > 16): split K over workgroups until there are >= 768 of them
-int64_t auto_ksplit(int64_t NT, int64_t KC) {
-  int64_t ks = 1;
-  while (NT * ks < 768 && KC >= 4 * 2 * (ks * 2)) ks *= 2;
-  return ks;
-}
 
 // v5 geometry (M <= 16): each of `groups` tile groups (a tile, or a gate/up
 // tile pair for GLU) is streamed by kw waves of one workgroup (in-LDS
@@ -166,20 +201,20 @@ Plan5 plan5_rope(Plan5 p, int64_t NT, int64_t rows) {
   return p;
 }
 
-Tensor gemv(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
-            const c10::optional<Tensor>& bias, int64_t epi, int64_t ksplit, int64_t act) {
+// rows 1 .. most: v5 up to 16 rows (ILLM_GEMV_V1=1: the many-row kernel for these too, A/B tests), the
+// skinny kernel from 17
+Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
+                   const c10::optional<Tensor>& bias, int64_t epi, int64_t ksplit, int64_t act, int64_t most) {
   TORCH_CHECK(x.is_cuda() && blob.is_cuda(), "gemv: GPU tensors expected");
   TORCH_CHECK(x.size(-1) == k, "gemv: x last dim ", x.size(-1), " != in_features ", k);
   c10::DeviceGuard g(x.device());
   const bool bf16 = is_bf16(x);
   Tensor xc = x.contiguous();
   const int64_t M = xc.numel() / k;
-  TORCH_CHECK(M >= 1 && M <= 64, "gemv handles 1..64 rows, got ", M);
+  TORCH_CHECK(M >= 1 && M <= most, "gemv handles 1..", most, " rows, got ", M);
   TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv: weight blob too small");
-  const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N;
   const int64_t KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
-  // M <= 16 runs v5 (ILLM_GEMV_V1=1 forces the general kernel, for A/B tests)
   const bool small = M <= 16 && getenv("ILLM_GEMV_V1") == nullptr;
 
   illm::GemvArgs a{};
@@ -204,11 +239,12 @@ Tensor gemv(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t
     if (small && p.shmem <= kMaxLds)
       a.nw = p.nw, launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);
     else
-      launch_gemv_any((int)fmt, bf16, mt, illm::EPI_GLU, dim3((unsigned)(NT / 2), 1), a);
+      launch_skinny_any((int)fmt, bf16, skinny_plan(M, NT, KC, false), illm::EPI_GLU, a);
     return out;
   }
   a.N = (int)n;
   Plan5 p5{};
+  SkinnyPlan q{};
   bool use5 = false;
   if (small) {
     p5 = plan5(M, NT, KC, true, ksplit);
@@ -219,12 +255,12 @@ Tensor gemv(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t
     a.cpk = (int)p5.cpk;
     a.nw = p5.nw;
   } else {
-    if (ksplit <= 0) ksplit = auto_ksplit(NT, KC);
-    ksplit = std::min<int64_t>(ksplit, KC);
+    q = skinny_plan(M, NT, KC, true, std::min<int64_t>(ksplit, KC));
+    ksplit = q.grid.y;
   }
   auto launch = [&](int e) {
     if (use5) launch_gemv5_any((int)fmt, bf16, p5.kw, e, dim3(p5.gx, (unsigned)ksplit), p5.shmem, a);
-    else launch_gemv_any((int)fmt, bf16, mt, e, dim3((unsigned)NT, (unsigned)ksplit), a);
+    else launch_skinny_any((int)fmt, bf16, q, e, a);
   };
   if (epi == illm::EPI_PARTIAL || ksplit > 1) {
     Tensor ws = at::empty({ksplit, M, n}, xc.options().dtype(at::kFloat));
@@ -245,6 +281,18 @@ Tensor gemv(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t
   a.bias = p16o(bias);
   launch(illm::EPI_STORE);
   return out;
+}
+
+Tensor gemv(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
+            const c10::optional<Tensor>& bias, int64_t epi, int64_t ksplit, int64_t act) {
+  return lowbit_rows(x, blob, fmt, n, k, bias, epi, ksplit, act, 64);
+}
+
+// x @ W^T (+ bias) (or the GLU of a gate/up weight) of a few hundred rows on the skinny kernel: several row
+// blocks over one weight stream
+Tensor gemm_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
+                 const c10::optional<Tensor>& bias, bool glu, int64_t act) {
+  return lowbit_rows(x, blob, fmt, n, k, bias, glu ? illm::EPI_GLU : illm::EPI_STORE, glu ? 1 : 0, act, 1 << 16);
 }
 
 // greedy decode head: the v5 GEMV stores the logits (T) and every wave writes
@@ -1721,6 +1769,7 @@ TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("quantize_device", &quantize_device);
   m.impl("dequantize_device", &dequantize_device);
   m.impl("gemv", &gemv);
+  m.impl("gemm_rows", &gemm_rows);
   m.impl("gemv_accum", &gemv_accum);
   m.impl("gemv_accum_norm", &gemv_accum_norm);
   m.impl("gemv_glu_ss", &gemv_glu_ss);

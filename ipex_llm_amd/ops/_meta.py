@@ -28,6 +28,13 @@ def _(x, blob, fmt, n, k, bias, epi, ksplit, act):
     return x.new_empty(shape)
 
 
+@register_fake("ipex_llm_amd::gemm_rows")
+def _(x, blob, fmt, n, k, bias, glu, act):
+    shape = list(x.shape)
+    shape[-1] = n // 2 if glu else n
+    return x.new_empty(shape)
+
+
 @register_fake("ipex_llm_amd::add_rms_norm")
 def _(x, partials, residual, w, eps, unit_offset, store_residual, zero_partials=False):
     if x is not None:

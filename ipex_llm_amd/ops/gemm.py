@@ -1,17 +1,16 @@
 """Prefill-size (M > 64) low-bit GEMM dispatch.
 
-Two paths: the MFMA kernel with in-register dequant (``csrc/hip/gemm.hip``:
-f16 MFMA, weights decoded straight from the tiled blob, never
-materialised), and dequantize to a transient dense weight + library GEMM
-(hipBLASLt).  Measured on MI355X at Llama-3-8B shapes (sym_int4, the fused
-kernel with its round-3 128 n x 64 m blocks below M = 1024,
-profiles/prefill_gemm_r3_small_tile6.jsonl): the fused kernel wins for the
-wide projections (M = 256: qkv 40 vs 53 us, gate_up 93 vs 129; M = 384:
-gate_up 130 vs 134) and for every shape at M <= 128 except the long-K down
-projection (M = 128: 113 vs 84 us -- its 4096-wide output gives few blocks
-for 14336-deep K); the library path wins above (M = 1024: qkv 64.7 vs 82,
-o 50 vs 62, gate_up 239 vs 318, down 138 vs 184).
-``ILLM_GEMM_LIB=1`` / ``ILLM_GEMM_FUSED=1`` force either path (A/B runs).
+Three paths: the skinny kernel (``csrc/hip/lowbit_skinny.cuh``: the decode
+kernel for 17 rows and up, weights streamed once, codes raw in the MFMA) while
+its row blocks fit one round of the chip; the MFMA kernel with in-register
+dequant (``csrc/hip/gemm.hip``: f16 MFMA, weights decoded straight from the
+tiled blob, never materialised) for the wide gate/up pairs above that; and
+dequantize to a transient dense weight + GEMM.  Measured on MI355X (Llama-3-8B,
+sym_int4, graph replays over weights that no cache holds), skinny against the
+better of the other two: M = 96 qkv 19 / 38 us, o 15 / 38, down 25 / 75,
+gate_up 47 / 56; M = 300 qkv 28 / 44, o 27 / 37, down 71 / 93, gate_up
+128 / 113; M = 512 o 28 / 38, down 86 / 104, qkv (two rounds) 52 / 48.
+``ILLM_GEMM_LIB=1`` / ``ILLM_GEMM_FUSED=1`` force either other path (A/B runs).
 """
 from __future__ import annotations
 
@@ -30,6 +29,29 @@ FUSED_LONG_K = 8192        # deeper K (down projections): library path from M > 
 FUSED_QKV_MAX_M = 256      # N >= 6144 (fused qkv) up to here
 FUSED_WIDE_MAX_M = 384     # N >= FUSED_WIDE_N (gate/up pairs) up to here
 FUSED_WIDE_N = 12288
+
+
+ROWS_MAX_M = 512           # skinny kernel up to here (from 512 rows on the dense paths are tiled for them)
+
+
+def rows_fit(M: int, n: int, fmt: int, glu: bool = False) -> bool:
+    """The skinny kernel's 64-row x 128-column blocks fit one round of the 256
+    CUs (a second round costs what the first did, and the compute-bound paths
+    are then ahead); formats with block minima, whose sums take a third more,
+    up to 5 / 8 of that.  Gate/up pairs up to 96 rows (Llama-3-8B, two rounds:
+    M = 96 47 / 56 us, M = 128 55 / 56), by the rows alone: a column shard of
+    a tensor-parallel model takes the kernel that the whole pair takes."""
+    if _USE_LIB or _USE_FUSED or M > ROWS_MAX_M:
+        return False
+    if glu:
+        return M <= 96
+    from ..quantize import qtypes as Q
+    blocks = (n + 127) // 128 * ((M + 63) // 64)
+    return blocks <= (160 if fmt in (Q.FMT_ASYM_INT4, Q.FMT_ASYM_INT5) else 256)
+
+
+def use_rows(x, M: int, n: int, fmt: int, glu: bool = False) -> bool:
+    return x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and rows_fit(M, n, fmt, glu)
 
 
 def use_fused(M: int, n: int, k: int = 0) -> bool:
@@ -72,7 +94,7 @@ def prefetch_dense(items, M: int, dtype) -> None:
         return
     ops = torch.ops.ipex_llm_amd
     for blob, fmt, n, k in items:
-        if not blob.is_cuda or use_fused(M, n, k):
+        if not blob.is_cuda or rows_fit(M, n, fmt) or use_fused(M, n, k):
             continue
         key = _key(blob, n, k, dtype)
         if key in _ready:
@@ -330,6 +352,8 @@ def lowbit_gemm(x, blob, fmt, n, k, bias=None):
     ops = torch.ops.ipex_llm_amd
     M = x.numel() // k
     bf16_bias = bias is None or bias.dtype == torch.bfloat16
+    if use_rows(x, M, n, fmt) and (bias is None or bias.dtype == x.dtype):
+        return ops.gemm_rows(x, blob, fmt, n, k, bias, False, 0)
     if use_g8(x, M, n, k, fmt) and bf16_bias:
         return ops.gemm8p_lowbit(x, blob, fmt, n, k, bias)
     if use_g8d(x, M, n, k) and bf16_bias:
@@ -353,6 +377,8 @@ def lowbit_gemm_glu(x, blob, fmt, n, k, act: int = 0):
     [M, 2I] round trip, no elementwise launches)."""
     ops = torch.ops.ipex_llm_amd
     M = x.numel() // k
+    if use_rows(x, M, n, fmt, glu=True):
+        return ops.gemm_rows(x, blob, fmt, n, k, None, True, act)
     if use_g8(x, M, n, k, fmt, glu=True):
         return ops.gemm8p_lowbit(x, blob, fmt, n, k, None, False, True, act)
     if use_g8d(x, M, n, k, glu=True) and act in (0, 1):
