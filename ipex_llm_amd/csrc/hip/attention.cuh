@@ -15,6 +15,7 @@
 // lengths and block tables are device tensors: the launch geometry depends
 // only on the max length bucket, so the whole thing is hipGraph-capturable.
 #pragma once
+#include <algorithm>
 #include <cstdlib>
 #include "../common/quant_block.h"
 #include "illm_device.h"

@@ -577,6 +577,285 @@ __global__ void __launch_bounds__(64 * NW, ILLM_V3_MINW(RQ)) attn_decode_v3_kern
   attn_v3_body<T, D, NW, RQ, FUSE>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, sm);
 }
 
+// ---- long contexts: several 32-key tiles per wave -------------------------
+// One tile per wave pays a workgroup's fixed chain (sequence length -> block
+// table -> K / V round trip -> max and sum over the waves -> partial) for every
+// 32 NW keys: 20 K keys x 3 sequences were 1896 workgroups in 7 rounds, 74 us
+// for 184 MB (2.5 TB/s).  Here a workgroup of 4 waves walks ``tiles`` tiles per
+// wave (tile = 128 keys of the workgroup, waves interleaved): running max /
+// sum / output in registers, the next tile's K requested behind the scores and
+// its V behind the LDS rows of this one, no barrier until the waves merge at
+// the end.  168 registers: 3 workgroups = 12 waves x 16 KB in flight per CU.
+// That case: 74 -> 55 us (3.3 TB/s).
+constexpr int V3L_NW = 4;
+
+template <typename T, int D, int RQ, bool FUSE>
+__global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const AttnDecodeArgs a, int tiles) {
+  constexpr int NW = V3L_NW;
+  constexpr int KSTEP = D / 32, DT = D / 16, VU = D / 8, KPJ = 64 / VU, VJ = V3_KPW / KPJ;
+  constexpr int SK = V3_KPW * NW;
+  static_assert(D == 64 || D == 128, "v3: head_dim 64 / 128");
+  static_assert(RQ == 0 || D == 128, "v3: fused RoPE needs head_dim 128");
+  __shared__ V3Smem<D, NW, RQ> sm;
+  const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int wv = threadIdx.x >> 6;
+  const int group = a.Hq / a.Hkv;
+  const int R = group * a.Tq;
+  const int k0 = split * SK * tiles;
+  int kw = k0 + V3_KPW * wv;                     // the wave's tile
+  uint16_t* vl = sm.vl;
+
+  int len = a.seq_lens[b];
+  auto entry = [&](int k) { return a.block_tables[(size_t)b * a.max_blocks + min(k / a.bs, a.max_blocks - 1)]; };
+  const int row = r16 < R ? r16 : 0;
+  const int t = row / group, h = kvh * group + row % group;
+  if ((int64_t)len > (int64_t)a.max_blocks * a.bs || (int64_t)a.nsplit * SPLIT < len) {
+    if (split == 0 && threadIdx.x == 0) kerr(a.err, ERR_SEQ_LEN);
+    len = min(min(len, a.max_blocks * a.bs), a.nsplit * SPLIT);
+  }
+  const size_t prow = (((size_t)b * a.Hq + h) * a.Tq + t) * a.nsplit + split;
+
+  if (k0 >= len) {
+    if (wv == 0 && g == 0 && r16 < R) {
+      if constexpr (FUSE) st8_sc1(a.part_ml + prow * 2, -INFINITY, 0.f);
+      else *(float2*)(a.part_ml + prow * 2) = make_float2(-INFINITY, 0.f);
+    }
+  } else {
+    // ---- q fragments (lane: row r16, dims 32 s + 8 g .. + 8)
+    uint4 qf[KSTEP];
+    if constexpr (RQ != 0) {
+      const V3Rope<T, D, RQ == 2> rp(a, b, g, true);
+      typename V3Rope<T, D, RQ == 2>::Raw raw;
+      typename V3Rope<T, D, RQ == 2>::CS cs;
+      rp.load(h * D, raw);
+      rp.load_cs(cs);
+      float v[KSTEP][8];
+      rp.vals(raw, v);
+      rp.frags(h * D, v, cs, a.rq_qscale, qf);
+      // the new token's k / v rows, appended by the wave whose tiles hold
+      // position len - 1 before it reads them (its own stores: in order)
+      const int nt = (len - 1 - k0) / V3_KPW;
+      if (nt % NW == wv && nt / NW < tiles) {
+        const int pos = len - 1, blk = entry(pos);
+        if (!bad_block(blk, a.num_blocks)) {
+          const size_t crow = (((size_t)blk * a.Hkv + kvh) * a.bs + pos % a.bs) * D;
+          rp.load((a.Hq + kvh) * D, raw);
+          rp.vals(raw, v);
+          uint4 kq[KSTEP];
+          rp.frags((a.Hq + kvh) * D, v, cs, 1.f, kq);
+          const int d0 = 8 * (lane % VU);
+          float4 f0, f1;
+          uint4 fb;
+          rp.vload((a.Hq + a.Hkv + kvh) * D + d0, f0, f1, fb);
+          float vv[8];
+          rp.vals8(f0, f1, fb, rp.rs(), vv);
+          if (r16 == 0)
+#pragma unroll
+            for (int s = 0; s < KSTEP; s++) *(uint4*)((uint16_t*)a.k_cache + crow + 32 * s + 8 * g) = kq[s];
+          if (lane < VU)
+            *(uint4*)((uint16_t*)a.v_cache + crow + d0) = make_uint4(pack2<T>(vv[0], vv[1]), pack2<T>(vv[2], vv[3]),
+                                                                   pack2<T>(vv[4], vv[5]), pack2<T>(vv[6], vv[7]));
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+    } else {
+      const uint16_t* qr = a.q + (((size_t)b * a.Tq + t) * a.Hq + h) * D;
+#pragma unroll
+      for (int s = 0; s < KSTEP; s++) qf[s] = *(const uint4*)(qr + 32 * s + 8 * g);
+    }
+    if (r16 >= R)
+#pragma unroll
+      for (int s = 0; s < KSTEP; s++) qf[s] = make_uint4(0, 0, 0, 0);
+
+    // ---- a tile's loads: rows past the sequence (or a bad block) read the tile's
+    // last valid row (block 0) and are masked by nvis
+    uint4 kf[2][KSTEP], vm[VJ];
+    int nvis = 0;
+    size_t base = 0;
+    int last = 0;
+    auto tile_at = [&](int blk) {
+      const int nkw = kw < len ? min(V3_KPW, len - kw) : 0;
+      const bool bad = nkw > 0 && bad_block(blk, a.num_blocks);
+      if (bad && lane == 0) kerr(a.err, ERR_BLOCK_ID);
+      nvis = bad ? 0 : nkw;
+      last = max(nvis, 1) - 1;
+      base = nvis > 0 ? (((size_t)blk * a.Hkv + kvh) * a.bs + kw % a.bs) * D : 0;
+    };
+    auto load_k = [&]() {
+      const uint16_t* kb = (const uint16_t*)a.k_cache + base;
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int s = 0; s < KSTEP; s++)
+          kf[kt][s] = *(const uint4*)(kb + (uint32_t)(min(kt * 16 + r16, last) * D + 32 * s + 8 * g));
+    };
+    auto load_v = [&]() {
+      const uint16_t* vb = (const uint16_t*)a.v_cache + base;
+#pragma unroll
+      for (int j = 0; j < VJ; j++)
+        vm[j] = *(const uint4*)(vb + (uint32_t)(min(j * KPJ + lane / VU, last) * D + 8 * (lane % VU)));
+    };
+
+    const int qpos = len - a.Tq + t;
+    const int win = a.sliding_window > 0 ? qpos - a.sliding_window : -1;
+    const float slope = a.alibi && r16 < R ? a.alibi[h] : 0.f;
+    float m = -INFINITY, l = 0.f;                // row r16: maximum; sum over this lane's keys
+    f32x4 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // tiles of this wave that hold keys (the first one runs in any case: fully masked if it holds none)
+    const int nt = max(1, min(tiles, (len - kw + SK - 1) / SK));
+
+    tile_at(entry(kw));
+    load_k();
+    load_v();
+    int blk_next = entry(kw + SK);
+    for (int it = 0; it < nt; it++) {
+      // ---- S^T tiles: lane holds (key = 16 kt + 4 g + i, row = r16)
+      f32x4 st[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KSTEP; s++) acc = mfma16<T>(kf[kt][s], qf[s], acc);
+        st[kt] = acc;
+      }
+      const int klim = min(nvis, qpos - kw + 1), kwc = kw;        // keys kk < klim are visible
+      // the V rows to the wave's own LDS rows (a masked tile's may be anything finite or not: P is 0 there,
+      // so they are cleared), then the next tile's loads into the freed registers
+      const uint32_t keep = nvis > 0 ? ~0u : 0u;
+      int ln = lane;
+      asm volatile("" : "+v"(ln));               // the LDS addresses are recomputed per tile: hoisted, they spill
+#pragma unroll
+      for (int j = 0; j < VJ; j++)
+        *(uint4*)(vl + pf_off<D>(V3_KPW * wv + j * KPJ + ln / VU, ln % VU)) =
+            make_uint4(vm[j].x & keep, vm[j].y & keep, vm[j].z & keep, vm[j].w & keep);
+      __builtin_amdgcn_sched_barrier(0);
+      if (it + 1 < nt) {
+        kw += SK;
+        tile_at(blk_next);
+        load_k();
+        load_v();
+        blk_next = entry(kw + SK);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) st[kt][i] *= a.scale;
+      if (a.softcap > 0.f) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) st[kt][i] = a.softcap * tanhf(st[kt][i] / a.softcap);
+      }
+      if (a.alibi) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) st[kt][i] += slope * (float)(kwc + kt * 16 + 4 * g + i);
+      }
+      float mt = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int kk = kt * 16 + 4 * g + i;
+          const bool ok = r16 < R && kk < klim && kwc + kk > win;
+          st[kt][i] = ok ? st[kt][i] : -INFINITY;
+          mt = fmaxf(mt, st[kt][i]);
+        }
+      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      const float mn = fmaxf(m, mt);
+      const float f = m == -INFINITY ? 0.f : __expf(m - mn);      // nothing summed yet: l and o are 0
+      m = mn;
+      l *= f;
+#pragma unroll
+      for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[d][i] *= f;
+      // ---- P (T precision, as the MFMA consumes it)
+      uint32_t pk[2][2];
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++) {
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          p[i] = m == -INFINITY ? 0.f : __expf(st[kt][i] - m);
+          l += p[i];
+        }
+        pk[kt][0] = pack2<T>(p[0], p[1]);
+        pk[kt][1] = pack2<T>(p[2], p[3]);
+      }
+      // ---- O^T += V^T P^T over the tile's 32 keys
+      asm volatile("" : "+v"(ln));
+      const int row0 = V3_KPW * wv + 4 * (ln >> 4) + ((ln & 15) >> 2), row1 = row0 + 16;
+      const uint4 pb = make_uint4(pk[0][0], pk[0][1], pk[1][0], pk[1][1]);
+#pragma unroll
+      for (int d = 0; d < DT; d++) {
+        const int col = 16 * d + 4 * (ln & 3);
+        const uint2 v0 = ds_read_tr16(vl + pf_off<D>(row0, col >> 3) + (col & 7));
+        const uint2 v1 = ds_read_tr16(vl + pf_off<D>(row1, col >> 3) + (col & 7));
+        o[d] = mfma16<T>(make_uint4(v0.x, v0.y, v1.x, v1.y), pb, o[d]);
+      }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    // ---- merge the waves: one common maximum, every wave's sums scaled to it
+    if (g == 0) sm.smx[wv][r16] = m;
+    __syncthreads();
+    float M = m;
+#pragma unroll
+    for (int w = 0; w < NW; w++) M = fmaxf(M, sm.smx[w][r16]);
+    const float f = m == -INFINITY ? 0.f : __expf(m - M);
+    if (g == 0) sm.sml[wv][r16] = l * f;
+    float* ob = (float*)vl;          // [NW][DT][64] float4: wave w's rows of vl (its own V rows, now read)
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+      *(float4*)(ob + ((size_t)(wv * DT + d) * 64 + lane) * 4) =
+          make_float4(o[d][0] * f, o[d][1] * f, o[d][2] * f, o[d][3] * f);
+    __syncthreads();
+    if (r16 < R) {
+      float L = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; w++) L += sm.sml[w][r16];
+      float* po = a.part_o + prow * D + 4 * g;
+#pragma unroll
+      for (int d = 0; d < DT; d++) {
+        if (d % NW != wv) continue;
+        float4 s4 = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+          const float4 u = *(const float4*)(ob + ((size_t)(w * DT + d) * 64 + lane) * 4);
+          s4.x += u.x; s4.y += u.y; s4.z += u.z; s4.w += u.w;
+        }
+        if constexpr (FUSE) st16_sc1(a.part_o, (size_t)(po - a.part_o) + 16 * d, s4);
+        else *(float4*)(po + 16 * d) = s4;
+      }
+      if (wv == 0 && g == 0) {
+        if constexpr (FUSE) st8_sc1(a.part_ml + prow * 2, M, L);
+        else *(float2*)(a.part_ml + prow * 2) = make_float2(M, L);
+      }
+    }
+  }
+  if constexpr (FUSE) {
+    // ---- the last workgroup of (b, kvh) to arrive merges every split
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's write-through stores are done
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int* ctr = a.v3_counters + (size_t)b * a.Hkv + kvh;
+      const int prev = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sm.s_last = prev == (int)gridDim.x - 1;
+      if (sm.s_last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!sm.s_last) return;
+    v3_combine<T, true>(a, b, kvh, gridDim.x, threadIdx.x, NW * 64);
+  }
+}
+
 // waves per workgroup: the most (>= 4) that still leaves >= ~2 workgroups per CU
 // (a function of the batch, kv heads and split grid only, so a multi-row
 // verify picks the same NW as one-token decoding of the same batch);
@@ -613,8 +892,35 @@ static void launch_v3_nw(const AttnDecodeArgs& a, hipStream_t st) {
   }
 }
 
+// tiles per wave of the long-context kernel (0: one tile per wave, the kernel above).  Fused-RoPE decode
+// only: with q from memory two 8-wave workgroups of the kernel above share a CU (108 - 118 registers) and
+// it is as fast.  One workgroup per CU, at most 8 tiles, at least 16 splits per sequence (ragged batches) --
+// whole decode layer of Llama-3-8B, one tile per wave -> this (us): 1 x 8000 keys 56.5 -> 54.1, 1 x 16000
+// 71.5 -> 60.9, 1 x 32000 91.9 -> 73.1, 4 x 4000 68.7 -> 66.4, 8 x 4000 88.8 -> 80.2, 3 x 20000 119 -> 98;
+// 8 x 2000 69.8 -> 70.8, so not below 48 splits.  (ILLM_ATTN_V3_TILES=n forces n; a function of batch, kv
+// heads and split grid only, as v3_pick_nw.)
+inline int v3_long_tiles(const AttnDecodeArgs& a, int rq) {
+  static const int env = getenv("ILLM_ATTN_V3_TILES") ? atoi(getenv("ILLM_ATTN_V3_TILES")) : -1;
+  if (env >= 0) return env;
+  if (rq == 0 || a.nsplit < 48) return 0;
+  const long wgs = (long)a.B * a.Hkv * ((a.nsplit * SPLIT + V3_KPW * V3L_NW - 1) / (V3_KPW * V3L_NW));
+  const long t = std::min<long>(std::min<long>((wgs + 255) / 256, 8), a.nsplit / 16);
+  return t >= 2 ? (int)t : 0;
+}
+
 template <typename T, int D, int RQ>
 static void launch_v3(const AttnDecodeArgs& a, hipStream_t st) {
+  if (const int tiles = v3_long_tiles(a, RQ)) {
+    const int keys = V3_KPW * V3L_NW * tiles, ns = (a.nsplit * SPLIT + keys - 1) / keys;
+    dim3 grid(ns, a.Hkv, a.B);
+    if (a.v3_counters != nullptr) {
+      hipLaunchKernelGGL((attn_decode_v3l_kernel<T, D, RQ, true>), grid, dim3(64 * V3L_NW), 0, st, a, tiles);
+    } else {
+      hipLaunchKernelGGL((attn_decode_v3l_kernel<T, D, RQ, false>), grid, dim3(64 * V3L_NW), 0, st, a, tiles);
+      hipLaunchKernelGGL((attn_combine_v3_kernel<T>), dim3(a.Hkv, a.B), dim3(256), 0, st, a, ns);
+    }
+    return;
+  }
   switch (v3_pick_nw(a)) {
     case 1: return launch_v3_nw<T, D, 1, RQ>(a, st);
     case 2: return launch_v3_nw<T, D, 2, RQ>(a, st);
