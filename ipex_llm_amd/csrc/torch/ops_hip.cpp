@@ -152,7 +152,9 @@ struct Plan5 {
   unsigned gx;
   int nw;
 };
-Plan5 plan5(int64_t rows, int64_t groups, int64_t KC, bool can_split, int64_t ks_req = 0, bool atomic = false) {
+// fmt >= 0: the plain (not expert-grouped) launches, whose rules also know the format.
+Plan5 plan5(int64_t rows, int64_t groups, int64_t KC, bool can_split, int64_t ks_req = 0, bool atomic = false,
+            int fmt = -1) {
   static const int kw_env = getenv("ILLM_GEMV5_KW") ? atoi(getenv("ILLM_GEMV5_KW")) : 0;
   static const int ks_env = getenv("ILLM_GEMV5_KS") ? atoi(getenv("ILLM_GEMV5_KS")) : 0;
   static const int nw_env = getenv("ILLM_GEMV5_NW") ? atoi(getenv("ILLM_GEMV5_NW")) : 0;
@@ -166,6 +168,10 @@ Plan5 plan5(int64_t rows, int64_t groups, int64_t KC, bool can_split, int64_t ks
     p.kw = 2;
     p.nw = rows <= 2 ? 4 : 8;
     while (p.kw > 1 && KC / p.kw < 4) p.kw /= 2;
+    // 8-bit codes whose 8-wave groups of 4 pairs just miss one round of the 256 CUs: 8 pairs each, no K
+    // split (Qwen2.5-7B gate/up, 296 -> 148 groups, fp8_e5m2: M = 5 36.5 -> 31.7 us, 8 38.3 -> 32.6, 12
+    // 40.7 -> 34.0; 4-bit codes 22.5 -> 23.5, so not for these)
+    if (fmt >= 0 && illm::fmt_bits(fmt) == 8 && p.nw == 8 && groups > 4 * 256 && groups <= 8 * 256) p.kw = 1;
   } else if (ks_req > 0) {
     p.ks = ks_req;
   } else {
@@ -177,6 +183,14 @@ Plan5 plan5(int64_t rows, int64_t groups, int64_t KC, bool can_split, int64_t ks
     // (16 x 7 vs 14 x 8), M = 8 9.6 vs 11.1 us (same sweep)
     const int64_t target = KC >= 64 ? 7 : 4;
     p.ks = std::min<int64_t>(atomic ? 32 : 16, std::max<int64_t>(1, (KC + target - 1) / target));
+    // ... but one round of 8-wave groups where every group streams through the generic loop (formats other
+    // than sym_int4, whose slices of <= 7 chunks have kernels of their own): [3584, 18944] fp8_e5m2 22 -> 9
+    // slices M = 1 19.1 -> 14.0 us, 5 21.2 -> 15.0 (4.7 TB/s), 8 22.2 -> 15.9; [4096, 14336] sym_int8 16 -> 8
+    // 15.7 -> 13.6 (M = 8 18.2 -> 15.3), nf4 12.3 -> 11.7 (14.5 -> 13.6), 4096 x 8192
+    // fp8_e5m2 12.0 -> 9.4 (14.5 -> 10.4); sym_int4 9.6 -> 10.5, and from [8192, 28672] (4 slices) no gain: nf4 at
+    // M = 8 40.1 -> 41.1
+    const int64_t round = 256 / ((groups + 7) / 8);
+    if (fmt >= 0 && fmt != illm::FMT_SYM_INT4 && KC >= 64 && round >= 8) p.nw = 8, p.ks = std::min(p.ks, round);
     // wide outputs (lm_head: 8016 tiles) already fill the chip: slabs only cost
     while (p.ks > 1 && groups * p.ks > 4096) p.ks /= 2;
     while (illm::gemv5_shmem_h((int)rows, (int)((KC + p.ks - 1) / p.ks)) > 65536 && p.ks < KC) p.ks *= 2;
@@ -235,7 +249,7 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
     a.N = (int)(n / 2);
     a.out = out.data_ptr();
     a.ldo = (int)(n / 2);
-    const Plan5 p = plan5(M, NT / 2, KC, false);
+    const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
     if (small && p.shmem <= kMaxLds)
       a.nw = p.nw, launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);
     else
@@ -247,7 +261,7 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   SkinnyPlan q{};
   bool use5 = false;
   if (small) {
-    p5 = plan5(M, NT, KC, true, ksplit);
+    p5 = plan5(M, NT, KC, true, ksplit, false, (int)fmt);
     use5 = p5.shmem <= kMaxLds;
   }
   if (use5) {
@@ -617,7 +631,7 @@ Tensor gemv_norm_in(const Tensor& acc_in, const Tensor& residual, Tensor& res_ou
     a.N = (int)(n / 2);
     a.out = out.data_ptr();
     a.ldo = (int)(n / 2);
-    const Plan5 p = plan5(M, NT / 2, KC, false);
+    const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
     TORCH_CHECK(p.shmem <= kMaxLds, "gemv_norm_in: K slice too large for LDS");
     a.nw = p.nw;
     launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);
@@ -630,7 +644,7 @@ Tensor gemv_norm_in(const Tensor& acc_in, const Tensor& residual, Tensor& res_ou
   a.out = acc_out->data_ptr();
   a.ldo = (int)n;
   const bool rope = set_rope(a, rope_cs, rope_pos, rope_cols, rope_d, M);
-  Plan5 p = plan5(M, NT, KC, true, 0, true);
+  Plan5 p = plan5(M, NT, KC, true, 0, true, (int)fmt);
   if (rope) p = plan5_rope(p, NT, M);
   TORCH_CHECK(p.shmem <= kMaxLds, "gemv_norm_in: K slice too large for LDS");
   a.cpk = (int)p.cpk;
@@ -665,7 +679,7 @@ void gemv_accum(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int
   a.out = acc.data_ptr();
   a.ldo = (int)n;
   const bool rope = set_rope(a, rope_cs, rope_pos, rope_cols, rope_d, M);
-  Plan5 p = plan5(M, NT, KC, true, ksplit, true);
+  Plan5 p = plan5(M, NT, KC, true, ksplit, true, (int)fmt);
   if (rope) p = plan5_rope(p, NT, M);
   a.cpk = (int)p.cpk;
   a.nw = p.nw;
@@ -713,7 +727,7 @@ void gemv_accum_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n
   a.N = (int)n;
   a.out = acc.data_ptr();
   a.ldo = (int)n;
-  Plan5 p = plan5(M, NT, KC, true, 0, true);
+  Plan5 p = plan5(M, NT, KC, true, 0, true, (int)fmt);
   p.kw = 1;                                   // column blocks of nw tiles: 64 / 128 columns
   p.gx = (unsigned)((NT + p.nw - 1) / p.nw);
   a.cpk = (int)p.cpk;
@@ -762,7 +776,7 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   a.N = (int)(n / 2);
   a.out = out.data_ptr();
   a.ldo = (int)(n / 2);
-  const Plan5 p = plan5(M, NT / 2, KC, false);
+  const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
   TORCH_CHECK(p.shmem <= kMaxLds, "gemv_glu_ss: x slice exceeds LDS");
   a.nw = p.nw;
   launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);
@@ -808,7 +822,7 @@ Tensor gemv_glu_in(const Tensor& part, const Tensor& blob, int64_t fmt, int64_t 
   a.lut_fmt = (int)fmt;
   a.N = (int)n;
   const bool atomic = acc.has_value() && acc->defined();
-  const Plan5 p = plan5(M, NT, KC, true, ksplit, atomic);
+  const Plan5 p = plan5(M, NT, KC, true, ksplit, atomic, (int)fmt);
   ksplit = p.ks;
   a.cpk = (int)p.cpk;
   a.nw = p.nw;
