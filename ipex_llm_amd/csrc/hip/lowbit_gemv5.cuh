@@ -807,7 +807,7 @@ __device__ __forceinline__ void gemv5_body(const GemvArgs& a, const G5Blk& blk) 
     const int mrow = min(r16, Mloc - 1);          // unused columns read a valid row (no masking)
     const uint16_t* xrow = xs + mrow * ldx + 8 * g;
     const float4* srow = sxs + mrow * (c1 - c0);
-    const uint32_t mask_s = a.nib_mask, magic_v = a.nib_magic;
+    const uint32_t mask_s = a.nib_mask, magic_v = opaque_v(a.nib_magic);
 
     auto compute_chunk = [&](const Chunk& ch, int c) {
       if constexpr ((ILLM_GEMV5_ABL & 1) != 0) {

@@ -10,11 +10,15 @@
 namespace illm {
 
 // packed-pair nibble extract (x & m) | c as ONE v_and_or_b32: hipcc splits
-// the pattern into v_and + v_or (gfx9 VOP3 takes no literal and one
-// constant-bus read), so the mask is an SGPR and the magic a VGPR operand
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t m_s, uint32_t c_v) {
+// the pattern into v_and + v_or where it sees the constants (gfx9 VOP3 takes no
+// literal and one constant-bus read), so the mask is a kernel argument (an SGPR)
+// and the magic an opaque VGPR (opaque_v).  Not written in asm: beside MFMA the
+// compiler places the wait states that a result's register needs before it is
+// written again, which it cannot for an asm statement
+__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t m_s, uint32_t c_v) { return (x & m_s) | c_v; }
+__device__ __forceinline__ uint32_t opaque_v(uint32_t x) {
   uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(m_s), "v"(c_v));
+  asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(x));
   return r;
 }
 

@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   for (int t = 0; t < SK_TPW; t++)
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint32_t mask_s = a.nib_mask, magic_v = a.nib_magic;
+  const uint32_t mask_s = a.nib_mask, magic_v = opaque_v(a.nib_magic);
   constexpr uint32_t cst = skinny_const2<DK, T>();
   const uint4 cA = make_uint4(cst, cst, cst, cst);
 
