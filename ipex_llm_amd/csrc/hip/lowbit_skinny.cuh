@@ -153,17 +153,21 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   constexpr uint32_t cst = skinny_const2<DK, T>();
   const uint4 cA = make_uint4(cst, cst, cst, cst);
 
-  auto compute = [&](const Chunk& ch, int buf) {
+  auto read_x = [&](uint4 (&B)[2][MT][2], int buf) {
     const uint16_t* xb = xs + (size_t)(buf * R + r16) * SK_STEP + kp * CHUNK_K;
 #pragma unroll
     for (int blk = 0; blk < 2; blk++) {
-      uint4 B[MT][2];
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
         const uint16_t* xm = xb + (size_t)mt * 16 * SK_STEP;
-        B[mt][0] = *(const uint4*)(xm + (((8 * blk + g) ^ r16) * 8));
-        B[mt][1] = *(const uint4*)(xm + (((8 * blk + 4 + g) ^ r16) * 8));
+        B[blk][mt][0] = *(const uint4*)(xm + (((8 * blk + g) ^ r16) * 8));
+        B[blk][mt][1] = *(const uint4*)(xm + (((8 * blk + 4 + g) ^ r16) * 8));
       }
+    }
+  };
+  auto compute = [&](const Chunk& ch, const uint4 (&B)[2][MT][2]) {
+#pragma unroll
+    for (int blk = 0; blk < 2; blk++) {
       uint4 A[SK_TPW][2];
 #pragma unroll
       for (int t = 0; t < SK_TPW; t++)
@@ -194,7 +198,7 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
       }
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
-        const uint4 B0 = B[mt][0], B1 = B[mt][1];
+        const uint4 B0 = B[blk][mt][0], B1 = B[blk][mt][1];
         const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
         f32x4 X = zero;
         if constexpr (NEEDX) {
@@ -222,6 +226,18 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   // flight (34 KB of 4-bit, 68 KB of 8-bit codes per CU).  Steps run in whole
   // groups of PF with no branch inside (hipcc keeps counted vmcnt waits); past
   // the slice's end they find zeros in the staged x.
+  //
+  // Two waves per SIMD leave the LDS reads (768 cycles of a 48-row step), the
+  // decoding (1040) and the matrix work (1152) mostly one behind the other.  From
+  // three row tiles on, a step reads all of its x first and stages the next
+  // before its products, so that the decoding runs while LDS answers and no wave
+  // waits for its own stores at the barrier, and half of the waves go first:
+  // fp8_e5m2 300 rows gate/up [37888, 3584] 139 -> 133 us, down [3584, 18944]
+  // 83.8 -> 79.8; sym_int4 48 rows gate/up 24.8 -> 24.3, down 15.4 -> 15.1.  Two
+  // row tiles measured slower so (gate/up at 32 rows 18.9 -> 19.6); a barrier per
+  // two steps (twice the LDS) gained nothing at any size.  Four-wave groups have no
+  // registers left for it (one spilled) and one wave per SIMD to order.
+  constexpr bool EARLY = MT >= 3 && NW == 8;
   uint4 xr[PF][XJ];
   Chunk ring[PF];
   load_x(xr[0], 0);
@@ -236,15 +252,25 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   store_x(xr[0], 0, 0);
   load_x(xr[0], PF);
   __syncthreads();
+  if (EARLY && wave < NW / 2) __builtin_amdgcn_s_setprio(1);
   for (int s0 = 0; s0 < nstep; s0 += PF) {
 #pragma unroll
     for (int u = 0; u < PF; u++) {
-      compute(ring[u], u & 1);
+      uint4 B[2][MT][2];
+      read_x(B, u & 1);
+      if constexpr (EARLY) {
+        __builtin_amdgcn_sched_barrier(0);
+        store_x(xr[(u + 1) % PF], s0 + u + 1, (u + 1) & 1);
+        load_x(xr[(u + 1) % PF], s0 + u + 1 + PF);
+      }
+      compute(ring[u], B);
       __builtin_amdgcn_sched_barrier(0);       // the ring slot is free only after its compute: no second copy of it
       load_w(ring[u], s0 + u + PF);
-      __builtin_amdgcn_sched_barrier(0);
-      store_x(xr[(u + 1) % PF], s0 + u + 1, (u + 1) & 1);
-      load_x(xr[(u + 1) % PF], s0 + u + 1 + PF);
+      if constexpr (!EARLY) {
+        __builtin_amdgcn_sched_barrier(0);
+        store_x(xr[(u + 1) % PF], s0 + u + 1, (u + 1) & 1);
+        load_x(xr[(u + 1) % PF], s0 + u + 1 + PF);
+      }
       __syncthreads();
     }
   }
