@@ -309,15 +309,26 @@ _AUTOTUNE = os.environ.get("ILLM_GEMM_AUTOTUNE", "1") == "1"
 _CHOICE: Dict[tuple, str] = {}
 
 
-def _time_ms(fn, reps: int = 3) -> float:
-    fn()
-    t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    t0.record()
-    for _ in range(reps):
+def _time_ms(fns, reps: int = 3, rounds: int = 3):
+    """best time of each candidate over rounds in turn.  One round alone is off by more
+    than the candidates differ (clocks still rising, the library's first calls): at
+    [6144, 4096] and 1024 rows it read 90 (8-phase) and 135 us (library) for what are 82
+    and 66, and the step of a 1024-token Llama-3-8B prompt was 18.3 to 19.2 ms from one
+    process to the next; in turn, 18.2 to 18.3.  Once per shape and process: 10 calls of
+    each candidate instead of 4"""
+    for fn in fns:
         fn()
-    t1.record()
-    t1.synchronize()
-    return t0.elapsed_time(t1) / reps
+    best = [float("inf")] * len(fns)
+    t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for _ in range(rounds):
+        for i, fn in enumerate(fns):
+            t0.record()
+            for _ in range(reps):
+                fn()
+            t1.record()
+            t1.synchronize()
+            best[i] = min(best[i], t0.elapsed_time(t1) / reps)
+    return best
 
 
 def _mbucket(M: int) -> int:
@@ -335,7 +346,7 @@ def _pick(key: tuple, g8d_fn, lib_fn, *more) -> str:
         if not _AUTOTUNE or torch.cuda.is_current_stream_capturing():
             return "g8d"
         names = ["g8d", "lib"] + [f"lib{i + 1}" for i in range(len(more))]
-        times = [_time_ms(f) for f in (g8d_fn, lib_fn) + more]
+        times = _time_ms((g8d_fn, lib_fn) + more)
         c = _CHOICE[key] = names[min(range(len(times)), key=times.__getitem__)]
         if os.environ.get("ILLM_GEMM_AUTOTUNE_LOG"):
             print(f"[gemm] M={key[0]} N={key[1]} K={key[2]} glu={key[3]}: "
