@@ -6,7 +6,7 @@ by the reference (`config.json: bigdl_transformers_low_bit=<name>`) resolve to
 the same format here.  What each id *means on the device* is ours: every format
 is described by a :class:`QFormat` record that drives the C++ quantizers
 (``csrc/cpu/quant.cpp``), the MI355X tile repacker and the HIP GEMV/GEMM
-decoders (``csrc/hip/lowbit_gemv.hip``).
+decoders (``csrc/hip/lowbit_gemv5.cuh``).
 """
 from __future__ import annotations
 
