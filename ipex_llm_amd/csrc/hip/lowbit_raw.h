@@ -70,6 +70,15 @@ __device__ __forceinline__ uint4 raw_a4(uint32_t u, uint32_t mask_s, uint32_t ma
   return r;
 }
 
+// dword c of raw_a4's fragment
+template <int DK, typename C>
+__device__ __forceinline__ uint32_t raw_a4_at(uint32_t u, int c, uint32_t mask_s, uint32_t magic_v, const uint32_t* lut2) {
+  if constexpr (DK == DK_INT4S || DK == DK_INT4A) return and_or(u >> (4 * c), mask_s, magic_v);
+  else if constexpr (DK == DK_LUT4) return lut2[(u >> (8 * c)) & 0xff];
+  const uint4 r = raw_a4<DK_FP4, C>(u, mask_s, magic_v, lut2);
+  return c == 0 ? r.x : c == 1 ? r.y : c == 2 ? r.z : r.w;
+}
+
 template <int DK, typename C>
 __device__ __forceinline__ uint32_t raw_pair8(uint32_t u, bool hi) {
   if constexpr (DK == DK_FP8E4) {

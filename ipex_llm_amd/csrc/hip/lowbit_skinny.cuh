@@ -10,27 +10,29 @@
 //     chunk (kp): codes go global -> registers in MFMA A-fragment order
 //     (formats.h), PF chunks of both tiles in flight per wave, and no weight
 //     is read twice by a row block;
-//   * x is staged through LDS once per workgroup and 256-k step (two buffers,
-//     the loads of a step requested two steps ahead), XOR-swizzled in 16-B
-//     pieces so the 16 rows of a fragment read fall on distinct banks;
-//   * codes stay raw in the A operand (exact in bf16 / f16); the block scale
-//     is applied to the f32 block sum.  The offset of the integer formats is
-//     one product of the block's x with the constant -offset: it comes out
-//     broadcast over the tile's rows, i.e. it IS the accumulator input of the
-//     code products (no per-row sums of x in memory, no subtract per value),
-//     shared by the wave's two tiles;
+//   * x is staged through LDS once per workgroup and 256-k step (three buffers: one is read, one is ahead, one is
+//     stored into), XOR-swizzled in 16-B pieces so the 16 rows of a fragment read fall on distinct banks;
+//   * x is the A operand and the codes are the B operand, raw (exact in bf16 / f16): a lane holds four rows of ONE
+//     column, so a (tile, chunk) takes one scale dword per lane where the other order takes four (a 16-B load of 16
+//     cycles in the address unit, as long as the codes' own);
+//   * the block scale is applied to the f32 block sum.  The offset of the integer formats is one product of the
+//     block's x with the constant -offset: it comes out broadcast over the tile's columns, i.e. it IS the
+//     accumulator input of the code products (no per-row sums of x in memory, no subtract per value), shared by the
+//     wave's two tiles;
+//   * loads through buffer descriptors (lane constant + scalar: no address registers that a load in flight holds),
+//     each in a place of its own among the products instead of in bursts, which stalled every wave of the step behind
+//     the address unit at once;
 //   * split-K over blockIdx.y writes f32 slabs summed by the consumer; row
 //     blocks of one column block get ids that share id % 8, so a weight chunk
 //     leaves HBM once per XCD.
-// MI355X, sym_int4, against the kernel it replaced (every wave read its own x
-// rows from L2 for one weight tile): gate/up [28672, 4096] 17 / 48 / 64 rows
-// 51 / 111 / 144 -> 21 / 25 / 30 us, down [4096, 14336] 29 / 65 / 84 -> 12 / 15
-// / 17, o [4096, 4096] 12 / 28 / 36 -> 6 / 8 / 10; fp8_e5m2 gate/up 51 / 108 /
-// 142 -> 25 / 28 / 32 (4.8 TB/s at 17 rows).  What bounds it now is a step's
-// own chain -- barrier, x fragments from LDS, products, scales, 0.6 to 0.9 us
-// with two waves per SIMD -- not the stream: two steps in flight measured
-// faster than four (o at 17 rows 5.9 vs 7.6 us, gate/up at 32 20.8 vs 22), and
-// 128 registers for twice the waves spilled (gate/up at 32 rows 32 us).
+// MI355X, us, back-to-back launches, bursts and four scales per lane / this: sym_int4 48 rows gate/up [28672, 4096]
+// 25.1 / 23.1, down [4096, 14336] 15.6 / 14.7, qkv [6144, 4096] 11.7 / 9.5, o [4096, 4096] 8.3 / 7.3; gate/up of 32
+// rows 20.2 / 18.6, 64 rows 30.3 / 27.6; fp8_e5m2 300 rows [3584, 18944] 78.4 / 67.5, [4608, 3584] 23.5 / 19.8; nf4
+// gate/up of 48 rows 27.1 / 23.4, asym_int4 27.1 / 25.2, sym_int8 29.5 / 28.5, fp4 21.2 / 19.4; the pair table of 128
+// rows [6144, 4096] 37.4 / 32.5.  What bounds it: issue, two waves per SIMD with 36 products (8 of an MFMA's 16 cycles
+// each) and some 110 vector instructions a step, 13.9 us of the 18.1 that 16 steps of the gate/up pair take, the
+// products alone 10.1.  Four steps of weights in flight measured no faster than three (23.9), nor did the bursts with
+// the next step's decoding and reads between the products (26.1).
 #pragma once
 #include <mutex>
 #include <type_traits>
@@ -58,6 +60,11 @@ __host__ __device__ constexpr uint32_t skinny_const2() {
        : (b ? 0x3F803F80u : 0x3C003C00u);
 }
 
+// 16 B per lane through a buffer descriptor (reads past its range return 0)
+__device__ __forceinline__ uint4 buf16(const __amdgpu_buffer_rsrc_t& r, uint32_t voff, int soff) {
+  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+
 // FINE (a table weight under bf16 x): every entry as a bf16 pair hi + lo, two products each.  An entry is then
 // 2^-17 off at most, where a bf16 table is 2^-9 and an f16 one 2^-12.  For the products of 65 rows and up that
 // a kernel with an f16 table served: nf4 [6144, 4096], one entry / a pair / that kernel, 80 rows 20.5 / 24.3 / 42.6
@@ -70,12 +77,12 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   constexpr bool NEEDX = OFFS || HASMIN;       // ... or the block minimum needs the sum of x
   constexpr int R = MT * 16;
   constexpr int SK_TILES = NW / SK_KW * SK_TPW;
-  constexpr int PF = 2;                        // steps of weights in flight, and that x is requested ahead
+  constexpr int RG = 3;                        // steps in the rings of weights (registers) and of x (LDS)
   constexpr int XJ = MT * 8 / NW;              // 16-B pieces of x per thread and step
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint16_t* xs = (uint16_t*)smem;                                 // [2][R][SK_STEP]
+  // x of three steps: [3][R][SK_STEP], then the table
   static_assert(!FINE || (DK == DK_LUT4 && std::is_same<T, BF16>::value), "the finer table: table formats in bf16");
-  uint32_t* lut2 = (uint32_t*)(smem + 2 * R * SK_STEP * 2);       // DK_LUT4 only: [256] (FINE: {hi, lo})
+  uint32_t* lut2 = (uint32_t*)(smem + 3 * R * SK_STEP * 2);       // DK_LUT4 only: [256] (FINE: {hi, lo})
   const uint2* lutf = (const uint2*)lut2;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // uniform: weight addresses live in SGPRs
@@ -118,47 +125,45 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
 
   // ---- weights: this wave's chunk of a step is c0 + 2 step + kp
   const size_t TB = (size_t)dk_tile_bytes(DK, KC);
-  const size_t soff = (size_t)KC * dk_code_chunk(DK), moff = soff + (size_t)16 * KC * 4;
-  const uint32_t lq = lane * 16, ls = g * 16;                     // lane's codes; rows 4g..4g+3 of a scale record
-  const uint8_t* tb[SK_TPW];
+  const uint32_t soff = (uint32_t)KC * dk_code_chunk(DK), moff = soff + 16 * KC * 4;
+  const uint32_t lq = lane * 16, ls = r16 * 4;                    // lane's codes; its column's scales
+  // through buffer descriptors: a load's address is a lane constant + a scalar, no register of its own to wait for
+  __amdgpu_buffer_rsrc_t wr[SK_TPW];
 #pragma unroll
-  for (int t = 0; t < SK_TPW; t++) tb[t] = a.w + (size_t)min(tile0 + t, NT - 1) * TB;
+  for (int t = 0; t < SK_TPW; t++)
+    wr[t] = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)min(tile0 + t, NT - 1) * TB), 0, (int)TB, 0x00020000);
   struct Chunk {
     uint4 q[SK_TPW][BITS / 4];
-    uint4 sc[SK_TPW];
-    uint4 mn[HASMIN ? SK_TPW : 1];
+    uint32_t sc[SK_TPW], mn[HASMIN ? SK_TPW : 1];
+  };
+  constexpr int WL = BITS / 4 + (HASMIN ? 2 : 1);                 // loads of a tile's chunk
+  auto load_w1 = [&](Chunk& ch, int step, int i) {                // load i of SK_TPW * WL
+    const int c = min(c0 + step * SK_KW + kp, c1 - 1), t = i / WL, j = i % WL;   // clamped: unconditional loads
+    if (j == 0) ch.sc[t] = __builtin_amdgcn_raw_buffer_load_b32(wr[t], soff + ls, c * 64, 0);
+    else if (j <= BITS / 4) ch.q[t][j - 1] = buf16(wr[t], lq + (j - 1) * 1024, c * dk_code_chunk(DK));
+    else ch.mn[t] = __builtin_amdgcn_raw_buffer_load_b32(wr[t], moff + ls, c * 64, 0);
   };
   auto load_w = [&](Chunk& ch, int step) {
-    const int c = min(c0 + step * SK_KW + kp, c1 - 1);            // clamped: unconditional loads
 #pragma unroll
-    for (int t = 0; t < SK_TPW; t++) {
-      const uint8_t* rec = tb[t] + (size_t)c * dk_code_chunk(DK);
-      ch.q[t][0] = *(const uint4*)(rec + lq);
-      if constexpr (BITS == 8) ch.q[t][1] = *(const uint4*)(rec + 1024 + lq);
-      ch.sc[t] = *(const uint4*)(tb[t] + soff + (size_t)c * 64 + ls);
-      if constexpr (HASMIN) ch.mn[t] = *(const uint4*)(tb[t] + moff + (size_t)c * 64 + ls);
-    }
+    for (int i = 0; i < SK_TPW * WL; i++) load_w1(ch, step, i);
   };
 
   // ---- x: thread -> rows tid / 32 + 16 j, 16-B piece tid % 32 of the step
   const int xr0 = tid >> 5, xc = tid & 31;
   const int kend = min(a.K, c1 * CHUNK_K);
-  uint32_t xo[XJ];                                                // byte offset of the row (host: < 4 GB)
+  const __amdgpu_buffer_rsrc_t xd =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)((uint32_t)a.M * (uint32_t)a.ldx * 2u), 0x00020000);
+  uint32_t xo[XJ];                                                // byte offset of the row's piece (host: < 4 GB)
 #pragma unroll
-  for (int j = 0; j < XJ; j++) xo[j] = (uint32_t)min(m0 + xr0 + NW * 2 * j, a.M - 1) * (uint32_t)a.ldx * 2u;
-  auto load_x = [&](uint4 (&xr)[XJ], int step) {                  // unconditional (clamped); store_x zeroes past the slice
-    const int k = (c0 + step * SK_KW) * CHUNK_K + xc * 8;
-    const uint32_t ko = k < a.K ? (uint32_t)k * 2u : 0u;
-#pragma unroll
-    for (int j = 0; j < XJ; j++) xr[j] = *(const uint4*)((const uint8_t*)a.x + (xo[j] + ko));
+  for (int j = 0; j < XJ; j++) xo[j] = (uint32_t)min(m0 + xr0 + NW * 2 * j, a.M - 1) * (uint32_t)a.ldx * 2u + xc * 16;
+  auto load_x1 = [&](int step, int j) {                           // past the slice: out of the descriptor's range, zeros
+    const int k = (c0 + step * SK_KW) * CHUNK_K;
+    return buf16(xd, k + xc * 8 < kend ? xo[j] + (uint32_t)k * 2u : ~0u, 0);
   };
   // piece p of row r lives at piece p ^ (r & 15) (within its half of the step)
-  auto store_x = [&](const uint4 (&xr)[XJ], int step, int buf) {
-    const uint32_t keep = (c0 + step * SK_KW) * CHUNK_K + xc * 8 < kend ? ~0u : 0u;
-#pragma unroll
-    for (int j = 0; j < XJ; j++)
-      *(uint4*)(xs + (size_t)(buf * R + xr0 + NW * 2 * j) * SK_STEP + ((xc & 16) | ((xc ^ (xr0 + NW * 2 * j)) & 15)) * 8) =
-          make_uint4(xr[j].x & keep, xr[j].y & keep, xr[j].z & keep, xr[j].w & keep);
+  auto store_x1 = [&](const uint4& v, uint32_t buf, int j) {
+    const int row = xr0 + NW * 2 * j;
+    *(uint4*)(smem + (buf + (uint32_t)row * SK_STEP * 2 + ((xc & 16) | ((xc ^ row) & 15)) * 16)) = v;
   };
 
   f32x4 acc[SK_TPW][MT];
@@ -170,208 +175,234 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   constexpr uint32_t cst = skinny_const2<DK, T>();
   const uint4 cA = make_uint4(cst, cst, cst, cst);
 
-  auto read_x = [&](uint4 (&B)[2][MT][2], int buf) {
-    const uint16_t* xb = xs + (size_t)(buf * R + r16) * SK_STEP + kp * CHUNK_K;
+  // ---- a phase = one 64-k block: products of the block's first 32 k (pass a), of its second (pass b), before them the
+  // offset products where the codes carry one.  Beside a pass' products, in program order between them: the scales of
+  // the block before, the decoding of the weights and the x reads of the pass after the next.
+  constexpr int NP = SK_TPW * MT;                                 // products of a pass
+  constexpr int NB1 = NEEDX ? 2 : 1;                              // (the offset products need both halves of x at once)
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 P[SK_TPW][MT], X[2][NEEDX ? MT : 1];
+  uint4 A[SK_TPW][2], lo[FINE ? SK_TPW : 1][2], B0[MT], B1[NB1][MT];
+  float d[2][SK_TPW], mn[2][HASMIN ? SK_TPW : 1];
 #pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
+  for (int t = 0; t < SK_TPW; t++)
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) {
-        const uint16_t* xm = xb + (size_t)mt * 16 * SK_STEP;
-        B[blk][mt][0] = *(const uint4*)(xm + (((8 * blk + g) ^ r16) * 8));
-        B[blk][mt][1] = *(const uint4*)(xm + (((8 * blk + 4 + g) ^ r16) * 8));
+    for (int mt = 0; mt < MT; mt++) P[t][mt] = zero;
+#pragma unroll
+  for (int t = 0; t < SK_TPW; t++) d[0][t] = d[1][t] = 0.f;
+  if constexpr (HASMIN) {
+#pragma unroll
+    for (int t = 0; t < SK_TPW; t++) mn[0][t] = mn[1][t] = 0.f;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) X[0][mt] = X[1][mt] = zero;
+  }
+  const uint32_t xl = (uint32_t)r16 * SK_STEP * 2 + kp * CHUNK_K * 2;
+  auto read_x = [&](uint32_t buf, int blk, int ss, int mt) {      // buf: byte offset of the step's x
+    return *(const uint4*)(smem + (buf + xl + (uint32_t)(((8 * blk + 4 * ss + g) ^ r16) * 16)) + mt * 16 * SK_STEP * 2);
+  };
+  auto decode = [&](const Chunk& ch, int blk, int ss, int t, int c) {   // dword c of a fragment
+    uint32_t v;
+    if constexpr (BITS == 4) {
+      const uint4& q = ch.q[t][0];
+      const uint32_t w = blk == 0 ? (ss == 0 ? q.x : q.y) : (ss == 0 ? q.z : q.w);
+      if constexpr (FINE) {
+        const uint2 e = lutf[(w >> (8 * c)) & 0xff];
+        v = e.x;
+        uint4& l = lo[t][ss];
+        (c == 0 ? l.x : c == 1 ? l.y : c == 2 ? l.z : l.w) = e.y;
+      } else {
+        v = raw_a4_at<DK, T>(w, c, mask_s, magic_v, lut2);
       }
+    } else {
+      const uint4& q = ch.q[t][blk];
+      const uint32_t w = ss == 0 ? (c < 2 ? q.x : q.y) : (c < 2 ? q.z : q.w);
+      v = raw_pair8<DK, T>(w, c & 1);
+    }
+    uint4& f = A[t][ss];
+    (c == 0 ? f.x : c == 1 ? f.y : c == 2 ? f.z : f.w) = v;
+  };
+  auto scales = [&](const Chunk& ch, int blk, int t) {
+    d[blk][t] = f16_to_f32((uint16_t)(ch.sc[t] >> (16 * blk)));
+    if constexpr (HASMIN) {
+      // times the sum of x: the offset product holds -offset * sum (exact power of two)
+      constexpr float f = OFFS ? -1.f / (std::is_same<T, BF16>::value ? 128.f : 1024.f) : 1.f;
+      mn[blk][t] = f * f16_to_f32((uint16_t)(ch.mn[t] >> (16 * blk)));
     }
   };
-  auto compute = [&](const Chunk& ch, const uint4 (&B)[2][MT][2]) {
+  auto scale_out = [&](int i, int blk) {                          // product i of block blk into the sums
+    const int mt = i / SK_TPW, t = i % SK_TPW;
 #pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
-      uint4 A[SK_TPW][2], lo[FINE ? SK_TPW : 1][2];
+    for (int e = 0; e < 4; e++) {
+      acc[t][mt][e] = __builtin_fmaf(d[blk][t], P[t][mt][e], acc[t][mt][e]);
+      if constexpr (HASMIN) acc[t][mt][e] = __builtin_fmaf(mn[blk][t], X[blk][mt][e], acc[t][mt][e]);
+    }
+  };
+  constexpr int LATE = NEEDX ? 0 : NP / 2;                        // products scaled in their own pass b; the rest in the next phase
+  // xb: this step's x, xn: the one of the next phase; ch: this chunk, nx: the next phase's
+  constexpr int PH = (NEEDX ? 2 * MT : 0) + 2 * NP;               // slots of a phase
+  auto phase = [&](const Chunk& ch, const Chunk& nx, int blk, uint32_t xb, uint32_t xn, auto&& fill) {
+    const int nblk = blk ^ 1;
+    if constexpr (NEEDX) {
 #pragma unroll
-      for (int t = 0; t < SK_TPW; t++)
+      for (int j = 0; j < 2 * MT; j++) {
+        const int mt = j % MT;
 #pragma unroll
-        for (int ss = 0; ss < 2; ss++) {
-          if constexpr (BITS == 4) {
-            const uint4& q = ch.q[t][0];
-            const uint32_t w = blk == 0 ? (ss == 0 ? q.x : q.y) : (ss == 0 ? q.z : q.w);
-            if constexpr (FINE) {
-              const uint2 e0 = lutf[w & 0xff], e1 = lutf[(w >> 8) & 0xff], e2 = lutf[(w >> 16) & 0xff], e3 = lutf[w >> 24];
-              A[t][ss] = make_uint4(e0.x, e1.x, e2.x, e3.x);
-              lo[t][ss] = make_uint4(e0.y, e1.y, e2.y, e3.y);
-            } else {
-              A[t][ss] = raw_a4<DK, T>(w, mask_s, magic_v, lut2);
-            }
-          } else {
-            const uint4& q = ch.q[t][blk];
-            A[t][ss] = ss == 0 ? raw_a8<DK, T>(q.x, q.y) : raw_a8<DK, T>(q.z, q.w);
-          }
-        }
-      float d[SK_TPW][4], mn[SK_TPW][4];
+        for (int i = j * NP / (2 * MT); i < (j + 1) * NP / (2 * MT); i++) scale_out(i, nblk);
+        X[blk][mt] = j < MT ? mfma16<T>(B0[mt], cA, zero) : mfma16<T>(B1[blk][mt], cA, X[blk][mt]);
+        fill(j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
-      for (int t = 0; t < SK_TPW; t++) {
-        const uint32_t sw[4] = {ch.sc[t].x, ch.sc[t].y, ch.sc[t].z, ch.sc[t].w};
+    for (int j = 0; j < NP; j++) {
+      const int mt = j / SK_TPW, t = j % SK_TPW;
+      if (!NEEDX && j + LATE < NP) scale_out(j + LATE, nblk);
+      P[t][mt] = mfma16<T>(B0[mt], A[t][0], OFFS ? X[blk][mt] : zero);
+      if (!NEEDX && j < MT) B1[0][j] = read_x(xb, blk, 1, j);
 #pragma unroll
-        for (int i = 0; i < 4; i++) d[t][i] = f16_to_f32((uint16_t)(sw[i] >> (16 * blk)));
-        if constexpr (HASMIN) {
-          // times the sum of x: the offset product holds -offset * sum (exact power of two)
-          constexpr float f = OFFS ? -1.f / (std::is_same<T, BF16>::value ? 128.f : 1024.f) : 1.f;
-          const uint32_t mw[4] = {ch.mn[t].x, ch.mn[t].y, ch.mn[t].z, ch.mn[t].w};
+      for (int c = j * 4 * SK_TPW / NP; c < (j + 1) * 4 * SK_TPW / NP; c++) decode(ch, blk, 1, c / 4, c % 4);
+      if (j >= NP - SK_TPW) scales(ch, blk, j - (NP - SK_TPW));
+      fill((NEEDX ? 2 * MT : 0) + j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (FINE) {
 #pragma unroll
-          for (int i = 0; i < 4; i++) mn[t][i] = f * f16_to_f32((uint16_t)(mw[i] >> (16 * blk)));
-        }
+      for (int j = 0; j < NP; j++) P[j % SK_TPW][j / SK_TPW] = mfma16<T>(B0[j / SK_TPW], lo[j % SK_TPW][0], P[j % SK_TPW][j / SK_TPW]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NP; j++) P[j % SK_TPW][j / SK_TPW] = mfma16<T>(B1[0][j / SK_TPW], lo[j % SK_TPW][1], P[j % SK_TPW][j / SK_TPW]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+      const int mt = j / SK_TPW, t = j % SK_TPW;
+      P[t][mt] = mfma16<T>(B1[NEEDX ? blk : 0][mt], A[t][1], P[t][mt]);
+      if (j < MT) {
+        B0[j] = read_x(xn, nblk, 0, j);
+        if constexpr (NEEDX) B1[nblk][j] = read_x(xn, nblk, 1, j);
       }
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) {
-        const uint4 B0 = B[blk][mt][0], B1 = B[blk][mt][1];
-        const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-        f32x4 X = zero;
-        if constexpr (NEEDX) {
-          X = mfma16<T>(cA, B0, zero);
-          X = mfma16<T>(cA, B1, X);
-        }
-#pragma unroll
-        for (int t = 0; t < SK_TPW; t++) {
-          f32x4 P = mfma16<T>(A[t][0], B0, OFFS ? X : zero);
-          P = mfma16<T>(A[t][1], B1, P);
-          if constexpr (FINE) {
-            P = mfma16<T>(lo[t][0], B0, P);
-            P = mfma16<T>(lo[t][1], B1, P);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            acc[t][mt][i] = __builtin_fmaf(d[t][i], P[i], acc[t][mt][i]);
-            if constexpr (HASMIN) acc[t][mt][i] = __builtin_fmaf(mn[t][i], X[i], acc[t][mt][i]);
-          }
-        }
-      }
+      for (int c = j * 4 * SK_TPW / NP; c < (j + 1) * 4 * SK_TPW / NP; c++) decode(nx, nblk, 0, c / 4, c % 4);
+      if (!NEEDX && j >= NP - LATE) scale_out(j - (NP - LATE), blk);
+      fill((NEEDX ? 2 * MT : 0) + NP + j);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  // ---- main loop.  Step s: stage x of s + 1 (requested PF steps before) into the
-  // buffer that step s - 1 read (every wave is past that step's barrier), request
-  // x of s + 1 + PF, compute s, request the weights of s + PF, barrier.  Loads
-  // retire in order, so the wait for x of s + 1 leaves PF steps of weights in
-  // flight (34 KB of 4-bit, 68 KB of 8-bit codes per CU).  Steps run in whole
-  // groups of PF with no branch inside (hipcc keeps counted vmcnt waits); past
-  // the slice's end they find zeros in the staged x.
-  //
-  // Two waves per SIMD leave the LDS reads (768 cycles of a 48-row step), the
-  // decoding (1040) and the matrix work (1152) mostly one behind the other.  From
-  // three row tiles on, a step reads all of its x first and stages the next
-  // before its products, so that the decoding runs while LDS answers and no wave
-  // waits for its own stores at the barrier, and half of the waves go first:
-  // fp8_e5m2 300 rows gate/up [37888, 3584] 139 -> 133 us, down [3584, 18944]
-  // 83.8 -> 79.8; sym_int4 48 rows gate/up 24.8 -> 24.3, down 15.4 -> 15.1.  Two
-  // row tiles measured slower so (gate/up at 32 rows 18.9 -> 19.6); a barrier per
-  // two steps (twice the LDS) gained nothing at any size.  Four-wave groups have no
-  // registers left for it (one spilled) and one wave per SIMD to order.
-  constexpr bool EARLY = MT >= 3 && NW == 8;
-  uint4 xr[PF][XJ];
-  Chunk ring[PF];
-  load_x(xr[0], 0);
-  __builtin_amdgcn_sched_barrier(0);           // (the order in which the loop requests and waits)
+  // ---- main loop.  Step s: store x of s + 2 (requested in step s - 1) into the buffer that step s - 1 read, request x
+  // of s + 3 and the weights of s + 2, two phases, barrier: what a step reads ahead from the next one's x was stored
+  // before the barrier behind it.
+  constexpr uint32_t XBUF = R * SK_STEP * 2;
+  uint4 xr[XJ];
+  Chunk ring[RG];
+  {
+    uint4 x1[XJ];
 #pragma unroll
-  for (int u = 0; u < PF; u++) {
-    load_w(ring[u], u);
+    for (int j = 0; j < XJ; j++) xr[j] = load_x1(0, j);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) x1[j] = load_x1(1, j);
+    __builtin_amdgcn_sched_barrier(0);         // (the order in which the loop requests and waits)
+    load_w(ring[0], 0);
     __builtin_amdgcn_sched_barrier(0);
-    if (u + 1 < PF) load_x(xr[u + 1], u + 1);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) store_x1(xr[j], 0, j);
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) xr[j] = load_x1(2, j);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(ring[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < XJ; j++) store_x1(x1[j], XBUF, j);
   }
-  store_x(xr[0], 0, 0);
-  load_x(xr[0], PF);
   __syncthreads();
-  if (EARLY && wave < NW / 2) __builtin_amdgcn_s_setprio(1);
-  for (int s0 = 0; s0 < nstep; s0 += PF) {
 #pragma unroll
-    for (int u = 0; u < PF; u++) {
-      uint4 B[2][MT][2];
-      read_x(B, u & 1);
-      if constexpr (EARLY) {
-        __builtin_amdgcn_sched_barrier(0);
-        store_x(xr[(u + 1) % PF], s0 + u + 1, (u + 1) & 1);
-        load_x(xr[(u + 1) % PF], s0 + u + 1 + PF);
-      }
-      compute(ring[u], B);
-      __builtin_amdgcn_sched_barrier(0);       // the ring slot is free only after its compute: no second copy of it
-      load_w(ring[u], s0 + u + PF);
-      if constexpr (!EARLY) {
-        __builtin_amdgcn_sched_barrier(0);
-        store_x(xr[(u + 1) % PF], s0 + u + 1, (u + 1) & 1);
-        load_x(xr[(u + 1) % PF], s0 + u + 1 + PF);
-      }
-      __syncthreads();
-    }
+  for (int j = 0; j < MT; j++) {
+    B0[j] = read_x(0, 0, 0, j);
+    if constexpr (NEEDX) B1[0][j] = read_x(0, 0, 1, j);
   }
+#pragma unroll
+  for (int c = 0; c < 4 * SK_TPW; c++) decode(ring[0], 0, 0, c / 4, c % 4);
+  constexpr int NL = SK_TPW * WL, LS = 2 * PH - 2 * XJ - 1;      // weight loads of a step, slots they are spread over
+  auto step = [&](int st, auto U) {
+    constexpr int u = decltype(U)::value;
+    auto fill = [&](int k) {                                      // slot k of the step's 2 PH
+      if (k < XJ) store_x1(xr[k], (u + 2) % RG * XBUF, k);
+      else if (k < 2 * XJ) xr[k - XJ] = load_x1(st + 3, k - XJ);
+#pragma unroll
+      for (int i = 0; i < NL; i++)
+        if (k == 2 * XJ + (i * LS) / NL) load_w1(ring[(u + 2) % RG], st + 2, i);
+    };
+    phase(ring[u], ring[u], 0, u * XBUF, u * XBUF, [&](int k) { fill(k); });
+    phase(ring[u], ring[(u + 1) % RG], 1, u * XBUF, (u + 1) % RG * XBUF, [&](int k) { fill(PH + k); });
+    __syncthreads();
+  };
+  int s0 = 0;
+  for (; s0 + RG <= nstep; s0 += RG) {                            // whole turns of the rings, no branch inside
+    step(s0, std::integral_constant<int, 0>{});
+    step(s0 + 1, std::integral_constant<int, 1>{});
+    step(s0 + 2, std::integral_constant<int, 2>{});
+  }
+  if (s0 < nstep) step(s0, std::integral_constant<int, 0>{});
+  if (s0 + 1 < nstep) step(s0 + 1, std::integral_constant<int, 1>{});
+#pragma unroll
+  for (int i = LATE; i < NP; i++) scale_out(i, 1);
 
-  // ---- the two k-parts through LDS (x is done: the last step's barrier is behind)
-  float4* red = (float4*)smem;                                    // [4][SK_TPW][MT][64]
-  if (kp == 1) {
+  // ---- the two k-parts through LDS (x is done: the last step's barrier is behind): each wave of a pair finishes two of
+  // the lane's four rows
+  float2* red = (float2*)smem;                                    // [NW / 2][2][SK_TPW][MT][64]
+  auto slot = [&](int part, int t, int mt) { return (((cg * 2 + part) * SK_TPW + t) * MT + mt) * 64 + lane; };
 #pragma unroll
-    for (int t = 0; t < SK_TPW; t++)
+  for (int t = 0; t < SK_TPW; t++)
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++)
-        red[((cg * SK_TPW + t) * MT + mt) * 64 + lane] =
-            make_float4(acc[t][mt][0], acc[t][mt][1], acc[t][mt][2], acc[t][mt][3]);
-  }
+    for (int mt = 0; mt < MT; mt++)
+      red[slot(kp ^ 1, t, mt)] = kp == 0 ? make_float2(acc[t][mt][2], acc[t][mt][3]) : make_float2(acc[t][mt][0], acc[t][mt][1]);
   __syncthreads();
-  if (kp != 0) return;
+  float o[SK_TPW][MT][2];                                         // first k-part + second, whichever wave adds them
 #pragma unroll
   for (int t = 0; t < SK_TPW; t++)
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      const float4 v = red[((cg * SK_TPW + t) * MT + mt) * 64 + lane];
-      acc[t][mt][0] += v.x; acc[t][mt][1] += v.y; acc[t][mt][2] += v.z; acc[t][mt][3] += v.w;
+      const float2 v = red[slot(kp, t, mt)];
+      o[t][mt][0] = kp == 0 ? acc[t][mt][0] + v.x : v.x + acc[t][mt][2];
+      o[t][mt][1] = kp == 0 ? acc[t][mt][1] + v.y : v.y + acc[t][mt][3];
     }
 
-  // ---- epilogue: lane holds columns 16 tile + 4 g + i of row m0 + 16 mt + r16
+  // ---- epilogue: lane holds column 16 tile + r16 of rows m0 + 16 mt + 4 g + 2 kp + e
+  const int mr = m0 + 4 * g + 2 * kp;
   if (epi == EPI_GLU) {
-    if (tile0 + 1 >= NT) return;                                  // whole gate / up pairs (NT even)
-    const int n0 = (tile0 / 2) * 16 + 4 * g;
-    if (n0 >= a.N) return;
+    const int n = (tile0 / 2) * 16 + r16;
+    if (tile0 + 1 >= NT || n >= a.N) return;                      // whole gate / up pairs (NT even)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      const int m = m0 + mt * 16 + r16;
-      if (m >= a.M) continue;
-      float o[4];
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float gv = acc[0][mt][i], uv = acc[1][mt][i];
-        o[i] = (a.act == 0 ? silu_f(gv) : gelu_tanh_f(gv)) * uv;
+      for (int e = 0; e < 2; e++) {
+        const int m = mr + mt * 16 + e;
+        const float gv = o[0][mt][e];
+        if (m < a.M) ((uint16_t*)a.out)[(size_t)m * a.ldo + n] = from_f32<T>((a.act == 0 ? silu_f(gv) : gelu_tanh_f(gv)) * o[1][mt][e]);
       }
-      uint16_t* y = (uint16_t*)a.out + (size_t)m * a.ldo + n0;
-      if (n0 + 3 < a.N && ((a.ldo | n0) & 3) == 0) *(uint2*)y = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
-      else for (int i = 0; i < 4 && n0 + i < a.N; i++) y[i] = from_f32<T>(o[i]);
-    }
     return;
   }
 #pragma unroll
   for (int t = 0; t < SK_TPW; t++) {
-    const int n0 = (tile0 + t) * 16 + 4 * g;
-    if (tile0 + t >= NT || n0 >= a.N) continue;
+    const int n = (tile0 + t) * 16 + r16;
+    if (tile0 + t >= NT || n >= a.N) continue;
+    const float bv = epi != EPI_PARTIAL && a.bias ? to_f32<T>(a.bias[n]) : 0.f;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      const int m = m0 + mt * 16 + r16;
-      if (m >= a.M) continue;
-      float o[4] = {acc[t][mt][0], acc[t][mt][1], acc[t][mt][2], acc[t][mt][3]};
-      if (epi == EPI_PARTIAL) {
-        float* ws = (float*)a.out + ((size_t)blockIdx.y * a.M + m) * a.N + n0;
-        if (n0 + 3 < a.N && (a.N & 3) == 0) *(float4*)ws = make_float4(o[0], o[1], o[2], o[3]);
-        else for (int i = 0; i < 4 && n0 + i < a.N; i++) ws[i] = o[i];
-      } else {
-        if (a.bias) {
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-          for (int i = 0; i < 4; i++) o[i] += n0 + i < a.N ? to_f32<T>(a.bias[n0 + i]) : 0.f;
-        }
-        uint16_t* y = (uint16_t*)a.out + (size_t)m * a.ldo + n0;
-        if (n0 + 3 < a.N && ((a.ldo | n0) & 3) == 0) *(uint2*)y = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
-        else for (int i = 0; i < 4 && n0 + i < a.N; i++) y[i] = from_f32<T>(o[i]);
+      for (int e = 0; e < 2; e++) {
+        const int m = mr + mt * 16 + e;
+        if (m >= a.M) continue;
+        if (epi == EPI_PARTIAL) ((float*)a.out)[((size_t)blockIdx.y * a.M + m) * a.N + n] = o[t][mt][e];
+        else ((uint16_t*)a.out)[(size_t)m * a.ldo + n] = from_f32<T>(o[t][mt][e] + bv);
       }
-    }
   }
 }
 
 // dynamic LDS of one workgroup; a kernel asking for more than 64 KiB has its
 // limit raised first (once per kernel)
-inline size_t skinny_shmem(int mt, int table) { return (size_t)2 * mt * 16 * SK_STEP * 2 + table; }
+inline size_t skinny_shmem(int mt, int table) { return (size_t)3 * mt * 16 * SK_STEP * 2 + table; }
 
 template <int DK, typename T, int MT, int NW, bool FINE = false>
 void launch_skinny_t(int epi, dim3 grid, const GemvArgs& a, hipStream_t st) {
