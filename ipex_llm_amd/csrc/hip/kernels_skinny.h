@@ -6,7 +6,7 @@
 
 namespace illm {
 
-// workgroup = nw waves (4 or 8) = nw weight tiles x 16 mt rows (mt 2 .. 4) x a.cpk chunks; grid =
+// workgroup = nw waves (4 or 8) = nw weight tiles x 16 mt rows (mt 1 .. 4) x a.cpk chunks; grid =
 // (column blocks x row blocks -- several row blocks: padded to groups of 8 column blocks or not at all --, slices)
 // fine: table formats under bf16 x keep their table as bf16 pairs hi + lo (mt 3, 4)
 template <int DK>

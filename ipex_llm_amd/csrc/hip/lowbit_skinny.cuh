@@ -1,5 +1,6 @@
-// Low-bit weight x bf16/f16 activation product for 17 .. a few hundred rows
-// (serving decode batches, speculative verify, short prompts) on gfx950 MFMA.
+// Low-bit weight x bf16/f16 activation product for up to a few hundred rows
+// (serving decode batches, speculative verify, short prompts) on gfx950 MFMA;
+// up to 16 rows beside the decode kernel (skinny16 in csrc/torch/ops_hip.cpp says when).
 //
 // Between the one-row-tile GEMV (lowbit_gemv5.cuh) and the compute-bound
 // prefill GEMM the weight stream still bounds the product (a Llama-3-8B
@@ -378,16 +379,38 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
 #pragma unroll
       for (int e = 0; e < 2; e++) {
         const int m = mr + mt * 16 + e;
-        const float gv = o[0][mt][e];
-        if (m < a.M) ((uint16_t*)a.out)[(size_t)m * a.ldo + n] = from_f32<T>((a.act == 0 ? silu_f(gv) : gelu_tanh_f(gv)) * o[1][mt][e]);
+        if (m >= a.M) continue;
+        // x of a deferred norm: its row's scale
+        const float rs = a.xpss ? rsqrtf(a.xpss[m] / (float)a.xpss_n + a.xpss_eps) : 1.f;
+        const float gv = o[0][mt][e] * rs, uv = o[1][mt][e] * rs;
+        ((uint16_t*)a.out)[(size_t)m * a.ldo + n] = from_f32<T>((a.act == 0 ? silu_f(gv) : gelu_tanh_f(gv)) * uv);
       }
     return;
   }
 #pragma unroll
   for (int t = 0; t < SK_TPW; t++) {
     const int n = (tile0 + t) * 16 + r16;
-    if (tile0 + t >= NT || n >= a.N) continue;
-    const float bv = epi != EPI_PARTIAL && a.bias ? to_f32<T>(a.bias[n]) : 0.f;
+    if (tile0 + t >= NT) continue;
+    const float bv = epi != EPI_PARTIAL && a.bias && n < a.N ? to_f32<T>(a.bias[n]) : 0.f;
+    if constexpr (MT == 1) {
+      if (epi == EPI_STORE && a.amax) {                           // maximum of the tile's stored values, first index on ties
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          const float v = to_f32<T>(from_f32<T>(o[t][0][e] + bv));
+          const bool on = n < a.N && v > -INFINITY;               // (false for NaN)
+          float best = on ? v : -INFINITY;
+          int at = on ? n : 0x7fffffff;
+#pragma unroll
+          for (int off = 1; off < 16; off <<= 1) {
+            const float ov = __shfl_xor(best, off, 64);
+            const int oi = __shfl_xor(at, off, 64);
+            if (ov > best || (ov == best && oi < at)) best = ov, at = oi;
+          }
+          if (r16 == 0 && mr + e < a.M) a.amax[(size_t)(tile0 + t) * a.M + mr + e] = make_float2(best, __int_as_float(at));
+        }
+      }
+    }
+    if (n >= a.N) continue;
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -422,11 +445,13 @@ void launch_skinny_t(int epi, dim3 grid, const GemvArgs& a, hipStream_t st) {
 template <int DK, typename T>
 void launch_skinny_mt(int mt, int nw, int epi, dim3 grid, const GemvArgs& a, hipStream_t st) {
   if (nw == 8) {
-    if (mt <= 2) launch_skinny_t<DK, T, 2, 8>(epi, grid, a, st);
+    if (mt == 1) launch_skinny_t<DK, T, 1, 8>(epi, grid, a, st);
+    else if (mt == 2) launch_skinny_t<DK, T, 2, 8>(epi, grid, a, st);
     else if (mt == 3) launch_skinny_t<DK, T, 3, 8>(epi, grid, a, st);
     else launch_skinny_t<DK, T, 4, 8>(epi, grid, a, st);
   } else {
-    if (mt <= 2) launch_skinny_t<DK, T, 2, 4>(epi, grid, a, st);
+    if (mt == 1) launch_skinny_t<DK, T, 1, 4>(epi, grid, a, st);
+    else if (mt == 2) launch_skinny_t<DK, T, 2, 4>(epi, grid, a, st);
     else if (mt == 3) launch_skinny_t<DK, T, 3, 4>(epi, grid, a, st);
     else launch_skinny_t<DK, T, 4, 4>(epi, grid, a, st);
   }

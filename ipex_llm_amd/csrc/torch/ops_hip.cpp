@@ -84,7 +84,7 @@ struct SkinnyPlan {
 };
 // The split with the least estimated time.  A CU runs one 8-wave or two 4-wave workgroups at a time; a
 // round of them takes 3 us (launch, first loads, epilogue) and 0.5 / 0.6 / 0.8 us per 128-k chunk at
-// 2 / 3 / 4 row tiles (MI355X: gate/up of Llama-3-8B, 32 chunks in one round, 21 / 25 / 30 us; two 4-wave
+// 2 / 3 / 4 row tiles, 0.4 at one (MI355X: gate/up of Llama-3-8B, 32 chunks in one round, 21 / 25 / 30 us; two 4-wave
 // groups 24 / 30 / 36, one alone on its CU about 0.65 of that: Qwen2.5-7B's 296 column blocks as 592 of
 // half the size 36 instead of 40 us, a [2048, 1024] gate/up 5.7 instead of 6.7); slabs cost their write
 // and read (4.5 TB/s) and the reduction.  Several row blocks of a column block run on one XCD, so that its
@@ -97,9 +97,9 @@ struct SkinnyPlan {
 SkinnyPlan skinny_plan(int fmt, bool fine, int64_t M, int64_t NT, int64_t KC, bool can_split, int64_t ks_req = 0) {
   SkinnyPlan best{};
   const int64_t MB = (M + 63) / 64;
-  const int mt = std::max<int>(2, (int)(((M + MB - 1) / MB + 15) / 16));
+  const int mt = (int)(((M + MB - 1) / MB + 15) / 16);
   const bool heavy = illm::fmt_has_min(fmt) || fmt == illm::FMT_SYM_INT8 || fmt == illm::FMT_SYM_INT5 || fine;
-  const double chunk = (mt == 2 ? 0.5 : mt == 3 ? 0.6 : 0.8) * (illm::fmt_has_min(fmt) ? 4. / 3. : 1.);
+  const double chunk = (mt == 1 ? 0.4 : mt == 2 ? 0.5 : mt == 3 ? 0.6 : 0.8) * (illm::fmt_has_min(fmt) ? 4. / 3. : 1.);
   const bool asked = can_split && ks_req > 0;
   const int64_t kmin = asked ? ks_req : 1, kmax = asked ? ks_req : can_split ? std::min<int64_t>((KC + 3) / 4, 64) : 1;
   double cost = 1e30;
@@ -265,6 +265,32 @@ Plan5 plan5_rope(Plan5 p, int64_t NT, int64_t rows) {
   return p;
 }
 
+// contiguous, and 16-byte aligned as the kernels' loads are (a view into a larger tensor may start anywhere)
+Tensor rows16(const Tensor& x) {
+  Tensor c = x.contiguous();
+  return ((uintptr_t)c.data_ptr() & 15) != 0 ? c.clone() : c;
+}
+
+// Up to 16 rows, input and output in memory: the skinny kernel's one row tile instead of v5, by the format and the
+// shape, so that a row keeps its bits beside any other rows (1 to 16).  Not table formats under bf16 (v5 keeps an f16
+// table, the skinny kernel one in the type of x).
+//   * gate/up: us at 1 / 4 / 8 / 16 rows, v5 and this: [28672, 4096] sym_int4 15.7 15.0 15.9 22.4 and 15.4 15.4 15.4
+//     15.5, asym_int4 18.7 19.0 21.0 25.1 and 16.9 16.6 16.7 16.0, [37888, 3584] sym_int4 18.7 21.3 22.3 34.8 and 18.4
+//     18.2 18.3 19.6, fp8_e5m2 28.7 30.4 31.8 34.3 and 28.6 29.1 29.3 29.9, [9728, 896] 6.9 8.5 8.9 9.5 and 4.8 5.0 5.1
+//     5.0.  8-bit codes over a long K stay: [57344, 8192] fp8_e5m2 85.4 78.9 81.8 and 86.6 82.9 83.6;
+//   * slabs and plain products of K up to 5120 and up to 8192 columns: [6144, 4096] sym_int4 6.4 7.2 7.5 8.4 and 6.3 6.3
+//     6.2 6.5, [4096, 4096] 5.5 5.9 6.1 6.7 and 5.2 5.3 5.3 5.4, [3584, 3584] fp8_e5m2 6.1 6.6 6.7 7.3 and 5.5 5.7 5.7
+//     5.7, [2048, 2048] 4.7 5.1 5.3 5.7 and 4.1 4.3 4.3 4.3.  Longer K and wider outputs stay where v5 is ahead at few
+//     rows ([4096, 14336] 8.8 8.7 9.2 10.3 and 9.9 9.9 9.9 10.1, [12288, 4096] 8.4 9.4 10.3 12.5 and 12.4 12.1 12.1 12.2);
+//   * ... and where v5 would cut K by the number of rows, as its x does not fit the LDS: [3584, 18944] at 16 rows 15.4
+//     and 11.2, [8192, 28672] 35.6 and 26.2, the head [128256, 4096] at 8 rows 129.7 and 54.6.
+bool skinny16(int fmt, bool bf16, int64_t M, int64_t NT, int64_t KC, int64_t epi, int64_t ksplit) {
+  if (bf16 && illm::fmt_to_dk(fmt) == illm::DK_LUT4) return false;
+  if (epi == illm::EPI_GLU) return KC < 64 || illm::fmt_bits(fmt) == 4;
+  if (KC <= 40 && NT <= 512) return true;
+  return ksplit <= 0 && plan5(M, NT, KC, true, 0, false, fmt).ks != plan5(1, NT, KC, true, 0, false, fmt).ks;
+}
+
 // rows 1 .. most: v5 up to 16 rows (ILLM_GEMV_V1=1: the many-row kernels for these too, A/B tests), the
 // skinny kernel from 17, the narrow one where it fits
 Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
@@ -273,13 +299,14 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   TORCH_CHECK(x.size(-1) == k, "gemv: x last dim ", x.size(-1), " != in_features ", k);
   c10::DeviceGuard g(x.device());
   const bool bf16 = is_bf16(x);
-  Tensor xc = x.contiguous();
+  Tensor xc = rows16(x);
   const int64_t M = xc.numel() / k;
   TORCH_CHECK(M >= 1 && M <= most, "gemv handles 1..", most, " rows, got ", M);
   TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv: weight blob too small");
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N;
   const int64_t KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
-  const bool small = M <= 16 && getenv("ILLM_GEMV_V1") == nullptr;
+  const bool one = M <= 16 && skinny16((int)fmt, bf16, M, NT, KC, epi, ksplit);
+  const bool small = M <= 16 && !one && getenv("ILLM_GEMV_V1") == nullptr;
 
   illm::GemvArgs a{};
   a.x = p16(xc);
@@ -302,7 +329,7 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
     const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
     if (small && p.shmem <= kMaxLds)
       a.nw = p.nw, launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);
-    else if (narrow_fit((int)fmt, M, NT / 2, KC, epi))
+    else if (!one && narrow_fit((int)fmt, M, NT / 2, KC, epi))
       launch_narrow_any((int)fmt, bf16, illm::EPI_GLU, dim3((unsigned)(NT / 2), 1), a);
     else
       launch_skinny_any((int)fmt, bf16, skinny_plan((int)fmt, fine, M, NT, KC, false), illm::EPI_GLU, a);
@@ -320,7 +347,7 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
     ksplit = p5.ks;
     a.cpk = (int)p5.cpk;
     a.nw = p5.nw;
-  } else if (narrow_fit((int)fmt, M, NT, KC, epi)) {
+  } else if (!one && narrow_fit((int)fmt, M, NT, KC, epi)) {
     narrow = true;
     ksplit = std::max<int64_t>(1, std::min<int64_t>(ksplit, KC));
   } else {
@@ -376,7 +403,7 @@ std::tuple<Tensor, Tensor> gemv_argmax(const Tensor& x, const Tensor& blob, int6
   TORCH_CHECK(x.is_cuda() && blob.is_cuda() && x.size(-1) == k, "gemv_argmax: GPU x [M, k]");
   c10::DeviceGuard g(x.device());
   const bool bf16 = is_bf16(x);
-  Tensor xc = x.contiguous();
+  Tensor xc = rows16(x);
   const int64_t M = xc.numel() / k;
   TORCH_CHECK(M >= 1 && M <= 16, "gemv_argmax: 1..16 rows");
   TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv_argmax: weight blob too small");
@@ -411,6 +438,13 @@ std::tuple<Tensor, Tensor> gemv_argmax(const Tensor& x, const Tensor& blob, int6
   TORCH_CHECK((int64_t)p.gx * tg >= nparts, "gemv_argmax: geometry");
   Tensor parts = at::empty({nparts, M, 2}, xc.options().dtype(at::kFloat));
   a.amax = (float2*)parts.data_ptr<float>();
+  // from 6 rows on v5's x (full K, one workgroup per CU then) holds the stream up: [128256, 4096] sym_int4 at 1 / 5 / 8 /
+  // 16 rows 53 / 55 / 76 / 99 us, the skinny kernel's one row tile 54 / 55 / 55 / 57; [152064, 3584] fp8_e5m2 94 / 104 /
+  // 109 / 126 and 101 / 103 / 104 / 107
+  if (M >= 6 && !(bf16 && illm::fmt_to_dk((int)fmt) == illm::DK_LUT4)) {
+    launch_skinny_any((int)fmt, bf16, skinny_plan((int)fmt, false, M, NT, KC, true, 1), illm::EPI_STORE, a);
+    return {out, parts};
+  }
   launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_STORE, dim3(p.gx, 1), p.shmem, a);
   return {out, parts};
 }
@@ -811,7 +845,7 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   TORCH_CHECK(x.is_cuda() && blob.is_cuda() && x.size(-1) == k, "gemv_glu_ss: GPU x [M, k]");
   c10::DeviceGuard g(x.device());
   const bool bf16 = is_bf16(x);
-  Tensor xc = x.contiguous();
+  Tensor xc = rows16(x);
   const int64_t M = xc.numel() / k;
   TORCH_CHECK(M >= 1 && M <= 16 && n % 32 == 0, "gemv_glu_ss: 1..16 rows, n a multiple of 32");
   TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.numel() >= M, "gemv_glu_ss: ss f32 [>= M]");
@@ -834,6 +868,10 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   a.N = (int)(n / 2);
   a.out = out.data_ptr();
   a.ldo = (int)(n / 2);
+  if (skinny16((int)fmt, bf16, M, NT, KC, illm::EPI_GLU, 1)) {
+    launch_skinny_any((int)fmt, bf16, skinny_plan((int)fmt, false, M, NT, KC, false), illm::EPI_GLU, a);
+    return out;
+  }
   const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
   TORCH_CHECK(p.shmem <= kMaxLds, "gemv_glu_ss: x slice exceeds LDS");
   a.nw = p.nw;
