@@ -8,8 +8,8 @@ tiled blob, never materialised) for the wide gate/up pairs above that; and
 dequantize to a transient dense weight + GEMM.  Measured on MI355X (Llama-3-8B,
 sym_int4, graph replays over weights that no cache holds), skinny against the
 better of the other two: M = 96 qkv 19 / 38 us, o 15 / 38, down 25 / 75,
-gate_up 47 / 56; M = 300 qkv 28 / 44, o 27 / 37, down 71 / 93, gate_up
-128 / 113; M = 512 o 28 / 38, down 86 / 104, qkv (two rounds) 52 / 48.
+gate_up 41 / 58; M = 300 qkv 28 / 44, o 27 / 37, down 71 / 93, gate_up
+119 / 112; M = 512 o 28 / 38, down 86 / 104, qkv (two rounds) 52 / 48.
 ``ILLM_GEMM_LIB=1`` / ``ILLM_GEMM_FUSED=1`` force either other path (A/B runs).
 """
 from __future__ import annotations
@@ -40,15 +40,22 @@ def rows_fit(M: int, n: int, fmt: int, glu: bool = False, k: int = 0) -> bool:
     are then ahead); formats with block minima, whose sums take a third more,
     up to 5 / 8 of that and 320 rows (asym_int5 [2048, 2048], 300 rows 17.5 /
     18.3 us, 384 rows 17.7 / 19.3), asym_int5 up to a half ([4096, 8192] 320
-    rows 62 / 57).  Gate/up pairs up to 96 rows (Llama-3-8B, two rounds: M = 96
-    47 / 56 us, M = 128 55 / 56), by the rows alone -- a column shard of a
-    tensor-parallel model takes the kernel that the whole pair takes -- but for
-    pairs of over three rounds where a round is short or has minima in integer bytes ([151936, 1024] sym_int4 80 / 70, fp4 77 / 62;
-    [57344, 8192] asym_int5 219 / 209, sym_int4 158 / 185)."""
+    rows 62 / 57).  Gate/up pairs by the rows alone -- a column shard of a
+    tensor-parallel model takes the kernel that the whole pair takes --: up to 96
+    rows (Llama-3-8B sym_int4, this / the fused kernel: M = 65 42 / 58 us, 96
+    41 / 58; two and more rounds would take 128 rows there, 49 / 58, but not in
+    [37888, 3584], 78 / 63), and 8-bit floats, whose codes have no offset, up to
+    512 (fp8_e5m2 [37888, 3584] M = 128 73 / 73, 300 118 / 128, 512 192 / 196;
+    e4m3 [28672, 4096] 50 / 58, 105 / 122, 152 / 168; not of K up to 1024,
+    [14336, 1024] M = 420 44 / 34).  Nor pairs of over three rounds where a round
+    is short or has minima in integer bytes ([151936, 1024] sym_int4 80 / 70,
+    fp4 77 / 62; [57344, 8192] asym_int5 219 / 209, sym_int4 158 / 185)."""
     if _USE_LIB or _USE_FUSED or M > ROWS_MAX_M:
         return False
     from ..quantize import qtypes as Q
     if glu:
+        if fmt in (Q.FMT_FP8E4, Q.FMT_FP8E5, Q.FMT_FP6) and not 0 < k <= 1024:
+            return True
         return M <= 96 and not (n > 49152 and (0 < k <= 1024 or fmt == Q.FMT_ASYM_INT5))
     blocks = (n + 127) // 128 * ((M + 63) // 64)
     if fmt in (Q.FMT_ASYM_INT4, Q.FMT_ASYM_INT5):

@@ -112,3 +112,21 @@ def test_x_that_starts_anywhere(cuda, at):
             else:
                 y, want = (op(t, blob, f, n, k, None, epi, 1, 0) for t in (x, x.clone()))
             assert torch.equal(y, want), (M, epi)
+
+
+@pytest.mark.parametrize("name", ["fp8_e4m3", "fp8_e5m2", "fp6"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_pairs_of_8_bit_floats(cuda, name, dtype):
+    """gate/up products of 97 to 512 rows: row blocks of every height, both sides of the rule"""
+    from ipex_llm_amd.models.decoder import deinterleave_glu
+    from ipex_llm_amd.ops.gemm import lowbit_gemm_glu, rows_take
+    f = get_format(name).fmt
+    torch.manual_seed(5)
+    for n, k in [(96, 1088), (4128, 1152), (320, 1024)]:
+        blob = ops.quantize(torch.randn(n, k, device=cuda) * 0.05, f)
+        W = R.dequantize_device_blob(blob, f, n, k).to(cuda).double()
+        for M in (97, 129, 300, 385, 511, 512, 513):
+            x = torch.randn(M, k, device=cuda).to(dtype)
+            assert rows_take(dtype, M, n, k, f, True) == (M <= 512 and k > 1024)
+            g, u = deinterleave_glu(x.double() @ W.t())
+            assert _rel(lowbit_gemm_glu(x, blob, f, n, k), torch.nn.functional.silu(g) * u) < 2 * STORE, (n, k, M)

@@ -66,3 +66,17 @@ def test_prefetch_asks_what_the_product_asks():
     assert not G.wants_dense(bf, 512, 2048, 4096, f) and G.wants_dense(bf, 512, 2048, 4096, f, glu=True)
     assert not G.wants_dense(bf, 90, 28672, 10240, f, glu=True) and G.wants_dense(bf, 97, 28672, 10240, f, glu=True)
     assert G.wants_dense(bf, 1024, 4096, 4096, f) and not G.wants_dense(bf, 100, 28672, 4096, f, glu=True)
+
+
+def test_pairs_of_8_bit_floats_up_to_512_rows():
+    """gate/up: by the rows alone (a column shard as the whole pair), but for a short K; other formats up to 96 rows"""
+    import torch
+    from ipex_llm_amd.quantize import get_format
+    for dt in (torch.bfloat16, torch.float16):
+        for n in (2048, 37888, 151936):
+            for name in ("fp8_e4m3", "fp8_e5m2", "fp6"):
+                f = get_format(name).fmt
+                assert all(G.rows_take(dt, M, n, 3584, f, True) for M in (1, 96, 97, 300, 512))
+                assert not G.rows_take(dt, 513, n, 3584, f, True) and not G.rows_take(dt, 97, n, 1024, f, True)
+            for name in ("sym_int4", "fp4", "sym_int8", "asym_int4"):
+                assert not G.rows_take(dt, 97, n, 3584, get_format(name).fmt, True)
