@@ -12,9 +12,10 @@
 //   * workgroup = 4 waves = 64 query rows of one head; wave w owns rows
 //     16w..16w+15.  Causal q-blocks are issued heaviest first;
 //   * K/V tiles of 64 keys are read once per workgroup straight from the
-//     paged cache (a 64-key tile never crosses a cache block, bs % 64 == 0),
-//     the next tile's loads in flight while the current one is computed,
-//     and staged in LDS as [key][D] rows with a 16-byte XOR swizzle;
+//     paged cache (a 64-key tile never crosses a cache block, bs % 64 == 0)
+//     into LDS as [key][D] rows with a 16-byte XOR swizzle, by LDS-DMA: the
+//     next tile is in flight while the current one is computed, with no
+//     register, conversion or LDS store in between;
 //   * swapped QK^T: S^T = K Q^T (A = K rows from LDS by ds_read_b128, B = the
 //     wave's Q rows kept in registers), so a lane holds 16 scores of ONE query
 //     row: the online-softmax row max / sum is a register reduction plus two
@@ -23,7 +24,22 @@
 //     converted to 16-bit (key order of the C layout, no lane movement), the
 //     A operand (V^T) comes from ds_read_b64_tr_b16 transposed reads of the
 //     row-major V tile in exactly that key order;
-//   * fp8 KV caches are converted to 16-bit while the tile is staged.
+//   * fp8 KV caches go through registers and are converted to 16-bit on the
+//     way to LDS.
+// What bounds it: up to a grid of two workgroups per CU, one tile's chain in a
+// wave (QK^T and PV each read the tile at LDS speed, 512 cycles, with the
+// softmax between them and the staging's wait and barrier after), not the
+// products.  Out of that chain came: the block-id round trip of every tile (ids
+// are read 64 at a time), the waits for the tile in flight that hipcc placed
+// before the first product (for Q, for zeros at the sequence end and for fp8
+// conversions beside the load), the LDS stores, and half of the vector
+// instructions (scale in one fma with the maximum, addresses by xor, row maximum
+// by lane swaps).  MI355X, 32 / 8 heads of 128, before -> after: 1024 rows 32.6 ->
+// 25.6 us, 8 x 1024 115 -> 100, 200 rows behind 1800 keys 56 -> 42, 300 rows of
+// 28 / 4 heads 12.8 -> 10.2, 1024 rows on an e5m2 cache 50 -> 31, the same error.
+// Slower or no better: keys of a tile split over 8 waves (23.5 at 1024 rows, 141 at
+// 8 x 1024), K and V half a tile apart with a second barrier (26.4, 99), the next
+// tile but one in flight, wave priorities around the products.
 #include <cstdlib>
 
 #include "../common/quant_block.h"
@@ -35,12 +51,15 @@ namespace illm {
 constexpr int PF_KT = 64;      // keys per tile
 constexpr int PF_QB = 64;      // query rows per workgroup
 
+// 8 cache elements as they lie, and as 16-bit values
+template <int KVF> struct pf_raw { typedef uint2 type; };
+template <> struct pf_raw<0> { typedef uint4 type; };
+
 template <typename T, int KVF>
-__device__ __forceinline__ uint4 pf_load8(const uint8_t* p, float scale) {
+__device__ __forceinline__ uint4 pf_cvt8(const typename pf_raw<KVF>::type& u, float scale) {
   if constexpr (KVF == 0) {
-    return *(const uint4*)p;
+    return u;
   } else {
-    const uint2 u = *(const uint2*)p;
     float v[8];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -56,18 +75,41 @@ __device__ __forceinline__ uint4 pf_load8(const uint8_t* p, float scale) {
   }
 }
 
+// LDS-DMA of a 16-bit tile: 16 bytes a lane, LDS side wave-uniform base + lane * 16 (asm, so that hipcc does not
+// drain it before every LDS read of the other buffer; the waits are written out)
+typedef int32_t pf_rsrc __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ pf_rsrc pf_make_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t p = (uint64_t)(uintptr_t)base;
+  return pf_rsrc{(int32_t)(uint32_t)p, (int32_t)((uint32_t)(p >> 32) & 0xffffu), (int32_t)bytes, 0x00020000};
+}
+
+__device__ __forceinline__ void pf_dma16(const pf_rsrc& rs, const uint8_t* lds, uint32_t voff, int soff) {
+  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)lds);
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(la), "v"(voff), "s"(rs), "s"(soff) : "memory", "m0");
+}
+
+// max over the four lanes of a query row (lane ^ 16, ^ 32)
+__device__ __forceinline__ float xmax(float v) {
+  auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+
 // HP = query heads per wave that share one kv head (GQA): every K fragment
 // read from LDS and every transposed V read feeds HP MFMAs.
 template <typename T, int D, int KVF, int HP, bool SOFTCAP>
-__global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs a) {
+__global__ void __launch_bounds__(256, 2) attn_prefill_kernel(const AttnPrefillArgs a) {
   constexpr int EB = KVF == 0 ? 2 : 1;            // cache bytes per element
   constexpr int KSTEP = D / 32;                   // MFMA k-steps over the head dim (QK^T)
   constexpr int DT = D / 16;                      // 16-wide d tiles of O^T
   constexpr int UPT = PF_KT * D / 8 / 256;        // 8-element staging units per thread per tile
-  // double-buffered K / V tiles: the next tile is written while the current
+  constexpr int TB = PF_KT * D * 2;               // bytes of a K or V tile in LDS
+  // double-buffered K / V tiles (K0, K1, V0, V1): the next tile is written while the current
   // one is read, one workgroup barrier per tile
-  __shared__ __attribute__((aligned(16))) uint16_t ks[2][PF_KT * D];
-  __shared__ __attribute__((aligned(16))) uint16_t vs[2][PF_KT * D];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * TB];
 
   // causal work per query block grows with its index.  Block order: heaviest
   // query blocks of every (head, batch) first (longest-processing-time first
@@ -80,8 +122,8 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
   const int rank = lin / nother, other = lin % nother;
   const int half = (nqb + 1) / 2;
   const int qb = (nqb * nother <= 512 && rank >= half) ? rank - half : nqb - 1 - rank;
-  const int h0 = (other % gridDim.y) * HP, b = other / gridDim.y;
-  const int kvh = h0 / (a.Hq / a.Hkv);
+  const int hh = other % gridDim.y, b = other / gridDim.y;
+  const int kvh = hh % a.Hkv, h0 = kvh * (a.Hq / a.Hkv) + hh / a.Hkv * HP;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r16 = lane & 15;
   const int L = a.seq_lens[b];
@@ -98,6 +140,16 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
   if (a.sliding_window > 0) kbeg = max(0, wg_q0 - a.sliding_window + 1) & ~(PF_KT - 1);
   const int ntile = kend > kbeg ? (kend - kbeg + PF_KT - 1) / PF_KT : 0;
 
+  if (ntile == 0) {                               // no key: zeros
+#pragma unroll
+    for (int j = 0; j < HP; j++)
+#pragma unroll
+      for (int d = 0; d < DT; d++)
+        if (qrow < Tq)
+          *(uint2*)(a.out + ((size_t)(b * Tq + qrow) * a.Hq + h0 + j) * D + 16 * d + 4 * g) = make_uint2(0u, 0u);
+    return;
+  }
+
   // Q fragments (B operand of S^T = K Q^T): row qrow, dims 32 s + 8 g .. + 7
   uint4 qf[HP][KSTEP];
 #pragma unroll
@@ -107,40 +159,77 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
     for (int s = 0; s < KSTEP; s++) qf[j][s] = *(const uint4*)(qp + 32 * s + 8 * g);
   }
 
-  // staging: unit u = tid + 256 j covers key u / (D / 8), chunk u % (D / 8)
-  auto tile_src = [&](int t, const uint8_t* cache) -> const uint8_t* {
-    const int k0 = kbeg + t * PF_KT;
-    int blk = a.block_tables[(size_t)b * a.max_blocks + k0 / a.bs];
+  // block ids: one load of 64 (lane i: block bi + i), read out lane by lane; an id and its tile
+  // loaded in one step are two round trips
+  const int* table = a.block_tables + (size_t)b * a.max_blocks;
+  const int blast = (kend - 1) / a.bs;
+  int bi = kbeg / a.bs, boff = kbeg % a.bs, bl = 0;       // block, offset and lane of the next tile to load
+  int bids = table[min(bi + lane, blast)];
+  size_t src = 0;                                         // its place in the caches, bytes
+  auto next_src = [&] {
+    int blk = __builtin_amdgcn_readlane(bids, bl);
     if (bad_block(blk, a.num_blocks)) {                  // read block 0 instead, report
       kerr(a.err, ERR_BLOCK_ID);
       blk = 0;
     }
-    return cache + (((size_t)blk * a.Hkv + kvh) * a.bs + (k0 % a.bs)) * D * EB;
+    src = (((size_t)blk * a.Hkv + kvh) * a.bs + boff) * D * EB;
+    boff += PF_KT;
+    if (boff == a.bs) {
+      boff = 0;
+      bi++;
+      if (++bl == 64) {
+        bids = table[min(bi + lane, blast)];
+        bl = 0;
+      }
+    }
   };
-  uint4 kreg[UPT], vreg[UPT];
+  // staging of a tile into buffer t & 1: 16-bit caches by LDS-DMA (piece i of a wave: 1 KB of LDS, the swizzle
+  // on the source side), fp8 through registers, converted on the way to LDS
+  using raw = typename pf_raw<KVF>::type;
+  raw kreg[KVF ? UPT : 1], vreg[KVF ? UPT : 1];
+  constexpr int RP = 512 / D;                     // rows of 1 KB
+  const int dr = wave * RP + lane / (D / 8);
+  const uint32_t doff = 2 * pf_off<D>(dr, lane % (D / 8));
   auto load_tile = [&](int t) {
-    const uint8_t* kp = tile_src(t, a.k_cache);
-    const uint8_t* vp = tile_src(t, a.v_cache);
-    const int k0 = kbeg + t * PF_KT;
+    next_src();
+    if constexpr (KVF == 0) {
+      const pf_rsrc rk = pf_make_rsrc(a.k_cache + src, TB), rv = pf_make_rsrc(a.v_cache + src, TB);
+      const uint8_t* dst = lds + (t & 1) * TB + wave * 1024;
 #pragma unroll
-    for (int j = 0; j < UPT; j++) {
-      const int u = tid + 256 * j;
-      const int r = u / (D / 8), c = u % (D / 8);
-      kreg[j] = pf_load8<T, KVF>(kp + ((size_t)r * D + c * 8) * EB, a.k_scale);
-      vreg[j] = pf_load8<T, KVF>(vp + ((size_t)r * D + c * 8) * EB, a.v_scale);
-      // slots past the sequence end hold stale bytes (possibly NaN patterns):
-      // p = 0 times NaN would still poison the P V product, so zero them
-      if (k0 + r >= L) kreg[j] = vreg[j] = make_uint4(0, 0, 0, 0);
+      for (int i = 0; i < TB / 4096; i++) pf_dma16(rk, dst + i * 4096, doff, i * 4096);
+#pragma unroll
+      for (int i = 0; i < TB / 4096; i++) pf_dma16(rv, dst + 2 * TB + i * 4096, doff, i * 4096);
+    } else {
+#pragma unroll
+      for (int j = 0; j < UPT; j++) {
+        const int u = tid + 256 * j;
+        kreg[j] = *(const raw*)(a.k_cache + src + (size_t)u * 8 * EB);
+        vreg[j] = *(const raw*)(a.v_cache + src + (size_t)u * 8 * EB);
+      }
     }
   };
-  auto store_tile = [&](int buf) {
+  // the tile is in LDS for every wave.  V slots past the sequence end hold stale bytes (possibly NaN
+  // patterns): p = 0 times NaN would still poison the P V product, so they are zeroed
+  auto finish_tile = [&](int t) {
+    const int buf = t & 1, last = L - (kbeg + t * PF_KT);       // rows of the tile that count
+    if constexpr (KVF == 0) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (last < PF_KT) {
+        __syncthreads();
+        for (int u = tid; u < PF_KT * D / 8; u += 256)
+          if (u / (D / 8) >= last) *(uint4*)(lds + (2 + buf) * TB + u * 16) = make_uint4(0, 0, 0, 0);
+      }
+    } else {
 #pragma unroll
-    for (int j = 0; j < UPT; j++) {
-      const int u = tid + 256 * j;
-      const int r = u / (D / 8), c = u % (D / 8);
-      *(uint4*)(ks[buf] + pf_off<D>(r, c)) = kreg[j];
-      *(uint4*)(vs[buf] + pf_off<D>(r, c)) = vreg[j];
+      for (int j = 0; j < UPT; j++) {
+        const int u = tid + 256 * j;
+        const int r = u / (D / 8), c = u % (D / 8);
+        const uint4 vv = pf_cvt8<T, KVF>(vreg[j], a.v_scale);
+        *(uint4*)(lds + buf * TB + 2 * pf_off<D>(r, c)) = pf_cvt8<T, KVF>(kreg[j], a.k_scale);
+        *(uint4*)(lds + (2 + buf) * TB + 2 * pf_off<D>(r, c)) = r < last ? vv : make_uint4(0, 0, 0, 0);
+      }
     }
+    __syncthreads();
   };
 
   f32x4 o[HP][DT];
@@ -154,18 +243,25 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
   const float sc = a.scale;
   constexpr float kLog2e = 1.4426950408889634f;
   const float sc2 = a.scale * kLog2e;
+  // scores in the exp2 domain: p = exp2(st * mul - m), one fma each; the maximum is taken before the
+  // factor, so a factor that is not positive and normal (and the soft cap) goes on beforehand and mul is 1
+  const bool pre = SOFTCAP || !(sc2 >= 1.17549435e-38f);
+  const float mul = pre ? 1.f : sc2;
 
-  if (ntile > 0) {
-    load_tile(0);
-    store_tile(0);
-  }
-  __syncthreads();
+  // LDS bytes of the lane's fragments: K row r16, chunk 4 s + g; V (transposed reads: lane 4 q + p of the
+  // 16-lane group g addresses row 4 g + q, columns 16 d + 4 p).  The swizzle is an xor of the chunk, so
+  // chunks s and d are an xor of bits 6.. and 5.. of the first one's address
+  const uint32_t ko = 2 * pf_off<D>(r16, g);
+  const uint32_t vo = 2 * pf_off<D>(4 * g + (r16 >> 2), (r16 & 3) >> 1) + 8 * (r16 & 1) + 2 * TB;
+
+  load_tile(0);
+  __builtin_amdgcn_s_waitcnt(0x0f70);           // Q too: a wait for it inside the loop would be one for the tile in flight
+  finish_tile(0);
   for (int t = 0; t < ntile; t++) {
-    const int buf = t & 1;
-    if (t + 1 < ntile) load_tile(t + 1);          // next tile in flight during the compute
+    const uint32_t bo = (t & 1) * TB;
+    // next tile in flight during the compute (its buffer: read last in tile t - 1, free since the barrier)
+    if (t + 1 < ntile) load_tile(t + 1);
     const int kt0 = kbeg + t * PF_KT;
-    const uint16_t* kb_ = ks[buf];
-    const uint16_t* vb_ = vs[buf];
     // tiles wholly below every query row of the workgroup need no mask
     const bool full = kt0 + PF_KT - 1 <= wg_q0 && kt0 + PF_KT <= L && a.sliding_window <= 0;
 
@@ -177,12 +273,12 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
       for (int j = 0; j < HP; j++) st[j][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < KSTEP; s++) {
-        const uint4 kf = *(const uint4*)(kb_ + pf_off<D>(16 * kb + r16, 4 * s + g));
+        const uint4 kf = *(const uint4*)(lds + ((ko + bo) ^ (s << 6)) + kb * 16 * D * 2);
 #pragma unroll
         for (int j = 0; j < HP; j++) st[j][kb] = mfma16<T>(kf, qf[j][s], st[j][kb]);
       }
     }
-    // ---- scale, soft-cap, causal / window / length mask, online softmax
+    // ---- soft-cap, causal / window / length mask, online softmax
     uint32_t pk[HP][4][2];                         // P^T fragments, 16-bit pairs
 #pragma unroll
     for (int j = 0; j < HP; j++) {
@@ -190,16 +286,14 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
       // a per-score branch (tanhf's own control flow inlined 16 times) split
       // the tile loop into ~100 basic blocks, so no MFMA / VALU interleaving
       // across them (rocprofv3: 3 SALU and 10 VALU per MFMA)
+      if (pre) {
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) {
+        for (int kb = 0; kb < 4; kb++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          // scores in the exp2 domain (scale * log2 e folded in): p = exp2(v - m)
-          float v;
-          if constexpr (SOFTCAP) v = a.softcap * tanhf(st[j][kb][i] * sc / a.softcap) * kLog2e;
-          else v = st[j][kb][i] * sc2;
-          st[j][kb][i] = v;
-        }
+          for (int i = 0; i < 4; i++) {
+            if constexpr (SOFTCAP) st[j][kb][i] = a.softcap * tanhf(st[j][kb][i] * sc / a.softcap) * kLog2e;
+            else st[j][kb][i] *= sc2;
+          }
       }
       if (!full) {
         const int win = a.sliding_window > 0 ? qpos - a.sliding_window : -1;
@@ -218,45 +312,37 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
       for (int kb = 0; kb < 4; kb++)
 #pragma unroll
         for (int i = 0; i < 4; i++) tmax = fmaxf(tmax, st[j][kb][i]);
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float mnew = fmaxf(mrow[j], tmax);
-      // nothing seen yet (mrow = -inf): exp2(-inf) = 0 clears the empty O; a row
-      // still fully masked keeps alpha 1 and a finite max of 0 for the exp2 below
-      const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow[j] - mnew);
-      const float msafe = mnew == -INFINITY ? 0.f : mnew;
-      mrow[j] = mnew;
-      // O rescale only when some row max of the wave moved (wave-uniform)
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+      tmax = xmax(tmax) * mul;
+      // O rescale only when some row max of the wave moved (wave-uniform).  Nothing seen yet
+      // (mrow = -inf): exp2(-inf) = 0 clears the empty O; a row still fully masked keeps alpha 1
+      if (__builtin_amdgcn_ballot_w64(tmax > mrow[j]) != 0) {
+        const float mnew = fmaxf(mrow[j], tmax);
+        const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow[j] - mnew);
+        mrow[j] = mnew;
         lpart[j] *= alpha;
 #pragma unroll
         for (int d = 0; d < DT; d++) {
           o[j][d][0] *= alpha; o[j][d][1] *= alpha; o[j][d][2] *= alpha; o[j][d][3] *= alpha;
         }
       }
+      const float msafe = mrow[j] == -INFINITY ? 0.f : mrow[j];     // a finite base for the exp2 below
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) {
         float p[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          p[i] = __builtin_amdgcn_exp2f(st[j][kb][i] - msafe);      // masked: exp2(-inf) = 0
-          lpart[j] += p[i];
-        }
+        for (int i = 0; i < 4; i++) p[i] = __builtin_amdgcn_exp2f(fmaf(st[j][kb][i], mul, -msafe));   // masked: 0
+        lpart[j] += (p[0] + p[1]) + (p[2] + p[3]);
         pk[j][kb][0] = pack2<T>(p[0], p[1]);
         pk[j][kb][1] = pack2<T>(p[2], p[3]);
       }
     }
-    // ---- O^T += V^T P^T over two 32-key steps (key blocks 2 ks, 2 ks + 1)
+    // ---- O^T += V^T P^T over two 32-key steps (key blocks 2 kk, 2 kk + 1)
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
-      // lane 4q + p of the 16-lane group g addresses row 16 kb + 4 g + q, columns 16 dt + 4 p
-      const int qq = r16 >> 2, pp = r16 & 3;
-      const int row0 = 16 * (2 * kk) + 4 * g + qq, row1 = row0 + 16;
 #pragma unroll
       for (int d = 0; d < DT; d++) {
-        const int col = 16 * d + 4 * pp;                     // element column; chunk col / 8
-        const uint2 v0 = ds_read_tr16(vb_ + pf_off<D>(row0, col >> 3) + (col & 7));
-        const uint2 v1 = ds_read_tr16(vb_ + pf_off<D>(row1, col >> 3) + (col & 7));
+        const uint8_t* vp = lds + ((vo + bo) ^ (d << 5)) + kk * 32 * D * 2;
+        const uint2 v0 = ds_read_tr16((const uint16_t*)vp), v1 = ds_read_tr16((const uint16_t*)(vp + 16 * D * 2));
         const uint4 va = make_uint4(v0.x, v0.y, v1.x, v1.y);
 #pragma unroll
         for (int j = 0; j < HP; j++) {
@@ -265,8 +351,7 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const AttnPrefillArgs
         }
       }
     }
-    if (t + 1 < ntile) store_tile(buf ^ 1);       // read last during tile t - 1: free since the barrier
-    __syncthreads();
+    if (t + 1 < ntile) finish_tile(t + 1);
   }
 
   // ---- normalise and store: lane holds O^T[16 d + 4 g + i][row r16]
@@ -305,10 +390,10 @@ static void launch_pf_d(const AttnPrefillArgs& a, hipStream_t st) {
   // HP = 2: two query heads of one kv head per wave, so every K fragment and
   // transposed V read from LDS feeds two MFMAs (even GQA group).  It halves
   // the grid, so it is taken when the halved grid still covers the chip
-  // twice (2 workgroups per CU).  Measured on MI355X (Llama-3-8B heads):
-  // T = 4096 266 -> 212 us, B = 8 x 1024 164 -> 120 us, T = 16 K 3.42 ->
-  // 2.46 ms (895 TFLOP/s); T = 1024 (256 workgroups) 30.3 -> 37.3 us, so HP = 1
-  // there.  ILLM_PREFILL_HP=1/2 forces either.
+  // twice (2 workgroups per CU).  Measured on MI355X (32 / 8 heads, HP = 1 / 2):
+  // T = 4096 200 / 170 us, B = 8 x 1024 125 / 100, 3 x 1024 50 / 44, T = 2048 (512
+  // workgroups) 59 / 63, with a window of 500 39 / 33; T = 1024 (256) 26 / 34, so
+  // HP = 1 there.  ILLM_PREFILL_HP=1/2 forces either.
   static const int hp_env = getenv("ILLM_PREFILL_HP") ? atoi(getenv("ILLM_PREFILL_HP")) : 0;
   const bool even = (a.Hq / a.Hkv) % 2 == 0;
   const long wg2 = (long)((a.Tq + PF_QB - 1) / PF_QB) * (a.Hq / 2) * a.B;
