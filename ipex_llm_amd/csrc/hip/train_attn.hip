@@ -76,18 +76,61 @@ __device__ __forceinline__ void ta_stage(const ta_rsrc& rs, uint32_t lds, int ro
   }
 }
 
+// Fragments of a tile at byte address `tile` (the swizzle is an xor of the 16-byte chunk, so chunk 4 s + g is an xor of
+// bits 6.. of chunk g's address, and columns 16 d.. of bits 5..).  Rows: 16 kb + r16 of the plain reads; of the
+// transposed ones lane 4 q + p of the 16-lane group g addresses row 16 kb + 4 g + q, columns 16 d + 4 p.  What bounds
+// these kernels is a tile's chain in a wave, whose vector part the addresses were half of: with them, one fma a score
+// and the row maximum by lane swaps, 8 x 512 forward 56.5 -> 50, backward 166 -> 160, 2048 rows 80 -> 69, 332 -> 286
+template <int D>
+struct FaFrag {
+  uint32_t ko, vo;
+  __device__ __forceinline__ FaFrag(int g, int r16)
+      : ko(2 * pf_off<D>(r16, g)), vo(2 * pf_off<D>(4 * g + (r16 >> 2), (r16 & 3) >> 1) + 8 * (r16 & 1)) {}
+  __device__ __forceinline__ uint4 row(const uint8_t* lds, uint32_t tile, int kb, int s) const {
+    return *(const uint4*)(lds + ((ko + tile) ^ (s << 6)) + kb * 16 * D * 2);
+  }
+  __device__ __forceinline__ uint4 col(const uint8_t* lds, uint32_t tile, int kk, int d) const {   // rows of blocks 2 kk, 2 kk + 1
+    const uint8_t* p = lds + ((vo + tile) ^ (d << 5)) + kk * 32 * D * 2;
+    const uint2 v0 = ds_read_tr16((const uint16_t*)p), v1 = ds_read_tr16((const uint16_t*)(p + 16 * D * 2));
+    return make_uint4(v0.x, v0.y, v1.x, v1.y);
+  }
+};
+
+// max over the four lanes of a query row (lane ^ 16, ^ 32)
+__device__ __forceinline__ float ta_xmax(float v) {
+  auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+
 __device__ __forceinline__ void ta_wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Workgroup -> (block in order of weight, head, batch).  Ids go round the 8 XCDs, so with the block fastest (grid x)
+// and 8 blocks (T = 512) every XCD had one weight: 64 keys against 512.  The heaviest blocks of all heads go first; a
+// grid that is resident at once (two workgroups per CU) runs its second half in ascending order, so the two of a CU
+// add up alike.  The query heads of one kv head stay on one XCD (their K / V share its L2).  MI355X, 32 / 8 heads of
+// 128, us, block fastest / this, forward and backward: 8 x 512 78 / 56.5, 195 / 166; 2 x 1024 70 / 45.5, 219 / 185;
+// 2 x 4096 735 / 495, 1930 / 1190
+__device__ __forceinline__ void ta_block(int& w, int& hh, int& b) {
+  const int nb = gridDim.x, nother = gridDim.y * gridDim.z;
+  const int lin = blockIdx.x + nb * (blockIdx.y + gridDim.y * blockIdx.z);
+  const int rank = lin / nother, other = lin % nother, half = (nb + 1) / 2;
+  w = nb * nother <= 512 && rank >= half ? nb - 1 - (rank - half) : rank;
+  hh = other % gridDim.y;
+  b = other / gridDim.y;
+}
 
 // ---- forward (with_dq = false) and dQ (with_dq = true) --------------------
 template <typename T, int D, bool BWD>
 __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
   constexpr int KSTEP = D / 32, DT = D / 16;
-  __shared__ __attribute__((aligned(16))) uint16_t ks[2][FA_KT * D];
-  __shared__ __attribute__((aligned(16))) uint16_t vs[2][FA_KT * D];
-  const int nqb = gridDim.x;
-  const int qb = a.causal ? nqb - 1 - blockIdx.x : blockIdx.x;     // causal: heaviest blocks first
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int kvh = h / (a.Hq / a.Hkv);
+  constexpr uint32_t TILE_B = FA_KT * D * 2;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * TILE_B];     // K0, K1, V0, V1
+  int rank, hh, b;
+  ta_block(rank, hh, b);
+  const int qb = gridDim.x - 1 - rank;                             // causal: the last blocks are the heaviest
+  const int kvh = hh % a.Hkv, h = kvh * (a.Hq / a.Hkv) + hh / a.Hkv;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r16 = lane & 15;
   // the forward also takes ragged T (encoders, inference): rows >= T load
@@ -120,8 +163,8 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
   const uint16_t* vbase = a.v + (size_t)b * a.vsb + (size_t)kvh * a.vsh;
   const ta_rsrc rk = ta_make_rsrc(kbase, (uint32_t)(((int64_t)(a.T - 1) * a.kst + D) * 2));
   const ta_rsrc rv = ta_make_rsrc(vbase, (uint32_t)(((int64_t)(a.T - 1) * a.vst + D) * 2));
-  const uint32_t ks_l = ta_lds_addr(ks), vs_l = ta_lds_addr(vs);
-  constexpr uint32_t TILE_B = FA_KT * D * 2;
+  const uint32_t ks_l = ta_lds_addr(lds), vs_l = ks_l + 2 * TILE_B;
+  const FaFrag<D> fr(g, r16);
   auto stage = [&](int t, int buf) {
     ta_stage<D>(rk, ks_l + buf * TILE_B, t * FA_KT, a.kst, a.T, wave, lane);
     ta_stage<D>(rv, vs_l + buf * TILE_B, t * FA_KT, a.vst, a.T, wave, lane);
@@ -133,6 +176,10 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
   float mrow = -INFINITY, lpart = 0.f;
   constexpr float kLog2e = 1.4426950408889634f;
   const float sc2 = a.scale * kLog2e;
+  // p = exp2(st * mul - m) in one fma; the maximum is taken before the factor, so one that is not positive and
+  // normal goes on beforehand
+  const bool pre = !BWD && !(sc2 >= 1.17549435e-38f);
+  const float mul = pre ? 1.f : sc2;
 
   stage(0, 0);
   // the Q / dO fragments (and LSE / delta) are consumed here, so hipcc's own
@@ -150,8 +197,7 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
     const int buf = t & 1;
     if (t + 1 < ntile) stage(t + 1, buf ^ 1);   // buffer last read in iteration t - 1
     const int kt0 = t * FA_KT;
-    const uint16_t* kb_ = ks[buf];
-    const uint16_t* vb_ = vs[buf];
+    const uint32_t kt = buf * TILE_B, vt = kt + 2 * TILE_B;
     const bool full = (!a.causal || kt0 + FA_KT - 1 <= qb * FA_QB) && kt0 + FA_KT <= a.T;
 
     // ---- S^T = K Q^T (and dP^T = V dO^T): lane holds keys 16 kb + 4 g + i of query qrow
@@ -162,49 +208,48 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
       if constexpr (BWD) dp[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < KSTEP; s++) {
-        const uint4 kf = *(const uint4*)(kb_ + pf_off<D>(16 * kb + r16, 4 * s + g));
-        st[kb] = mfma16<T>(kf, qf[s], st[kb]);
-        if constexpr (BWD) {
-          const uint4 vf = *(const uint4*)(vb_ + pf_off<D>(16 * kb + r16, 4 * s + g));
-          dp[kb] = mfma16<T>(vf, df[s], dp[kb]);
-        }
+        st[kb] = mfma16<T>(fr.row(lds, kt, kb, s), qf[s], st[kb]);
+        if constexpr (BWD) dp[kb] = mfma16<T>(fr.row(lds, vt, kb, s), df[s], dp[kb]);
       }
     }
     uint32_t pk[4][2];                         // forward: P^T; backward: dS^T (16-bit pairs)
     if constexpr (!BWD) {
+      if (pre) {
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++)
+        for (int kb = 0; kb < 4; kb++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          float v = st[kb][i] * sc2;
-          const int key = kt0 + 16 * kb + 4 * g + i;
-          if (!full && ((a.causal && key > qrow) || key >= a.T)) v = -INFINITY;
-          st[kb][i] = v;
-        }
+          for (int i = 0; i < 4; i++) st[kb][i] *= sc2;
+      }
+      if (!full) {
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int key = kt0 + 16 * kb + 4 * g + i;
+            if ((a.causal && key > qrow) || key >= a.T) st[kb][i] = -INFINITY;
+          }
+      }
       float tmax = -INFINITY;
 #pragma unroll
       for (int kb = 0; kb < 4; kb++)
 #pragma unroll
         for (int i = 0; i < 4; i++) tmax = fmaxf(tmax, st[kb][i]);
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float mnew = fmaxf(mrow, tmax);
-      const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow - mnew);
-      const float msafe = mnew == -INFINITY ? 0.f : mnew;
-      mrow = mnew;
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+      tmax = ta_xmax(tmax) * mul;
+      if (__builtin_amdgcn_ballot_w64(tmax > mrow) != 0) {
+        const float mnew = fmaxf(mrow, tmax);
+        const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow - mnew);
+        mrow = mnew;
         lpart *= alpha;
 #pragma unroll
         for (int d = 0; d < DT; d++) { o[d][0] *= alpha; o[d][1] *= alpha; o[d][2] *= alpha; o[d][3] *= alpha; }
       }
+      const float msafe = mrow == -INFINITY ? 0.f : mrow;
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) {
         float p[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          p[i] = __builtin_amdgcn_exp2f(st[kb][i] - msafe);
-          lpart += p[i];
-        }
+        for (int i = 0; i < 4; i++) p[i] = __builtin_amdgcn_exp2f(fmaf(st[kb][i], mul, -msafe));
+        lpart += (p[0] + p[1]) + (p[2] + p[3]);
         pk[kb][0] = pack2<T>(p[0], p[1]);
         pk[kb][1] = pack2<T>(p[2], p[3]);
       }
@@ -215,7 +260,7 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
         float ds[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float p = __builtin_amdgcn_exp2f(st[kb][i] * sc2 - lse2);
+          float p = __builtin_amdgcn_exp2f(fmaf(st[kb][i], sc2, -lse2));
           if (!full && kt0 + 16 * kb + 4 * g + i > qrow) p = 0.f;
           ds[i] = p * (dp[kb][i] - delta);
         }
@@ -224,20 +269,11 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
       }
     }
     // ---- O^T += V^T P^T  /  dQ^T += K^T dS^T (two 32-key steps)
-    const uint16_t* tb = BWD ? kb_ : vb_;
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
-      const int qq = r16 >> 2, pp = r16 & 3;
-      const int row0 = 16 * (2 * kk) + 4 * g + qq, row1 = row0 + 16;
+      const uint4 pb = make_uint4(pk[2 * kk][0], pk[2 * kk][1], pk[2 * kk + 1][0], pk[2 * kk + 1][1]);
 #pragma unroll
-      for (int d = 0; d < DT; d++) {
-        const int col = 16 * d + 4 * pp;
-        const uint2 v0 = ds_read_tr16(tb + pf_off<D>(row0, col >> 3) + (col & 7));
-        const uint2 v1 = ds_read_tr16(tb + pf_off<D>(row1, col >> 3) + (col & 7));
-        const uint4 va = make_uint4(v0.x, v0.y, v1.x, v1.y);
-        const uint4 pb = make_uint4(pk[2 * kk][0], pk[2 * kk][1], pk[2 * kk + 1][0], pk[2 * kk + 1][1]);
-        o[d] = mfma16<T>(va, pb, o[d]);
-      }
+      for (int d = 0; d < DT; d++) o[d] = mfma16<T>(fr.col(lds, BWD ? kt : vt, kk, d), pb, o[d]);
     }
     ta_wait_vm0();                               // tile t + 1 landed (this wave's pieces)
     __syncthreads();
@@ -270,17 +306,15 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
 template <typename T, int D>
 __global__ void __launch_bounds__(256) fa_dkdv_kernel(const TrainAttnArgs a) {
   constexpr int KSTEP = D / 32, DT = D / 16;
-  __shared__ __attribute__((aligned(16))) uint16_t qs[2][FA_QB * D];
-  __shared__ __attribute__((aligned(16))) uint16_t os[2][FA_QB * D];   // dO tile
+  constexpr uint32_t TILE_B = FA_QB * D * 2;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * TILE_B];     // Q0, Q1, dO0, dO1
   __shared__ float ls[2][2 * FA_QB];                                   // LSE2, delta of the tile's rows
-  const int nkb = gridDim.x;
-  const int kb = blockIdx.x;                                           // key block (light ones last: causal)
-  const int kvh = blockIdx.y, b = blockIdx.z;
+  int kb, kvh, b;                                                      // key block (causal: the first ones are the heaviest)
+  ta_block(kb, kvh, b);
   const int G = a.Hq / a.Hkv;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r16 = lane & 15;
   const int key = kb * FA_KT + wave * 16 + r16;                        // this lane's key (B operand column)
-  (void)nkb;
   // K / V fragments: B operands of S = Q K^T and dP = dO V^T
   uint4 kf[KSTEP], vf[KSTEP];
   {
@@ -296,8 +330,8 @@ __global__ void __launch_bounds__(256) fa_dkdv_kernel(const TrainAttnArgs a) {
   const int nqb = a.T / FA_QB - qb0;
   const int nwork = G * nqb;                                           // (head, query block) pairs
   float lreg = 0.f;
-  const uint32_t qs_l = ta_lds_addr(qs), os_l = ta_lds_addr(os);
-  constexpr uint32_t TILE_B = FA_QB * D * 2;
+  const uint32_t qs_l = ta_lds_addr(lds), os_l = qs_l + 2 * TILE_B;
+  const FaFrag<D> fr(g, r16);
   auto load_tile = [&](int w, int buf) {
     const int hh = kvh * G + w / nqb, qb = qb0 + w % nqb;
     const uint16_t* qp = a.q + (size_t)b * a.qsb + (size_t)hh * a.qsh;
@@ -332,8 +366,7 @@ __global__ void __launch_bounds__(256) fa_dkdv_kernel(const TrainAttnArgs a) {
     if (w + 1 < nwork) load_tile(w + 1, buf ^ 1);
     const int qb = qb0 + w % nqb;
     const bool diag = a.causal && qb == kb;
-    const uint16_t* qb_ = qs[buf];
-    const uint16_t* ob_ = os[buf];
+    const uint32_t qt_ = buf * TILE_B, ot_ = qt_ + 2 * TILE_B;
     // ---- S = Q K^T, dP = dO V^T: lane holds query rows 16 qt + 4 g + i for key `key`
     uint32_t pk[4][2], dk16[4][2];
 #pragma unroll
@@ -341,16 +374,14 @@ __global__ void __launch_bounds__(256) fa_dkdv_kernel(const TrainAttnArgs a) {
       f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, p = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ss = 0; ss < KSTEP; ss++) {
-        const uint4 qa = *(const uint4*)(qb_ + pf_off<D>(16 * qt + r16, 4 * ss + g));
-        const uint4 oa = *(const uint4*)(ob_ + pf_off<D>(16 * qt + r16, 4 * ss + g));
-        s = mfma16<T>(qa, kf[ss], s);
-        p = mfma16<T>(oa, vf[ss], p);
+        s = mfma16<T>(fr.row(lds, qt_, qt, ss), kf[ss], s);
+        p = mfma16<T>(fr.row(lds, ot_, qt, ss), vf[ss], p);
       }
       float pv[4], dsv[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int qr = 16 * qt + 4 * g + i;                           // row within the tile
-        float pr = __builtin_amdgcn_exp2f(s[i] * sc2 - ls[buf][qr]);
+        float pr = __builtin_amdgcn_exp2f(fmaf(s[i], sc2, -ls[buf][qr]));
         if (diag && wave * 16 + r16 > qr) pr = 0.f;                    // key > query (same block offsets)
         pv[i] = pr;
         dsv[i] = pr * (p[i] - ls[buf][FA_QB + qr]);
@@ -363,19 +394,12 @@ __global__ void __launch_bounds__(256) fa_dkdv_kernel(const TrainAttnArgs a) {
     // ---- dV += P^T dO, dK += dS^T Q over two 32-row query steps
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
-      const int qq = r16 >> 2, pp = r16 & 3;
-      const int row0 = 16 * (2 * kk) + 4 * g + qq, row1 = row0 + 16;
       const uint4 pa = make_uint4(pk[2 * kk][0], pk[2 * kk][1], pk[2 * kk + 1][0], pk[2 * kk + 1][1]);
       const uint4 da = make_uint4(dk16[2 * kk][0], dk16[2 * kk][1], dk16[2 * kk + 1][0], dk16[2 * kk + 1][1]);
 #pragma unroll
       for (int d = 0; d < DT; d++) {
-        const int col = 16 * d + 4 * pp;
-        const uint2 o0 = ds_read_tr16(ob_ + pf_off<D>(row0, col >> 3) + (col & 7));
-        const uint2 o1 = ds_read_tr16(ob_ + pf_off<D>(row1, col >> 3) + (col & 7));
-        const uint2 q0 = ds_read_tr16(qb_ + pf_off<D>(row0, col >> 3) + (col & 7));
-        const uint2 q1 = ds_read_tr16(qb_ + pf_off<D>(row1, col >> 3) + (col & 7));
-        dv[d] = mfma16<T>(pa, make_uint4(o0.x, o0.y, o1.x, o1.y), dv[d]);
-        dk[d] = mfma16<T>(da, make_uint4(q0.x, q0.y, q1.x, q1.y), dk[d]);
+        dv[d] = mfma16<T>(pa, fr.col(lds, ot_, kk, d), dv[d]);
+        dk[d] = mfma16<T>(da, fr.col(lds, qt_, kk, d), dk[d]);
       }
     }
     ta_wait_vm0();                               // Q / dO tiles and the LSE / delta row of w + 1
