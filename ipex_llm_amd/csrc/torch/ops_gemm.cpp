@@ -123,6 +123,40 @@ Tensor gemm_bf16(const Tensor& x, const Tensor& w, const c10::optional<Tensor>& 
   return out_opt.has_value() ? out : out.view(shape);
 }
 
+// the automatic split-K factor, and the product as that many f32 slabs [S, M, N] (S >= 2) for a consumer that sums them
+int64_t gemm_bf16_split(int64_t M, int64_t N, int64_t K) { return M > 0 && N > 0 ? g8_auto_split(M, N, K) : 1; }
+
+Tensor gemm_bf16_slabs(const Tensor& x, const Tensor& w) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
+                  x.dim() == 2 && w.dim() == 2 && w.stride(1) == 1 && w.stride(0) % 8 == 0,
+              "gemm_bf16_slabs: bf16 GPU x [M, K], w [N, K] of whole 16-byte rows");
+  const int64_t M = x.size(0), K = w.size(1), N = w.size(0);
+  TORCH_CHECK(x.size(1) == K && K % 64 == 0 && K > 0, "gemm_bf16_slabs: K must match and be a multiple of 64");
+  const int64_t S = gemm_bf16_split(M, N, K);
+  TORCH_CHECK(S > 1, "gemm_bf16_slabs: a product that is not split");
+  c10::DeviceGuard g(x.device());
+  Tensor x2 = x.stride(1) != 1 || x.stride(0) % 8 != 0 ? x.contiguous() : x;
+  const int64_t xb = (M - 1) * x2.stride(0) * 2 + K * 2, wb = (N - 1) * w.stride(0) * 2 + K * 2;
+  TORCH_CHECK(xb < (int64_t)UINT32_MAX && wb < (int64_t)UINT32_MAX, "gemm_bf16_slabs: operands over 4 GiB");
+  Tensor ws = at::empty({S, M, N}, x.options().dtype(at::kFloat));
+  illm::G8Args a{};
+  a.x = (const uint16_t*)x2.data_ptr();
+  a.w = (const uint16_t*)w.data_ptr();
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.ldx = (int)x2.stride(0);
+  a.ldw = (int)w.stride(0);
+  a.ldo = (int)N;
+  a.x_bytes = (uint32_t)xb;
+  a.w_bytes = (uint32_t)wb;
+  a.w_fmt = -1;
+  a.ksplit = (int)S;
+  a.ws = ws.data_ptr<float>();
+  illm::launch_gemm8p(a, cur_stream());
+  return ws;
+}
+
 // low-bit weights (tiled device blob, sym_int4 / nf4 / nf3) decoded to bf16
 // in LDS inside the same 8-phase GEMM: y = x @ dequant(W)^T (+ bias)
 Tensor gemm8p_lowbit(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
@@ -173,11 +207,14 @@ Tensor gemm8p_lowbit(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("x_to_f16_rowscale(Tensor x) -> Tensor[]");
   m.def("gemm_bf16(Tensor x, Tensor w, Tensor? bias=None, bool out_f32=False, int kernel=0, bool glu=False, int act=0, int ksplit=-1, Tensor(a!)? out=None, bool accumulate=False) -> Tensor");
+  m.def("gemm_bf16_split(int m, int n, int k) -> int", &gemm_bf16_split);
+  m.def("gemm_bf16_slabs(Tensor x, Tensor w) -> Tensor");
   m.def("gemm8p_lowbit(Tensor x, Tensor blob, int fmt, int n, int k, Tensor? bias=None, bool out_f32=False, bool glu=False, int act=0) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("x_to_f16_rowscale", &x_to_f16_rowscale);
   m.impl("gemm_bf16", &gemm_bf16);
+  m.impl("gemm_bf16_slabs", &gemm_bf16_slabs);
   m.impl("gemm8p_lowbit", &gemm8p_lowbit);
 }

@@ -394,6 +394,13 @@ Tensor gemm_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, in
   return lowbit_rows(x, blob, fmt, n, k, bias, glu ? illm::EPI_GLU : illm::EPI_STORE, glu ? 1 : 0, act, 1 << 16, fine);
 }
 
+// ... as f32 slabs [S, M, n] for a consumer that sums them
+Tensor gemm_rows_slabs(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, bool fine) {
+  TORCH_CHECK(!fine || (is_bf16(x) && x.numel() > 64 * k && illm::fmt_to_dk((int)fmt) == illm::DK_LUT4),
+              "gemm_rows_slabs: the finer table serves table formats, bf16 and 65 rows and up");
+  return lowbit_rows(x, blob, fmt, n, k, c10::nullopt, illm::EPI_PARTIAL, 0, 0, 1 << 16, fine);
+}
+
 // greedy decode head: the v5 GEMV stores the logits (T) and every wave writes
 // the argmax {max, index} of its columns per row (parts [nparts, M, 2] f32),
 // which decode_advance reduces instead of re-reading the [M, V] logits.
@@ -1884,6 +1891,7 @@ TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("dequantize_device", &dequantize_device);
   m.impl("gemv", &gemv);
   m.impl("gemm_rows", &gemm_rows);
+  m.impl("gemm_rows_slabs", &gemm_rows_slabs);
   m.impl("gemv_accum", &gemv_accum);
   m.impl("gemv_accum_norm", &gemv_accum_norm);
   m.impl("gemv_glu_ss", &gemv_glu_ss);

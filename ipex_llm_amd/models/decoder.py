@@ -501,6 +501,15 @@ class NativeCausalLM(nn.Module):
             out, _ = ops.add_rms_norm(None, residual, norm_w, s.rms_eps, partials=part,
                                       unit_offset=s.norm_unit_offset)
             return out
+        part = None
+        if (type(proj) is LowBitLinear and proj.bias is None and proj.g_idx_map is None and post_norm_w is None
+                and self.tp_group is None and proj.mp_group is None and x.dim() == 2 and x.dtype == residual.dtype
+                and ops.native_gpu(x) and not (proj._forward_hooks or proj._forward_pre_hooks)):
+            from ..ops.gemm import lowbit_slabs
+            part = lowbit_slabs(x, proj.weight, proj.fmt, proj.out_features, proj.in_features)
+        if part is not None:
+            out, _ = ops.add_rms_norm(None, residual, norm_w, s.rms_eps, partials=part, unit_offset=s.norm_unit_offset)
+            return out
         y = proj(x)
         if self.tp_group is not None and not getattr(proj, "mp_group", None):
             from ..parallel.comm import all_reduce_inplace

@@ -35,6 +35,16 @@ def _(x, blob, fmt, n, k, bias, glu, act, fine=False):
     return x.new_empty(shape)
 
 
+@register_fake("ipex_llm_amd::gemm_rows_slabs")
+def _(x, blob, fmt, n, k, fine=False):
+    return x.new_empty((1, x.numel() // k, n), dtype=torch.float32)
+
+
+@register_fake("ipex_llm_amd::gemm_bf16_slabs")
+def _(x, w):
+    return x.new_empty((2, x.shape[0], w.shape[0]), dtype=torch.float32)
+
+
 @register_fake("ipex_llm_amd::add_rms_norm")
 def _(x, partials, residual, w, eps, unit_offset, store_residual, zero_partials=False):
     if x is not None:

@@ -437,6 +437,29 @@ def lowbit_gemm(x, blob, fmt, n, k, bias=None):
     return F.linear(x, w, bias)
 
 
+def lowbit_slabs(x, blob, fmt, n, k):
+    """x @ W^T of more rows than the decode kernels take as the f32 slabs [S, M, n]
+    of a split K for :func:`add_rms_norm` to sum -- it rounds the sum as the pass
+    over the slabs that this saves does, so with the same bits --, or None where
+    :func:`lowbit_gemm` takes a dense product that it does not split.  Pass and
+    norm / norm alone, us: fp8_e5m2 [3584, 18944] of 300 rows 10.1 / 5.9, the dense
+    [4096, 14336] of 1024 rows 22.5 / 16.2."""
+    ops = torch.ops.ipex_llm_amd
+    M = x.numel() // k
+    if torch.is_grad_enabled() and x.requires_grad:
+        return None
+    if use_rows(x, M, n, k, fmt):
+        return ops.gemm_rows_slabs(x, blob, fmt, n, k, rows_fine(x.dtype, M, n, k, fmt))
+    if use_g8(x, M, n, k, fmt) or not use_g8d(x, M, n, k) or ops.gemm_bf16_split(M, n, k) < 2:
+        return None
+
+    def dw():
+        return _dense_weight(blob, fmt, n, k, x.dtype)
+    if _pick((M, n, k, False, 0), lambda: ops.gemm_bf16(x, dw()), lambda: F.linear(x, dw())) == "lib":
+        return None
+    return ops.gemm_bf16_slabs(x, dw())
+
+
 def lowbit_gemm_glu(x, blob, fmt, n, k, act: int = 0):
     """act(x @ Wg^T) * (x @ Wu^T) for a tile-interleaved gate/up weight at
     prefill M: the fused kernel applies the activation in its epilogue (no
