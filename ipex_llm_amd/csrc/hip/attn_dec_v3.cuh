@@ -589,7 +589,8 @@ __global__ void __launch_bounds__(64 * NW, ILLM_V3_MINW(RQ)) attn_decode_v3_kern
 // tile's K requested behind the scores and its V behind the LDS rows of this
 // one, no barrier until the waves merge at the end.  168 registers: 3
 // workgroups = 12 waves x 16 KB in flight per CU.
-// That case: 74 -> 55 us (3.3 TB/s).
+// That case: 74 -> 55 us (3.3 TB/s); with the first block id read beside the length and the first tile requested ahead
+// of q (which also took the spills away), 51 -> 45 on the card that timed these (4.1 TB/s).
 constexpr int V3L_NW = 4;
 
 template <typename T, int D, int RQ, bool FUSE>
@@ -611,6 +612,7 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
 
   int len = a.seq_lens[b];
   auto entry = [&](int k) { return a.block_tables[(size_t)b * a.max_blocks + min(k / a.bs, a.max_blocks - 1)]; };
+  int blk_next = entry(kw);                      // with the length, not behind it
   const int row = r16 < R ? r16 : 0;
   const int t = row / group, h = kvh * group + row % group;
   if ((int64_t)len > (int64_t)a.max_blocks * a.bs || (int64_t)a.nsplit * SPLIT < len) {
@@ -625,6 +627,47 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
       else *(float2*)(a.part_ml + prow * 2) = make_float2(-INFINITY, 0.f);
     }
   } else {
+    // ---- a tile's loads: rows past the sequence (or a bad block) read the tile's
+    // last valid row (block 0) and are masked by nvis
+    uint4 kf[2][KSTEP], vm[VJ];
+    int nvis = 0;
+    size_t base = 0;
+    int last = 0;
+    auto tile_at = [&](int blk) {
+      const int nkw = kw < len ? min(V3_KPW, len - kw) : 0;
+      const bool bad = nkw > 0 && bad_block(blk, a.num_blocks);
+      if (bad && lane == 0) kerr(a.err, ERR_BLOCK_ID);
+      nvis = bad ? 0 : nkw;
+      last = max(nvis, 1) - 1;
+      base = nvis > 0 ? (((size_t)blk * a.Hkv + kvh) * a.bs + kw % a.bs) * D : 0;
+    };
+    auto load_k = [&]() {
+      const uint16_t* kb = (const uint16_t*)a.k_cache + base;
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int s = 0; s < KSTEP; s++)
+          kf[kt][s] = *(const uint4*)(kb + (uint32_t)(min(kt * 16 + r16, last) * D + 32 * s + 8 * g));
+    };
+    auto load_v = [&]() {
+      const uint16_t* vb = (const uint16_t*)a.v_cache + base;
+#pragma unroll
+      for (int j = 0; j < VJ; j++)
+        vm[j] = *(const uint4*)(vb + (uint32_t)(min(j * KPJ + lane / VU, last) * D + 8 * (lane % VU)));
+    };
+
+    // tiles of this wave that hold keys (the first one runs in any case: fully masked if it holds none)
+    const int nt = max(1, (len - kw + step - 1) / step);
+    // the first tile is requested before q, whose columns are then a round trip beside it, not ahead of it; not where
+    // the new token's rows are appended to it first, nor beside the registers of the rotation
+    const bool appends = RQ != 0 && (len - 1) / SK % (int)gridDim.x == split && (len - 1) % SK / V3_KPW == wv;
+    const bool early = RQ != 1 && !(appends && nt == 1);          // wave-uniform
+    if (early) {
+      tile_at(blk_next);
+      load_k();
+      load_v();
+    }
+
     // ---- q fragments (lane: row r16, dims 32 s + 8 g .. + 8)
     uint4 qf[KSTEP];
     if constexpr (RQ != 0) {
@@ -638,7 +681,7 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
       rp.frags(h * D, v, cs, a.rq_qscale, qf);
       // the new token's k / v rows, appended by the wave whose tiles hold
       // position len - 1 before it reads them (its own stores: in order)
-      if ((len - 1) / SK % (int)gridDim.x == split && (len - 1) % SK / V3_KPW == wv) {
+      if (appends) {
         const int pos = len - 1, blk = entry(pos);
         if (!bad_block(blk, a.num_blocks)) {
           const size_t crow = (((size_t)blk * a.Hkv + kvh) * a.bs + pos % a.bs) * D;
@@ -670,35 +713,12 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
 #pragma unroll
       for (int s = 0; s < KSTEP; s++) qf[s] = make_uint4(0, 0, 0, 0);
 
-    // ---- a tile's loads: rows past the sequence (or a bad block) read the tile's
-    // last valid row (block 0) and are masked by nvis
-    uint4 kf[2][KSTEP], vm[VJ];
-    int nvis = 0;
-    size_t base = 0;
-    int last = 0;
-    auto tile_at = [&](int blk) {
-      const int nkw = kw < len ? min(V3_KPW, len - kw) : 0;
-      const bool bad = nkw > 0 && bad_block(blk, a.num_blocks);
-      if (bad && lane == 0) kerr(a.err, ERR_BLOCK_ID);
-      nvis = bad ? 0 : nkw;
-      last = max(nvis, 1) - 1;
-      base = nvis > 0 ? (((size_t)blk * a.Hkv + kvh) * a.bs + kw % a.bs) * D : 0;
-    };
-    auto load_k = [&]() {
-      const uint16_t* kb = (const uint16_t*)a.k_cache + base;
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-        for (int s = 0; s < KSTEP; s++)
-          kf[kt][s] = *(const uint4*)(kb + (uint32_t)(min(kt * 16 + r16, last) * D + 32 * s + 8 * g));
-    };
-    auto load_v = [&]() {
-      const uint16_t* vb = (const uint16_t*)a.v_cache + base;
-#pragma unroll
-      for (int j = 0; j < VJ; j++)
-        vm[j] = *(const uint4*)(vb + (uint32_t)(min(j * KPJ + lane / VU, last) * D + 8 * (lane % VU)));
-    };
-
+    if (!early) {
+      tile_at(blk_next);
+      load_k();
+      load_v();
+    }
+    blk_next = entry(kw + step);
     const int qpos = len - a.Tq + t;
     const int win = a.sliding_window > 0 ? qpos - a.sliding_window : -1;
     const int win0 = a.sliding_window > 0 ? len - a.Tq - a.sliding_window : -1;   // keys up to here: no row sees them
@@ -707,13 +727,6 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
     f32x4 o[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // tiles of this wave that hold keys (the first one runs in any case: fully masked if it holds none)
-    const int nt = max(1, (len - kw + step - 1) / step);
-
-    tile_at(entry(kw));
-    load_k();
-    load_v();
-    int blk_next = entry(kw + step);
     for (int it = 0; it < nt; it++) {
       // ---- S^T tiles: lane holds (key = 16 kt + 4 g + i, row = r16)
       f32x4 st[2];
