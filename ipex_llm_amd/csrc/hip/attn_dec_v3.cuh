@@ -29,7 +29,7 @@
 // Row r of the P V MFMA depends only on row r of P, and each split's
 // reductions run in a fixed key order: a multi-row verify (speculative decoding)
 // reduces every row exactly like one-token decoding with the same NW, as long as
-// both take q from memory (fused RoPE of long contexts: v3_long_grid).
+// both take q from memory; the kernel with several tiles per wave, too (v3_long_grid: which batches run it).
 #pragma once
 
 namespace illm {
@@ -908,25 +908,37 @@ static void launch_v3_nw(const AttnDecodeArgs& a, hipStream_t st) {
   }
 }
 
-// workgroups per (sequence, kv head) of the long-context kernel (0: one tile per wave, the kernel above).  Fused-
-// RoPE decode only: with q from memory two 8-wave workgroups of the kernel above share a CU (108 - 118 registers)
-// and it is as fast or faster below some 8 K keys (4 x 4000 18 us, this 21), so a one-token step of a model with
-// dense projections and a multi-row verify keep one kernel and one order of reduction; a verify of a low-bit model
-// reduces in another order than its fused step, whose q, k and v are sums of f32 atomics in no fixed order anyway.
+// workgroups per (sequence, kv head) of the kernel with several tiles per wave (0: one tile per wave, the kernel above).
 //
-// For sequences of the grid's full length: the CU with the most workgroups has n = ceil(workgroups / 256) of them,
-// each t tiles and about 0.7 tiles' time to start and merge, and where the lengths differ the longest workgroup ends
-// the launch (0.2 t); t from 2 to 8 with the least n (t + 0.7) + 0.2 t.  Attention of Llama-3-8B heads, sequences of
-// half to all of these keys, one tile per wave / t 2 .. 8 (us), the chosen one marked: 4 x 4000 24.8 / 22.5 25.5
-// [22.5] 23.4 25.3 27.2 28.7; 8 x 6000 56.3 / 48.9 46.3 41.9 45.4 [40.4] 42.8 45.6; 16 x 3500 62.7 / 52.2 53.6 48.5
-// 49.8 53.3 [46.7] 49.0; 1 x 16000 36.8 / 30.1 29.9 [24.3] 25.7 27.3 28.9 29.0; 3 x 20000 77.7 / 68.6 64.0 61.8
-// [53.9] 57.9 62.3 54.5.  Not below 48 splits (8 x 2000: layer 69.8 -> 70.8), nor for few workgroups just above
-// (4 x 3200 19.2 / 20.8).  (ILLM_ATTN_V3_TILES=t forces t; a function of batch, kv heads and split grid only.)
+// q from memory (a batch past the fused RoPE, dense projections, a multi-row verify: one rule by batch, kv heads and
+// split grid, so a one-token step and a verify of the same batch keep one kernel and one order of reduction): from 256
+// pairs of sequence and kv head on as many as make 768, which are resident at once (three per CU), where the kernel
+// above needs rounds.  Sequences of half to all of the keys, 32 / 8 heads, one tile per wave / this, us: 48 x 700 32.2 /
+// 30.8, 48 x 400 23.9 / 21.2, 48 x 1200 48.0 / 47.1, 64 x 300 26.7 / 20.8, 56 x 800 47.6 / 39.4, 64 x 900 54.6 / 46.1,
+// 128 x 200 44.0 / 30.5, 36 x 300 19.8 / 16.2, 32 x 768 30.0 / 25.0, 32 x 1800 53.9 / 45.7, but 40 x 1500 48.2 / 48.8 (two
+// and a half per CU); 28 / 4 heads 96 x 300 22.6 / 19.1, 32 / 32 heads 64 x 500 98.6 / 90.5.  Not below: 24 x 512 15.5 /
+// 16.5, 24 x 1024 25.5 / 25.8, 28 / 4 heads 48 x 700 20.0 / 20.7; nor where a workgroup has one tile or the grid two: 64 x
+// 128 13.5 / 14.2, 32 x 100 10.4 / 11.9, 28 / 4 heads 64 x 300 14.7 / 15.6.
+//
+// Fused-RoPE decode, 48 splits and more, for sequences of the grid's full length: the CU with the most workgroups has
+// n = ceil(workgroups / 256) of them, each t tiles and about 0.7 tiles' time to start and merge, and where the lengths
+// differ the longest workgroup ends the launch (0.2 t); t from 2 to 8 with the least n (t + 0.7) + 0.2 t.  Attention of
+// 32 / 8 heads, sequences of half to all of these keys, one tile per wave / t 2 .. 8 (us), the chosen one marked:
+// 4 x 4000 24.6 / 19.0 21.2 [19.9] 20.8 21.2 22.7 24.4; 8 x 6000 48.3 / 39.8 39.1 35.8 37.1 [34.9] 36.6 39.1; 16 x 3500
+// 47.8 / 41.5 40.4 40.1 38.1 41.3 [38.7] 38.9; 1 x 16000 30.9 / 22.0 19.8 [17.9] 17.7 18.5 19.8 18.2; 3 x 20000 72.5 /
+// 52.7 46.6 45.4 [41.0] 41.9 45.4 41.1.  Not below 48 splits (8 x 2000: layer 69.8 -> 70.8), nor for few workgroups just
+// above (4 x 3200 19.2 / 20.8).  (ILLM_ATTN_V3_TILES=t forces t; a function of batch, kv heads and split grid only.)
 inline int v3_long_grid(const AttnDecodeArgs& a, int rq) {
   static const int env = getenv("ILLM_ATTN_V3_TILES") ? atoi(getenv("ILLM_ATTN_V3_TILES")) : -1;
   const long all = (a.nsplit * SPLIT + V3_KPW * V3L_NW - 1) / (V3_KPW * V3L_NW);
   if (env >= 0) return env == 0 ? 0 : (int)((all + env - 1) / env);
-  if (rq == 0 || a.nsplit < 48 || (a.nsplit < 56 && (long)a.B * a.Hkv * all < 1024)) return 0;
+  if (rq == 0) {
+    const long pairs = (long)a.B * a.Hkv;
+    if (pairs < 256) return 0;
+    const long s = pairs < 768 ? 768 / pairs : 1;
+    return all >= 3 && all > s ? (int)s : 0;
+  }
+  if (a.nsplit < 48 || (a.nsplit < 56 && (long)a.B * a.Hkv * all < 1024)) return 0;
   long best = 0, cost = 0;
   for (long t = 2; t <= 8; t++) {
     const long s = (all + t - 1) / t, c = ((long)a.B * a.Hkv * s + 255) / 256 * (10 * t + 7) + 2 * t;
