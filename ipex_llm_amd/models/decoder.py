@@ -346,7 +346,8 @@ class NativeCausalLM(nn.Module):
             # every query row is reduced exactly as in one-token decoding
             # (greedy speculative output == plain greedy output; the fused step
             # of a low-bit model sums q, k and v in no fixed order, and from
-            # some 3 K keys on runs a kernel of its own, v3_long_grid)
+            # some 3 K keys, or its verify from 256 pairs of sequence and kv
+            # head on, runs another kernel, v3_long_grid)
             c = 16 // group
             qv = q.view(meta.B, meta.Tq, s.num_heads, s.head_dim)
             outs = []
