@@ -271,6 +271,15 @@ Tensor rows16(const Tensor& x) {
   return ((uintptr_t)c.data_ptr() & 15) != 0 ? c.clone() : c;
 }
 
+// The head (32000 columns and up) of 1 to 16 rows on the skinny kernel, whichever of its entries is called: by format and
+// shape alone, so that a sequence's logits do not change with the sequences beside it, and only where no number of rows is
+// slower for it.  v5 / this, us at 1 / 2 / 4 / 8 / 16 rows, weights that no cache holds: asym_int4 [128256, 4096] 60.3 61.0
+// 67.1 76.9 95.9 / 56.7 57.1 57.1 58.0 59.5, [152064, 3584] 63.1 66.1 74.3 78.8 97.5 / 63.1 62.7 62.8 62.1 65.1, [32000,
+// 4096] 17.8 18.5 18.6 20.7 25.8 / 18.0 18.0 18.1 18.1 18.3; K of 3072 19.5 / 20.6 at one row.  The others pay for their
+// few rows: [128256, 4096] sym_int4 51.5 52.0 72.6 93.3 / 56.8 54.5 55.2 57.0 at 1 / 4 / 8 / 16, fp4 51.1 57.6 63.7 75.8 /
+// 55.6 55.3 54.4 56.0, fp8_e5m2 87.2 90.5 99.2 112.1 / 94.9 92.3 94.3 95.2.
+bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4 && KC >= 28 && NT >= 2000; }
+
 // Up to 16 rows, input and output in memory: the skinny kernel's one row tile instead of v5, by the format and the
 // shape, so that a row keeps its bits beside any other rows (1 to 16).  Not table formats under bf16 (v5 keeps an f16
 // table, the skinny kernel one in the type of x).
@@ -283,12 +292,22 @@ Tensor rows16(const Tensor& x) {
 //     5.7, [2048, 2048] 4.7 5.1 5.3 5.7 and 4.1 4.3 4.3 4.3.  Longer K and wider outputs stay where v5 is ahead at few
 //     rows ([4096, 14336] 8.8 8.7 9.2 10.3 and 9.9 9.9 9.9 10.1, [12288, 4096] 8.4 9.4 10.3 12.5 and 12.4 12.1 12.1 12.2);
 //   * ... and where v5 would cut K by the number of rows, as its x does not fit the LDS: [3584, 18944] at 16 rows 15.4
-//     and 11.2, [8192, 28672] 35.6 and 26.2, the head [128256, 4096] at 8 rows 129.7 and 54.6.
+//     and 11.2, [8192, 28672] 35.6 and 26.2, the head [128256, 4096] at 8 rows 129.7 and 54.6 (these rows' bits change
+//     with the number of rows on either path);
+//   * ... and the heads of head16.
 bool skinny16(int fmt, bool bf16, int64_t M, int64_t NT, int64_t KC, int64_t epi, int64_t ksplit) {
   if (bf16 && illm::fmt_to_dk(fmt) == illm::DK_LUT4) return false;
   if (epi == illm::EPI_GLU) return KC < 64 || illm::fmt_bits(fmt) == 4;
   if (KC <= 40 && NT <= 512) return true;
+  if (head16(fmt, NT, KC)) return true;
   return ksplit <= 0 && plan5(M, NT, KC, true, 0, false, fmt).ks != plan5(1, NT, KC, true, 0, false, fmt).ks;
+}
+
+// whether the skinny kernel takes a product of up to 16 rows (what the tests of the rule ask for)
+bool skinny_takes(int64_t M, int64_t n, int64_t k, int64_t fmt, bool glu, bool bf16, int64_t ksplit) {
+  TORCH_CHECK(M >= 1 && M <= 16 && n >= 1 && k >= 1, "skinny_takes: 1..16 rows");
+  return skinny16((int)fmt, bf16, M, illm::pad_to(n, illm::TILE_N) / illm::TILE_N, illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K,
+                  glu ? illm::EPI_GLU : illm::EPI_STORE, ksplit);
 }
 
 // rows 1 .. most: v5 up to 16 rows (ILLM_GEMV_V1=1: the many-row kernels for these too, A/B tests), the
@@ -401,10 +420,10 @@ Tensor gemm_rows_slabs(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t
   return lowbit_rows(x, blob, fmt, n, k, c10::nullopt, illm::EPI_PARTIAL, 0, 0, 1 << 16, fine);
 }
 
-// greedy decode head: the v5 GEMV stores the logits (T) and every wave writes
-// the argmax {max, index} of its columns per row (parts [nparts, M, 2] f32),
-// which decode_advance reduces instead of re-reading the [M, V] logits.
-// Split-K 1 (the stored values are final); M <= 16.
+// greedy decode head: the product (v5, or the skinny kernel where head16 says so) stores the
+// logits (T) and writes the argmax {max, index} of every 16-column tile per row (parts [nparts,
+// M, 2] f32), which decode_advance reduces instead of re-reading the [M, V] logits.
+// Split-K 1 (the stored values are final); M <= 16, a K whose rows fit v5's LDS for either kernel.
 std::tuple<Tensor, Tensor> gemv_argmax(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
                                        const c10::optional<Tensor>& bias) {
   TORCH_CHECK(x.is_cuda() && blob.is_cuda() && x.size(-1) == k, "gemv_argmax: GPU x [M, k]");
@@ -445,10 +464,7 @@ std::tuple<Tensor, Tensor> gemv_argmax(const Tensor& x, const Tensor& blob, int6
   TORCH_CHECK((int64_t)p.gx * tg >= nparts, "gemv_argmax: geometry");
   Tensor parts = at::empty({nparts, M, 2}, xc.options().dtype(at::kFloat));
   a.amax = (float2*)parts.data_ptr<float>();
-  // from 6 rows on v5's x (full K, one workgroup per CU then) holds the stream up: [128256, 4096] sym_int4 at 1 / 5 / 8 /
-  // 16 rows 53 / 55 / 76 / 99 us, the skinny kernel's one row tile 54 / 55 / 55 / 57; [152064, 3584] fp8_e5m2 94 / 104 /
-  // 109 / 126 and 101 / 103 / 104 / 107
-  if (M >= 6 && !(bf16 && illm::fmt_to_dk((int)fmt) == illm::DK_LUT4)) {
+  if (head16((int)fmt, NT, KC)) {
     launch_skinny_any((int)fmt, bf16, skinny_plan((int)fmt, false, M, NT, KC, true, 1), illm::EPI_STORE, a);
     return {out, parts};
   }
@@ -1872,6 +1888,7 @@ int* illm_kernel_err(const c10::Device& dev) { return kernel_err(dev); }
 
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("skinny_geometry(int M, int n, int k, int fmt, bool glu, int ksplit, bool fine=False) -> int[]", &skinny_geometry);
+  m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
 }
 
 TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {

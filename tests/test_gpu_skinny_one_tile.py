@@ -114,6 +114,28 @@ def test_x_that_starts_anywhere(cuda, at):
             assert torch.equal(y, want), (M, epi)
 
 
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "nf4", "fp8_e5m2"])
+@pytest.mark.parametrize("n,k", [(32000, 3584), (32016, 4096), (1008, 4096)])
+def test_a_heads_rows_do_not_see_each_other(cuda, name, n, k):
+    """one kernel for 1 to 16 rows: the logits and tile maxima of a row are the same bits beside any other rows, and
+    those of the plain product where the skinny kernel takes the head"""
+    f = get_format(name).fmt
+    torch.manual_seed(6)
+    blob = ops.quantize(torch.randn(n, k, device=cuda) * 0.05, f)
+    x = torch.randn(16, k, device=cuda).bfloat16()
+    one, parts = torch.ops.ipex_llm_amd.gemv_argmax(x[:1], blob, f, n, k, None)
+    assert _rel(one, x[:1].double() @ R.dequantize_device_blob(blob, f, n, k).to(cuda).double().t()) < 2 * STORE
+    tiles = torch.nn.functional.pad(one.float(), (0, -n % 16), value=float("-inf")).view(-1, 16)
+    assert torch.equal(parts[:, 0, 0], tiles.amax(-1))
+    assert torch.equal(parts[:, 0, 1].contiguous().view(torch.int32), torch.arange(tiles.shape[0], device=cuda).int() * 16
+                       + (tiles == tiles.amax(-1, keepdim=True)).float().argmax(-1).int())
+    for M in (2, 5, 6, 8, 15, 16):
+        y, p = torch.ops.ipex_llm_amd.gemv_argmax(x[:M], blob, f, n, k, None)
+        assert torch.equal(y[:1], one) and torch.equal(p[:, :1], parts), M
+        if torch.ops.ipex_llm_amd.skinny_takes(1, n, k, f, False, True):
+            assert torch.equal(torch.ops.ipex_llm_amd.gemv(x[:M], blob, f, n, k, None, 0, 0, 0)[:1], one), M
+
+
 @pytest.mark.parametrize("name", ["fp8_e4m3", "fp8_e5m2", "fp6"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_pairs_of_8_bit_floats(cuda, name, dtype):

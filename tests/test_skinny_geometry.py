@@ -34,3 +34,12 @@ def test_finer_table(n, k):
         mt, nw, cpk, _, slices = torch.ops.ipex_llm_amd.skinny_geometry(M, n, k, get_format("nf4").fmt, False, 0, True)
         assert mt == 3 or (mt, nw) == (4, 8)
         assert cpk * slices >= -(-k // 128)
+
+
+@pytest.mark.parametrize("k", [3584, 4096, 8192])
+def test_heads_by_format_and_shape(k):
+    """the kernel of an asym_int4 head of 1 to 16 rows does not depend on their number"""
+    import torch
+    ops.require()
+    for n in (32000, 128256, 152064):
+        assert all(torch.ops.ipex_llm_amd.skinny_takes(M, n, k, get_format("asym_int4").fmt, False, True) for M in range(1, 17)), n
