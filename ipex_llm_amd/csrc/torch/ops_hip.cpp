@@ -98,6 +98,7 @@ SkinnyPlan skinny_plan(int fmt, bool fine, int64_t M, int64_t NT, int64_t KC, bo
   SkinnyPlan best{};
   const int64_t MB = (M + 63) / 64;
   const int mt = (int)(((M + MB - 1) / MB + 15) / 16);
+  const int64_t rows = mt == 1 ? 1 : M;           // 1 to 16 rows: one split of K, a row keeps its bits beside any others
   const bool heavy = illm::fmt_has_min(fmt) || fmt == illm::FMT_SYM_INT8 || fmt == illm::FMT_SYM_INT5 || fine;
   const double chunk = (mt == 1 ? 0.4 : mt == 2 ? 0.5 : mt == 3 ? 0.6 : 0.8) * (illm::fmt_has_min(fmt) ? 4. / 3. : 1.);
   const bool asked = can_split && ks_req > 0;
@@ -119,7 +120,7 @@ SkinnyPlan skinny_plan(int fmt, bool fine, int64_t M, int64_t NT, int64_t KC, bo
       const double plain = rounds_of(NB * MB * ks, slots);
       const double shared = MB == 1 ? plain : rounds_of((NB + 7) / 8 * MB * ks, slots / 8);
       const double rounds = std::min(plain, shared);
-      const double c = rounds * (nw == 8 ? 3. + cpk * chunk : 2.5 + 1.15 * cpk * chunk) + (ks > 1 ? 2.5 + ks * M * NT * 16 * 8 / 4.5e6 : 0.);
+      const double c = rounds * (nw == 8 ? 3. + cpk * chunk : 2.5 + 1.15 * cpk * chunk) + (ks > 1 ? 2.5 + ks * rows * NT * 16 * 8 / 4.5e6 : 0.);
       if (c < cost) {
         cost = c;
         best = SkinnyPlan{mt, nw, (int)cpk, dim3((unsigned)(MB > 1 && shared <= plain ? padded : NB * MB), (unsigned)ks), fine};
@@ -287,10 +288,13 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 //     15.5, asym_int4 18.7 19.0 21.0 25.1 and 16.9 16.6 16.7 16.0, [37888, 3584] sym_int4 18.7 21.3 22.3 34.8 and 18.4
 //     18.2 18.3 19.6, fp8_e5m2 28.7 30.4 31.8 34.3 and 28.6 29.1 29.3 29.9, [9728, 896] 6.9 8.5 8.9 9.5 and 4.8 5.0 5.1
 //     5.0.  8-bit codes over a long K stay: [57344, 8192] fp8_e5m2 85.4 78.9 81.8 and 86.6 82.9 83.6;
-//   * slabs and plain products of K up to 5120 and up to 8192 columns: [6144, 4096] sym_int4 6.4 7.2 7.5 8.4 and 6.3 6.3
-//     6.2 6.5, [4096, 4096] 5.5 5.9 6.1 6.7 and 5.2 5.3 5.3 5.4, [3584, 3584] fp8_e5m2 6.1 6.6 6.7 7.3 and 5.5 5.7 5.7
-//     5.7, [2048, 2048] 4.7 5.1 5.3 5.7 and 4.1 4.3 4.3 4.3.  Longer K and wider outputs stay where v5 is ahead at few
-//     rows ([4096, 14336] 8.8 8.7 9.2 10.3 and 9.9 9.9 9.9 10.1, [12288, 4096] 8.4 9.4 10.3 12.5 and 12.4 12.1 12.1 12.2);
+//   * slabs and plain products of K 2048 to 5120 and up to 2048 columns, of 8-bit codes from K 3584 on up to 4096 (4 bits: K
+//     to 4096).  Weights that no cache holds, v5 / this, us at 1 / 2 / 4 / 8 / 16 rows, slabs: sym_int4 [2048, 4096] 4.8 4.9
+//     5.2 5.4 5.9 / 4.6 4.7 4.8 4.7 4.8, asym_int4 [1024, 3584] 0.94 to 0.78 of v5, fp8_e5m2 [2048, 2048] 5.1 5.2 5.4 5.6 6.1 /
+//     4.3 4.4 4.4 4.5 4.5, [4096, 4096] 6.7 6.9 7.0 7.2 7.6 / 6.5 6.6 6.5 6.5 6.6.  Wider outputs and little K are slower at
+//     one and two rows or at all: sym_int4 [4096, 4096] 5.4 5.5 5.7 5.9 6.5 / 5.9 6.0 6.0 6.0 6.0, [7168, 5120] 7.5 7.6 8.9 10.0
+//     12.1 / 9.7 9.1 9.2 9.1 9.2, [2048, 1536] 4.4 4.5 4.8 5.0 5.5 / 6.1 6.3 6.3 6.3 6.3, fp8_e5m2 [6144, 2048] 6.0 5.9 6.4 6.6
+//     7.1 / 7.7 7.8 7.8 7.8 7.8; a K of 14336 8.8 8.7 9.2 10.3 / 9.9 9.9 9.9 10.1 (sym_int4 [4096, 14336], 1 / 4 / 8 / 16);
 //   * ... and where v5 would cut K by the number of rows, as its x does not fit the LDS: [3584, 18944] at 16 rows 15.4
 //     and 11.2, [8192, 28672] 35.6 and 26.2, the head [128256, 4096] at 8 rows 129.7 and 54.6 (these rows' bits change
 //     with the number of rows on either path);
@@ -298,7 +302,7 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 bool skinny16(int fmt, bool bf16, int64_t M, int64_t NT, int64_t KC, int64_t epi, int64_t ksplit) {
   if (bf16 && illm::fmt_to_dk(fmt) == illm::DK_LUT4) return false;
   if (epi == illm::EPI_GLU) return KC < 64 || illm::fmt_bits(fmt) == 4;
-  if (KC <= 40 && NT <= 512) return true;
+  if (KC >= 16 && (illm::fmt_bits(fmt) == 4 ? KC <= 32 && NT <= 128 : KC <= 40 && NT <= (KC < 28 ? 128 : 256))) return true;
   if (head16(fmt, NT, KC)) return true;
   return ksplit <= 0 && plan5(M, NT, KC, true, 0, false, fmt).ks != plan5(1, NT, KC, true, 0, false, fmt).ks;
 }

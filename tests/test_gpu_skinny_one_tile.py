@@ -114,6 +114,21 @@ def test_x_that_starts_anywhere(cuda, at):
             assert torch.equal(y, want), (M, epi)
 
 
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "sym_int8", "fp8_e5m2"])
+@pytest.mark.parametrize("n,k", [(2048, 4096), (1040, 2112), (4096, 5120), (6144, 4096), (8192, 4096), (5120, 5120)])
+def test_rows_do_not_see_each_other(cuda, name, n, k):
+    """plain products and their slabs, on both sides of the rule"""
+    f = get_format(name).fmt
+    torch.manual_seed(7)
+    blob = ops.quantize(torch.randn(n, k, device=cuda) * 0.05, f)
+    x = torch.randn(16, k, device=cuda).bfloat16()
+    for epi in (0, 1):
+        one = torch.ops.ipex_llm_amd.gemv(x[:1], blob, f, n, k, None, epi, 0, 0)
+        for M in (2, 7, 8, 10, 11, 13, 16):
+            y = torch.ops.ipex_llm_amd.gemv(x[:M], blob, f, n, k, None, epi, 0, 0)
+            assert torch.equal(y[:, :1] if epi else y[:1], one), (epi, M)
+
+
 @pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "nf4", "fp8_e5m2"])
 @pytest.mark.parametrize("n,k", [(32000, 3584), (32016, 4096), (1008, 4096)])
 def test_a_heads_rows_do_not_see_each_other(cuda, name, n, k):

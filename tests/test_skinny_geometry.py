@@ -43,3 +43,22 @@ def test_heads_by_format_and_shape(k):
     ops.require()
     for n in (32000, 128256, 152064):
         assert all(torch.ops.ipex_llm_amd.skinny_takes(M, n, k, get_format("asym_int4").fmt, False, True) for M in range(1, 17)), n
+
+
+# every kind of decoder, both sides of the rule's borders; not products whose K v5 cuts by the rows (of 5248 and up, wide outputs)
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "fp4", "sym_int8", "asym_int5", "fp8_e4m3", "fp8_e5m2"])
+def test_one_kernel_and_split_for_16_rows(name):
+    """the kernel and the slabs of a product of 1 to 16 rows do not depend on their number"""
+    import torch
+    ops.require()
+    f, o = get_format(name).fmt, torch.ops.ipex_llm_amd
+    for n in (16, 1024, 2048, 2064, 4096, 4112, 4608, 6144, 8192, 8208):
+        for k in (64, 1920, 2048, 2176, 3456, 3584, 4096, 4224, 5120):
+            if n > 6144 and k > 4096:
+                continue
+            takes = {o.skinny_takes(M, n, k, f, False, True) for M in range(1, 17)}
+            assert len(takes) == 1, (n, k)
+            if takes == {True}:
+                assert len({tuple(o.skinny_geometry(M, n, k, f, False, 0)) for M in range(1, 17)}) == 1, (n, k)
+    for takes, n, k in [(True, 2048, 2048), (False, 6144, 4096), (False, 1024, 1536), (False, 4096, 2048)]:
+        assert o.skinny_takes(1, n, k, f, False, True) == takes, (n, k)
