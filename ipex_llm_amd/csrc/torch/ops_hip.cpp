@@ -145,9 +145,9 @@ void launch_skinny_any(int fmt, bool bf16, const SkinnyPlan& p, int epi, const i
   ILLM_DK_SWITCH(fmt, illm::launch_skinny_dk<DKV>(bf16, p.mt, p.nw, epi, p.grid, a, st, p.fine));
 }
 // lowbit_narrow.cuh instead of the skinny kernel: one workgroup per CU at most (it reads x once per tile), and
-//   * up to 16 rows: a K that the decode kernel's LDS does not hold (gate/up of K 8192 from 9 rows on; the skinny
-//     kernel's second row tile is empty): [8192, 8192] sym_int4 22.5 -> 19 us, nf4 30 -> 19; [16384, 8192], 512
-//     groups, 23 / 29;
+//   * up to 16 rows: a K that the decode kernel's LDS does not hold (gate/up of K 8192 from 9 rows on) and skinny16 does
+//     not take: [8192, 8192] at 9 / 12 / 16 rows, this and the skinny kernel's one row tile, sym_int4 18.3 19.4 21.0 / 18.7
+//     18.6 18.7 us, asym_int4 17.3 18.9 21.4 / 19.1 19.2 19.2, fp4 17.0 18.3 20.6 / 18.2 18.2 18.2;
 //   * so little K that the skinny kernel's chain of steps is all there is.  Its steps come in groups of 4 chunks: K
 //     up to 256 is half a group ([1024, 256] sym_int4 17 rows 4.7 -> 4.0 us, asym_int4 64 rows 8.4 -> 6.7), up to
 //     512 a whole one (4.7 / 4.8: stays), up to 1024 two ([1024, 1024] 17 rows 5.8 -> 4.9, asym_int4 33 rows 8.4 ->
@@ -284,10 +284,17 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 // Up to 16 rows, input and output in memory: the skinny kernel's one row tile instead of v5, by the format and the
 // shape, so that a row keeps its bits beside any other rows (1 to 16).  Not table formats under bf16 (v5 keeps an f16
 // table, the skinny kernel one in the type of x).
-//   * gate/up: us at 1 / 4 / 8 / 16 rows, v5 and this: [28672, 4096] sym_int4 15.7 15.0 15.9 22.4 and 15.4 15.4 15.4
-//     15.5, asym_int4 18.7 19.0 21.0 25.1 and 16.9 16.6 16.7 16.0, [37888, 3584] sym_int4 18.7 21.3 22.3 34.8 and 18.4
-//     18.2 18.3 19.6, fp8_e5m2 28.7 30.4 31.8 34.3 and 28.6 29.1 29.3 29.9, [9728, 896] 6.9 8.5 8.9 9.5 and 4.8 5.0 5.1
-//     5.0.  8-bit codes over a long K stay: [57344, 8192] fp8_e5m2 85.4 78.9 81.8 and 86.6 82.9 83.6;
+//   * gate/up, where no number of rows is slower by more than the runs differ.  v5's chain of one pair is the shorter at one
+//     and two rows (K cut in two within a group, deeper prefetch), so few pairs stay there unless K is short or decoding is
+//     long (minima, tables, integer bytes); with more than a round of its groups, one of 4 waves per CU and 2 pairs each, the
+//     stream counts.  Weights that no cache holds, v5 / this, us at 1 / 2 / 4 / 16 rows: sym_int4 [28672, 4096] 15.8 15.9
+//     15.7 22.8 / 15.7 16.1 15.7 16.2, [37888, 3584] 19.0 19.2 22.2 35.2 / 17.7 17.9 17.8 19.3, [18944, 2048] 9.4 9.4 9.5 11.2 /
+//     8.7 8.7 8.7 8.8, [28672, 8192] 26.8 28.6 28.0 26.5 / 26.0 26.3 26.0 26.5; asym_int4 [7168, 4096] 12.0 12.7 17.0 23.1 /
+//     11.8 11.9 12.0 12.0; fp8_e5m2 [37888, 3584] 28.7 28.3 30.5 34.3 / 29.7 28.6 28.8 29.8, [7168, 2048] 7.4 7.9 11.1 13.3 /
+//     7.5 7.7 7.8 7.7.  Not so: sym_int4 [7168, 4096] 9.4 9.6 12.7 20.4 / 11.2 11.4 11.4 11.5, [14336, 2048] 7.3 7.2 9.1 11.0 /
+//     7.7 7.8 7.9 7.8, [18944, 8192] 23.7 25.0 25.7 27.4 / 26.6 26.6 26.6 27.4, fp4 [7168, 8192] 13.8 15.2 20.6 21.1 / 18.6 18.7
+//     18.8 18.8, fp8_e5m2 [7168, 4096] 10.9 11.7 17.3 21.5 / 12.1 12.3 12.4 12.5, sym_int8 [7168, 7168] 17.6 18.7 28.6 20.6 /
+//     20.5 20.6 21.0 21.2;
 //   * slabs and plain products of K 2048 to 5120 and up to 2048 columns, of 8-bit codes from K 3584 on up to 4096 (4 bits: K
 //     to 4096).  Weights that no cache holds, v5 / this, us at 1 / 2 / 4 / 8 / 16 rows, slabs: sym_int4 [2048, 4096] 4.8 4.9
 //     5.2 5.4 5.9 / 4.6 4.7 4.8 4.7 4.8, asym_int4 [1024, 3584] 0.94 to 0.78 of v5, fp8_e5m2 [2048, 2048] 5.1 5.2 5.4 5.6 6.1 /
@@ -301,7 +308,16 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 //   * ... and the heads of head16.
 bool skinny16(int fmt, bool bf16, int64_t M, int64_t NT, int64_t KC, int64_t epi, int64_t ksplit) {
   if (bf16 && illm::fmt_to_dk(fmt) == illm::DK_LUT4) return false;
-  if (epi == illm::EPI_GLU) return KC < 64 || illm::fmt_bits(fmt) == 4;
+  if (epi == illm::EPI_GLU) {
+    const bool rounds = NT > 1024;                 // pairs of more than one v5 group per CU
+    if (illm::fmt_bits(fmt) == 8) {
+      const bool ints = fmt == illm::FMT_SYM_INT8 || fmt == illm::FMT_SYM_INT5 || fmt == illm::FMT_ASYM_INT5;
+      return KC <= 16 || (KC <= 32 && NT >= 768) || (KC <= 28 && ints);
+    }
+    if (fmt == illm::FMT_SYM_INT4) return KC <= 4 || (KC <= 32 && rounds) || (KC <= 64 && NT >= 1728);
+    if (fmt == illm::FMT_FP4) return KC <= 8 || (KC <= 16 && rounds);
+    return KC <= 32 || rounds;                     // minima; tables under f16
+  }
   if (KC >= 16 && (illm::fmt_bits(fmt) == 4 ? KC <= 32 && NT <= 128 : KC <= 40 && NT <= (KC < 28 ? 128 : 256))) return true;
   if (head16(fmt, NT, KC)) return true;
   return ksplit <= 0 && plan5(M, NT, KC, true, 0, false, fmt).ks != plan5(1, NT, KC, true, 0, false, fmt).ks;

@@ -62,3 +62,20 @@ def test_one_kernel_and_split_for_16_rows(name):
                 assert len({tuple(o.skinny_geometry(M, n, k, f, False, 0)) for M in range(1, 17)}) == 1, (n, k)
     for takes, n, k in [(True, 2048, 2048), (False, 6144, 4096), (False, 1024, 1536), (False, 4096, 2048)]:
         assert o.skinny_takes(1, n, k, f, False, True) == takes, (n, k)
+
+
+# sym_int4 and fp4 pairs of few columns or a long K are slower at one and two rows (the times are beside the rule)
+@pytest.mark.parametrize("name,takes,stays", [
+    ("sym_int4", [(28672, 4096), (37888, 3584), (16416, 2048), (28672, 8192), (1024, 512)], [(7168, 4096), (14336, 2048), (3584, 8192), (18944, 8192), (28672, 12288)]),
+    ("asym_int4", [(28672, 4096), (7168, 4096), (18944, 8192)], [(7168, 8192), (4096, 5120)]),
+    ("fp4", [(37888, 2048), (9728, 1024)], [(7168, 4096), (8192, 8192), (28672, 4096)]),
+    ("fp8_e5m2", [(37888, 3584), (28672, 4096), (7168, 2048)], [(7168, 4096), (28672, 7168)]),
+    ("sym_int8", [(28672, 4096), (7168, 3584)], [(7168, 4096), (7168, 7168)]),
+    ("nf4", [], [(28672, 4096), (1024, 512)])])
+def test_pairs_by_format_and_shape(name, takes, stays):
+    import torch
+    ops.require()
+    f, o = get_format(name).fmt, torch.ops.ipex_llm_amd
+    for want, shapes in ((True, takes), (False, stays)):
+        for n, k in shapes:
+            assert {o.skinny_takes(M, n, k, f, True, True, 1) for M in range(1, 17)} == {want}, (n, k)
