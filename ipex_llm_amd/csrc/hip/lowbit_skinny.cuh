@@ -41,13 +41,10 @@
 #include "../common/quant_block.h"
 #include "gemv_args.h"
 #include "illm_device.h"
+#include "kernels_skinny.h"
 #include "lowbit_raw.h"
 
 namespace illm {
-
-constexpr int SK_KW = 2;                       // waves along K
-constexpr int SK_TPW = 2;                      // weight tiles per wave
-constexpr int SK_STEP = SK_KW * CHUNK_K;       // k per step
 
 // constant of the offset product: -offset for the formats whose codes carry
 // one, 1 for unsigned codes with a block minimum (the plain sum of x)
@@ -423,13 +420,10 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   }
 }
 
-// dynamic LDS of one workgroup; a kernel asking for more than 64 KiB has its
-// limit raised first (once per kernel)
-inline size_t skinny_shmem(int mt, int table) { return (size_t)3 * mt * 16 * SK_STEP * 2 + table; }
-
+// a kernel asking for more than 64 KiB of dynamic LDS has its limit raised first (once per kernel)
 template <int DK, typename T, int MT, int NW, bool FINE = false>
 void launch_skinny_t(int epi, dim3 grid, const GemvArgs& a, hipStream_t st) {
-  const size_t shmem = skinny_shmem(MT, DK != DK_LUT4 ? 0 : FINE ? 2048 : 1024);
+  const size_t shmem = skinny_shmem(MT, skinny_table(DK == DK_LUT4, FINE));
   if (shmem > 64 * 1024) {
     static std::once_flag once;
     std::call_once(once, [&] {

@@ -76,24 +76,29 @@ Tensor dequantize_device(const Tensor& blob, int64_t fmt, int64_t n, int64_t k, 
     default: TORCH_CHECK(false, "gemv: unsupported fmt ", fmt);              \
   }
 
+constexpr size_t kLdsPerCu = 160 * 1024;
 // geometry of lowbit_skinny.cuh: workgroups of nw tiles x 16 mt rows x cpk chunks
 struct SkinnyPlan {
   int mt, nw, cpk;
   dim3 grid;
   bool fine;                    // a table weight's table as bf16 pairs
 };
-// The split with the least estimated time.  A CU runs one 8-wave or two 4-wave workgroups at a time; a
-// round of them takes 3 us (launch, first loads, epilogue) and 0.5 / 0.6 / 0.8 us per 128-k chunk at
-// 2 / 3 / 4 row tiles, 0.4 at one (MI355X: gate/up of Llama-3-8B, 32 chunks in one round, 21 / 25 / 30 us; two 4-wave
-// groups 24 / 30 / 36, one alone on its CU about 0.65 of that: Qwen2.5-7B's 296 column blocks as 592 of
-// half the size 36 instead of 40 us, a [2048, 1024] gate/up 5.7 instead of 6.7); slabs cost their write
+// The split with the least estimated time.  A CU runs one 8-wave workgroup at a time, or two of 4 waves where the x
+// rings of both fit its LDS: to three row tiles; at four, 98 KB each, one.  A round of 8-wave groups takes 3 us (launch,
+// first loads, epilogue) and 0.4 / 0.5 / 0.6 / 0.8 us per 128-k chunk at 1 / 2 / 3 / 4 row tiles, one of 4-wave pairs 2.5
+// us and 1.15 of that per chunk, a 4-wave group alone on its CU 0.65 of a pair's round (MI355X: gate/up of Llama-3-8B,
+// sym_int4, 32 chunks in one round of 8 waves, 18.6 / 23.1 / 27.6 at 2 / 3 / 4 row tiles: the figures are some 15 % on
+// the high side, alike for all).  Counting pairs of four row tiles that did not fit, us, 4-wave groups taken / 8-wave:
+// sym_int4 [37888, 3584] 49 rows 49.5 / 42.6, 128 rows 77.6 / 63.6, [4608, 3584] 49 rows 12.4 / 8.5, [6144, 4096] 512
+// rows 51.0 / 45.9, [10240, 8192] 256 rows 97 / 82, fp8_e5m2 [8192, 1024] 300 rows 20.9 / 17.9; up to 256 of them, one
+// per CU, they stay ahead ([4096, 4096] 256 rows 18.2 / 22.7, [4608, 3584] 192 rows 16.4 / 20.9).  Slabs cost their write
 // and read (4.5 TB/s) and the reduction.  Several row blocks of a column block run on one XCD, so that its
 // weights leave HBM once, and the rounds are those of the fullest XCD; column blocks that do not divide by 8
 // can leave XCDs idle, and where that costs a round the blocks go over all of them ([1280, 8192] sym_int4 512
-// rows 38.8 -> 26.4 us, [3584, 18944] 192 rows 70 -> 49, [256, 4096] sym_int8 512 rows 20.8 -> 12.9).  Block minima take a third more per chunk, and their 4-wave kernel
-// of 4 row tiles, like the integer bytes' and the fine table's one, spills 27 to 38 registers in the loop: 8
-// waves only.  ks_req > 0: that many slabs as asked (any number up to KC; the search on its own stops at 64,
-// where the slabs alone cost more than the slices save).
+// rows 38.8 -> 26.4 us, [3584, 18944] 192 rows 70 -> 49, [256, 4096] sym_int8 512 rows 20.8 -> 12.9).  Block minima take a
+// third more per chunk; their 4-wave kernel of 4 row tiles, like the integer bytes' one, spills 15 to 37 registers in the
+// loop (sym_int4's 5), and the fine table has none: 8 waves only.  ks_req > 0: that many slabs as asked (any number up to
+// KC; the search on its own stops at 64, where the slabs alone cost more than the slices save).
 SkinnyPlan skinny_plan(int fmt, bool fine, int64_t M, int64_t NT, int64_t KC, bool can_split, int64_t ks_req = 0) {
   SkinnyPlan best{};
   const int64_t MB = (M + 63) / 64;
@@ -105,15 +110,19 @@ SkinnyPlan skinny_plan(int fmt, bool fine, int64_t M, int64_t NT, int64_t KC, bo
   const int64_t kmin = asked ? ks_req : 1, kmax = asked ? ks_req : can_split ? std::min<int64_t>((KC + 3) / 4, 64) : 1;
   double cost = 1e30;
   for (int nw = 8; nw >= (heavy && mt == 4 ? 8 : 4); nw -= 4) {
-    const int64_t NB = (NT + nw - 1) / nw, slots = 256 * 8 / nw;
+    const int64_t NB = (NT + nw - 1) / nw;
+    const bool lut = illm::fmt_to_dk(fmt) == illm::DK_LUT4;
+    const bool pair = nw == 4 && 2 * illm::skinny_shmem(mt, illm::skinny_table(lut, fine)) <= kLdsPerCu;
+    const int64_t slots = pair ? 512 : 256;
     int64_t last = 0;
     for (int64_t k = kmin; k <= kmax; k++) {
       int64_t ks = k, cpk = (KC + k - 1) / k;
       if (asked) cpk = (cpk + 1) / 2 * 2;
-      else cpk = (cpk + 3) / 4 * 4, ks = (KC + cpk - 1) / cpk;     // the kernel's two steps of two chunks
+      else cpk = (cpk + 3) / 4 * 4, ks = (KC + cpk - 1) / cpk;     // (the search's grain; the kernel takes any even number)
       if (cpk == last) continue;
       last = cpk;
-      auto rounds_of = [nw](int64_t wg, int64_t s) {
+      auto rounds_of = [nw, pair](int64_t wg, int64_t s) {
+        if (nw == 4 && !pair) return 0.65 * ((wg + s - 1) / s);
         return wg / s + (wg % s == 0 ? 0. : nw == 4 && wg % s <= s / 2 ? 0.65 : 1.);
       };
       const int64_t padded = (NB + 7) / 8 * 8 * MB;

@@ -43,9 +43,9 @@ def rows_fit(M: int, n: int, fmt: int, glu: bool = False, k: int = 0) -> bool:
     rows 62 / 57).  Gate/up pairs by the rows alone -- a column shard of a
     tensor-parallel model takes the kernel that the whole pair takes --: up to 96
     rows (Llama-3-8B sym_int4, this / the fused kernel: M = 65 42 / 58 us, 96
-    41 / 58; two and more rounds would take 128 rows there, 49 / 58, but not in
-    [37888, 3584], 78 / 63), and 8-bit floats, whose codes have no offset, up to
-    512 (fp8_e5m2 [37888, 3584] M = 128 73 / 73, 300 118 / 128, 512 192 / 196;
+    41 / 58; two and more rounds would take 128 rows there, 49 / 58, not in
+    [37888, 3584], 64 / 63), and 8-bit floats, whose codes have no offset, up to
+    512 (fp8_e5m2 [37888, 3584] M = 128 62 / 73, 300 118 / 128, 512 192 / 196;
     e4m3 [28672, 4096] 50 / 58, 105 / 122, 152 / 168; not of K up to 1024,
     [14336, 1024] M = 420 44 / 34).  Nor pairs of over three rounds where a round
     is short or has minima in integer bytes ([151936, 1024] sym_int4 80 / 70,

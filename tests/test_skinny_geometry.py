@@ -79,3 +79,17 @@ def test_pairs_by_format_and_shape(name, takes, stays):
     for want, shapes in ((True, takes), (False, stays)):
         for n, k in shapes:
             assert {o.skinny_takes(M, n, k, f, True, True, 1) for M in range(1, 17)} == {want}, (n, k)
+
+
+@pytest.mark.parametrize("name", ["sym_int4", "fp4", "nf4", "fp8_e5m2"])
+def test_resident_groups(name):
+    """four row tiles take 98 KB of LDS: one workgroup per CU, so more than 256 of 4 waves are rounds"""
+    import torch
+    ops.require()
+    geometry, f = torch.ops.ipex_llm_amd.skinny_geometry, get_format(name).fmt
+    for M, n, k, glu in [(49, 37888, 3584, True), (64, 37888, 3584, True), (128, 37888, 3584, True), (49, 4608, 3584, False),
+                         (64, 4608, 3584, False), (512, 6144, 4096, False), (300, 8192, 1024, False), (256, 10240, 8192, False)]:
+        mt, nw = geometry(M, n, k, f, glu, 0)[:2]
+        assert (mt, nw) == (4, 8), (M, n, k)
+    assert geometry(256, 4096, 4096, f, False, 0)[:2] == [4, 4] and geometry(192, 4608, 3584, f, False, 0)[:2] == [4, 4]
+    assert geometry(48, 6144, 4096, f, False, 0)[0] == 3                     # (three row tiles: two 4-wave groups fit)
