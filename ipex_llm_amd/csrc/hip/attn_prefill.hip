@@ -45,6 +45,7 @@
 #include "../common/quant_block.h"
 #include "illm_device.h"
 #include "kernels.h"
+#include "lds_dma.h"
 
 namespace illm {
 
@@ -73,21 +74,6 @@ __device__ __forceinline__ uint4 pf_cvt8(const typename pf_raw<KVF>::type& u, fl
     }
     return make_uint4(pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]), pack2<T>(v[4], v[5]), pack2<T>(v[6], v[7]));
   }
-}
-
-// LDS-DMA of a 16-bit tile: 16 bytes a lane, LDS side wave-uniform base + lane * 16 (asm, so that hipcc does not
-// drain it before every LDS read of the other buffer; the waits are written out)
-typedef int32_t pf_rsrc __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ pf_rsrc pf_make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t p = (uint64_t)(uintptr_t)base;
-  return pf_rsrc{(int32_t)(uint32_t)p, (int32_t)((uint32_t)(p >> 32) & 0xffffu), (int32_t)bytes, 0x00020000};
-}
-
-__device__ __forceinline__ void pf_dma16(const pf_rsrc& rs, const uint8_t* lds, uint32_t voff, int soff) {
-  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)lds);
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(la), "v"(voff), "s"(rs), "s"(soff) : "memory", "m0");
 }
 
 // max over the four lanes of a query row (lane ^ 16, ^ 32)
@@ -193,12 +179,12 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(const AttnPrefillA
   auto load_tile = [&](int t) {
     next_src();
     if constexpr (KVF == 0) {
-      const pf_rsrc rk = pf_make_rsrc(a.k_cache + src, TB), rv = pf_make_rsrc(a.v_cache + src, TB);
+      const dma_rsrc rk = make_dma_rsrc(a.k_cache + src, TB), rv = make_dma_rsrc(a.v_cache + src, TB);
       const uint8_t* dst = lds + (t & 1) * TB + wave * 1024;
 #pragma unroll
-      for (int i = 0; i < TB / 4096; i++) pf_dma16(rk, dst + i * 4096, doff, i * 4096);
+      for (int i = 0; i < TB / 4096; i++) lds_dma16(rk, lds_addr(dst + i * 4096), doff, i * 4096);
 #pragma unroll
-      for (int i = 0; i < TB / 4096; i++) pf_dma16(rv, dst + 2 * TB + i * 4096, doff, i * 4096);
+      for (int i = 0; i < TB / 4096; i++) lds_dma16(rv, lds_addr(dst + 2 * TB + i * 4096), doff, i * 4096);
     } else {
 #pragma unroll
       for (int j = 0; j < UPT; j++) {

@@ -45,6 +45,7 @@
 #include "gemv_args.h"
 #include "illm_device.h"
 #include "kernels_g8.h"
+#include "lds_dma.h"
 #include "mfg_common.h"
 
 namespace illm {
@@ -55,23 +56,10 @@ constexpr int IMG = 256 * ROWB;         // one operand image, 32 KB
 constexpr int BUFB = 2 * IMG;           // A + B images of one K-tile
 constexpr int LDS_BYTES = 2 * BUFB;     // two buffers, 128 KB
 
-typedef int32_t g8_rsrc __attribute__((ext_vector_type(4)));
-
-// buffer descriptor: base, num_records = bytes (reads past it return 0)
-__device__ __forceinline__ g8_rsrc make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t p = (uint64_t)(uintptr_t)base;
-  return g8_rsrc{(int32_t)(uint32_t)p, (int32_t)((uint32_t)(p >> 32) & 0xffffu), (int32_t)bytes, 0x00020000};
-}
-
-// 16-B LDS-DMA per lane (LDS side: wave-uniform base + lane * 16).  Issued
-// from inline asm ON PURPOSE: hipcc cannot tell these LDS writes from the
-// fragment ds_reads of the other buffer and would otherwise drain vmcnt(0)
-// before every phase's reads (measured in the .s) -- the counted
-// `s_waitcnt vmcnt(N)` + barrier below are the only ordering they need.
-__device__ __forceinline__ void dma16(const g8_rsrc& rs, const uint8_t* lds, uint32_t voff, int soff) {
-  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)lds);
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(la), "v"(voff), "s"(rs), "s"(soff) : "memory", "m0");
+// 16-B LDS-DMA per lane (lds_dma.h): the counted `s_waitcnt vmcnt(N)` +
+// barrier below are the only ordering they need.
+__device__ __forceinline__ void dma16(const dma_rsrc& rs, const uint8_t* lds, uint32_t voff, int soff) {
+  lds_dma16(rs, lds_addr(lds), voff, soff);
 }
 
 // image row of half-tile h, half-tile row q in [0, 128)
@@ -172,7 +160,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(const G8Args a) {
       xo[h][i] = (uint32_t)(m0 + ra) * (uint32_t)a.ldx * ES + 16u * (uint32_t)(c ^ ((ra >> 1) & 7));
       wo[h][i] = DENSE ? (uint32_t)(n0 + rb) * (uint32_t)a.ldw * ES + 16u * (uint32_t)(c ^ ((rb >> 1) & 7)) : 0u;
     }
-  const g8_rsrc rx = make_rsrc(a.x, a.x_bytes), rw = make_rsrc(a.w, a.w_bytes);
+  const dma_rsrc rx = make_dma_rsrc(a.x, a.x_bytes), rw = make_dma_rsrc(a.w, a.w_bytes);
   auto a_img = [&](int t) -> uint8_t* { return smem + L::A0 + (t & 1) * L::ASTR; };
   auto b_img = [&](int t) -> uint8_t* { return smem + L::B0 + (t & 1) * L::BSTR; };
   auto stage_a = [&](int h, int t) {          // half-tile A_h of k-tile t -> buffer t & 1

@@ -34,6 +34,7 @@
 #include "../common/quant_block.h"
 #include "gemv_args.h"
 #include "illm_device.h"
+#include "lds_dma.h"
 #include "lowbit_raw.h"
 
 namespace illm {
@@ -93,7 +94,6 @@ __device__ __forceinline__ uint4 ldw16(const uint8_t* p) {
 // no VGPR round trip, every row requested at once) for launches whose x slice
 // needs more than one batch of register-staged loads per thread (the batch-8
 // gate/up GEMV: 64 KB per workgroup, two dependent L2 round trips before).
-// Issued from inline asm like the 8-phase GEMM's (gemm_8p.hip dma16).
 #ifndef ILLM_GEMV5_XDMA
 #define ILLM_GEMV5_XDMA 1
 #endif
@@ -103,16 +103,6 @@ __device__ __forceinline__ uint4 ldw16(const uint8_t* p) {
 #ifndef ILLM_GEMV5_EARLYX
 #define ILLM_GEMV5_EARLYX 1
 #endif
-typedef int32_t gv5_rsrc __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ gv5_rsrc gv5_make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t p = (uint64_t)(uintptr_t)base;
-  return gv5_rsrc{(int32_t)(uint32_t)p, (int32_t)((uint32_t)(p >> 32) & 0xffffu), (int32_t)bytes, 0x00020000};
-}
-__device__ __forceinline__ void gv5_dma16(const gv5_rsrc& rs, const void* lds, uint32_t voff) {
-  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)lds);
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(la), "v"(voff), "s"(rs) : "memory", "m0");
-}
 
 // per-workgroup timeline stamps (tools/probe/gemv5_probe.hip PROBE_MODE=s,
 // built with its own definition): 0 entry, 1 x staged, 2 chunks computed,
@@ -340,10 +330,10 @@ __device__ __forceinline__ void gemv5_body(const GemvArgs& a, const G5Blk& blk) 
   }
   if (dma_x) {
     const int per_row = (xvpr + 63) >> 6, nins = Mloc * per_row;
-    const gv5_rsrc rx = gv5_make_rsrc(a.x, (uint32_t)((size_t)a.M * a.ldx * 2));
+    const dma_rsrc rx = make_dma_rsrc(a.x, (uint32_t)((size_t)a.M * a.ldx * 2));
     for (int i = wave; i < nins; i += NW) {      // wave-uniform: one whole row piece per instruction
       const int m = i / per_row, j = i - m * per_row;
-      gv5_dma16(rx, xs + m * ldx + j * 512, (uint32_t)(((size_t)m * a.ldx + kbase + j * 512 + lane * 8) * 2));
+      lds_dma16(rx, lds_addr(xs + m * ldx + j * 512), (uint32_t)(((size_t)m * a.ldx + kbase + j * 512 + lane * 8) * 2));
     }
   }
   asm volatile("" ::: "memory");             // the ring loads stay behind these

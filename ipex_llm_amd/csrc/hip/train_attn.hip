@@ -28,6 +28,7 @@
 
 #include "illm_device.h"
 #include "kernels_train.h"
+#include "lds_dma.h"
 
 namespace illm {
 
@@ -43,23 +44,10 @@ constexpr int FA_QB = 64;   // query rows per workgroup (forward / dQ)
 // writing physical chunk p of row r fetches logical chunk p ^ (r & MSK).  No
 // register staging (the register form spilled to scratch and waited on its
 // own loads), the next tile in flight across the compute of the current one.
-// Issued from inline asm so hipcc does not drain vmcnt before the LDS reads.
-typedef int32_t ta_rsrc __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ ta_rsrc ta_make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t p = (uint64_t)(uintptr_t)base;
-  return ta_rsrc{(int32_t)(uint32_t)p, (int32_t)((uint32_t)(p >> 32) & 0xffffu), (int32_t)bytes, 0x00020000};
-}
-
-__device__ __forceinline__ uint32_t ta_lds_addr(const void* p) {
-  return __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p);
-}
-
 // rows row0 .. row0 + 63 (clamped to nrows - 1) of a tensor with row stride
 // `rstride` elements -> LDS tile at byte address `lds` (wave-uniform)
 template <int D>
-__device__ __forceinline__ void ta_stage(const ta_rsrc& rs, uint32_t lds, int row0, int64_t rstride, int nrows,
+__device__ __forceinline__ void ta_stage(const dma_rsrc& rs, uint32_t lds, int row0, int64_t rstride, int nrows,
                                          int wave, int lane) {
   constexpr int CH = D / 8, MSK = CH >= 16 ? 15 : CH - 1;
   constexpr int RPI = 64 / CH;                    // rows per wave instruction
@@ -70,9 +58,7 @@ __device__ __forceinline__ void ta_stage(const ta_rsrc& rs, uint32_t lds, int ro
     const int r = idx * RPI + lane / CH, pch = lane % CH;
     const int srow = min(row0 + r, nrows - 1);
     const uint32_t voff = (uint32_t)((int64_t)srow * rstride * 2) + (uint32_t)((pch ^ (r & MSK)) * 16);
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds + (uint32_t)(idx * RPI * D * 2));   // wave-uniform
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(m0), "v"(voff), "s"(rs), "s"(0) : "memory", "m0");
+    lds_dma16(rs, __builtin_amdgcn_readfirstlane(lds + (uint32_t)(idx * RPI * D * 2)), voff);   // wave-uniform
   }
 }
 
@@ -161,9 +147,9 @@ __global__ void __launch_bounds__(256) fa_q_kernel(const TrainAttnArgs a) {
 
   const uint16_t* kbase = a.k + (size_t)b * a.ksb + (size_t)kvh * a.ksh;
   const uint16_t* vbase = a.v + (size_t)b * a.vsb + (size_t)kvh * a.vsh;
-  const ta_rsrc rk = ta_make_rsrc(kbase, (uint32_t)(((int64_t)(a.T - 1) * a.kst + D) * 2));
-  const ta_rsrc rv = ta_make_rsrc(vbase, (uint32_t)(((int64_t)(a.T - 1) * a.vst + D) * 2));
-  const uint32_t ks_l = ta_lds_addr(lds), vs_l = ks_l + 2 * TILE_B;
+  const dma_rsrc rk = make_dma_rsrc(kbase, (uint32_t)(((int64_t)(a.T - 1) * a.kst + D) * 2));
+  const dma_rsrc rv = make_dma_rsrc(vbase, (uint32_t)(((int64_t)(a.T - 1) * a.vst + D) * 2));
+  const uint32_t ks_l = lds_addr(lds), vs_l = ks_l + 2 * TILE_B;
   const FaFrag<D> fr(g, r16);
   auto stage = [&](int t, int buf) {
     ta_stage<D>(rk, ks_l + buf * TILE_B, t * FA_KT, a.kst, a.T, wave, lane);
@@ -330,15 +316,15 @@ __global__ void __launch_bounds__(256) fa_dkdv_kernel(const TrainAttnArgs a) {
   const int nqb = a.T / FA_QB - qb0;
   const int nwork = G * nqb;                                           // (head, query block) pairs
   float lreg = 0.f;
-  const uint32_t qs_l = ta_lds_addr(lds), os_l = qs_l + 2 * TILE_B;
+  const uint32_t qs_l = lds_addr(lds), os_l = qs_l + 2 * TILE_B;
   const FaFrag<D> fr(g, r16);
   auto load_tile = [&](int w, int buf) {
     const int hh = kvh * G + w / nqb, qb = qb0 + w % nqb;
     const uint16_t* qp = a.q + (size_t)b * a.qsb + (size_t)hh * a.qsh;
     const uint16_t* dp = a.dout + (size_t)b * a.dsb + (size_t)hh * a.dsh;
-    ta_stage<D>(ta_make_rsrc(qp, (uint32_t)(((int64_t)(a.T - 1) * a.qst + D) * 2)), qs_l + buf * TILE_B,
+    ta_stage<D>(make_dma_rsrc(qp, (uint32_t)(((int64_t)(a.T - 1) * a.qst + D) * 2)), qs_l + buf * TILE_B,
                 qb * FA_QB, a.qst, a.T, wave, lane);
-    ta_stage<D>(ta_make_rsrc(dp, (uint32_t)(((int64_t)(a.T - 1) * a.dst + D) * 2)), os_l + buf * TILE_B,
+    ta_stage<D>(make_dma_rsrc(dp, (uint32_t)(((int64_t)(a.T - 1) * a.dst + D) * 2)), os_l + buf * TILE_B,
                 qb * FA_QB, a.dst, a.T, wave, lane);
     if (tid < 2 * FA_QB) {
       const size_t ri = ((size_t)b * a.Hq + hh) * a.T + qb * FA_QB + (tid & (FA_QB - 1));
