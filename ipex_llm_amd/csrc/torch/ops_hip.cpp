@@ -339,6 +339,38 @@ bool skinny_takes(int64_t M, int64_t n, int64_t k, int64_t fmt, bool glu, bool b
                   glu ? illm::EPI_GLU : illm::EPI_STORE, ksplit);
 }
 
+// the kernel and the slabs of a plain product or its partial sums (epi: not GLU)
+struct RowsRoute {
+  bool use5, narrow;
+  Plan5 p5;
+  SkinnyPlan q;
+  int64_t ksplit;
+};
+RowsRoute rows_route(int fmt, bool bf16, bool fine, int64_t M, int64_t NT, int64_t KC, int64_t epi, int64_t ksplit) {
+  RowsRoute r{};
+  const bool one = M <= 16 && skinny16(fmt, bf16, M, NT, KC, epi, ksplit);
+  if (M <= 16 && !one && getenv("ILLM_GEMV_V1") == nullptr) {
+    r.p5 = plan5(M, NT, KC, true, ksplit, false, fmt);
+    r.use5 = r.p5.shmem <= kMaxLds;
+  }
+  if (r.use5) {
+    r.ksplit = r.p5.ks;
+  } else if (!one && narrow_fit(fmt, M, NT, KC, epi)) {
+    r.narrow = true;
+    r.ksplit = std::max<int64_t>(1, std::min<int64_t>(ksplit, KC));
+  } else {
+    r.q = skinny_plan(fmt, fine, M, NT, KC, true, std::min<int64_t>(ksplit, KC));
+    r.ksplit = r.q.grid.y;
+  }
+  return r;
+}
+// slabs of gemv's partial sums and of gemm_rows_slabs (shape propagation)
+int64_t gemv_slabs(int64_t M, int64_t n, int64_t k, int64_t fmt, bool bf16, int64_t ksplit, bool fine) {
+  TORCH_CHECK(M >= 1 && n >= 1 && k >= 1, "gemv_slabs: sizes");
+  return rows_route((int)fmt, bf16, fine, M, illm::pad_to(n, illm::TILE_N) / illm::TILE_N,
+                    illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K, illm::EPI_PARTIAL, ksplit).ksplit;
+}
+
 // rows 1 .. most: v5 up to 16 rows (ILLM_GEMV_V1=1: the many-row kernels for these too, A/B tests), the
 // skinny kernel from 17, the narrow one where it fits
 Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k,
@@ -353,8 +385,6 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv: weight blob too small");
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N;
   const int64_t KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
-  const bool one = M <= 16 && skinny16((int)fmt, bf16, M, NT, KC, epi, ksplit);
-  const bool small = M <= 16 && !one && getenv("ILLM_GEMV_V1") == nullptr;
 
   illm::GemvArgs a{};
   a.x = p16(xc);
@@ -374,6 +404,8 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
     a.N = (int)(n / 2);
     a.out = out.data_ptr();
     a.ldo = (int)(n / 2);
+    const bool one = M <= 16 && skinny16((int)fmt, bf16, M, NT, KC, epi, ksplit);
+    const bool small = M <= 16 && !one && getenv("ILLM_GEMV_V1") == nullptr;
     const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
     if (small && p.shmem <= kMaxLds)
       a.nw = p.nw, launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);
@@ -384,28 +416,16 @@ Tensor lowbit_rows(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
     return out;
   }
   a.N = (int)n;
-  Plan5 p5{};
-  SkinnyPlan q{};
-  bool use5 = false, narrow = false;
-  if (small) {
-    p5 = plan5(M, NT, KC, true, ksplit, false, (int)fmt);
-    use5 = p5.shmem <= kMaxLds;
-  }
-  if (use5) {
-    ksplit = p5.ks;
-    a.cpk = (int)p5.cpk;
-    a.nw = p5.nw;
-  } else if (!one && narrow_fit((int)fmt, M, NT, KC, epi)) {
-    narrow = true;
-    ksplit = std::max<int64_t>(1, std::min<int64_t>(ksplit, KC));
-  } else {
-    q = skinny_plan((int)fmt, fine, M, NT, KC, true, std::min<int64_t>(ksplit, KC));
-    ksplit = q.grid.y;
+  const RowsRoute r = rows_route((int)fmt, bf16, fine, M, NT, KC, epi, ksplit);
+  ksplit = r.ksplit;
+  if (r.use5) {
+    a.cpk = (int)r.p5.cpk;
+    a.nw = r.p5.nw;
   }
   auto launch = [&](int e) {
-    if (use5) launch_gemv5_any((int)fmt, bf16, p5.kw, e, dim3(p5.gx, (unsigned)ksplit), p5.shmem, a);
-    else if (narrow) launch_narrow_any((int)fmt, bf16, e, dim3((unsigned)NT, (unsigned)ksplit), a);
-    else launch_skinny_any((int)fmt, bf16, q, e, a);
+    if (r.use5) launch_gemv5_any((int)fmt, bf16, r.p5.kw, e, dim3(r.p5.gx, (unsigned)ksplit), r.p5.shmem, a);
+    else if (r.narrow) launch_narrow_any((int)fmt, bf16, e, dim3((unsigned)NT, (unsigned)ksplit), a);
+    else launch_skinny_any((int)fmt, bf16, r.q, e, a);
   };
   if (epi == illm::EPI_PARTIAL || ksplit > 1) {
     Tensor ws = at::empty({ksplit, M, n}, xc.options().dtype(at::kFloat));
@@ -1918,6 +1938,7 @@ int* illm_kernel_err(const c10::Device& dev) { return kernel_err(dev); }
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("skinny_geometry(int M, int n, int k, int fmt, bool glu, int ksplit, bool fine=False) -> int[]", &skinny_geometry);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
+  m.def("gemv_slabs(int M, int n, int k, int fmt, bool bf16, int ksplit=0, bool fine=False) -> int", &gemv_slabs);
 }
 
 TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {

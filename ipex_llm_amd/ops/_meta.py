@@ -18,11 +18,17 @@ def _(blob, fmt, n, k, dtype, transpose=False):
     return blob.new_empty((k, n) if transpose else (n, k), dtype=dtype)
 
 
+def _slabs(M, split):
+    """slabs of a product whose split of K the launch plan chooses by its sizes: unknown where the rows are"""
+    return split(M) if isinstance(M, int) else torch.library.get_ctx().new_dynamic_size()
+
+
 @register_fake("ipex_llm_amd::gemv")
 def _(x, blob, fmt, n, k, bias, epi, ksplit, act):
     M = x.numel() // k
     if epi == 1:
-        return x.new_empty((max(ksplit, 1), M, n), dtype=torch.float32)
+        S = _slabs(M, lambda m: torch.ops.ipex_llm_amd.gemv_slabs(m, n, k, fmt, x.dtype == torch.bfloat16, ksplit))
+        return x.new_empty((S, M, n), dtype=torch.float32)
     shape = list(x.shape)
     shape[-1] = n // 2 if epi == 2 else n
     return x.new_empty(shape)
@@ -37,12 +43,15 @@ def _(x, blob, fmt, n, k, bias, glu, act, fine=False):
 
 @register_fake("ipex_llm_amd::gemm_rows_slabs")
 def _(x, blob, fmt, n, k, fine=False):
-    return x.new_empty((1, x.numel() // k, n), dtype=torch.float32)
+    M = x.numel() // k
+    S = _slabs(M, lambda m: torch.ops.ipex_llm_amd.gemv_slabs(m, n, k, fmt, x.dtype == torch.bfloat16, 0, fine))
+    return x.new_empty((S, M, n), dtype=torch.float32)
 
 
 @register_fake("ipex_llm_amd::gemm_bf16_slabs")
 def _(x, w):
-    return x.new_empty((2, x.shape[0], w.shape[0]), dtype=torch.float32)
+    M, N, K = x.shape[0], w.shape[0], w.shape[1]
+    return x.new_empty((_slabs(M, lambda m: torch.ops.ipex_llm_amd.gemm_bf16_split(m, N, K)), M, N), dtype=torch.float32)
 
 
 @register_fake("ipex_llm_amd::add_rms_norm")

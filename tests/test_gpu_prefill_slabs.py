@@ -44,3 +44,16 @@ def test_products_that_are_not_split(cuda):
     assert gemm.lowbit_slabs(x[:70].requires_grad_(), blob, f, 8192, 256) is None
     with pytest.raises(RuntimeError, match="not split"):
         torch.ops.ipex_llm_amd.gemm_bf16_slabs(x, torch.randn(8192, 256, device=cuda).bfloat16())
+
+
+@pytest.mark.parametrize("qtype", ["sym_int4", "asym_int4", "nf4", "sym_int8", "fp8_e5m2"])
+def test_slabs_of_every_route(cuda, qtype):
+    """the number of slabs that shape propagation names is the launch's: decode, one-tile, narrow and skinny kernels"""
+    f, o = get_format(qtype).fmt, torch.ops.ipex_llm_amd
+    for n, k in [(1040, 2048), (4096, 4096), (512, 256), (8200, 1088), (48, 18944)]:
+        blob = ops.quantize(torch.randn(n, k, device=cuda) * 0.05, f)
+        for M in (1, 7, 16, 17, 40, 64, 65, 300):
+            x = torch.randn(M, k, device=cuda).bfloat16()
+            for ks in (0, 3) if M <= 64 else (0,):
+                y = o.gemv(x, blob, f, n, k, None, 1, ks, 0) if M <= 64 else o.gemm_rows_slabs(x, blob, f, n, k)
+                assert y.shape == (o.gemv_slabs(M, n, k, f, True, ks), M, n)

@@ -1,5 +1,7 @@
 """Measured GEMM dispatch bookkeeping (ops/gemm.py _pick): row buckets and the
 cached per-shape choice (the timing itself needs a GPU: tests/test_gpu_kernels.py)."""
+import pytest
+
 from ipex_llm_amd.ops import gemm as G
 
 
@@ -80,3 +82,38 @@ def test_pairs_of_8_bit_floats_up_to_512_rows():
                 assert not G.rows_take(dt, 513, n, 3584, f, True) and not G.rows_take(dt, 97, n, 1024, f, True)
             for name in ("sym_int4", "fp4", "sym_int8", "asym_int4"):
                 assert not G.rows_take(dt, 97, n, 3584, get_format(name).fmt, True)
+
+
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "fp8_e5m2"])
+def test_traced_slabs_are_the_plans(name):
+    """partial sums under tracing have as many slabs as the launch plan makes, also where that is neither one nor two"""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    import ipex_llm_amd.ops as ops
+    from ipex_llm_amd.quantize import get_format
+    ops.require()
+    f, o, seen = get_format(name).fmt, torch.ops.ipex_llm_amd, set()
+    with FakeTensorMode():
+        for M, n, k in [(1, 4096, 4096), (16, 2048, 2048), (20, 1024, 256), (48, 4096, 14336), (300, 3584, 18944), (300, 3584, 3584), (65, 512, 512)]:
+            x, blob = torch.empty(M, k, dtype=torch.bfloat16, device="cuda"), torch.empty(64, dtype=torch.uint8, device="cuda")
+            S = o.gemv_slabs(M, n, k, f, True)
+            seen.add(S)
+            assert (o.gemv(x, blob, f, n, k, None, 1, 0, 0) if M <= 64 else o.gemm_rows_slabs(x, blob, f, n, k)).shape == (S, M, n)
+            assert o.gemv(x[:1], blob, f, n, k, None, 1, 3, 0).shape[0] == o.gemv_slabs(1, n, k, f, True, 3)
+        assert max(seen) > 2
+        for M, N, K in [(1024, 4096, 14336), (512, 4096, 4096), (1024, 6144, 4096)]:
+            y = o.gemm_bf16_slabs(*(torch.empty(r, K, dtype=torch.bfloat16, device="cuda") for r in (M, N)))
+            assert y.shape == (o.gemm_bf16_split(M, N, K), M, N)
+
+
+def test_traced_slabs_of_unknown_rows():
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.symbolic_shapes import ShapeEnv
+    import ipex_llm_amd.ops as ops
+    ops.require()
+    env = ShapeEnv()
+    with FakeTensorMode(shape_env=env):
+        x = torch.empty(env.create_unbacked_symint(), 64, dtype=torch.bfloat16, device="cuda")
+        y = torch.ops.ipex_llm_amd.gemm_rows_slabs(x, torch.empty(64, dtype=torch.uint8, device="cuda"), 0, 96, 64)
+        assert isinstance(y.shape[0], torch.SymInt) and y.shape[2] == 96
