@@ -31,4 +31,12 @@ void launch_attn_decode(bool bf16, const AttnDecodeArgs& a, hipStream_t st) {
   if (bf16) launch_t<BF16>(a, st); else launch_t<F16>(a, st);
 }
 
+int attn_decode_groups(int B, int Hkv, int nsplit) {
+  AttnDecodeArgs a{};
+  a.B = B;
+  a.Hkv = Hkv;
+  a.nsplit = nsplit;
+  return v3_long_grid(a, 0);
+}
+
 }  // namespace illm

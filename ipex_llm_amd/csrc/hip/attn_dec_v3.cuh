@@ -918,7 +918,13 @@ static void launch_v3_nw(const AttnDecodeArgs& a, hipStream_t st) {
 // 128 x 200 44.0 / 30.5, 36 x 300 19.8 / 16.2, 32 x 768 30.0 / 25.0, 32 x 1800 53.9 / 45.7, but 40 x 1500 48.2 / 48.8 (two
 // and a half per CU); 28 / 4 heads 96 x 300 22.6 / 19.1, 32 / 32 heads 64 x 500 98.6 / 90.5.  Not below: 24 x 512 15.5 /
 // 16.5, 24 x 1024 25.5 / 25.8, 28 / 4 heads 48 x 700 20.0 / 20.7; nor where a workgroup has one tile or the grid two: 64 x
-// 128 13.5 / 14.2, 32 x 100 10.4 / 11.9, 28 / 4 heads 64 x 300 14.7 / 15.6.
+// 128 13.5 / 14.2, 32 x 100 10.4 / 11.9, 28 / 4 heads 64 x 300 14.7 / 15.6; nor where 8-wave groups of one tile per wave are
+// one round themselves (32 x 400 16.4 / 17.3, 28 / 4 heads 64 x 400 16.8 / 18.7), nor with 9 to 12 tiles a pair where two
+// workgroups a pair leave many CUs two of their three (33 x 1500 42.8 / 46.6, 28 / 4 heads 72 x 1200 37.1 / 41.0, 80 x 1200
+// 41.7 / 44.2; longer ones are even, 40 x 2500 78.2 / 76.0).  Some 4 % behind it is at 33 x 2500 and 28 / 4 heads 96 x 1200 in
+// one run of two.  Lengths that differ more: 31 of 500 tokens and one of 16000 137 / 78, 95 and one 424 / 209, 39 of 500 and
+// one of 16000 170 / 110, 56 of 300 and 8 of 8000 160 / 107 (most groups of a grid made for the longest find no keys; more
+// workgroups for these is open: 12 tiles each measured 60, 90, 69 and 75, 8 tiles 76, 193, 73 and 94).
 //
 // Fused-RoPE decode, 48 splits and more, for sequences of the grid's full length: the CU with the most workgroups has
 // n = ceil(workgroups / 256) of them, each t tiles and about 0.7 tiles' time to start and merge, and where the lengths
@@ -936,6 +942,8 @@ inline int v3_long_grid(const AttnDecodeArgs& a, int rq) {
     const long pairs = (long)a.B * a.Hkv;
     if (pairs < 256) return 0;
     const long s = pairs < 768 ? 768 / pairs : 1;
+    if (pairs * ((a.nsplit * SPLIT + 8 * V3_KPW - 1) / (8 * V3_KPW)) <= 512) return 0;
+    if (s == 2 && pairs < 336 && all > 8 && all <= 12) return 0;
     return all >= 3 && all > s ? (int)s : 0;
   }
   if (a.nsplit < 48 || (a.nsplit < 56 && (long)a.B * a.Hkv * all < 1024)) return 0;

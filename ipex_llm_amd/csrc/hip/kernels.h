@@ -210,6 +210,8 @@ struct AttnDecodeArgs {
   int* v3_counters;
 };
 void launch_attn_decode(bool bf16, const AttnDecodeArgs& a, hipStream_t st);
+// workgroups per (sequence, kv head) of several tiles per wave, q from memory (0: one tile per wave)
+int attn_decode_groups(int B, int Hkv, int nsplit);
 
 // ---- prefill / long-query attention over the paged cache (attn_prefill.hip)
 struct AttnPrefillArgs {

@@ -1938,6 +1938,10 @@ int* illm_kernel_err(const c10::Device& dev) { return kernel_err(dev); }
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("skinny_geometry(int M, int n, int k, int fmt, bool glu, int ksplit, bool fine=False) -> int[]", &skinny_geometry);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
+  m.def("attn_decode_groups(int batch, int kv_heads, int nsplit) -> int", [](int64_t b, int64_t h, int64_t n) -> int64_t {
+    TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_groups: sizes");
+    return illm::attn_decode_groups((int)b, (int)h, (int)n);
+  });
   m.def("gemv_slabs(int M, int n, int k, int fmt, bool bf16, int ksplit=0, bool fine=False) -> int", &gemv_slabs);
 }
 
