@@ -507,7 +507,7 @@ class NativeCausalLM(nn.Module):
                 and self.tp_group is None and proj.mp_group is None and x.dim() == 2 and x.dtype == residual.dtype
                 and ops.native_gpu(x) and not (proj._forward_hooks or proj._forward_pre_hooks)):
             from ..ops.gemm import lowbit_slabs
-            part = lowbit_slabs(x, proj.weight, proj.fmt, proj.out_features, proj.in_features)
+            part = lowbit_slabs(x, proj.weight, proj.fmt, proj.out_features, proj.in_features, least=2)
         if part is not None:
             out, _ = ops.add_rms_norm(None, residual, norm_w, s.rms_eps, partials=part, unit_offset=s.norm_unit_offset)
             return out

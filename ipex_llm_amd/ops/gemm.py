@@ -437,19 +437,25 @@ def lowbit_gemm(x, blob, fmt, n, k, bias=None):
     return F.linear(x, w, bias)
 
 
-def lowbit_slabs(x, blob, fmt, n, k):
+def lowbit_slabs(x, blob, fmt, n, k, least=1):
     """x @ W^T of more rows than the decode kernels take as the f32 slabs [S, M, n]
     of a split K for :func:`add_rms_norm` to sum -- it rounds the sum as the pass
     over the slabs that this saves does, so with the same bits --, or None where
-    :func:`lowbit_gemm` takes a dense product that it does not split.  Pass and
-    norm / norm alone, us: fp8_e5m2 [3584, 18944] of 300 rows 10.1 / 5.9, the dense
-    [4096, 14336] of 1024 rows 22.5 / 16.2."""
+    the skinny kernel makes fewer than ``least`` or :func:`lowbit_gemm` takes a dense
+    product that it does not split.  Product and norm, us, of slabs / of the 16-bit
+    result: fp8_e5m2 [3584, 18944] of 300 rows, three slabs, 70.3 / 73.9; a product in
+    one piece has no pass to save, and its slab is twice the bytes: [3584, 3584] of 300
+    rows 24.9 / 24.0, sym_int4 [4096, 14336] of 512 rows 86.3 / 83.8.  Pass and norm /
+    norm alone of the dense [4096, 14336] of 1024 rows 22.5 / 16.2."""
     ops = torch.ops.ipex_llm_amd
     M = x.numel() // k
     if torch.is_grad_enabled() and x.requires_grad:
         return None
     if use_rows(x, M, n, k, fmt):
-        return ops.gemm_rows_slabs(x, blob, fmt, n, k, rows_fine(x.dtype, M, n, k, fmt))
+        fine = rows_fine(x.dtype, M, n, k, fmt)
+        if least > 1 and ops.gemv_slabs(M, n, k, fmt, x.dtype == torch.bfloat16, 0, fine) < least:
+            return None
+        return ops.gemm_rows_slabs(x, blob, fmt, n, k, fine)
     if use_g8(x, M, n, k, fmt) or not use_g8d(x, M, n, k) or ops.gemm_bf16_split(M, n, k) < 2:
         return None
 

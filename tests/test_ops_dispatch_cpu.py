@@ -106,6 +106,21 @@ def test_traced_slabs_are_the_plans(name):
             assert y.shape == (o.gemm_bf16_split(M, N, K), M, N)
 
 
+def test_a_product_in_one_piece_leaves_no_slabs_to_the_norm():
+    """the decoder asks for two slabs at least: of one, f32 and written and read once more, the norm saves nothing"""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    import ipex_llm_amd.ops as ops
+    ops.require()
+    with FakeTensorMode():
+        blob = torch.empty(64, dtype=torch.uint8, device="cuda")
+        for M, n, k, S in [(300, 3584, 3584, 1), (512, 4096, 14336, 1), (300, 3584, 18944, 3), (128, 4096, 4096, 2)]:
+            x = torch.empty(M, k, dtype=torch.bfloat16, device="cuda")
+            part = G.lowbit_slabs(x, blob, 6 if n == 3584 else 0, n, k, least=2)
+            assert (part is None) if S == 1 else part.shape == (S, M, n), (M, n, k)
+            assert G.lowbit_slabs(x, blob, 6 if n == 3584 else 0, n, k).shape == (S, M, n)
+
+
 def test_traced_slabs_of_unknown_rows():
     import torch
     from torch._subclasses.fake_tensor import FakeTensorMode
