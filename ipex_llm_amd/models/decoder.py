@@ -243,6 +243,13 @@ class NativeLayer(nn.Module):
         self.post_feedforward_layernorm = nn.Parameter(post_ff, requires_grad=False) if post_ff is not None else None
 
 
+def _watched(mod: nn.Module) -> bool:
+    """something of the program's own sees a call of the module: its hooks, those of
+    all modules, a forward of its own"""
+    return bool(mod._forward_hooks or mod._forward_pre_hooks or "forward" in mod.__dict__
+                or nn.modules.module._has_any_global_hook())
+
+
 def linear(x: torch.Tensor, mod: nn.Module) -> torch.Tensor:
     return mod(x)
 
@@ -505,7 +512,7 @@ class NativeCausalLM(nn.Module):
         part = None
         if (type(proj) is LowBitLinear and proj.bias is None and proj.g_idx_map is None and post_norm_w is None
                 and self.tp_group is None and proj.mp_group is None and x.dim() == 2 and x.dtype == residual.dtype
-                and ops.native_gpu(x) and not (proj._forward_hooks or proj._forward_pre_hooks)):
+                and ops.native_gpu(x) and not _watched(proj)):
             from ..ops.gemm import lowbit_slabs
             part = lowbit_slabs(x, proj.weight, proj.fmt, proj.out_features, proj.in_features, least=2)
         if part is not None:
