@@ -8,9 +8,9 @@
 // copy, beside 11 GFLOP), so the split is made for the stream:
 //   * workgroup = NW = 8 (4) waves = 128 (64) output columns x R = MT * 16 rows;
 //     wave (cg, kp) owns two 16-column weight tiles (cg) and every second 128-k
-//     chunk (kp): codes go global -> registers in MFMA A-fragment order
-//     (formats.h), PF chunks of both tiles in flight per wave, and no weight
-//     is read twice by a row block;
+//     chunk (kp): codes go global -> registers in MFMA fragment order
+//     (formats.h), a ring of three chunks of both tiles per wave, requested two
+//     steps ahead, and no weight is read twice by a row block;
 //   * x is staged through LDS once per workgroup and 256-k step (three buffers: one is read, one is ahead, one is
 //     stored into), XOR-swizzled in 16-B pieces so the 16 rows of a fragment read fall on distinct banks;
 //   * x is the A operand and the codes are the B operand, raw (exact in bf16 / f16): a lane holds four rows of ONE
