@@ -940,11 +940,14 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   a.N = (int)(n / 2);
   a.out = out.data_ptr();
   a.ldo = (int)(n / 2);
-  if (skinny16((int)fmt, bf16, M, NT, KC, illm::EPI_GLU, 1)) {
+  const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
+  // the skinny kernel also for rows whose x v5's LDS does not hold: 4 bits, a K of 8192 from 9 rows on; 8-bit codes of such
+  // a K and tables under bf16 have no kernel for them
+  const bool other = (illm::fmt_bits((int)fmt) == 4 || KC < 64) && !(bf16 && illm::fmt_to_dk((int)fmt) == illm::DK_LUT4);
+  if (skinny16((int)fmt, bf16, M, NT, KC, illm::EPI_GLU, 1) || (other && p.shmem > kMaxLds)) {
     launch_skinny_any((int)fmt, bf16, skinny_plan((int)fmt, false, M, NT, KC, false), illm::EPI_GLU, a);
     return out;
   }
-  const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
   TORCH_CHECK(p.shmem <= kMaxLds, "gemv_glu_ss: x slice exceeds LDS");
   a.nw = p.nw;
   launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_GLU, dim3(p.gx, 1), p.shmem, a);

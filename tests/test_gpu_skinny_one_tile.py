@@ -57,6 +57,25 @@ def test_rows_and_tails(cuda, name, dtype):
                 assert _rel(y, want) < 2 * STORE, (n, k, M)
 
 
+@pytest.mark.parametrize("name,k,takes", [("sym_int4", 8192, True), ("asym_int4", 8192, True), ("fp4", 12288, True),
+                                          ("fp8_e5m2", 5120, True), ("fp8_e5m2", 8192, False), ("nf4", 8192, False)])
+def test_rows_that_the_decode_kernel_cannot_hold(cuda, name, k, takes):
+    """the pair of a deferred norm: taken by the skinny kernel where its rule leaves it to a kernel without the LDS for it"""
+    from ipex_llm_amd.models.decoder import deinterleave_glu
+    f, n = get_format(name).fmt, 1024
+    torch.manual_seed(8)
+    blob = ops.quantize(torch.randn(n, k, device=cuda) * 0.05, f)
+    W = R.dequantize_device_blob(blob, f, n, k).to(cuda).double()
+    for M in (5, 16):
+        x, ss = torch.randn(M, k, device=cuda).bfloat16(), torch.rand(M, device=cuda) * k + 1.0
+        if M == 16 and not takes:
+            with pytest.raises(RuntimeError, match="exceeds LDS"):
+                ops.gemv_glu_ss(x, blob, f, n, k, 0, ss, k, 1e-5)
+            continue
+        g, u = deinterleave_glu(x.double() @ W.t() * torch.rsqrt(ss.double() / k + 1e-5)[:, None])
+        assert _rel(ops.gemv_glu_ss(x, blob, f, n, k, 0, ss, k, 1e-5), torch.nn.functional.silu(g) * u) < 2 * STORE, M
+
+
 @pytest.mark.parametrize("name", ["sym_int4", "sym_int8", "fp8_e5m2"])
 def test_split_by_rows(cuda, name):
     """a long K whose x does not fit the decode kernel's LDS at these rows, and one just below"""
