@@ -293,7 +293,7 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 // Up to 16 rows, input and output in memory: the skinny kernel's one row tile instead of v5, by the format and the
 // shape, so that a row keeps its bits beside any other rows (1 to 16).  Not table formats under bf16 (v5 keeps an f16
 // table, the skinny kernel one in the type of x).
-//   * gate/up, where no number of rows is slower by more than the runs differ.  v5's chain of one pair is the shorter at one
+//   * gate/up, where one and two rows do not pay for the others.  v5's chain of one pair is the shorter at one
 //     and two rows (K cut in two within a group, deeper prefetch), so few pairs stay there unless K is short or decoding is
 //     long (minima, tables, integer bytes); with more than a round of its groups, one of 4 waves per CU and 2 pairs each, the
 //     stream counts.  Weights that no cache holds, v5 / this, us at 1 / 2 / 4 / 16 rows: sym_int4 [28672, 4096] 15.8 15.9
@@ -303,7 +303,8 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 //     7.5 7.7 7.8 7.7.  Not so: sym_int4 [7168, 4096] 9.4 9.6 12.7 20.4 / 11.2 11.4 11.4 11.5, [14336, 2048] 7.3 7.2 9.1 11.0 /
 //     7.7 7.8 7.9 7.8, [18944, 8192] 23.7 25.0 25.7 27.4 / 26.6 26.6 26.6 27.4, fp4 [7168, 8192] 13.8 15.2 20.6 21.1 / 18.6 18.7
 //     18.8 18.8, fp8_e5m2 [7168, 4096] 10.9 11.7 17.3 21.5 / 12.1 12.3 12.4 12.5, sym_int8 [7168, 7168] 17.6 18.7 28.6 20.6 /
-//     20.5 20.6 21.0 21.2;
+//     20.5 20.6 21.0 21.2.  What it does take is behind at 8-bit [28672, 3584] (two rows 19.7 / 21.0) and sym_int4 [49152, 6144]
+//     (one row 30.4 / 32.5), by 3 % and less elsewhere;
 //   * slabs and plain products of K 2048 to 5120 and up to 2048 columns, of 8-bit codes from K 3584 on up to 4096 (4 bits: K
 //     to 4096).  Weights that no cache holds, v5 / this, us at 1 / 2 / 4 / 8 / 16 rows, slabs: sym_int4 [2048, 4096] 4.8 4.9
 //     5.2 5.4 5.9 / 4.6 4.7 4.8 4.7 4.8, asym_int4 [1024, 3584] 0.94 to 0.78 of v5, fp8_e5m2 [2048, 2048] 5.1 5.2 5.4 5.6 6.1 /
@@ -311,9 +312,9 @@ bool head16(int fmt, int64_t NT, int64_t KC) { return fmt == illm::FMT_ASYM_INT4
 //     one and two rows or at all: sym_int4 [4096, 4096] 5.4 5.5 5.7 5.9 6.5 / 5.9 6.0 6.0 6.0 6.0, [7168, 5120] 7.5 7.6 8.9 10.0
 //     12.1 / 9.7 9.1 9.2 9.1 9.2, [2048, 1536] 4.4 4.5 4.8 5.0 5.5 / 6.1 6.3 6.3 6.3 6.3, fp8_e5m2 [6144, 2048] 6.0 5.9 6.4 6.6
 //     7.1 / 7.7 7.8 7.8 7.8 7.8; a K of 14336 8.8 8.7 9.2 10.3 / 9.9 9.9 9.9 10.1 (sym_int4 [4096, 14336], 1 / 4 / 8 / 16);
-//   * ... and where v5 would cut K by the number of rows, as its x does not fit the LDS: [3584, 18944] at 16 rows 15.4
-//     and 11.2, [8192, 28672] 35.6 and 26.2, the head [128256, 4096] at 8 rows 129.7 and 54.6 (these rows' bits change
-//     with the number of rows on either path);
+//   * ... and where v5 would cut K by the number of rows, as its x does not fit the LDS: sym_int4 [3584, 18944] at 16 rows
+//     16.3 and 11.7, [8192, 28672] 35.5 and 26.2, the plain product of the head [128256, 4096] at 8 / 16 rows 62.9 86.6 and
+//     51.9 53.5 (these rows' bits change with the number of rows on either path);
 //   * ... and the heads of head16.
 bool skinny16(int fmt, bool bf16, int64_t M, int64_t NT, int64_t KC, int64_t epi, int64_t ksplit) {
   if (bf16 && illm::fmt_to_dk(fmt) == illm::DK_LUT4) return false;
