@@ -286,6 +286,9 @@ void launch_decode_advance(bool bf16, const uint16_t* logits, int B, int V, int6
                            int64_t* pos, const int32_t* block_tables, int max_blocks, int bs, int64_t* slots,
                            int32_t* seq_lens, const int64_t* pos_offset, int* err, hipStream_t st,
                            const float* parts = nullptr, int nparts = 0);
+void launch_decode_set_state(const int64_t* ids, const int64_t* pos, const int64_t* off, int64_t* ids_out,
+                             int64_t* pos_out, int64_t* off_out, const int32_t* block_tables, int max_blocks, int bs,
+                             int64_t* slots, int32_t* seq_lens, int B, int* err, hipStream_t st);
 
 // ---- one-shot / two-shot xGMI peer all-reduce (allreduce.hip) -------------
 constexpr int AR_MAX_RANKS = 8;

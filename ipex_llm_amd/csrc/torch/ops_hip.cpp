@@ -1912,6 +1912,29 @@ void decode_advance(const c10::optional<Tensor>& logits, Tensor& ids, Tensor& ne
                               hp ? (int)parts->size(0) : 0);
 }
 
+// a decode step's tokens, positions and position offsets (none: zeros) with the slots and key counts they give
+void decode_set_state(const Tensor& ids, const Tensor& pos, const c10::optional<Tensor>& off, Tensor& ids_out,
+                      Tensor& pos_out, Tensor& off_out, const Tensor& block_tables, int64_t bs, Tensor& slots,
+                      Tensor& seq_lens) {
+  c10::DeviceGuard g(pos_out.device());
+  const int64_t B = pos_out.numel();
+  const bool ho = off.has_value() && off->defined();
+  const Tensor* longs[] = {&ids, &pos, ho ? &*off : &pos, &ids_out, &pos_out, &off_out, &slots};
+  for (const Tensor* t : longs)
+    TORCH_CHECK(t->is_cuda() && t->device() == pos_out.device() && t->scalar_type() == at::kLong && t->is_contiguous() &&
+                t->numel() == B, "decode_set_state: int64 [B] on one GPU");
+  TORCH_CHECK(seq_lens.device() == pos_out.device() && seq_lens.scalar_type() == at::kInt && seq_lens.is_contiguous() &&
+              seq_lens.numel() == B && block_tables.device() == pos_out.device() && block_tables.scalar_type() == at::kInt &&
+              block_tables.is_contiguous() && block_tables.dim() == 2 && block_tables.size(0) == B && bs > 0,
+              "decode_set_state: int32 lengths [B] and block tables [B, blocks]");
+  if (B == 0) return;
+  illm::launch_decode_set_state(ids.data_ptr<int64_t>(), pos.data_ptr<int64_t>(), ho ? off->data_ptr<int64_t>() : nullptr,
+                                ids_out.data_ptr<int64_t>(), pos_out.data_ptr<int64_t>(), off_out.data_ptr<int64_t>(),
+                                block_tables.data_ptr<int32_t>(), (int)block_tables.size(1), (int)bs,
+                                slots.data_ptr<int64_t>(), seq_lens.data_ptr<int32_t>(), (int)B, kernel_err(pos_out.device()),
+                                cur_stream());
+}
+
 // stream bytes [offset, offset + nbytes) of t's storage through the caches
 // (Infinity-Cache warm-up for the next reader); nbytes < 0 -> to the end
 void l3_prefetch(const Tensor& t, int64_t offset, int64_t nbytes, int64_t wgs) {
@@ -1953,6 +1976,7 @@ TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("gemv_glu_in", &gemv_glu_in);
   m.impl("decode_advance", &decode_advance);
   m.impl("gemv_argmax", &gemv_argmax);
+  m.impl("decode_set_state", &decode_set_state);
   m.impl("embed_rms_norm", &embed_rms_norm);
   m.impl("l3_prefetch", &l3_prefetch);
   m.impl("rope_kv_fused", &rope_kv_fused);

@@ -139,7 +139,18 @@ class DecodeStep:
         self.pos.copy_(pos0)
         self._refresh()
 
+    def _state_like(self, t) -> bool:
+        """what one launch can read: int64 [B] on the step's GPU, no memory of the step's own state"""
+        return (isinstance(t, torch.Tensor) and t.device == self.pos.device and t.dtype == torch.long
+                and t.shape == self.pos.shape and t.is_contiguous()
+                and all(t.untyped_storage().data_ptr() != s.untyped_storage().data_ptr()
+                        for s in (self.ids, self.pos, self.off, self.slots)))
+
     def set_state(self, ids: torch.Tensor, pos: torch.Tensor, off: Optional[torch.Tensor] = None):
+        if self.native_glue and all(self._state_like(t) for t in (ids, pos, off) if t is not None):
+            torch.ops.ipex_llm_amd.decode_set_state(ids, pos, off, self.ids, self.pos, self.off, self.block_tables,
+                                                    self.cache.bs, self.slots, self.seq_lens)
+            return
         self.ids.copy_(ids)
         self.pos.copy_(pos)
         if off is not None:
