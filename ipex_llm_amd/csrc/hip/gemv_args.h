@@ -1,6 +1,7 @@
 // Host/device-shared argument block and enums of the low-bit GEMV
 // (lowbit_gemv5.cuh, lowbit_skinny.cuh).  No device code: included by the torch op wrappers.
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "../common/formats.h"
@@ -109,6 +110,9 @@ struct GemvArgs {
   const float* xpss;
   int xpss_n;
   float xpss_eps;
+  // > 0: xpss is [M][xpss_parts], parts of the rows' sums (lowbit_fullk.cuh); GLU launches and, scaling their sums
+  // before they are rotated or added, plain EPI_ATOMIC ones (parts a multiple of 4)
+  int xpss_parts;
   // NeoX RoPE applied to the split-K partial sums before the atomic add
   // (rotation is linear, so the accumulator ends up holding rotated q / k):
   // output columns [0, rcols) are heads of rD dims, rotated at position
@@ -138,5 +142,25 @@ struct GemvArgs {
   float* lss;
   int lunit;
 };
+
+// lowbit_fullk.cuh: h = rnd(rnd(x W^T) + res) -> res_out, rnd(w * h) -> xo, sums of squares of h by 16 columns -> ss
+struct FullkArgs {
+  const uint16_t* x;       // [M, ldx] activations
+  int M, K, ldx;
+  const uint8_t* w;        // device blob (formats.h)
+  int N, KC;
+  int lut_fmt;             // DK_LUT4: FMT_NF4 / FMT_NF3
+  const uint16_t* res;     // [M, N]
+  uint16_t* res_out;       // [M, N], not res
+  const uint16_t* nw;      // [N] norm weight (unit: stored as w - 1)
+  int unit;
+  uint16_t* xo;            // [M, N]
+  float* ss;               // [M, ceil(N / 16)]
+  float* zero;             // [M, N] to clear (an accumulator whose readers ran earlier in the stream), or null
+  uint32_t nib_mask, nib_magic;
+};
+
+template <int DK>
+void launch_fullk_dk(bool bf16, const FullkArgs& a, hipStream_t st);
 
 }  // namespace illm

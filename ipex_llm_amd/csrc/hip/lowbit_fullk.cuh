@@ -1,5 +1,25 @@
 // Low-bit weight x bf16/f16 activations of 1 to 16 rows with the residual add and the deferred RMSNorm behind it (a
 // decode step's o and down projections) on gfx950 MFMA: one workgroup finishes 16 output columns.
+//
+// A projection of 9 to 70 MB at few rows is bound by its chain of latencies, not by its bytes: launch, x from L2, weights,
+// sum over K, and -- where K is cut over workgroups -- f32 atomics, a ticket and the sums read back before the row can be
+// finished, 3 to 5 us of a 5 us product.  So K is not cut over workgroups:
+//   * a workgroup is one 16-column tile, its 8 waves take an eighth of K each and meet once, in LDS; every wave stages its
+//     own x (a piece = 4 chunks of 128 k; 2 from 9 rows on) in an LDS region of its own, so nothing waits for another wave
+//     before the end, and requests its weights before it needs x: all of them where K is one piece a wave (to K = 4096), two
+//     pieces ahead else.  A request out of range is not free (its turn in the address unit, 1 us over the 24 of a wave of
+//     K = 4096 whose ring was 16 chunks deep), hence the exact ends;
+//   * x is the A operand, raw codes the B operand, and the offset a product of x with a constant (lowbit_skinny.cuh): one
+//     scale per lane, one dword load for the four chunks of a piece;
+//   * the rows' sums of squares go out as one number per tile, which the consumer's waves add (RowParts): no atomics, the
+//     same bits each time.
+// Alone, weights that no cache holds, us at 1 / 3 / 8 / 16 rows, split-K with atomics and the last group finishing the rows
+// / this: sym_int4 [4096, 4096] 7.9 8.0 8.9 12.0 / 4.6 4.6 4.8 5.7, asym_int4 8.9 9.2 10.5 13.6 / 4.7 4.8 5.2 6.1, fp8_e5m2
+// [3584, 3584] 9.2 9.4 10.3 12.7 / 4.6 4.8 5.2 6.3 (the split-K product without its rows 6.6 6.8 7.3 8.3).  A long K is
+// bound by x, which every workgroup reads in full (sym_int4 [4096, 14336] 8.8 / 10.1 / 11.9 / 13.2, of 58 MB of x at 8 rows:
+// row_norm_takes in csrc/torch/ops_hip.cpp).  16 waves, or pieces four ahead, were slower.  A decode step of Llama-3-8B
+// sym_int4, 1024 tokens, 1 / 4 / 8 rows: 1572 1844 1981 -> 1499 1635 1809 us, Qwen2.5-7B fp8_e5m2 1 / 5 rows 2149 2372 -> 1995
+// 2182, sym_int4 4 rows 1976 -> 1533.
 #pragma once
 #include <mutex>
 #include <type_traits>
@@ -15,13 +35,14 @@ namespace illm {
 __host__ __device__ constexpr int fullk_pc(int mr) { return mr <= 8 ? 4 : 2; }
 __host__ __device__ constexpr int fullk_row(int mr) { return fullk_pc(mr) * CHUNK_K * 2 + 16; }
 // staged x of every wave, the waves' sums, the pair table
-__host__ __device__ constexpr size_t fullk_shmem(int mr, int nw, bool lut) {
-  return (size_t)nw * mr * fullk_row(mr) + (size_t)nw * mr * 16 * 4 + (lut ? 1024 : 0);
+constexpr int FULLK_NW = 8;                                       // waves of a workgroup, each an eighth of K
+__host__ __device__ constexpr size_t fullk_shmem(int mr, bool lut) {
+  return (size_t)FULLK_NW * mr * fullk_row(mr) + (size_t)FULLK_NW * mr * 16 * 4 + (lut ? 1024 : 0);
 }
 
-// MR: rows of the instantiation (1, 2, 4, 8, 16), a.M <= MR
-template <int DK, typename T, int MR, int NW>
-__global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a) {
+// MR: rows of the instantiation (1, 2, 4, 8, 16), a.M <= MR; RG: pieces of weights in flight, no more than a wave has
+template <int DK, typename T, int MR, int RG>
+__global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const FullkArgs a) {
   using C = typename std::conditional<DK == DK_LUT4, F16, T>::type;   // product type: table formats keep an f16 table
   constexpr int BITS = dk_bits(DK);
   constexpr bool HASMIN = dk_has_min(DK);
@@ -29,7 +50,7 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
   constexpr bool NEEDX = OFFS || HASMIN;
   constexpr int PC = fullk_pc(MR), ROW = fullk_row(MR);
   constexpr int XL = MR * PC / 4;                                 // 1-KB loads of a piece of x (PC chunks of MR rows)
-  constexpr int QL = BITS / 4;
+  constexpr int QL = BITS / 4, NW = FULLK_NW;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -76,37 +97,44 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
   const __amdgpu_buffer_rsrc_t wd =
       __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)tile * TB), 0, (int)TB, 0x00020000);
   const uint32_t soff = (uint32_t)KC * dk_code_chunk(DK), moff = soff + 16u * (uint32_t)KC * 4u;
-  struct Chunk {
-    uint4 q[QL];
-    uint32_t sc, mn[HASMIN ? 1 : 0 + 1];
+  struct Piece {
+    uint4 q[PC][QL];
+    uint32_t sc, mn;                                              // chunk c + lane / 16, column lane % 16
   };
-  auto load_w = [&](Chunk& ch, int c) {                           // past the wave's range: no memory traffic, zeros
-    const bool on = c < c1;
-    const uint32_t cb = (uint32_t)c * dk_code_chunk(DK), cs = (uint32_t)c * 64u;
+  const int cl = g & (PC - 1);
+  auto load_w1 = [&](Piece& w, int c, int i) {                    // (past the wave's range: zeros)
+    const uint32_t cb = (uint32_t)(c + i) * dk_code_chunk(DK) + (uint32_t)lane * 16u;
 #pragma unroll
     for (int j = 0; j < QL; j++)
-      ch.q[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-          wd, on ? cb + (uint32_t)lane * 16u + j * 1024u : ~0u, 0, 2));
-    ch.sc = __builtin_amdgcn_raw_buffer_load_b32(wd, on ? soff + cs + (uint32_t)r16 * 4u : ~0u, 0, 0);
-    if constexpr (HASMIN) ch.mn[0] = __builtin_amdgcn_raw_buffer_load_b32(wd, on ? moff + cs + (uint32_t)r16 * 4u : ~0u, 0, 0);
+      w.q[i][j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wd, c + i < c1 ? cb + j * 1024u : ~0u, 0, 2));
+  };
+  auto load_sc = [&](Piece& w, int c) {
+    const uint32_t cs = c + cl < c1 ? soff + (uint32_t)(c + cl) * 64u + (uint32_t)r16 * 4u : ~0u;
+    w.sc = __builtin_amdgcn_raw_buffer_load_b32(wd, cs, 0, 0);
+    if constexpr (HASMIN) w.mn = __builtin_amdgcn_raw_buffer_load_b32(wd, c + cl < c1 ? cs + (moff - soff) : ~0u, 0, 0);
   };
 
-  uint4 xv[XL];
-  load_x(xv, 0);
+  constexpr int XV = MR <= 4 ? RG : 1;                            // pieces of x ahead
+  uint4 xv[XV][XL];
+#pragma unroll
+  for (int u = 0; u < XV; u++) load_x(xv[u], u);
   // what the last step reads: requested now
   const int om = tid >> 4, on = tile * 16 + r16;                  // output of threads below 16 M
   const bool fin = tid < a.M * 16 && on < a.N;
   uint16_t res16 = 0, nw16 = 0;
   if (fin) {
+    if (a.zero) a.zero[(size_t)om * a.N + on] = 0.f;
     res16 = a.res[(size_t)om * a.N + on];
     nw16 = a.nw[on];
   }
   asm volatile("" ::: "memory");
-  Chunk ring[2][PC];
+  Piece ring[RG];
 #pragma unroll
-  for (int u = 0; u < 2; u++)
+  for (int u = 0; u < RG; u++) {
+    load_sc(ring[u], c0 + u * PC);
 #pragma unroll
-    for (int i = 0; i < PC; i++) load_w(ring[u][i], c0 + u * PC + i);
+    for (int i = 0; i < PC; i++) load_w1(ring[u], c0 + u * PC, i);
+  }
 
   if constexpr (DK == DK_LUT4) {
     for (int i = tid; i < 256; i += NW * 64) lut2[i] = pack2<F16>(hd_lut4(a.lut_fmt, i & 15), hd_lut4(a.lut_fmt, i >> 4));
@@ -118,7 +146,10 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
   const uint8_t* xf = xs + min(r16, MR - 1) * ROW + g * 16;       // rows past MR repeat the last one: never stored
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 acc = zero;
-  auto compute = [&](const Chunk& ch, int i) {
+  auto compute = [&](const Piece& w, int i) {
+    const uint4(&q)[QL] = w.q[i];
+    const int from = (16 * i + r16) * 4;
+    const uint32_t sc = __builtin_amdgcn_ds_bpermute(from, w.sc), mnw = HASMIN ? __builtin_amdgcn_ds_bpermute(from, w.mn) : 0;
 #pragma unroll
     for (int blk = 0; blk < 2; blk++) {
       const uint4 B0 = *(const uint4*)(xf + i * 256 + blk * 128), B1 = *(const uint4*)(xf + i * 256 + blk * 128 + 64);
@@ -129,40 +160,65 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
       }
       uint4 A0, A1;
       if constexpr (BITS == 4) {
-        A0 = raw_a4<DK, C>(blk == 0 ? ch.q[0].x : ch.q[0].z, mask_s, magic_v, lut2);
-        A1 = raw_a4<DK, C>(blk == 0 ? ch.q[0].y : ch.q[0].w, mask_s, magic_v, lut2);
+        A0 = raw_a4<DK, C>(blk == 0 ? q[0].x : q[0].z, mask_s, magic_v, lut2);
+        A1 = raw_a4<DK, C>(blk == 0 ? q[0].y : q[0].w, mask_s, magic_v, lut2);
       } else {
-        A0 = raw_a8<DK, C>(ch.q[blk].x, ch.q[blk].y);
-        A1 = raw_a8<DK, C>(ch.q[blk].z, ch.q[blk].w);
+        A0 = raw_a8<DK, C>(q[blk].x, q[blk].y);
+        A1 = raw_a8<DK, C>(q[blk].z, q[blk].w);
       }
       f32x4 P = mfma16<C>(B0, A0, OFFS ? X : zero);
       P = mfma16<C>(B1, A1, P);
-      const float d = f16_to_f32((uint16_t)(ch.sc >> (16 * blk)));
+      const float d = f16_to_f32((uint16_t)(sc >> (16 * blk)));
 #pragma unroll
       for (int e = 0; e < 4; e++) acc[e] = __builtin_fmaf(d, P[e], acc[e]);
       if constexpr (HASMIN) {
         // X holds const * sum of x (const an exact power of two)
         constexpr float f = OFFS ? -1.f / (std::is_same<C, BF16>::value ? 128.f : 1024.f) : 1.f;
-        const float mn = f * f16_to_f32((uint16_t)(ch.mn[0] >> (16 * blk)));
+        const float mn = f * f16_to_f32((uint16_t)(mnw >> (16 * blk)));
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[e] = __builtin_fmaf(mn, X[e], acc[e]);
       }
     }
   };
 
+  const int np = ((KC + NW - 1) / NW + PC - 1) / PC;              // pieces of the longest wave (host: RG <= np)
   // LDS operations of a wave are done in order: piece p + 1 is stored behind the reads of piece p without a wait
-  auto piece = [&](Chunk (&ch)[PC], int c) {
-    store_x(xv);
-    load_x(xv, (c - c0) / PC + 1);
+  auto piece = [&](auto U, int p, auto more) {
+    Piece& w = ring[decltype(U)::value];
+    uint4(&v)[XL] = xv[decltype(U)::value % XV];
+    const int c = c0 + p * PC;
+    asm volatile("" ::: "memory");
+    store_x(v);
+    asm volatile("" ::: "memory");
+    if (decltype(more)::value || (XV < RG && p + 1 < np)) load_x(v, p + XV);
 #pragma unroll
     for (int i = 0; i < PC; i++) {
-      if (c + i < c1) compute(ch[i], i);
-      load_w(ch[i], c + 2 * PC + i);
+      if (c + i < c1) compute(w, i);
+      if constexpr (decltype(more)::value) load_w1(w, c + RG * PC, i);
     }
+    if constexpr (decltype(more)::value) load_sc(w, c + RG * PC);
   };
-  for (int c = c0; c < c1; c += 2 * PC) {
-    piece(ring[0], c);
-    if (c + PC < c1) piece(ring[1], c + PC);
+  // requests run RG pieces ahead and stop at the last one: a load out of range costs its turn in the address unit
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  constexpr std::integral_constant<int, 0> u0{};
+  constexpr std::integral_constant<int, RG - 1> u1{};
+  if constexpr (RG == 1) {
+    piece(u0, 0, no);
+  } else {
+    int p = 0;
+    for (; p + 4 <= np; p += 2) {
+      piece(u0, p, yes);
+      piece(u1, p + 1, yes);
+    }
+    if (p + 3 == np) {
+      piece(u0, p, yes);
+      piece(u1, p + 1, no);
+      piece(u0, p + 2, no);
+    } else {
+      piece(u0, p, no);
+      piece(u1, p + 1, no);
+    }
   }
 
   // ---- the waves' sums, in the order of K; lane holds column r16 of rows 4 g + e
@@ -189,34 +245,39 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
   if (r16 == 0) a.ss[(size_t)om * gridDim.x + tile] = ss;
 }
 
-template <int DK, typename T, int MR, int NW>
+template <int DK, typename T, int MR, int RG>
 void launch_fullk_t(const FullkArgs& a, hipStream_t st) {
-  constexpr size_t shmem = fullk_shmem(MR, NW, DK == DK_LUT4);
+  constexpr size_t shmem = fullk_shmem(MR, DK == DK_LUT4);
   if (shmem > 64 * 1024) {
     static std::once_flag once;
     std::call_once(once, [&] {
-      if (hipFuncSetAttribute((const void*)lowbit_fullk_kernel<DK, T, MR, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      if (hipFuncSetAttribute((const void*)lowbit_fullk_kernel<DK, T, MR, RG>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)shmem) != hipSuccess)
         (void)hipGetLastError();
     });
   }
-  hipLaunchKernelGGL((lowbit_fullk_kernel<DK, T, MR, NW>), dim3((a.N + 15) / 16), dim3(NW * 64), shmem, st, a);
+  hipLaunchKernelGGL((lowbit_fullk_kernel<DK, T, MR, RG>), dim3((a.N + 15) / 16), dim3(FULLK_NW * 64), shmem, st, a);
 }
-template <int DK, typename T, int NW>
+template <int DK, typename T, int MR>
+void launch_fullk_r(const FullkArgs& a, hipStream_t st) {
+  if ((a.KC + FULLK_NW - 1) / FULLK_NW <= fullk_pc(MR)) launch_fullk_t<DK, T, MR, 1>(a, st);
+  else launch_fullk_t<DK, T, MR, 2>(a, st);
+}
+template <int DK, typename T>
 void launch_fullk_m(const FullkArgs& a, hipStream_t st) {
-  if (a.M == 1) launch_fullk_t<DK, T, 1, NW>(a, st);
-  else if (a.M == 2) launch_fullk_t<DK, T, 2, NW>(a, st);
-  else if (a.M <= 4) launch_fullk_t<DK, T, 4, NW>(a, st);
-  else if (a.M <= 8) launch_fullk_t<DK, T, 8, NW>(a, st);
-  else launch_fullk_t<DK, T, 16, NW>(a, st);
+  if (a.M == 1) launch_fullk_r<DK, T, 1>(a, st);
+  else if (a.M == 2) launch_fullk_r<DK, T, 2>(a, st);
+  else if (a.M <= 4) launch_fullk_r<DK, T, 4>(a, st);
+  else if (a.M <= 8) launch_fullk_r<DK, T, 8>(a, st);
+  else launch_fullk_r<DK, T, 16>(a, st);
 }
 template <int DK>
-void launch_fullk_dk(bool bf16, int nw, const FullkArgs& a0, hipStream_t st) {
+void launch_fullk_dk(bool bf16, const FullkArgs& a0, hipStream_t st) {
   FullkArgs a = a0;
   a.nib_mask = 0x000F000Fu;
   a.nib_magic = bf16 && DK != DK_LUT4 ? Raw<BF16>::k4 : Raw<F16>::k4;
-  if (bf16) nw == 16 ? launch_fullk_m<DK, BF16, 16>(a, st) : launch_fullk_m<DK, BF16, 8>(a, st);
-  else nw == 16 ? launch_fullk_m<DK, F16, 16>(a, st) : launch_fullk_m<DK, F16, 8>(a, st);
+  if (bf16) launch_fullk_m<DK, BF16>(a, st);
+  else launch_fullk_m<DK, F16>(a, st);
 }
 
 }  // namespace illm

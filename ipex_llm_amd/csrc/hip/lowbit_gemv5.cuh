@@ -272,8 +272,11 @@ __device__ __forceinline__ void gemv5_body(const GemvArgs& a, const G5Blk& blk) 
   // GLU over a deferred-norm input staged elsewhere (gemv5_norm_out): the
   // row's sum of squares, requested first, used by the epilogue
   float xss_raw = 0.f;
+  constexpr bool PARTS = (EPI == EPI_GLU || EPI == EPI_ATOMIC) && !MOE;   // ... or its parts (lowbit_fullk.cuh)
+  RowParts<NW> parts;
+  if constexpr (PARTS) parts.request(a, wave, lane);
   if constexpr (EPI == EPI_GLU)
-    if (a.xpss != nullptr && a.xpart == nullptr) xss_raw = a.xpss[orow_of(min(r16, Mloc - 1))];
+    if (a.xpss != nullptr && a.xpart == nullptr && a.xpss_parts == 0) xss_raw = a.xpss[orow_of(min(r16, Mloc - 1))];
   // ---- zero a consumed atomic accumulator (its readers ran earlier in the
   // stream), spread over every workgroup of the grid (up to ~1 MB at M = 8)
   if (a.nzero) {
@@ -773,6 +776,7 @@ __device__ __forceinline__ void gemv5_body(const GemvArgs& a, const G5Blk& blk) 
       commit_x(v, val);
     }
   }
+  if constexpr (PARTS) parts.finish(a, wave, lane, ninv);
   __syncthreads();
   ILLM_GEMV5_STAMP(1);
 #ifdef ILLM_GEMV5_DUMP
@@ -968,6 +972,7 @@ __device__ __forceinline__ void gemv5_body(const GemvArgs& a, const G5Blk& blk) 
           const float pv = tbuf[d < half ? v + half : v - half];
           val = d < half ? val * c - pv * sn : val * c + pv * sn;
         }
+        if (a.xpss_parts > 0) val *= ninv[m];      // (the rotation is linear)
         __hip_atomic_fetch_add(ws + (size_t)m * a.N + n, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
@@ -982,7 +987,7 @@ __device__ __forceinline__ void gemv5_body(const GemvArgs& a, const G5Blk& blk) 
   const int m = orow_of(r16);
   if constexpr (EPI == EPI_GLU) {
     float o[4];
-    const float rs = defer ? ninv[r16]
+    const float rs = defer || a.xpss_parts > 0 ? ninv[r16]
                            : (a.xpss != nullptr && a.xpart == nullptr ? rsqrtf(xss_raw / (float)a.xpss_n + a.xpss_eps)
                                                                       : 1.f);
 #pragma unroll

@@ -104,10 +104,53 @@ __device__ __forceinline__ uint32_t raw_pair8(uint32_t u, bool hi) {
   }
 }
 
+// constant of the offset product: -offset for the formats whose codes carry
+// one, 1 for unsigned codes with a block minimum (the plain sum of x)
+template <int DK, typename T>
+__host__ __device__ constexpr uint32_t raw_const2() {
+  constexpr bool b = std::is_same<T, BF16>::value;
+  // bf16 -136 / -128 / 1, f16 -1032 / -1024 / -128 / 1
+  return DK == DK_INT4S ? (b ? 0xC308C308u : 0xE408E408u)
+       : DK == DK_INT4A ? (b ? 0xC300C300u : 0xE400E400u)
+       : DK == DK_INT8S ? (b ? 0xC300C300u : 0xD800D800u)
+       : (b ? 0x3F803F80u : 0x3C003C00u);
+}
+
 template <int DK, typename C>
 __device__ __forceinline__ uint4 raw_a8(uint32_t lo, uint32_t hi) {
   return make_uint4(raw_pair8<DK, C>(lo, false), raw_pair8<DK, C>(lo, true), raw_pair8<DK, C>(hi, false),
                     raw_pair8<DK, C>(hi, true));
 }
+
+// 1 / rms of the rows of a deferred norm from parts of their sums of squares (GemvArgs::xpss_parts): wave w sums rows w, w
+// + NW ..  request() comes ahead of the other loads; a launch without parts asks for nothing (an empty descriptor).
+template <int NW>
+struct RowParts {
+  static constexpr int R = 16 / NW;
+  f32x4 v[R];
+  __device__ __forceinline__ void request(const GemvArgs& a, int wave, int lane) {
+    const int n = a.xpss_parts;
+    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)a.xpss, 0, n > 0 ? a.M * n * 4 : 0, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int m = wave + i * NW;
+      v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+          rd, lane * 4 < n ? (uint32_t)(m * n + lane * 4) * 4u : ~0u, 0, 0));
+    }
+  }
+  __device__ __forceinline__ void finish(const GemvArgs& a, int wave, int lane, float* inv) const {
+    const int n = a.xpss_parts;
+    if (n <= 0) return;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int m = wave + i * NW;
+      if (m >= a.M) continue;
+      float s = (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+      for (int j = 256 + lane; j < n; j += 64) s += a.xpss[(size_t)m * n + j];
+      s = wave_sum(s);
+      if (lane == 0) inv[m] = rsqrtf(s / (float)a.xpss_n + a.xpss_eps);
+    }
+  }
+};
 
 }  // namespace illm

@@ -46,18 +46,6 @@
 
 namespace illm {
 
-// constant of the offset product: -offset for the formats whose codes carry
-// one, 1 for unsigned codes with a block minimum (the plain sum of x)
-template <int DK, typename T>
-__host__ __device__ constexpr uint32_t skinny_const2() {
-  constexpr bool b = std::is_same<T, BF16>::value;
-  // bf16 -136 / -128 / 1, f16 -1032 / -1024 / -128 / 1
-  return DK == DK_INT4S ? (b ? 0xC308C308u : 0xE408E408u)
-       : DK == DK_INT4A ? (b ? 0xC300C300u : 0xE400E400u)
-       : DK == DK_INT8S ? (b ? 0xC300C300u : 0xD800D800u)
-       : (b ? 0x3F803F80u : 0x3C003C00u);
-}
-
 // 16 B per lane through a buffer descriptor (reads past its range return 0)
 __device__ __forceinline__ uint4 buf16(const __amdgpu_buffer_rsrc_t& r, uint32_t voff, int soff) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
@@ -109,6 +97,11 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   const int cpk = a.cpk;                                          // chunks per split-K slice (even)
   const int c0 = blockIdx.y * cpk, c1 = min(KC, c0 + cpk);
   const int nstep = (c1 - c0 + SK_KW - 1) / SK_KW;
+
+  // x of a deferred norm: its rows' sums of squares, summed behind the first requests (one row tile: 1 to 16 rows)
+  __shared__ float rsum[MT == 1 ? 16 : 1];
+  RowParts<NW> parts;
+  if constexpr (MT == 1) parts.request(a, wave, lane);
 
   if constexpr (DK == DK_LUT4) {
     if (tid < 256) {
@@ -170,7 +163,7 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint32_t mask_s = a.nib_mask, magic_v = opaque_v(a.nib_magic);
-  constexpr uint32_t cst = skinny_const2<DK, T>();
+  constexpr uint32_t cst = raw_const2<DK, T>();
   const uint4 cA = make_uint4(cst, cst, cst, cst);
 
   // ---- a phase = one 64-k block: products of the block's first 32 k (pass a), of its second (pass b), before them the
@@ -313,6 +306,7 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
 #pragma unroll
     for (int j = 0; j < XJ; j++) store_x1(x1[j], XBUF, j);
   }
+  if constexpr (MT == 1) parts.finish(a, wave, lane, rsum);
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < MT; j++) {
@@ -378,7 +372,8 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
         const int m = mr + mt * 16 + e;
         if (m >= a.M) continue;
         // x of a deferred norm: its row's scale
-        const float rs = a.xpss ? rsqrtf(a.xpss[m] / (float)a.xpss_n + a.xpss_eps) : 1.f;
+        const float rs = MT == 1 && a.xpss_parts > 0 ? rsum[m & 15]
+                         : a.xpss ? rsqrtf(a.xpss[m] / (float)a.xpss_n + a.xpss_eps) : 1.f;
         const float gv = o[0][mt][e] * rs, uv = o[1][mt][e] * rs;
         ((uint16_t*)a.out)[(size_t)m * a.ldo + n] = from_f32<T>((a.act == 0 ? silu_f(gv) : gelu_tanh_f(gv)) * uv);
       }

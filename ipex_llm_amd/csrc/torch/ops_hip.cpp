@@ -818,9 +818,21 @@ Tensor gemv_norm_in(const Tensor& acc_in, const Tensor& residual, Tensor& res_ou
   return *acc_out;
 }
 
+// parts of the rows' sums of squares of a deferred-norm input (gemv_row_norm)
+void set_parts(illm::GemvArgs& a, const Tensor& ss, int64_t M, int64_t ss_n, double eps) {
+  TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.is_contiguous() && ss.dim() == 2 && ss.size(0) == M &&
+              ss.size(1) % 4 == 0 && ss.size(1) > 0 && ss.size(1) < (1 << 20) && ss_n > 0 && ((uintptr_t)ss.data_ptr() & 15) == 0,
+              "sums of squares: f32 [M, parts], parts a multiple of 4");
+  a.xpss = ss.data_ptr<float>();
+  a.xpss_parts = (int)ss.size(1);
+  a.xpss_n = (int)ss_n;
+  a.xpss_eps = (float)eps;
+}
+
 void gemv_accum(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, Tensor& acc,
                 int64_t ksplit, const c10::optional<Tensor>& zero, const c10::optional<Tensor>& rope_cs,
-                const c10::optional<Tensor>& rope_pos, int64_t rope_cols, int64_t rope_d) {
+                const c10::optional<Tensor>& rope_pos, int64_t rope_cols, int64_t rope_d,
+                const c10::optional<Tensor>& xss, int64_t xss_n, double xss_eps) {
   TORCH_CHECK(x.is_cuda() && blob.is_cuda() && acc.is_cuda(), "gemv_accum: GPU tensors expected");
   c10::DeviceGuard g(x.device());
   const bool bf16 = is_bf16(x);
@@ -849,6 +861,7 @@ void gemv_accum(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int
   a.cpk = (int)p.cpk;
   a.nw = p.nw;
   set_zero(a, zero);
+  if (xss.has_value() && xss->defined()) set_parts(a, *xss, M, xss_n, xss_eps);
   TORCH_CHECK(p.shmem <= kMaxLds, "gemv_accum: K slice too large for LDS");
   launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_ATOMIC, dim3(p.gx, (unsigned)p.ks), p.shmem, a);
 }
@@ -911,6 +924,74 @@ void gemv_accum_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n
   launch_gemv5_any((int)fmt, bf16, p.kw, illm::EPI_ATOMIC, dim3(p.gx, (unsigned)p.ks), p.shmem, a);
 }
 
+// A down projection that finishes its rows (gemv_row_norm) instead of adding slices of K with atomics for the next
+// layer's qkv launch to normalise: by what a decode step of that shape and format measured (MI355X, Llama-3-8B / Qwen2.5-7B
+// layers, us a step, slices / rows).  Every workgroup reads all of x, so 16 columns of a long K pay in x what they save in
+// atomics:
+//   * 8-bit codes: sym_int8 [4096, 14336] 4 / 8 / 16 rows 2326 2512 2915 / 2321 2489 2829; fp8_e5m2 [3584, 18944] 1 / 5 / 8
+//     / 16 rows 2081 2222 2285 2545 / 1995 2182 2240 2528; alone [8192, 28672] 5 rows 48 / 44;
+//   * 4-bit codes, one workgroup per CU (alone [5120, 13824] 1 row 10.4 / 12.4, [8192, 28672] 3 rows 25.9 / 28.4): asym_int4
+//     [4096, 14336] 9 / 16 rows 2143 2432 / 2070 2338;
+//   * ... not 3 to 8 rows of sym_int4 in slices of up to 7 chunks, which have kernels of their own ([4096, 14336] 1 / 2 / 3 /
+//     4 / 8 / 10 / 16 rows 1523 1546 1584 1635 1809 2011 2528 / 1499 1535 1586 1641 1850 1942 2440; [3584, 18944], slices of
+//     14, 1 / 4 / 8 rows 1588 1600 1762 / 1516 1533 1698);
+//   * ... nor 3 to 12 rows of tables (nf4 [4096, 14336] 4 / 8 / 9 / 16 rows 2123 2416 2579 2958 / 2157 2490 2620 2925).
+bool row_norm_takes(int64_t M, int64_t n, int64_t k, int64_t fmt) {
+  TORCH_CHECK(M >= 1 && n >= 1 && k >= 1, "row_norm_takes: sizes");
+  const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N, KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
+  if (M > 16) return false;
+  if (illm::fmt_bits((int)fmt) == 8) return true;
+  if (NT > 256) return false;
+  if (M <= 2) return true;
+  if (illm::fmt_to_dk((int)fmt) == illm::DK_LUT4) return M > 12;
+  if (fmt != illm::FMT_SYM_INT4 || M > 8) return true;
+  const Plan5 p = plan5(M, NT, KC, true, 0, true, (int)fmt);
+  return p.cpk > 7;
+}
+
+// lowbit_fullk.cuh: x W^T of 1..16 rows, the residual add, the deferred-norm input of the next product and the parts of
+// its rows' sums of squares
+void gemv_row_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, const Tensor& residual,
+                   Tensor& res_out, const Tensor& norm_w, bool unit_offset, Tensor& xo, Tensor& ss,
+                   const c10::optional<Tensor>& zero) {
+  TORCH_CHECK(x.is_cuda() && blob.is_cuda() && x.size(-1) == k, "gemv_row_norm: GPU x [M, k]");
+  c10::DeviceGuard g(x.device());
+  const bool bf16 = is_bf16(x);
+  Tensor xc = rows16(x);
+  const int64_t M = xc.numel() / k, NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N;
+  TORCH_CHECK(M >= 1 && M <= 16 && k % 8 == 0, "gemv_row_norm: 1..16 rows, k a multiple of 8");
+  for (const Tensor* t : {&residual, (const Tensor*)&res_out, &norm_w, (const Tensor*)&xo})
+    TORCH_CHECK(t->device() == x.device() && t->scalar_type() == x.scalar_type() && t->is_contiguous() &&
+                t->numel() == (t == &norm_w ? n : M * n),
+                "gemv_row_norm: residual / res_out / xo [M, n] and norm weight [n] in x's dtype");
+  TORCH_CHECK(res_out.data_ptr() != residual.data_ptr() && xo.data_ptr() != xc.data_ptr(),
+              "gemv_row_norm: res_out / xo must not alias residual / x");
+  TORCH_CHECK(ss.device() == x.device() && ss.scalar_type() == at::kFloat && ss.is_contiguous() && ss.numel() == M * NT,
+              "gemv_row_norm: ss f32 [M, ", NT, "]");
+  TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv_row_norm: weight blob too small");
+  illm::FullkArgs a{};
+  a.x = p16(xc);
+  a.M = (int)M;
+  a.K = a.ldx = (int)k;
+  a.w = blob.data_ptr<uint8_t>();
+  a.N = (int)n;
+  a.KC = (int)(illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K);
+  a.lut_fmt = (int)fmt;
+  a.res = p16(residual);
+  a.res_out = m16(res_out);
+  a.nw = p16(norm_w);
+  a.unit = unit_offset ? 1 : 0;
+  a.xo = m16(xo);
+  a.ss = ss.data_ptr<float>();
+  if (zero.has_value() && zero->defined()) {
+    TORCH_CHECK(zero->device() == x.device() && zero->scalar_type() == at::kFloat && zero->is_contiguous() &&
+                zero->numel() == M * n, "gemv_row_norm: zero f32 [M, n]");
+    a.zero = zero->data_ptr<float>();
+  }
+  hipStream_t st = cur_stream();
+  ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, a, st));
+}
+
 // gate/up GLU GEMV over a deferred-norm input (gemv_accum_norm's xo): the row
 // scale rsqrt(ss[m] / ss_n + eps) is applied to gate and up before the activation
 Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, int64_t act,
@@ -921,7 +1002,8 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   Tensor xc = rows16(x);
   const int64_t M = xc.numel() / k;
   TORCH_CHECK(M >= 1 && M <= 16 && n % 32 == 0, "gemv_glu_ss: 1..16 rows, n a multiple of 32");
-  TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.numel() >= M, "gemv_glu_ss: ss f32 [>= M]");
+  const bool parted = ss.dim() == 2;                               // [M, parts] of gemv_row_norm
+  TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && (parted || ss.numel() >= M), "gemv_glu_ss: ss f32 [>= M]");
   TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv_glu_ss: weight blob too small");
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N;
   const int64_t KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
@@ -934,9 +1016,13 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   a.KC = (int)KC;
   a.act = (int)act;
   a.lut_fmt = (int)fmt;
-  a.xpss = ss.data_ptr<float>();
-  a.xpss_n = (int)ss_n;
-  a.xpss_eps = (float)eps;
+  if (parted) {
+    set_parts(a, ss, M, ss_n, eps);
+  } else {
+    a.xpss = ss.data_ptr<float>();
+    a.xpss_n = (int)ss_n;
+    a.xpss_eps = (float)eps;
+  }
   Tensor out = at::empty({M, n / 2}, xc.options());
   a.N = (int)(n / 2);
   a.out = out.data_ptr();
@@ -1964,6 +2050,7 @@ int* illm_kernel_err(const c10::Device& dev) { return kernel_err(dev); }
 
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("skinny_geometry(int M, int n, int k, int fmt, bool glu, int ksplit, bool fine=False) -> int[]", &skinny_geometry);
+  m.def("row_norm_takes(int M, int n, int k, int fmt) -> bool", &row_norm_takes);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
   m.def("attn_decode_groups(int batch, int kv_heads, int nsplit) -> int", [](int64_t b, int64_t h, int64_t n) -> int64_t {
     TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_groups: sizes");
@@ -1993,6 +2080,7 @@ TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("gemm_rows_slabs", &gemm_rows_slabs);
   m.impl("gemv_accum", &gemv_accum);
   m.impl("gemv_accum_norm", &gemv_accum_norm);
+  m.impl("gemv_row_norm", &gemv_row_norm);
   m.impl("gemv_glu_ss", &gemv_glu_ss);
   m.impl("gemv_norm_in", &gemv_norm_in);
   m.impl("gemm_glu", &gemm_glu);

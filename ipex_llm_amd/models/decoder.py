@@ -197,6 +197,10 @@ DEFER_MLP_ACC = __import__("os").environ.get("ILLM_DEFER_MLP_ACC", "0") == "1"
 # add_rms_norm launch between attention and MLP (ILLM_ONORM=0 restores it)
 ONORM = __import__("os").environ.get("ILLM_ONORM", "1") != "0"
 ONORM_MIN_M = int(__import__("os").environ.get("ILLM_ONORM_MIN_M", "5"))
+# the o projection (and the down projection, where row_norm_takes in csrc/torch/ops_hip.cpp says so) in launches that
+# finish their rows: residual add, the deferred-norm input of the next launch and the parts of its sums of squares
+# (ops.gemv_row_norm), no atomics and no accumulator to clear.  ILLM_ROW_NORM=0: the split-K launches above
+ROW_NORM = __import__("os").environ.get("ILLM_ROW_NORM", "1") != "0"
 # decode batches up to this size take the fused-RoPE attention (qkv accumulated
 # atomically into one slab read by the attention, re-zeroed by its combine).
 # Measured on MI355X (Llama-3-8B, L=1024): batch 1 1.960 -> 1.910 ms/token,
@@ -545,6 +549,19 @@ class NativeCausalLM(nn.Module):
     def _defer_ok(self, ref: torch.Tensor, T: int) -> bool:
         return DEFER_NORM and T <= min(ACC_MAX_M, DEFER_MAX_M)
 
+    def _row_norm_ok(self) -> bool:
+        """o and down projections whose launch finishes its rows: 16-column tiles, sums of squares in whole fours"""
+        ok = self.__dict__.get("_row_norm_layers")
+        if ok is None:
+            ok = (ROW_NORM and not self._oproj_combine and not DEFER_MLP_ACC
+                  and self.spec.hidden_size % 64 == 0
+                  and all(m.mp_group is None and m.in_features % 8 == 0 and m.out_features == self.spec.hidden_size
+                          for L in self.layers for m in (L.self_attn.o_proj, L.mlp.down_proj))
+                  and all(w.dtype == self.dtype and w.is_contiguous()
+                          for L in self.layers for w in (L.input_layernorm, L.post_attention_layernorm)))
+            self.__dict__["_row_norm_layers"] = ok
+        return ok and self.tp_group is None
+
     def _norm_in_ok(self, ref: torch.Tensor, T: int) -> bool:
         lim = max(NORM_IN_MAX_M, DEFER_MAX_M if self._defer_ok(ref, T) else 0)
         if not (self._norm_in_env and T <= min(ACC_MAX_M, lim) and ref.is_cuda
@@ -697,6 +714,8 @@ class NativeCausalLM(nn.Module):
             if ss_zeroed is not ss_all:
                 ss_all.zero_()
         ss_q = None                     # sums of squares of the current layer's qkv input (deferred)
+        row_norm = defer and self._row_norm_ok()        # o / down that finish their rows (ops.gemv_row_norm)
+        x_ss = None                     # (sums of squares by 16 columns, n, eps) of x: a deferred-norm qkv input
         zero_gu = None                  # consumed gate/up accumulator (batch > DEFER_GLU_MAX_M), zeroed next
         # fused-RoPE decode attention (batch <= ROPE_IN_MAX_M, one token each): the qkv
         # GEMV accumulates into one atomic slab that the attention reads and the
@@ -744,8 +763,8 @@ class NativeCausalLM(nn.Module):
                         residual, consumed, pend = r2, pend, None
                     else:
                         ops.gemv_accum(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, part,
-                                       zero=zero_next, rope=qrope)
-                        zero_next = None
+                                       zero=zero_next, rope=qrope, xss=x_ss)
+                        zero_next = x_ss = None
                     qkv_acc = part
                     part = part.unsqueeze(0)
                 else:
@@ -778,7 +797,10 @@ class NativeCausalLM(nn.Module):
                 H = o.out_features
                 accP, accD = self._acc(H, T, x.device, "P"), self._acc(H, T, x.device, "D")
                 zero_qkv = None
-                onorm = (ONORM and defer and ONORM_MIN_M <= T and not (T > DEFER_GLU_MAX_M and DEFER_MLP_ACC)
+                fin_o = row_norm
+                fin_d = (row_norm and li + 1 < len(self.layers)
+                         and torch.ops.ipex_llm_amd.row_norm_takes(T, H, mlp.down_proj.in_features, mlp.down_proj.fmt))
+                onorm = (ONORM and defer and not row_norm and ONORM_MIN_M <= T and not (T > DEFER_GLU_MAX_M and DEFER_MLP_ACC)
                          and o.mp_group is None and o.bias is None and H % 4 == 0
                          and not (rope_in and self._oproj_combine and o.bias is None))
                 if rope_in and self._oproj_combine and o.bias is None:
@@ -796,7 +818,14 @@ class NativeCausalLM(nn.Module):
                     zero_qkv = qkv_acc
                 else:
                     a = a_rope if rope_in else self._attention(li, attn, q, meta, cache)
-                    if onorm:
+                    if fin_o:
+                        # o_proj + residual add + deferred-norm staging of the gate/up input
+                        r2 = nxt_res(residual)
+                        xo, sp = self._acc(H, T, x.device, "XO", self.dtype), self._acc((H + 15) // 16, T, x.device, "SP")
+                        ops.gemv_row_norm(a, o.weight, o.fmt, H, o.in_features, residual, r2,
+                                          layer.post_attention_layernorm, s.norm_unit_offset, xo, sp, zero=consumed)
+                        residual = r2
+                    elif onorm:
                         # o_proj + residual add + deferred-norm staging of the gate/up input
                         r2 = nxt_res(residual)
                         xo = self._acc(H, T, x.device, "XO", self.dtype)
@@ -806,9 +835,21 @@ class NativeCausalLM(nn.Module):
                         residual = r2
                     else:
                         ops.gemv_accum(a, o.weight, o.fmt, H, o.in_features, accP, 0, zero=consumed)
-                self._reduce(accP, o)
+                if not fin_o:
+                    self._reduce(accP, o)
                 gu, dn = mlp.gate_up_proj, mlp.down_proj
-                if onorm:
+                if fin_o:
+                    act = ops.gemv_glu_ss(xo, gu.weight, gu.fmt, gu.out_features, gu.in_features, s.act, sp,
+                                          s.hidden_size, s.rms_eps)
+                    if fin_d:
+                        r2 = nxt_res(residual)
+                        x, sp = self._acc(H, T, x.device, "XD", self.dtype), self._acc((H + 15) // 16, T, x.device, "SPD")
+                        ops.gemv_row_norm(act, dn.weight, dn.fmt, H, dn.in_features, residual, r2,
+                                          self.layers[li + 1].input_layernorm, s.norm_unit_offset, x, sp)
+                        residual, consumed, x_ss = r2, None, (sp, s.hidden_size, s.rms_eps)
+                        continue
+                    ops.gemv_accum(act, dn.weight, dn.fmt, dn.out_features, dn.in_features, accD, 0)
+                elif onorm:
                     act = ops.gemv_glu_ss(xo, gu.weight, gu.fmt, gu.out_features, gu.in_features, s.act,
                                           ss_all[2 * li + 1], s.hidden_size, s.rms_eps)
                     ops.gemv_accum(act, dn.weight, dn.fmt, dn.out_features, dn.in_features, accD, 0, zero=zero_qkv)

@@ -18,7 +18,7 @@ __all__ = [
     "fp8_quantize_weight", "dense_linear", "check_kernel_errors", "KernelError", "repack_to_device", "repack_from_device", "lowbit_matmul",
     "gemv_partials", "gemv_glu", "add_rms_norm", "rms_norm", "layer_norm", "rope_kv",
     "attn_decode", "glu", "attn_softmax_", "moe_topk", "reduce_partials", "to_fp8_bytes", "GEMV_MAX_M", "gather_kv",
-    "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_glu_ss",
+    "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_row_norm", "gemv_glu_ss",
     "attn_decode_split", "gemv_attn", "gemv_norm_in", "attn_decode_rope", "attn_decode_rope_split", "attn_prefill", "moe_group_topk",
 ]
 
@@ -225,22 +225,53 @@ def gemv_partials(x, blob, fmt, n, k, ksplit: int) -> torch.Tensor:
     return _ops().gemv(x, blob, fmt, n, k, None, 1, ksplit, 0)
 
 
+def _row_scale(ss: torch.Tensor, M: int, ss_n: int, eps: float) -> torch.Tensor:
+    """1 / rms [M, 1] of a deferred norm from its rows' sums of squares: [M] or, from ``gemv_row_norm``, parts [M, parts]"""
+    s = ss[:M].float()
+    return torch.rsqrt((s.sum(-1) if ss.dim() == 2 else s) / ss_n + eps)[:, None]
+
+
 def gemv_accum(x, blob, fmt, n, k, acc: torch.Tensor, ksplit: int = 0,
-               zero: Optional[torch.Tensor] = None, rope=None) -> torch.Tensor:
+               zero: Optional[torch.Tensor] = None, rope=None, xss=None) -> torch.Tensor:
     """acc [M, n] f32 (zero on entry) += x @ W^T via split-K f32 atomics; the
     consumer (add_rms_norm / rope_kv_fused with zero_*=True) re-zeroes it, or
     a later launch does through ``zero`` (a buffer whose readers are done).
     ``rope`` = (cos_sin [max_pos, D/2, 2], pos [M], rotated columns, D): NeoX
     RoPE applied to each split's partial before its atomic add (rotation is
-    linear), so ``acc`` ends up holding rotated q / k."""
+    linear), so ``acc`` ends up holding rotated q / k.  ``xss`` = (ss [M, parts],
+    n, eps) of ``gemv_row_norm``: the rows' scale rsqrt(sum / n + eps)."""
     if _native(x):
         rc, rp, rn, rd = rope if rope is not None else (None, None, 0, 0)
-        _ops().gemv_accum(x, blob, fmt, n, k, acc, ksplit, zero, rc, rp, rn, rd)
+        ss, ss_n, eps = xss if xss is not None else (None, 0, 0.0)
+        _ops().gemv_accum(x, blob, fmt, n, k, acc, ksplit, zero, rc, rp, rn, rd, ss, ss_n, eps)
         return acc
     if zero is not None:
         zero.zero_()
-    acc += _rope_cols(lowbit_matmul(x, blob, fmt, n, k).float(), rope, x.dtype).view_as(acc)
+    y = lowbit_matmul(x, blob, fmt, n, k).float().view_as(acc)
+    if xss is not None:
+        y = y * _row_scale(xss[0], y.shape[0], xss[1], xss[2])
+    acc += _rope_cols(y, rope, x.dtype).view_as(acc)
     return acc
+
+
+def gemv_row_norm(x, blob, fmt, n, k, residual: torch.Tensor, res_out: torch.Tensor, norm_w: torch.Tensor,
+                  unit_offset: bool, xo: torch.Tensor, ss: torch.Tensor, zero: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """One launch without atomics for ``gemv_accum_norm``'s results: res_out = rnd(rnd(x W^T) + residual), xo = rnd(w *
+    res_out), ss [M, ceil(n / 16)] = the sums of squares of res_out by 16 columns (consumers: ``gemv_glu_ss``, ``gemv_accum``
+    with ``xss``).  ``zero`` f32 [M, n] is cleared."""
+    if _native(x):
+        _ops().gemv_row_norm(x, blob, fmt, n, k, residual, res_out, norm_w, unit_offset, xo, ss, zero)
+        return xo
+    if zero is not None:
+        zero.zero_()
+    y = lowbit_matmul(x, blob, fmt, n, k).float().view_as(res_out)
+    h = (y.to(residual.dtype).float() + residual.float()).to(residual.dtype)
+    res_out.copy_(h)
+    w = norm_w.float() + 1.0 if unit_offset else norm_w.float()
+    xo.copy_((w.to(residual.dtype).float() * h.float()).to(residual.dtype))
+    sq = F.pad(h.float().pow(2), (0, -n % 16))
+    ss.copy_(sq.view(h.shape[0], -1, 16).sum(-1))
+    return xo
 
 
 def gemv_accum_norm(x, blob, fmt, n, k, acc: torch.Tensor, ctr: torch.Tensor, residual: torch.Tensor,
@@ -269,12 +300,12 @@ def gemv_accum_norm(x, blob, fmt, n, k, acc: torch.Tensor, ctr: torch.Tensor, re
 
 def gemv_glu_ss(x, blob, fmt, n, k, act: int, ss: torch.Tensor, ss_n: int, eps: float) -> torch.Tensor:
     """act(s x Wg^T) * (s x Wu^T) with s = rsqrt(ss / ss_n + eps) per row: the
-    gate/up GEMV over ``gemv_accum_norm``'s deferred-norm input."""
+    gate/up GEMV over ``gemv_accum_norm``'s (ss [M]) or ``gemv_row_norm``'s (ss [M, parts]) deferred-norm input."""
     if _native(x):
         return _ops().gemv_glu_ss(x, blob, fmt, n, k, act, ss, ss_n, eps)
     from ..models.decoder import deinterleave_glu
     M = x.numel() // k
-    inv = torch.rsqrt(ss[:M].float() / ss_n + eps)[:, None]
+    inv = _row_scale(ss, M, ss_n, eps)
     g, u = deinterleave_glu(lowbit_matmul(x, blob, fmt, n, k).float())
     g, u = g * inv, u * inv
     return ((F.silu(g) if act == 0 else F.gelu(g, approximate="tanh")) * u).to(x.dtype).contiguous()

@@ -1,0 +1,127 @@
+"""The product that finishes its rows (residual add, deferred-norm input, sums of squares by 16 columns) and the launches
+that take its parts, against f64 over the dequantized weights.
+
+Bounds: rounding to 16 bits moves a value by half a step at most, 2^-8 (bf16) or 2^-11 (f16) of itself, and the residual
+add rounds the product first, hence two roundings; beside them the error of the 32-bit sums, 2^-18 of the sum of
+magnitudes for the up to 2^11 additions of one of them, and of the f16 table of the table formats, whose entries are
+2^-11 of themselves off at most."""
+import pytest
+import torch
+
+import ipex_llm_amd.ops as ops
+from ipex_llm_amd.quantize import qtypes as Q
+
+pytestmark = pytest.mark.gpu
+
+HALF = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+# edges: one chunk, fewer chunks than waves, K inside a chunk, ends of a piece of 4 (2) chunks and of two pieces ahead (K of
+# 4096, 4224, 8192, 8320, 12416 over 8 waves), a last tile of 4 columns, the widest K
+SHAPES = [(64, 128), (64, 192), (132, 640), (64, 1088), (320, 2048), (64, 2176), (192, 4096), (64, 4224), (128, 8192),
+          (64, 8320), (64, 12416), (64, 28672)]
+
+
+def fmt_of(q):
+    return Q.get_format(Q.resolve_qtype(q)).fmt
+
+
+def make(q, n, k, M, dtype, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    fmt = fmt_of(q)
+    blob = ops.quantize(torch.randn(n, k, device="cuda", generator=g) * 0.05, fmt)
+    w = ops.dequantize(blob, fmt, n, k, torch.float32).double()
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)        # noqa: E731
+    return fmt, blob, w, r(M, k), r(M, n), r(n)
+
+
+def check(q, n, k, M, dtype, unit=False):
+    fmt, blob, w, x, res, nw = make(q, n, k, M, dtype)
+    NT = (n + 15) // 16
+    full = torch.full((M + 2, n), 7.0, device="cuda", dtype=dtype)              # a row before and behind each output
+    full2, ss = full.clone(), torch.full((M + 2, NT), 7.0, device="cuda")
+    clear = torch.ones(M + 2, n, device="cuda")
+    ops.gemv_row_norm(x, blob, fmt, n, k, res, full[1:-1], nw, unit, full2[1:-1], ss[1:-1], zero=clear[1:-1])
+    for t in (full, full2, ss):
+        assert (t[0] == 7).all() and (t[-1] == 7).all()
+    assert (clear[1:-1] == 0).all() and (clear[0] == 1).all() and (clear[-1] == 1).all()
+    h, xo, ss = full[1:-1], full2[1:-1], ss[1:-1]
+    y = x.double() @ w.t()
+    scale = (x.double().abs() @ w.abs().t())
+    e = HALF[dtype]
+    bound = (y.abs() + (y + res.double()).abs()) * e * 1.01 + scale * (2.0 ** -11 if q in ("nf4", "nf3") else 2.0 ** -18)
+    assert ((h.double() - (y + res.double())).abs() <= bound).all()
+    wv = (nw.double() + 1).to(dtype).double() if unit else nw.double()
+    want = wv * h.double()
+    assert ((xo.double() - want).abs() <= want.abs() * e * 1.001 + 1e-7).all()
+    sq = torch.nn.functional.pad(h.double().pow(2), (0, -n % 16)).view(M, NT, 16).sum(-1)
+    assert torch.allclose(ss.double(), sq, rtol=2e-6, atol=1e-12)
+    # the same bits again, and with other rows beside a row
+    h2, xo2, ss2 = torch.empty_like(h), torch.empty_like(h), torch.empty_like(ss)
+    ops.gemv_row_norm(x, blob, fmt, n, k, res, h2, nw, unit, xo2, ss2)
+    assert torch.equal(h, h2) and torch.equal(xo, xo2) and torch.equal(ss, ss2)
+    h1, xo1, ss1 = h[-1:].clone(), xo[-1:].clone(), ss[-1:].clone()
+    ops.gemv_row_norm(x[-1:], blob, fmt, n, k, res[-1:].clone(), h1, nw, unit, xo1, ss1)
+    assert torch.equal(h1, h[-1:]) and torch.equal(xo1, xo[-1:]) and torch.equal(ss1, ss[-1:])
+
+
+@pytest.mark.parametrize("n,k", SHAPES)
+@pytest.mark.parametrize("q", ["sym_int4", "asym_int4", "fp8_e5m2"])
+def test_shapes(n, k, q):
+    for M in (1, 8, 9):
+        check(q, n, k, M, torch.bfloat16)
+
+
+@pytest.mark.parametrize("q", ["sym_int4", "asym_int4", "nf4", "nf3", "fp4", "sym_int8", "sym_int5", "asym_int5",
+                               "fp8_e4m3", "fp8_e5m2", "fp6"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_formats_and_rows(q, dtype):
+    for M in (1, 2, 3, 4, 5, 8, 9, 16):
+        check(q, 80, 4480, M, dtype, unit=M == 3)
+
+
+def test_refused():
+    fmt, blob, _, x, res, nw = make("sym_int4", 64, 256, 4, torch.bfloat16)
+    ro, xo, ss = torch.empty_like(res), torch.empty_like(res), torch.empty(4, 4, device="cuda")
+    ok = lambda **k: dict(dict(x=x, residual=res, res_out=ro, norm_w=nw, xo=xo, ss=ss), **k)   # noqa: E731
+
+    def call(x, residual, res_out, norm_w, xo, ss):
+        ops.gemv_row_norm(x, blob, fmt, 64, 256, residual, res_out, norm_w, False, xo, ss)
+    call(**ok())
+    for bad in (dict(res_out=res), dict(ss=ss[:, :3].contiguous()), dict(ss=ss.half()), dict(norm_w=nw.float()),
+                dict(residual=res[:3]), dict(xo=xo.t()), dict(x=torch.cat([x] * 5))):
+        with pytest.raises(RuntimeError):
+            call(**ok(**bad))
+
+
+@pytest.mark.parametrize("q,n,k", [("sym_int4", 1024, 512), ("fp8_e5m2", 512, 1024), ("nf4", 256, 512),
+                                   ("sym_int4", 28672, 4096), ("asym_int4", 256, 1088)])
+@pytest.mark.parametrize("M", [1, 3, 8, 16])
+def test_consumers_add_the_parts(q, n, k, M):
+    """gate/up (decode and skinny kernels) and the rotated qkv sums: the launch on parts against the one on whole sums"""
+    fmt, blob, w, x, _, _ = make(q, n, k, M, torch.bfloat16, 1)
+    parts = torch.rand(M, k // 16, device="cuda") * 16
+    whole = parts.double().sum(-1)
+    a = ops.gemv_glu_ss(x, blob, fmt, n, k, 0, parts, k, 1e-5)
+    b = ops.gemv_glu_ss(x, blob, fmt, n, k, 0, whole.float(), k, 1e-5)
+    assert torch.allclose(a.double(), b.double(), rtol=2.0 ** -7, atol=1e-6)   # a scale 1e-7 off: a step in the last place
+    if n > 4096:
+        return
+    D, cols = 128, n // 256 * 128
+    tab = torch.randn(64, D // 2, 2, device="cuda")
+    pos = torch.randint(0, 64, (M,), device="cuda")
+    acc = torch.zeros(M, n, device="cuda")
+    ops.gemv_accum(x, blob, fmt, n, k, acc, rope=(tab, pos, cols, D), xss=(parts, k, 1e-5))
+    y = (x.double() @ w.t()) * torch.rsqrt(whole / k + 1e-5)[:, None]
+    cs = tab[pos].to(torch.bfloat16).double()
+    c, s = (torch.cat([cs[..., i]] * 2, -1)[:, None] for i in (0, 1))
+    r = y[:, :cols].reshape(M, -1, D)
+    y[:, :cols] = (r * c + torch.cat([-r[..., D // 2:], r[..., :D // 2]], -1) * s).reshape(M, cols)
+    assert ((acc.double() - y).norm() / y.norm()).item() < (2e-3 if q == "nf4" else 1e-5)   # (an f16 table)
+
+
+def test_rule():
+    """a down projection finishes its rows: 8 bits; 4 bits of at most one workgroup per CU but for what row_norm_takes names"""
+    f = lambda M, n, k, q: torch.ops.ipex_llm_amd.row_norm_takes(M, n, k, fmt_of(q))      # noqa: E731
+    assert [f(M, 4096, 14336, "sym_int4") for M in (1, 2, 3, 8, 9, 16, 17)] == [True, True, False, False, True, True, False]
+    assert [f(M, 4096, 14336, "nf4") for M in (1, 2, 3, 12, 13)] == [True, True, False, False, True]
+    assert f(8, 3584, 18944, "sym_int4") and f(8, 8192, 28672, "fp8_e5m2") and f(4, 4096, 14336, "asym_int4")
+    assert not f(1, 5120, 13824, "sym_int4")
