@@ -143,24 +143,4 @@ struct GemvArgs {
   int lunit;
 };
 
-// lowbit_fullk.cuh: h = rnd(rnd(x W^T) + res) -> res_out, rnd(w * h) -> xo, sums of squares of h by 16 columns -> ss
-struct FullkArgs {
-  const uint16_t* x;       // [M, ldx] activations
-  int M, K, ldx;
-  const uint8_t* w;        // device blob (formats.h)
-  int N, KC;
-  int lut_fmt;             // DK_LUT4: FMT_NF4 / FMT_NF3
-  const uint16_t* res;     // [M, N]
-  uint16_t* res_out;       // [M, N], not res
-  const uint16_t* nw;      // [N] norm weight (unit: stored as w - 1)
-  int unit;
-  uint16_t* xo;            // [M, N]
-  float* ss;               // [M, ceil(N / 16)]
-  float* zero;             // [M, N] to clear (an accumulator whose readers ran earlier in the stream), or null
-  uint32_t nib_mask, nib_magic;
-};
-
-template <int DK>
-void launch_fullk_dk(bool bf16, const FullkArgs& a, hipStream_t st);
-
 }  // namespace illm

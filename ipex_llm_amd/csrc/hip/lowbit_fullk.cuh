@@ -1,25 +1,28 @@
-// Low-bit weight x bf16/f16 activations of 1 to 16 rows with the residual add and the deferred RMSNorm behind it (a
-// decode step's o and down projections) on gfx950 MFMA: one workgroup finishes 16 output columns.
+// Low-bit weight x bf16/f16 activations of 1 to 16 rows in launches that finish their rows (a decode step's projections) on
+// gfx950 MFMA: o and down with the residual add and the deferred RMSNorm behind them, qkv with bias and rotation, gate/up
+// with the activation.  One workgroup finishes 16 output columns (qkv: the two halves of 16 columns of a head; gate/up: a
+// pair of tiles).
 //
 // A projection of 9 to 70 MB at few rows is bound by its chain of latencies, not by its bytes: launch, x from L2, weights,
 // sum over K, and -- where K is cut over workgroups -- f32 atomics, a ticket and the sums read back before the row can be
 // finished, 3 to 5 us of a 5 us product.  So K is not cut over workgroups:
-//   * a workgroup is one 16-column tile, its 8 waves take an eighth of K each and meet once, in LDS; every wave stages its
-//     own x (a piece = 4 chunks of 128 k; 2 from 9 rows on) in an LDS region of its own, so nothing waits for another wave
-//     before the end, and requests its weights before it needs x: all of them where K is one piece a wave (to K = 4096), two
-//     pieces ahead else.  A request out of range is not free (its turn in the address unit, 1 us over the 24 of a wave of
-//     K = 4096 whose ring was 16 chunks deep), hence the exact ends;
-//   * x is the A operand, raw codes the B operand, and the offset a product of x with a constant (lowbit_skinny.cuh): one
-//     scale per lane, one dword load for the four chunks of a piece;
+//   * a workgroup's 8 waves take an eighth of K each and meet once, in LDS; every wave stages its own x (a piece = 4 chunks
+//     of 128 k; 2 from 9 rows on) in an LDS region of its own, so nothing waits for another wave before the end, and
+//     requests its weights before it needs x: all of them where K is one piece a wave (to K = 4096), two pieces ahead else.
+//     A request out of range is not free (its turn in the address unit, 1 us over the 24 of a wave of K = 4096 whose ring
+//     was 16 chunks deep), hence the exact ends;
+//   * x is the A operand, raw codes the B operand, and the offset a product of x with a constant (lowbit_skinny.cuh), shared
+//     by the workgroup's tiles: one scale per lane, one dword load for the four chunks of a piece;
 //   * the rows' sums of squares go out as one number per tile, which the consumer's waves add (RowParts): no atomics, the
 //     same bits each time.
 // Alone, weights that no cache holds, us at 1 / 3 / 8 / 16 rows, split-K with atomics and the last group finishing the rows
 // / this: sym_int4 [4096, 4096] 7.9 8.0 8.9 12.0 / 4.6 4.6 4.8 5.7, asym_int4 8.9 9.2 10.5 13.6 / 4.7 4.8 5.2 6.1, fp8_e5m2
 // [3584, 3584] 9.2 9.4 10.3 12.7 / 4.6 4.8 5.2 6.3 (the split-K product without its rows 6.6 6.8 7.3 8.3).  A long K is
-// bound by x, which every workgroup reads in full (sym_int4 [4096, 14336] 8.8 / 10.1 / 11.9 / 13.2, of 58 MB of x at 8 rows:
-// row_norm_takes in csrc/torch/ops_hip.cpp).  16 waves, or pieces four ahead, were slower.  A decode step of Llama-3-8B
-// sym_int4, 1024 tokens, 1 / 4 / 8 rows: 1572 1844 1981 -> 1499 1635 1809 us, Qwen2.5-7B fp8_e5m2 1 / 5 rows 2149 2372 -> 1995
-// 2182, sym_int4 4 rows 1976 -> 1533.
+// bound by x, which every workgroup reads in full (sym_int4 [4096, 14336] 8.8 / 10.1 / 11.9 / 13.2, of 58 MB of x at 8 rows;
+// the rules row_norm_takes, row_rope_takes and glu_rows_takes of csrc/torch/ops_hip.cpp, with qkv's and gate/up's figures).
+// 16 waves, or pieces four ahead, were slower.  A decode step, us: Llama-3-8B sym_int4,
+// 1024 tokens, 1 / 4 / 8 rows 1572 1844 1981, with o and down here 1499 1635 1809, and qkv 1473 1599 1774, and gate/up 1379
+// 1551 1769; Qwen2.5-7B fp8_e5m2, 1 / 5 rows 2149 2372, 1995 2182, 1887 2014, 1704 1886.
 #pragma once
 #include <mutex>
 #include <type_traits>
@@ -27,6 +30,7 @@
 #include "../common/quant_block.h"
 #include "gemv_args.h"
 #include "illm_device.h"
+#include "kernels_fullk.h"
 #include "lowbit_raw.h"
 
 namespace illm {
@@ -36,12 +40,13 @@ __host__ __device__ constexpr int fullk_pc(int mr) { return mr <= 8 ? 4 : 2; }
 __host__ __device__ constexpr int fullk_row(int mr) { return fullk_pc(mr) * CHUNK_K * 2 + 16; }
 // staged x of every wave, the waves' sums, the pair table
 constexpr int FULLK_NW = 8;                                       // waves of a workgroup, each an eighth of K
-__host__ __device__ constexpr size_t fullk_shmem(int mr, bool lut) {
-  return (size_t)FULLK_NW * mr * fullk_row(mr) + (size_t)FULLK_NW * mr * 16 * 4 + (lut ? 1024 : 0);
+constexpr int fullk_tiles(int epi) { return epi == FK_NORM ? 1 : 2; }
+__host__ __device__ constexpr size_t fullk_shmem(int mr, int tiles, bool lut) {
+  return (size_t)FULLK_NW * mr * fullk_row(mr) + (size_t)tiles * FULLK_NW * mr * 16 * 4 + (lut ? 1024 : 0);
 }
 
 // MR: rows of the instantiation (1, 2, 4, 8, 16), a.M <= MR; RG: pieces of weights in flight, no more than a wave has
-template <int DK, typename T, int MR, int RG>
+template <int DK, typename T, int MR, int RG, int EPI>
 __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const FullkArgs a) {
   using C = typename std::conditional<DK == DK_LUT4, F16, T>::type;   // product type: table formats keep an f16 table
   constexpr int BITS = dk_bits(DK);
@@ -50,16 +55,17 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
   constexpr bool NEEDX = OFFS || HASMIN;
   constexpr int PC = fullk_pc(MR), ROW = fullk_row(MR);
   constexpr int XL = MR * PC / 4;                                 // 1-KB loads of a piece of x (PC chunks of MR rows)
-  constexpr int QL = BITS / 4, NW = FULLK_NW;
+  constexpr int QL = BITS / 4, NW = FULLK_NW, NT = fullk_tiles(EPI);
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   uint8_t* xs = smem + (size_t)wave * MR * ROW;                   // this wave's alone: no barrier before the sums
-  float* red = (float*)(smem + (size_t)NW * MR * ROW);            // [NW][MR][16]
-  uint32_t* lut2 = (uint32_t*)(red + NW * MR * 16);
+  float* red = (float*)(smem + (size_t)NW * MR * ROW);            // [NT][NW][MR][16]
+  uint32_t* lut2 = (uint32_t*)(red + NT * NW * MR * 16);
 
-  const int tile = blockIdx.x, KC = a.KC;
+  const int KC = a.KC, ht = EPI == FK_ROPE ? a.rD / 32 : 1;       // FK_ROPE: tiles of a head's half
+  const int tile0 = EPI == FK_NORM ? blockIdx.x : EPI == FK_GLU ? 2 * blockIdx.x : blockIdx.x / ht * 2 * ht + blockIdx.x % ht;
   const int c0 = (int)((uint32_t)wave * KC / NW), c1 = (int)((uint32_t)(wave + 1) * KC / NW);
 
   // x: piece p of the wave is chunks c0 + PC p ..; rows past M and k past K or the wave's range: out of the descriptor, 0
@@ -94,24 +100,31 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
 
   // weights: two pieces in flight
   const size_t TB = (size_t)dk_tile_bytes(DK, KC);
-  const __amdgpu_buffer_rsrc_t wd =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)tile * TB), 0, (int)TB, 0x00020000);
+  __amdgpu_buffer_rsrc_t wd[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+    wd[t] = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)(tile0 + t * ht) * TB), 0, (int)TB, 0x00020000);
   const uint32_t soff = (uint32_t)KC * dk_code_chunk(DK), moff = soff + 16u * (uint32_t)KC * 4u;
   struct Piece {
-    uint4 q[PC][QL];
-    uint32_t sc, mn;                                              // chunk c + lane / 16, column lane % 16
+    uint4 q[PC][NT][QL];
+    uint32_t sc[NT], mn[NT];                                      // chunk c + lane / 16, column lane % 16
   };
   const int cl = g & (PC - 1);
   auto load_w1 = [&](Piece& w, int c, int i) {                    // (past the wave's range: zeros)
     const uint32_t cb = (uint32_t)(c + i) * dk_code_chunk(DK) + (uint32_t)lane * 16u;
 #pragma unroll
-    for (int j = 0; j < QL; j++)
-      w.q[i][j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wd, c + i < c1 ? cb + j * 1024u : ~0u, 0, 2));
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int j = 0; j < QL; j++)
+        w.q[i][t][j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wd[t], c + i < c1 ? cb + j * 1024u : ~0u, 0, 2));
   };
   auto load_sc = [&](Piece& w, int c) {
     const uint32_t cs = c + cl < c1 ? soff + (uint32_t)(c + cl) * 64u + (uint32_t)r16 * 4u : ~0u;
-    w.sc = __builtin_amdgcn_raw_buffer_load_b32(wd, cs, 0, 0);
-    if constexpr (HASMIN) w.mn = __builtin_amdgcn_raw_buffer_load_b32(wd, c + cl < c1 ? cs + (moff - soff) : ~0u, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      w.sc[t] = __builtin_amdgcn_raw_buffer_load_b32(wd[t], cs, 0, 0);
+      if constexpr (HASMIN) w.mn[t] = __builtin_amdgcn_raw_buffer_load_b32(wd[t], c + cl < c1 ? cs + (moff - soff) : ~0u, 0, 0);
+    }
   };
 
   constexpr int XV = MR <= 4 ? RG : 1;                            // pieces of x ahead
@@ -119,13 +132,30 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
 #pragma unroll
   for (int u = 0; u < XV; u++) load_x(xv[u], u);
   // what the last step reads: requested now
-  const int om = tid >> 4, on = tile * 16 + r16;                  // output of threads below 16 M
+  const int om = tid >> 4, on = tile0 * 16 + r16;                 // output of threads below 16 M; its (first) column
   const bool fin = tid < a.M * 16 && on < a.N;
   uint16_t res16 = 0, nw16 = 0;
-  if (fin) {
-    if (a.zero) a.zero[(size_t)om * a.N + on] = 0.f;
-    res16 = a.res[(size_t)om * a.N + on];
-    nw16 = a.nw[on];
+  float2 cs = make_float2(1.f, 0.f);
+  float bias[NT] = {};
+  RowParts<NW> parts;
+  __shared__ float rscale[EPI == FK_NORM ? 1 : 16];
+  if constexpr (EPI == FK_NORM) {
+    if (fin) {
+      if (a.zero) a.zero[(size_t)om * a.N + on] = 0.f;
+      res16 = a.res[(size_t)om * a.N + on];
+      nw16 = a.nw[on];
+    }
+  } else {
+    parts.request(a, wave, lane);
+    if constexpr (EPI == FK_ROPE) {
+      if (fin) {
+        if (on < a.rcols) cs = ((const float2*)a.rcs)[(size_t)a.rpos[om] * (a.rD / 2) + on % a.rD];
+        if (a.bias) {
+#pragma unroll
+          for (int t = 0; t < NT; t++) bias[t] = to_f32<T>(a.bias[on + t * ht * 16]);
+        }
+      }
+    }
   }
   asm volatile("" ::: "memory");
   Piece ring[RG];
@@ -145,11 +175,17 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
   const uint4 cA = make_uint4(cst, cst, cst, cst);
   const uint8_t* xf = xs + min(r16, MR - 1) * ROW + g * 16;       // rows past MR repeat the last one: never stored
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-  f32x4 acc = zero;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) acc[t] = zero;
   auto compute = [&](const Piece& w, int i) {
-    const uint4(&q)[QL] = w.q[i];
     const int from = (16 * i + r16) * 4;
-    const uint32_t sc = __builtin_amdgcn_ds_bpermute(from, w.sc), mnw = HASMIN ? __builtin_amdgcn_ds_bpermute(from, w.mn) : 0;
+    uint32_t sc[NT], mnw[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      sc[t] = __builtin_amdgcn_ds_bpermute(from, w.sc[t]);
+      mnw[t] = HASMIN ? __builtin_amdgcn_ds_bpermute(from, w.mn[t]) : 0;
+    }
 #pragma unroll
     for (int blk = 0; blk < 2; blk++) {
       const uint4 B0 = *(const uint4*)(xf + i * 256 + blk * 128), B1 = *(const uint4*)(xf + i * 256 + blk * 128 + 64);
@@ -158,25 +194,29 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
         X = mfma16<C>(B0, cA, X);
         X = mfma16<C>(B1, cA, X);
       }
-      uint4 A0, A1;
-      if constexpr (BITS == 4) {
-        A0 = raw_a4<DK, C>(blk == 0 ? q[0].x : q[0].z, mask_s, magic_v, lut2);
-        A1 = raw_a4<DK, C>(blk == 0 ? q[0].y : q[0].w, mask_s, magic_v, lut2);
-      } else {
-        A0 = raw_a8<DK, C>(q[blk].x, q[blk].y);
-        A1 = raw_a8<DK, C>(q[blk].z, q[blk].w);
-      }
-      f32x4 P = mfma16<C>(B0, A0, OFFS ? X : zero);
-      P = mfma16<C>(B1, A1, P);
-      const float d = f16_to_f32((uint16_t)(sc >> (16 * blk)));
 #pragma unroll
-      for (int e = 0; e < 4; e++) acc[e] = __builtin_fmaf(d, P[e], acc[e]);
-      if constexpr (HASMIN) {
-        // X holds const * sum of x (const an exact power of two)
-        constexpr float f = OFFS ? -1.f / (std::is_same<C, BF16>::value ? 128.f : 1024.f) : 1.f;
-        const float mn = f * f16_to_f32((uint16_t)(mnw >> (16 * blk)));
+      for (int t = 0; t < NT; t++) {
+        const uint4(&q)[QL] = w.q[i][t];
+        uint4 A0, A1;
+        if constexpr (BITS == 4) {
+          A0 = raw_a4<DK, C>(blk == 0 ? q[0].x : q[0].z, mask_s, magic_v, lut2);
+          A1 = raw_a4<DK, C>(blk == 0 ? q[0].y : q[0].w, mask_s, magic_v, lut2);
+        } else {
+          A0 = raw_a8<DK, C>(q[blk].x, q[blk].y);
+          A1 = raw_a8<DK, C>(q[blk].z, q[blk].w);
+        }
+        f32x4 P = mfma16<C>(B0, A0, OFFS ? X : zero);
+        P = mfma16<C>(B1, A1, P);
+        const float d = f16_to_f32((uint16_t)(sc[t] >> (16 * blk)));
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[e] = __builtin_fmaf(mn, X[e], acc[e]);
+        for (int e = 0; e < 4; e++) acc[t][e] = __builtin_fmaf(d, P[e], acc[t][e]);
+        if constexpr (HASMIN) {
+          // X holds const * sum of x (const an exact power of two)
+          constexpr float f = OFFS ? -1.f / (std::is_same<C, BF16>::value ? 128.f : 1024.f) : 1.f;
+          const float mn = f * f16_to_f32((uint16_t)(mnw[t] >> (16 * blk)));
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[t][e] = __builtin_fmaf(mn, X[e], acc[t][e]);
+        }
       }
     }
   };
@@ -223,61 +263,89 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
 
   // ---- the waves' sums, in the order of K; lane holds column r16 of rows 4 g + e
 #pragma unroll
-  for (int e = 0; e < 4; e++)
-    if (4 * g + e < MR) red[(wave * MR + 4 * g + e) * 16 + r16] = acc[e];
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (4 * g + e < MR) red[((t * NW + wave) * MR + 4 * g + e) * 16 + r16] = acc[t][e];
+  if constexpr (EPI != FK_NORM) parts.finish(a, wave, lane, rscale);
   __syncthreads();
   if (tid >= a.M * 16) return;                                    // (whole 16-lane groups)
-  float y = 0.f;
+  float y[NT];
 #pragma unroll
-  for (int w = 0; w < NW; w++) y += red[(w * MR + om) * 16 + r16];
-  auto rnd = [](float v) { return to_f32<T>(from_f32<T>(v)); };
-  float h = 0.f;
-  if (fin) {
-    float wv = to_f32<T>(nw16);
-    if (a.unit) wv = rnd(1.f + wv);
-    h = rnd(rnd(y) + to_f32<T>(res16));
-    a.res_out[(size_t)om * a.N + on] = from_f32<T>(h);
-    a.xo[(size_t)om * a.N + on] = from_f32<T>(wv * h);
+  for (int t = 0; t < NT; t++) {
+    y[t] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) y[t] += red[((t * NW + w) * MR + om) * 16 + r16];
   }
-  float ss = h * h;
+  const float rs = EPI != FK_NORM && a.xpss_parts > 0 ? rscale[om & 15] : 1.f;
+  auto rnd = [](float v) { return to_f32<T>(from_f32<T>(v)); };
+  if constexpr (EPI == FK_NORM) {
+    float h = 0.f;
+    if (fin) {
+      float wv = to_f32<T>(nw16);
+      if (a.unit) wv = rnd(1.f + wv);
+      h = rnd(rnd(y[0]) + to_f32<T>(res16));
+      a.res_out[(size_t)om * a.N + on] = from_f32<T>(h);
+      a.xo[(size_t)om * a.N + on] = from_f32<T>(wv * h);
+    }
+    float ss = h * h;
 #pragma unroll
-  for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 16);
-  if (r16 == 0) a.ss[(size_t)om * gridDim.x + tile] = ss;
+    for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 16);
+    if (r16 == 0) a.ss[(size_t)om * gridDim.x + tile0] = ss;
+  } else if constexpr (EPI == FK_ROPE) {
+    if (!fin) return;
+    const float c = rnd(cs.x), sn = rnd(cs.y);                    // as the model casts its tables
+    const float y0 = __builtin_fmaf(y[0], rs, bias[0]), y1 = __builtin_fmaf(y[NT - 1], rs, bias[NT - 1]);
+    float* o = a.out32 + (size_t)om * a.N + on;
+    o[0] = __builtin_fmaf(-y1, sn, y0 * c);                       // (spelled out: one rounding in every instantiation)
+    o[ht * 16] = __builtin_fmaf(y0, sn, y1 * c);
+  } else {
+    const float gv = y[0] * rs, uv = y[NT - 1] * rs;
+    const int n = blockIdx.x * 16 + r16;
+    if (fin) a.xo[(size_t)om * (a.N / 2) + n] = from_f32<T>((a.act == 0 ? silu_f(gv) : gelu_tanh_f(gv)) * uv);
+  }
 }
 
-template <int DK, typename T, int MR, int RG>
+template <int DK, typename T, int MR, int RG, int EPI>
 void launch_fullk_t(const FullkArgs& a, hipStream_t st) {
-  constexpr size_t shmem = fullk_shmem(MR, DK == DK_LUT4);
+  constexpr int NT = fullk_tiles(EPI);
+  constexpr size_t shmem = fullk_shmem(MR, NT, DK == DK_LUT4);
   if (shmem > 64 * 1024) {
     static std::once_flag once;
     std::call_once(once, [&] {
-      if (hipFuncSetAttribute((const void*)lowbit_fullk_kernel<DK, T, MR, RG>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)shmem) != hipSuccess)
+      if (hipFuncSetAttribute((const void*)lowbit_fullk_kernel<DK, T, MR, RG, EPI>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
         (void)hipGetLastError();
     });
   }
-  hipLaunchKernelGGL((lowbit_fullk_kernel<DK, T, MR, RG>), dim3((a.N + 15) / 16), dim3(FULLK_NW * 64), shmem, st, a);
+  hipLaunchKernelGGL((lowbit_fullk_kernel<DK, T, MR, RG, EPI>), dim3(((a.N + 15) / 16) / NT), dim3(FULLK_NW * 64), shmem, st, a);
 }
-template <int DK, typename T, int MR>
+template <int DK, typename T, int MR, int EPI>
 void launch_fullk_r(const FullkArgs& a, hipStream_t st) {
-  if ((a.KC + FULLK_NW - 1) / FULLK_NW <= fullk_pc(MR)) launch_fullk_t<DK, T, MR, 1>(a, st);
-  else launch_fullk_t<DK, T, MR, 2>(a, st);
+  if ((a.KC + FULLK_NW - 1) / FULLK_NW <= fullk_pc(MR)) launch_fullk_t<DK, T, MR, 1, EPI>(a, st);
+  else launch_fullk_t<DK, T, MR, 2, EPI>(a, st);
+}
+template <int DK, typename T, int EPI>
+void launch_fullk_m(const FullkArgs& a, hipStream_t st) {
+  if (a.M == 1) launch_fullk_r<DK, T, 1, EPI>(a, st);
+  else if (a.M == 2) launch_fullk_r<DK, T, 2, EPI>(a, st);
+  else if (a.M <= 4) launch_fullk_r<DK, T, 4, EPI>(a, st);
+  else if (a.M <= 8) launch_fullk_r<DK, T, 8, EPI>(a, st);
+  else launch_fullk_r<DK, T, 16, EPI>(a, st);
 }
 template <int DK, typename T>
-void launch_fullk_m(const FullkArgs& a, hipStream_t st) {
-  if (a.M == 1) launch_fullk_r<DK, T, 1>(a, st);
-  else if (a.M == 2) launch_fullk_r<DK, T, 2>(a, st);
-  else if (a.M <= 4) launch_fullk_r<DK, T, 4>(a, st);
-  else if (a.M <= 8) launch_fullk_r<DK, T, 8>(a, st);
-  else launch_fullk_r<DK, T, 16>(a, st);
+void launch_fullk_e(int epi, const FullkArgs& a, hipStream_t st) {
+  if (epi == FK_NORM) launch_fullk_m<DK, T, FK_NORM>(a, st);
+  else if (epi == FK_ROPE) launch_fullk_m<DK, T, FK_ROPE>(a, st);
+  else launch_fullk_m<DK, T, FK_GLU>(a, st);
 }
 template <int DK>
-void launch_fullk_dk(bool bf16, const FullkArgs& a0, hipStream_t st) {
+void launch_fullk_dk(bool bf16, int epi, const FullkArgs& a0, hipStream_t st) {
   FullkArgs a = a0;
   a.nib_mask = 0x000F000Fu;
   a.nib_magic = bf16 && DK != DK_LUT4 ? Raw<BF16>::k4 : Raw<F16>::k4;
-  if (bf16) launch_fullk_m<DK, BF16>(a, st);
-  else launch_fullk_m<DK, F16>(a, st);
+  if (bf16) launch_fullk_e<DK, BF16>(epi, a, st);
+  else launch_fullk_e<DK, F16>(epi, a, st);
 }
 
 }  // namespace illm

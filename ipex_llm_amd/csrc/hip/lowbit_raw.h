@@ -128,7 +128,8 @@ template <int NW>
 struct RowParts {
   static constexpr int R = 16 / NW;
   f32x4 v[R];
-  __device__ __forceinline__ void request(const GemvArgs& a, int wave, int lane) {
+  template <typename A>
+  __device__ __forceinline__ void request(const A& a, int wave, int lane) {
     const int n = a.xpss_parts;
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)a.xpss, 0, n > 0 ? a.M * n * 4 : 0, 0x00020000);
 #pragma unroll
@@ -138,7 +139,8 @@ struct RowParts {
           rd, lane * 4 < n ? (uint32_t)(m * n + lane * 4) * 4u : ~0u, 0, 0));
     }
   }
-  __device__ __forceinline__ void finish(const GemvArgs& a, int wave, int lane, float* inv) const {
+  template <typename A>
+  __device__ __forceinline__ void finish(const A& a, int wave, int lane, float* inv) const {
     const int n = a.xpss_parts;
     if (n <= 0) return;
 #pragma unroll

@@ -10,6 +10,7 @@
 
 #include "../common/formats.h"
 #include "../hip/kernels.h"
+#include "../hip/kernels_fullk.h"
 #include "../hip/kernels_skinny.h"
 #include "../hip/gemv_args.h"
 
@@ -819,7 +820,8 @@ Tensor gemv_norm_in(const Tensor& acc_in, const Tensor& residual, Tensor& res_ou
 }
 
 // parts of the rows' sums of squares of a deferred-norm input (gemv_row_norm)
-void set_parts(illm::GemvArgs& a, const Tensor& ss, int64_t M, int64_t ss_n, double eps) {
+template <typename A>
+void set_parts(A& a, const Tensor& ss, int64_t M, int64_t ss_n, double eps) {
   TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.is_contiguous() && ss.dim() == 2 && ss.size(0) == M &&
               ss.size(1) % 4 == 0 && ss.size(1) > 0 && ss.size(1) < (1 << 20) && ss_n > 0 && ((uintptr_t)ss.data_ptr() & 15) == 0,
               "sums of squares: f32 [M, parts], parts a multiple of 4");
@@ -932,17 +934,20 @@ void gemv_accum_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n
 //     / 16 rows 2081 2222 2285 2545 / 1995 2182 2240 2528; alone [8192, 28672] 5 rows 48 / 44;
 //   * 4-bit codes, one workgroup per CU (alone [5120, 13824] 1 row 10.4 / 12.4, [8192, 28672] 3 rows 25.9 / 28.4): asym_int4
 //     [4096, 14336] 9 / 16 rows 2143 2432 / 2070 2338;
-//   * ... not 3 to 8 rows of sym_int4 in slices of up to 7 chunks, which have kernels of their own ([4096, 14336] 1 / 2 / 3 /
+//   * ... of few rows only where the next qkv launch adds slices too (not stored: it takes its input from the sums on its
+//     way, below), as that launch gains more from an input in memory than this one loses (alone, slices then sums / rows then
+//     gemv_rope: sym_int4 [4096, 14336] + [6144, 4096] 4 rows 9.0 + 7.6 / 10.4 + 5.9, 8 rows 9.8 + 9.1 / 11.9 + 6.4, nf4 8 rows
+//     14.1 + 12.2 / 16.0 + 9.4): not 3 to 8 rows of sym_int4 in slices of up to 7 chunks, which have kernels of their own ([4096, 14336] 1 / 2 / 3 /
 //     4 / 8 / 10 / 16 rows 1523 1546 1584 1635 1809 2011 2528 / 1499 1535 1586 1641 1850 1942 2440; [3584, 18944], slices of
 //     14, 1 / 4 / 8 rows 1588 1600 1762 / 1516 1533 1698);
 //   * ... nor 3 to 12 rows of tables (nf4 [4096, 14336] 4 / 8 / 9 / 16 rows 2123 2416 2579 2958 / 2157 2490 2620 2925).
-bool row_norm_takes(int64_t M, int64_t n, int64_t k, int64_t fmt) {
+bool row_norm_takes(int64_t M, int64_t n, int64_t k, int64_t fmt, bool stored) {
   TORCH_CHECK(M >= 1 && n >= 1 && k >= 1, "row_norm_takes: sizes");
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N, KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
   if (M > 16) return false;
   if (illm::fmt_bits((int)fmt) == 8) return true;
   if (NT > 256) return false;
-  if (M <= 2) return true;
+  if (M <= 2 || stored) return true;
   if (illm::fmt_to_dk((int)fmt) == illm::DK_LUT4) return M > 12;
   if (fmt != illm::FMT_SYM_INT4 || M > 8) return true;
   const Plan5 p = plan5(M, NT, KC, true, 0, true, (int)fmt);
@@ -989,7 +994,73 @@ void gemv_row_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
     a.zero = zero->data_ptr<float>();
   }
   hipStream_t st = cur_stream();
-  ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, a, st));
+  ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, illm::FK_NORM, a, st));
+}
+
+// A decode step's qkv projection that stores its rotated rows (gemv_rope) instead of adding slices of K: all, but few rows
+// of a K past one piece a wave at 4 bits, where x is not all requested at once.  Alone, weights that no cache holds, slices
+// (their input in memory) / this, us at 1 / 4 / 8 / 16 rows: sym_int4 [6144, 4096] 6.5 7.1 8.4 11.1 / 5.6 5.9 6.4 7.9, [4608,
+// 3584] 5.0 5.3 6.7 8.6 / 4.9 5.1 5.8 7.3, [3072, 2048] 4.4 4.7 5.9 8.0 / 4.0 4.2 4.7 4.9, nf4 [6144, 4096] 9.5 10.4 11.9 14.9 /
+// 7.9 8.5 9.4 11.0, sym_int8 12.8 14.6 16.0 20.1 / 8.0 8.0 8.3 12.2, fp8_e5m2 [4608, 3584] 7.6 8.3 8.9 11.2 / 5.9 5.9 6.6 9.3,
+// [10240, 8192] 23.2 25.3 27.1 42.0 / 20.9 21.7 25.8 32.2; sym_int4 [10240, 8192] 12.8 13.5 16.4 25.3 / 14.8 15.5 19.6 22.5.
+bool row_rope_takes(int64_t M, int64_t n, int64_t k, int64_t fmt) {
+  TORCH_CHECK(M >= 1 && n >= 1 && k >= 1, "row_rope_takes: sizes");
+  return M <= 16 && (illm::fmt_bits((int)fmt) == 8 || k <= 4096 || M > 8);
+}
+
+// lowbit_fullk.cuh: out [M, n] f32 = x W^T of 1..16 rows (times the rows' scale of a deferred norm, plus bias), columns below
+// rope_cols rotated: what gemv_accum adds up, stored
+void gemv_rope(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, const c10::optional<Tensor>& bias,
+               Tensor& out, const Tensor& rope_cs, const Tensor& rope_pos, int64_t rope_cols, int64_t rope_d,
+               const c10::optional<Tensor>& xss, int64_t xss_n, double xss_eps) {
+  TORCH_CHECK(x.is_cuda() && blob.is_cuda() && x.size(-1) == k, "gemv_rope: GPU x [M, k]");
+  c10::DeviceGuard g(x.device());
+  const bool bf16 = is_bf16(x);
+  Tensor xc = rows16(x);
+  const int64_t M = xc.numel() / k;
+  TORCH_CHECK(M >= 1 && M <= 16 && k % 8 == 0, "gemv_rope: 1..16 rows, k a multiple of 8");
+  TORCH_CHECK(out.device() == x.device() && out.scalar_type() == at::kFloat && out.is_contiguous() && out.numel() == M * n,
+              "gemv_rope: out f32 [M, n]");
+  TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv_rope: weight blob too small");
+  TORCH_CHECK(!bias.has_value() || !bias->defined() || (bias->device() == x.device() && bias->scalar_type() == x.scalar_type() &&
+              bias->is_contiguous() && bias->numel() == n), "gemv_rope: bias [n] in x's dtype");
+  illm::GemvArgs r{};
+  r.N = (int)n;
+  set_rope(r, rope_cs, rope_pos, rope_cols, rope_d, M);
+  TORCH_CHECK(n % rope_d == 0 && rope_pos.is_contiguous() && rope_cs.device() == x.device() && rope_pos.device() == x.device(),
+              "gemv_rope: whole heads");
+  illm::FullkArgs a{};
+  a.x = p16(xc);
+  a.M = (int)M;
+  a.K = a.ldx = (int)k;
+  a.w = blob.data_ptr<uint8_t>();
+  a.N = (int)n;
+  a.KC = (int)(illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K);
+  a.lut_fmt = (int)fmt;
+  a.out32 = out.data_ptr<float>();
+  a.bias = p16o(bias);
+  a.rcs = r.rcs;
+  a.rpos = r.rpos;
+  a.rcols = r.rcols;
+  a.rD = r.rD;
+  if (xss.has_value() && xss->defined()) set_parts(a, *xss, M, xss_n, xss_eps);
+  hipStream_t st = cur_stream();
+  ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, illm::FK_ROPE, a, st));
+}
+
+// gate/up of 1 to 8 rows over gemv_row_norm's parts on lowbit_fullk.cuh: a K of one piece a wave, so that everything is
+// requested at once.  v5 or the skinny kernel (skinny16) / this, weights that no cache holds, us at 1 / 4 / 8 rows: sym_int4
+// [28672, 4096] 16.4 16.4 15.7 / 13.2 14.1 16.3, [37888, 3584] 19.0 18.8 19.2 / 14.4 15.3 18.2, [7168, 4096] 9.6 12.9 15.0 /
+// 5.9 6.1 6.6, [1024, 512] 4.3 4.7 4.9 / 3.5 3.7 4.2, asym_int4 [28672, 4096] 16.2 16.4 16.3 / 14.3 15.3 16.9, [37888, 3584]
+// 20.1 20.5 20.9 / 16.2 18.4 19.3, fp4 15.2 15.6 17.4 / 12.8 13.3 15.2, nf4 22.8 23.1 25.7 / 18.6 19.6 22.6, sym_int8 25.4 25.3
+// 25.3 / 22.1 22.8 24.4, fp8_e5m2 [37888, 3584] 31.2 31.5 31.6 / 23.7 24.5 26.1 (5.9 TB/s), [7168, 4096] 11.9 17.9 19.6 / 7.6
+// 8.0 8.5.  Every pair of tiles reads all of x, so from 5 rows on not where the skinny kernel has one round of workgroups (the
+// two [28672, 4096] above at 8 rows), and not from 9 (28.3 / 16.0 at 16).  A longer K: [27648, 5120] 19.8 19.7 19.1 / 20.9 22.1
+// 28.4, nf4 [57344, 8192] 66 71 81 / 78 84 100.
+bool glu_rows_takes(int64_t M, int64_t NT, int64_t k, int fmt) {
+  if (M > 8 || k > 4096 || k % 8 != 0) return false;
+  const bool ints = fmt == illm::FMT_SYM_INT4 || fmt == illm::FMT_ASYM_INT4;
+  return M <= 4 || !(ints && NT > 1024 && NT <= 2048);
 }
 
 // gate/up GLU GEMV over a deferred-norm input (gemv_accum_norm's xo): the row
@@ -1027,6 +1098,22 @@ Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   a.N = (int)(n / 2);
   a.out = out.data_ptr();
   a.ldo = (int)(n / 2);
+  if (parted && glu_rows_takes(M, NT, k, (int)fmt)) {
+    illm::FullkArgs f{};
+    f.x = a.x;
+    f.M = (int)M;
+    f.K = f.ldx = (int)k;
+    f.w = a.w;
+    f.N = (int)n;
+    f.KC = (int)KC;
+    f.lut_fmt = (int)fmt;
+    f.xo = m16(out);
+    f.act = (int)act;
+    set_parts(f, ss, M, ss_n, eps);
+    hipStream_t st = cur_stream();
+    ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, illm::FK_GLU, f, st));
+    return out;
+  }
   const Plan5 p = plan5(M, NT / 2, KC, false, 0, false, (int)fmt);
   // the skinny kernel also for rows whose x v5's LDS does not hold: 4 bits, a K of 8192 from 9 rows on; 8-bit codes of such
   // a K and tables under bf16 have no kernel for them
@@ -2050,7 +2137,8 @@ int* illm_kernel_err(const c10::Device& dev) { return kernel_err(dev); }
 
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("skinny_geometry(int M, int n, int k, int fmt, bool glu, int ksplit, bool fine=False) -> int[]", &skinny_geometry);
-  m.def("row_norm_takes(int M, int n, int k, int fmt) -> bool", &row_norm_takes);
+  m.def("row_norm_takes(int M, int n, int k, int fmt, bool stored=False) -> bool", &row_norm_takes);
+  m.def("row_rope_takes(int M, int n, int k, int fmt) -> bool", &row_rope_takes);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
   m.def("attn_decode_groups(int batch, int kv_heads, int nsplit) -> int", [](int64_t b, int64_t h, int64_t n) -> int64_t {
     TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_groups: sizes");
@@ -2081,6 +2169,7 @@ TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("gemv_accum", &gemv_accum);
   m.impl("gemv_accum_norm", &gemv_accum_norm);
   m.impl("gemv_row_norm", &gemv_row_norm);
+  m.impl("gemv_rope", &gemv_rope);
   m.impl("gemv_glu_ss", &gemv_glu_ss);
   m.impl("gemv_norm_in", &gemv_norm_in);
   m.impl("gemm_glu", &gemm_glu);

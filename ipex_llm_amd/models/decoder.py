@@ -562,6 +562,17 @@ class NativeCausalLM(nn.Module):
             self.__dict__["_row_norm_layers"] = ok
         return ok and self.tp_group is None
 
+    def _row_rope_ok(self, T: int) -> bool:
+        """every layer's qkv projection in a launch that stores its rotated rows, its input in memory: that launch needs no
+        sums pending, so every down projection but the last has to finish its rows"""
+        H, D = self.spec.hidden_size, self.spec.head_dim
+        t = torch.ops.ipex_llm_amd
+        return all(q.in_features % 8 == 0 and q.out_features % D == 0
+                   and t.row_rope_takes(T, q.out_features, q.in_features, q.fmt)
+                   and (i == 0 or t.row_norm_takes(T, H, d.in_features, d.fmt, True))
+                   for i, (q, d) in enumerate(zip((L.self_attn.qkv_proj for L in self.layers),
+                                                  [None] + [L.mlp.down_proj for L in self.layers])))
+
     def _norm_in_ok(self, ref: torch.Tensor, T: int) -> bool:
         lim = max(NORM_IN_MAX_M, DEFER_MAX_M if self._defer_ok(ref, T) else 0)
         if not (self._norm_in_env and T <= min(ACC_MAX_M, lim) and ref.is_cuda
@@ -722,7 +733,9 @@ class NativeCausalLM(nn.Module):
         # combine launch re-zeroes
         rope_ok = self._rope_in_ok(meta, cache) and self._qkv_native(residual)
         prerot = (GEMV_ROPE and rope_ok and T <= ACC_MAX_M and s.rot_dim == s.head_dim and not s.rope_interleaved
-                  and s.head_dim in (64, 128) and self._qkv_bias_free())
+                  and s.head_dim in (64, 128))
+        row_rope = prerot and row_norm and self._row_rope_ok(T)       # bias and rotation ahead of the store
+        prerot = row_rope or (prerot and self._qkv_bias_free())
         rope_in = rope_ok and (T <= ROPE_IN_MAX_M or prerot)
         qrope = (self.rope_cache, pos, (s.num_heads + s.num_kv_heads) * s.head_dim, s.head_dim) if prerot else None
         nxt_res = lambda r: res_pp[1] if r is res_pp[0] else res_pp[0]
@@ -761,6 +774,10 @@ class NativeCausalLM(nn.Module):
                                          ss=ss_q, rope=qrope, zero=zero_gu)
                         zero_gu = None
                         residual, consumed, pend = r2, pend, None
+                    elif row_rope:
+                        ops.gemv_rope(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, qp.bias, part, qrope,
+                                      xss=x_ss)
+                        x_ss = None
                     else:
                         ops.gemv_accum(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, part,
                                        zero=zero_next, rope=qrope, xss=x_ss)
@@ -776,7 +793,7 @@ class NativeCausalLM(nn.Module):
                                       cache.v_scale, meta.pos_offset, zero_part=T <= ACC_MAX_M,
                                       pss=ss_q, pss_n=s.hidden_size, pss_eps=s.rms_eps)
                 elif not (norm_in and self._oproj_combine and attn.o_proj.bias is None):
-                    a_rope = ops.attn_decode_rope(qkv_acc, qp.bias, self.rope_cache, pos, cache.k[li], cache.v[li],
+                    a_rope = ops.attn_decode_rope(qkv_acc, None if row_rope else qp.bias, self.rope_cache, pos, cache.k[li], cache.v[li],
                                                   meta.block_tables, meta.seq_lens, meta.nsplit, s.scale,
                                                   s.attn_softcap, attn.sliding_window, s.num_heads, s.rot_dim,
                                                   s.rope_interleaved, 1.0, x.dtype, pss=ss_q,
@@ -799,7 +816,8 @@ class NativeCausalLM(nn.Module):
                 zero_qkv = None
                 fin_o = row_norm
                 fin_d = (row_norm and li + 1 < len(self.layers)
-                         and torch.ops.ipex_llm_amd.row_norm_takes(T, H, mlp.down_proj.in_features, mlp.down_proj.fmt))
+                         and torch.ops.ipex_llm_amd.row_norm_takes(T, H, mlp.down_proj.in_features, mlp.down_proj.fmt,
+                                                                     row_rope))
                 onorm = (ONORM and defer and not row_norm and ONORM_MIN_M <= T and not (T > DEFER_GLU_MAX_M and DEFER_MLP_ACC)
                          and o.mp_group is None and o.bias is None and H % 4 == 0
                          and not (rope_in and self._oproj_combine and o.bias is None))

@@ -18,7 +18,7 @@ __all__ = [
     "fp8_quantize_weight", "dense_linear", "check_kernel_errors", "KernelError", "repack_to_device", "repack_from_device", "lowbit_matmul",
     "gemv_partials", "gemv_glu", "add_rms_norm", "rms_norm", "layer_norm", "rope_kv",
     "attn_decode", "glu", "attn_softmax_", "moe_topk", "reduce_partials", "to_fp8_bytes", "GEMV_MAX_M", "gather_kv",
-    "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_row_norm", "gemv_glu_ss",
+    "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_row_norm", "gemv_rope", "gemv_glu_ss",
     "attn_decode_split", "gemv_attn", "gemv_norm_in", "attn_decode_rope", "attn_decode_rope_split", "attn_prefill", "moe_group_topk",
 ]
 
@@ -252,6 +252,23 @@ def gemv_accum(x, blob, fmt, n, k, acc: torch.Tensor, ksplit: int = 0,
         y = y * _row_scale(xss[0], y.shape[0], xss[1], xss[2])
     acc += _rope_cols(y, rope, x.dtype).view_as(acc)
     return acc
+
+
+def gemv_rope(x, blob, fmt, n, k, bias: Optional[torch.Tensor], out: torch.Tensor, rope, xss=None) -> torch.Tensor:
+    """out [M, n] f32 = x @ W^T (times the rows' scale of ``xss``, see ``gemv_accum``) (+ bias), its first columns rotated
+    (``rope`` as in ``gemv_accum``), stored by one launch that reads all of K."""
+    rc, rp, rn, rd = rope
+    if _native(x):
+        ss, ss_n, eps = xss if xss is not None else (None, 0, 0.0)
+        _ops().gemv_rope(x, blob, fmt, n, k, bias, out, rc, rp, rn, rd, ss, ss_n, eps)
+        return out
+    y = lowbit_matmul(x, blob, fmt, n, k).float().view_as(out)
+    if xss is not None:
+        y = y * _row_scale(xss[0], y.shape[0], xss[1], xss[2])
+    if bias is not None:
+        y = y + bias.float()
+    out.copy_(_rope_cols(y, rope, x.dtype).view_as(out))
+    return out
 
 
 def gemv_row_norm(x, blob, fmt, n, k, residual: torch.Tensor, res_out: torch.Tensor, norm_w: torch.Tensor,
