@@ -201,6 +201,11 @@ ONORM_MIN_M = int(__import__("os").environ.get("ILLM_ONORM_MIN_M", "5"))
 # finish their rows: residual add, the deferred-norm input of the next launch and the parts of its sums of squares
 # (ops.gemv_row_norm), no atomics and no accumulator to clear.  ILLM_ROW_NORM=0: the split-K launches above
 ROW_NORM = __import__("os").environ.get("ILLM_ROW_NORM", "1") != "0"
+# ... up to this many sequences where every launch of the step does so (hidden sizes up to 4096).  A step, us, 8 launches a
+# layer with slabs, rope and norm launches of their own / 5: Llama-3-8B sym_int4, 1024 tokens, 10 / 16 sequences 2260 2473 /
+# 1871 2316, 500 tokens, 9 / 16 sequences, asym_int4 2199 2343 / 1795 1984, nf4 2785 3049 / 2544 2788, sym_int8 2655 2807 /
+# 2368 2570; Qwen2.5-7B fp8_e5m2 10 / 16 sequences 2514 2630 / 2245 2387
+ROW_NORM_MAX_M = int(__import__("os").environ.get("ILLM_ROW_NORM_MAX_M", "16"))
 # decode batches up to this size take the fused-RoPE attention (qkv accumulated
 # atomically into one slab read by the attention, re-zeroed by its combine).
 # Measured on MI355X (Llama-3-8B, L=1024): batch 1 1.960 -> 1.910 ms/token,
@@ -546,8 +551,8 @@ class NativeCausalLM(nn.Module):
                 and self.layers[0].input_layernorm.dtype == e.dtype and self.spec.hidden_size % 8 == 0
                 and ops.native_gpu(ids))
 
-    def _defer_ok(self, ref: torch.Tensor, T: int) -> bool:
-        return DEFER_NORM and T <= min(ACC_MAX_M, DEFER_MAX_M)
+    def _defer_ok(self, ref: torch.Tensor, T: int, rows: bool = False) -> bool:
+        return DEFER_NORM and (rows or T <= min(ACC_MAX_M, DEFER_MAX_M))
 
     def _row_norm_ok(self) -> bool:
         """o and down projections whose launch finishes its rows: 16-column tiles, sums of squares in whole fours"""
@@ -562,20 +567,33 @@ class NativeCausalLM(nn.Module):
             self.__dict__["_row_norm_layers"] = ok
         return ok and self.tp_group is None
 
+    def _rows_ok(self, T: int, meta: "AttnMeta", cache) -> bool:
+        """more sequences than the split-K launches serve, up to 16: every launch of the step finishes its rows (or is the
+        skinny gate/up, whose product of up to 4096 k has a kernel for every format)"""
+        s, ref = self.spec, self.layers[0].input_layernorm
+        return (ACC_MAX_M < T <= ROW_NORM_MAX_M and DEFER_NORM and s.hidden_size <= 4096 and self._rope_in_ok(meta, cache)
+                and GEMV_ROPE and s.rot_dim == s.head_dim and not s.rope_interleaved and s.head_dim in (64, 128)
+                and self._norm_in_ok(ref, T, True) and self._qkv_native(ref)
+                and self._row_norm_ok() and self._row_rope_ok(T))
+
     def _row_rope_ok(self, T: int) -> bool:
         """every layer's qkv projection in a launch that stores its rotated rows, its input in memory: that launch needs no
         sums pending, so every down projection but the last has to finish its rows"""
+        known = self.__dict__.setdefault("_row_rope_rows", {})
+        if T in known:
+            return known[T]
         H, D = self.spec.hidden_size, self.spec.head_dim
         t = torch.ops.ipex_llm_amd
-        return all(q.in_features % 8 == 0 and q.out_features % D == 0
+        known[T] = all(q.in_features % 8 == 0 and q.out_features % D == 0
                    and t.row_rope_takes(T, q.out_features, q.in_features, q.fmt)
                    and (i == 0 or t.row_norm_takes(T, H, d.in_features, d.fmt, True))
                    for i, (q, d) in enumerate(zip((L.self_attn.qkv_proj for L in self.layers),
                                                   [None] + [L.mlp.down_proj for L in self.layers])))
+        return known[T]
 
-    def _norm_in_ok(self, ref: torch.Tensor, T: int) -> bool:
+    def _norm_in_ok(self, ref: torch.Tensor, T: int, rows: bool = False) -> bool:
         lim = max(NORM_IN_MAX_M, DEFER_MAX_M if self._defer_ok(ref, T) else 0)
-        if not (self._norm_in_env and T <= min(ACC_MAX_M, lim) and ref.is_cuda
+        if not (self._norm_in_env and (rows or T <= min(ACC_MAX_M, lim)) and ref.is_cuda
                 and not self.spec.sandwich_norm and not self._attn_fuse and not self._glu_in_enabled
                 and self.spec.hidden_size % 8 == 0 and ops.native_gpu(ref)):
             return False
@@ -691,10 +709,11 @@ class NativeCausalLM(nn.Module):
         s = self.spec
         T = ids.shape[0]
         ss_zeroed = None
+        rows = self._rows_ok(T, meta, cache)
         if hidden_in is None and self._embed_norm_ok(ids):
             # one launch: embedding gather (the residual stream), the first
             # layer's RMSNorm and the zeroing of the step's deferred-norm sums
-            defer0 = self._norm_in_ok(self.embed_tokens, T) and self._defer_ok(self.embed_tokens, T)
+            defer0 = self._norm_in_ok(self.embed_tokens, T, rows) and self._defer_ok(self.embed_tokens, T, rows)
             ss_zeroed = self._acc(T, 2 * len(self.layers), ids.device, "SS") if defer0 else None
             residual, x = torch.ops.ipex_llm_amd.embed_rms_norm(ids.contiguous(), self.embed_tokens,
                                                                self.layers[0].input_layernorm, s.rms_eps,
@@ -713,12 +732,12 @@ class NativeCausalLM(nn.Module):
         # norm-in decode: the down projection's atomic accumulator stays pending
         # and the next layer's qkv GEMV adds + normalises it in its prologue;
         # the residual ping-pongs between two buffers (written by one workgroup)
-        norm_in = self._norm_in_ok(residual, T)
+        norm_in = self._norm_in_ok(residual, T, rows)
         pend = None                     # accumulator awaiting residual-add + norm
         consumed = None                 # accumulator read by the last launch: zeroed by the next GEMV
         res_pp = (residual, torch.empty_like(residual)) if norm_in else None
         # deferred norm: per-(layer, norm) row sums of squares, zeroed once per step
-        defer = norm_in and self._defer_ok(residual, T)
+        defer = norm_in and self._defer_ok(residual, T, rows)
         ss_all = None
         if defer:
             ss_all = self._acc(T, 2 * len(self.layers), x.device, "SS")
@@ -732,7 +751,7 @@ class NativeCausalLM(nn.Module):
         # GEMV accumulates into one atomic slab that the attention reads and the
         # combine launch re-zeroes
         rope_ok = self._rope_in_ok(meta, cache) and self._qkv_native(residual)
-        prerot = (GEMV_ROPE and rope_ok and T <= ACC_MAX_M and s.rot_dim == s.head_dim and not s.rope_interleaved
+        prerot = (GEMV_ROPE and rope_ok and (rows or T <= ACC_MAX_M) and s.rot_dim == s.head_dim and not s.rope_interleaved
                   and s.head_dim in (64, 128))
         row_rope = prerot and row_norm and self._row_rope_ok(T)       # bias and rotation ahead of the store
         prerot = row_rope or (prerot and self._qkv_bias_free())
@@ -816,8 +835,8 @@ class NativeCausalLM(nn.Module):
                 zero_qkv = None
                 fin_o = row_norm
                 fin_d = (row_norm and li + 1 < len(self.layers)
-                         and torch.ops.ipex_llm_amd.row_norm_takes(T, H, mlp.down_proj.in_features, mlp.down_proj.fmt,
-                                                                     row_rope))
+                         and (row_rope or torch.ops.ipex_llm_amd.row_norm_takes(T, H, mlp.down_proj.in_features,
+                                                                                mlp.down_proj.fmt)))
                 onorm = (ONORM and defer and not row_norm and ONORM_MIN_M <= T and not (T > DEFER_GLU_MAX_M and DEFER_MLP_ACC)
                          and o.mp_group is None and o.bias is None and H % 4 == 0
                          and not (rope_in and self._oproj_combine and o.bias is None))

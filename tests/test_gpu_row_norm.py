@@ -121,6 +121,7 @@ def test_consumers_add_the_parts(q, n, k, M):
 
 def test_rule():
     """a down projection finishes its rows: 8 bits; 4 bits of at most one workgroup per CU but for what row_norm_takes names"""
+    ops.require()
     f = lambda M, n, k, q: torch.ops.ipex_llm_amd.row_norm_takes(M, n, k, fmt_of(q))      # noqa: E731
     assert [f(M, 4096, 14336, "sym_int4") for M in (1, 2, 3, 8, 9, 16, 17)] == [True, True, False, False, True, True, False]
     assert [f(M, 4096, 14336, "nf4") for M in (1, 2, 3, 12, 13)] == [True, True, False, False, True]
@@ -195,3 +196,75 @@ def test_gate_up_rows(q, n, k):
         # every value rounded, by half a step of itself at most, from 32-bit sums, and the tables' entries
         rel = ((got.double() - want).norm() / want.norm()).item()
         assert rel <= HALF[dtype] + (2.0 ** -10 if q == "nf4" else 2.0 ** -16), (M, rel)
+
+
+@pytest.mark.parametrize("B", [1, 5, 8, 9, 16, 17])
+@pytest.mark.parametrize("q,bias", [("sym_int4", True), ("fp8_e5m2", False)])
+def test_step_of_many_sequences(B, q, bias):
+    """a decode step on either side of every rule by rows, captured and replayed, against the same step in f32"""
+    from transformers import LlamaConfig, Qwen2Config
+    from ipex_llm_amd.engine.runner import Engine
+    from ipex_llm_amd.models.builder import random_native_model
+    import __graft_entry__ as G
+    dev = torch.device("cuda")
+    cfg = (Qwen2Config if bias else LlamaConfig)(vocab_size=512, hidden_size=1024, intermediate_size=2560,
+                                                 num_hidden_layers=3, num_attention_heads=8, num_key_value_heads=2,
+                                                 max_position_embeddings=512)
+    torch.manual_seed(1)
+    m = random_native_model(cfg, q, dev, torch.bfloat16, seed=0)
+    if bias:
+        for L in m.layers:
+            qkv = L.self_attn.qkv_proj
+            qkv.bias = torch.nn.Parameter(torch.randn(qkv.out_features, device=dev, dtype=torch.bfloat16) * 0.2, False)
+    eng = Engine(m)
+    n, steps = 40, 3
+    eng._ensure_cache(B, 64)
+    seqs = [eng.new_sequence(64) for _ in range(B)]
+    prompts = torch.randint(0, 512, (B, n), generator=torch.Generator().manual_seed(7))
+    eng.prefill_batch(seqs, prompts)
+    st = eng.decode_step_obj(seqs, 64, False, True)
+    toks = torch.randint(0, 512, (B, steps), generator=torch.Generator().manual_seed(8))
+    got = []
+    st.set_state(toks[:, 0].to(dev), torch.full((B,), n, device=dev))
+    for i in range(steps):
+        st.ids.copy_(toks[:, i])
+        st.step()
+        got.append(st.logits.float().cpu().clone())
+    W = [L.self_attn.qkv_proj.bias for L in m.layers]
+    for b in {0, B - 1}:
+        ref = _reference(m, torch.cat([prompts[b], toks[b]]), W, G)[n:n + steps]
+        out = torch.stack([g[b] for g in got])
+        assert ((out - ref).norm() / ref.norm()).item() < 3e-2      # 16-bit activations through three layers, as smoke()
+
+
+def _reference(m, ids, biases, G):
+    """``__graft_entry__``'s f32 forward with the qkv bias"""
+    if biases[0] is None:
+        return G._fp32_reference(m, ids)
+    import torch.nn.functional as F
+    from ipex_llm_amd.models.decoder import deinterleave_glu
+    s = m.spec
+
+    def rms(x, w):
+        return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + s.rms_eps) * w.float().cpu()
+    T = ids.shape[0]
+    x = m.embed_tokens.float().cpu()[ids]
+    fr = torch.arange(T, dtype=torch.float32)[:, None] * m.inv_freq.float().cpu()[None]
+    cos, sin = torch.cat([fr.cos()] * 2, -1), torch.cat([fr.sin()] * 2, -1)
+
+    def rope(t):
+        a, b = t.chunk(2, -1)
+        return t * cos[:, None] + torch.cat([-b, a], -1) * sin[:, None]
+    nh, nkv, hd = s.num_heads, s.num_kv_heads, s.head_dim
+    W = lambda mod: mod.dequantize(torch.float32).cpu()              # noqa: E731
+    for L in m.layers:
+        qkv = rms(x, L.input_layernorm) @ W(L.self_attn.qkv_proj).t() + L.self_attn.qkv_proj.bias.float().cpu()
+        q, k, v = qkv.split([nh * hd, nkv * hd, nkv * hd], -1)
+        q, k, v = rope(q.view(T, nh, hd)), rope(k.view(T, nkv, hd)), v.view(T, nkv, hd)
+        k, v = k.repeat_interleave(nh // nkv, 1), v.repeat_interleave(nh // nkv, 1)
+        o = F.scaled_dot_product_attention(q.transpose(0, 1), k.transpose(0, 1), v.transpose(0, 1), is_causal=True,
+                                           scale=s.scale)
+        x = x + o.transpose(0, 1).reshape(T, -1) @ W(L.self_attn.o_proj).t()
+        g, u = deinterleave_glu(rms(x, L.post_attention_layernorm) @ W(L.mlp.gate_up_proj).t())
+        x = x + (F.silu(g) * u) @ W(L.mlp.down_proj).t()
+    return rms(x, m.norm) @ W(m.lm_head).t()
