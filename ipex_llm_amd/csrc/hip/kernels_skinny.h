@@ -10,8 +10,8 @@ namespace illm {
 constexpr int SK_KW = 2;                       // waves along K
 constexpr int SK_TPW = 2;                      // weight tiles per wave
 constexpr int SK_STEP = SK_KW * CHUNK_K;       // k per step
-// dynamic LDS of a workgroup: x of three steps and the table (bytes)
-constexpr size_t skinny_shmem(int mt, int table) { return (size_t)3 * mt * 16 * SK_STEP * 2 + table; }
+// dynamic LDS of a workgroup: x of three steps, the table and, of one row tile, the rows' scales (bytes)
+constexpr size_t skinny_shmem(int mt, int table) { return (size_t)3 * mt * 16 * SK_STEP * 2 + table + (mt == 1 ? 64 : 0); }
 constexpr int skinny_table(bool lut, bool fine) { return !lut ? 0 : fine ? 2048 : 1024; }
 
 // workgroup = nw waves (4 or 8) = nw weight tiles x 16 mt rows (mt 1 .. 4) x a.cpk chunks; grid =

@@ -98,8 +98,9 @@ __global__ void __launch_bounds__(NW * 64, 2) lowbit_skinny_kernel(const GemvArg
   const int c0 = blockIdx.y * cpk, c1 = min(KC, c0 + cpk);
   const int nstep = (c1 - c0 + SK_KW - 1) / SK_KW;
 
-  // x of a deferred norm: its rows' sums of squares, summed behind the first requests (one row tile: 1 to 16 rows)
-  __shared__ float rsum[MT == 1 ? 16 : 1];
+  // x of a deferred norm: its rows' sums of squares, summed behind the first requests (one row tile: 1 to 16 rows; the sums
+  // of more cost the gate/up product of 48 rows what the norm launch took)
+  float* rsum = (float*)(smem + 3 * R * SK_STEP * 2 + skinny_table(DK == DK_LUT4, FINE));
   RowParts<NW> parts;
   if constexpr (MT == 1) parts.request(a, wave, lane);
 
