@@ -6,7 +6,7 @@
 // A projection of 9 to 70 MB at few rows is bound by its chain of latencies, not by its bytes: launch, x from L2, weights,
 // sum over K, and -- where K is cut over workgroups -- f32 atomics, a ticket and the sums read back before the row can be
 // finished, 3 to 5 us of a 5 us product.  So K is not cut over workgroups:
-//   * a workgroup's 8 waves take an eighth of K each and meet once, in LDS; every wave stages its own x (a piece = 4 chunks
+//   * a workgroup's 8 (16) waves take an eighth (a 16th) of K each and meet once, in LDS; every wave stages its own x (a piece = 4 chunks
 //     of 128 k; 2 from 9 rows on) in an LDS region of its own, so nothing waits for another wave before the end, and
 //     requests its weights before it needs x: all of them where K is one piece a wave (to K = 4096), two pieces ahead else.
 //     A request out of range is not free (its turn in the address unit, 1 us over the 24 of a wave of K = 4096 whose ring
@@ -20,7 +20,7 @@
 // [3584, 3584] 9.2 9.4 10.3 12.7 / 4.6 4.8 5.2 6.3 (the split-K product without its rows 6.6 6.8 7.3 8.3).  A long K is
 // bound by x, which every workgroup reads in full (sym_int4 [4096, 14336] 8.8 / 10.1 / 11.9 / 13.2, of 58 MB of x at 8 rows;
 // the rules row_norm_takes, row_rope_takes and glu_rows_takes of csrc/torch/ops_hip.cpp, with qkv's and gate/up's figures).
-// 16 waves, or pieces four ahead, were slower.  A decode step, us: Llama-3-8B sym_int4,
+// 16 waves of a K that 8 hold in one piece, or pieces four ahead, were slower.  A decode step, us: Llama-3-8B sym_int4,
 // 1024 tokens, 1 / 4 / 8 rows 1572 1844 1981, with o and down here 1499 1635 1809, and qkv 1473 1599 1774, and gate/up 1379
 // 1551 1769; Qwen2.5-7B fp8_e5m2, 1 / 5 rows 2149 2372, 1995 2182, 1887 2014, 1704 1886.
 #pragma once
@@ -41,13 +41,14 @@ __host__ __device__ constexpr int fullk_row(int mr) { return fullk_pc(mr) * CHUN
 // staged x of every wave, the waves' sums, the pair table
 constexpr int FULLK_NW = 8;                                       // waves of a workgroup, each an eighth of K
 constexpr int fullk_tiles(int epi) { return epi == FK_NORM ? 1 : 2; }
-__host__ __device__ constexpr size_t fullk_shmem(int mr, int tiles, bool lut) {
-  return (size_t)FULLK_NW * mr * fullk_row(mr) + (size_t)tiles * FULLK_NW * mr * 16 * 4 + (lut ? 1024 : 0);
+__host__ __device__ constexpr size_t fullk_shmem(int mr, int nw, int tiles, bool lut) {
+  return (size_t)nw * mr * fullk_row(mr) + (size_t)tiles * nw * mr * 16 * 4 + (lut ? 1024 : 0);
 }
 
-// MR: rows of the instantiation (1, 2, 4, 8, 16), a.M <= MR; RG: pieces of weights in flight, no more than a wave has
-template <int DK, typename T, int MR, int RG, int EPI>
-__global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const FullkArgs a) {
+// MR: rows of the instantiation (1, 2, 4, 8, 16), a.M <= MR; RG: pieces of weights in flight, no more than a wave has; NW:
+// waves
+template <int DK, typename T, int MR, int RG, int EPI, int NW = FULLK_NW>
+__global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a) {
   using C = typename std::conditional<DK == DK_LUT4, F16, T>::type;   // product type: table formats keep an f16 table
   constexpr int BITS = dk_bits(DK);
   constexpr bool HASMIN = dk_has_min(DK);
@@ -55,7 +56,7 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
   constexpr bool NEEDX = OFFS || HASMIN;
   constexpr int PC = fullk_pc(MR), ROW = fullk_row(MR);
   constexpr int XL = MR * PC / 4;                                 // 1-KB loads of a piece of x (PC chunks of MR rows)
-  constexpr int QL = BITS / 4, NW = FULLK_NW, NT = fullk_tiles(EPI);
+  constexpr int QL = BITS / 4, NT = fullk_tiles(EPI);
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -306,24 +307,31 @@ __global__ void __launch_bounds__(FULLK_NW * 64) lowbit_fullk_kernel(const Fullk
   }
 }
 
-template <int DK, typename T, int MR, int RG, int EPI>
+template <int DK, typename T, int MR, int RG, int EPI, int NW = FULLK_NW>
 void launch_fullk_t(const FullkArgs& a, hipStream_t st) {
   constexpr int NT = fullk_tiles(EPI);
-  constexpr size_t shmem = fullk_shmem(MR, NT, DK == DK_LUT4);
+  constexpr size_t shmem = fullk_shmem(MR, NW, NT, DK == DK_LUT4);
   if (shmem > 64 * 1024) {
     static std::once_flag once;
     std::call_once(once, [&] {
-      if (hipFuncSetAttribute((const void*)lowbit_fullk_kernel<DK, T, MR, RG, EPI>,
+      if (hipFuncSetAttribute((const void*)lowbit_fullk_kernel<DK, T, MR, RG, EPI, NW>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
         (void)hipGetLastError();
     });
   }
-  hipLaunchKernelGGL((lowbit_fullk_kernel<DK, T, MR, RG, EPI>), dim3(((a.N + 15) / 16) / NT), dim3(FULLK_NW * 64), shmem, st, a);
+  hipLaunchKernelGGL((lowbit_fullk_kernel<DK, T, MR, RG, EPI, NW>), dim3(((a.N + 15) / 16) / NT), dim3(NW * 64), shmem, st, a);
 }
 template <int DK, typename T, int MR, int EPI>
 void launch_fullk_r(const FullkArgs& a, hipStream_t st) {
-  if ((a.KC + FULLK_NW - 1) / FULLK_NW <= fullk_pc(MR)) launch_fullk_t<DK, T, MR, 1, EPI>(a, st);
-  else launch_fullk_t<DK, T, MR, 2, EPI>(a, st);
+  if ((a.KC + FULLK_NW - 1) / FULLK_NW <= fullk_pc(MR)) return launch_fullk_t<DK, T, MR, 1, EPI>(a, st);
+  // down projections of few rows whose K is two pieces for each of 16 waves: what hides the second piece is the other
+  // waves, where their registers (128) hold it.  8 / 16 waves, us at 1 / 2 / 3 rows: sym_int4 [4096, 14336] 9.1 9.1 10.3 /
+  // 8.4 8.6 9.2, sym_int8 14.1 14.4 / 13.0 13.4 (3 rows spill: 15.1 / 21.4); three pieces, [3584, 18944], sym_int4 10.0 10.6
+  // 11.6 / 10.3 10.6 11.3, fp8_e5m2 13.7 14.0 / 14.2 14.6; tables 12.6 12.9 / 13.3 14.2
+  if constexpr (EPI == FK_NORM && MR <= (dk_bits(DK) == 4 ? 4 : 2) && DK != DK_LUT4) {
+    if (a.KC > 16 * fullk_pc(MR) && a.KC <= 32 * fullk_pc(MR)) return launch_fullk_t<DK, T, MR, 2, EPI, 16>(a, st);
+  }
+  launch_fullk_t<DK, T, MR, 2, EPI>(a, st);
 }
 template <int DK, typename T, int EPI>
 void launch_fullk_m(const FullkArgs& a, hipStream_t st) {

@@ -33,7 +33,7 @@ def make(q, n, k, M, dtype, seed=0):
     return fmt, blob, w, r(M, k), r(M, n), r(n)
 
 
-def check(q, n, k, M, dtype, unit=False):
+def check(q, n, k, M, dtype, unit=False, alone=True):
     fmt, blob, w, x, res, nw = make(q, n, k, M, dtype)
     NT = (n + 15) // 16
     full = torch.full((M + 2, n), 7.0, device="cuda", dtype=dtype)              # a row before and behind each output
@@ -58,6 +58,8 @@ def check(q, n, k, M, dtype, unit=False):
     h2, xo2, ss2 = torch.empty_like(h), torch.empty_like(h), torch.empty_like(ss)
     ops.gemv_row_norm(x, blob, fmt, n, k, res, h2, nw, unit, xo2, ss2)
     assert torch.equal(h, h2) and torch.equal(xo, xo2) and torch.equal(ss, ss2)
+    if not alone:
+        return
     h1, xo1, ss1 = h[-1:].clone(), xo[-1:].clone(), ss[-1:].clone()
     ops.gemv_row_norm(x[-1:], blob, fmt, n, k, res[-1:].clone(), h1, nw, unit, xo1, ss1)
     assert torch.equal(h1, h[-1:]) and torch.equal(xo1, xo[-1:]) and torch.equal(ss1, ss[-1:])
@@ -67,7 +69,15 @@ def check(q, n, k, M, dtype, unit=False):
 @pytest.mark.parametrize("q", ["sym_int4", "asym_int4", "fp8_e5m2"])
 def test_shapes(n, k, q):
     for M in (1, 8, 9):
-        check(q, n, k, M, torch.bfloat16)
+        check(q, n, k, M, torch.bfloat16, alone=not 8192 < k <= 16384)
+
+
+# 16 waves: from a K of 8 chunks a wave on, two pieces each at most
+@pytest.mark.parametrize("k", [8192, 8256, 14336, 16384, 16448])
+@pytest.mark.parametrize("q", ["sym_int4", "asym_int4", "nf4", "fp4", "sym_int8", "asym_int5", "fp8_e5m2"])
+def test_sixteen_waves(q, k):
+    for M, dtype in ((1, torch.bfloat16), (2, torch.float16), (3, torch.bfloat16), (4, torch.bfloat16)):
+        check(q, 48, k, M, dtype, alone=False)      # (a row's waves, so its sums, go by the number of rows here)
 
 
 @pytest.mark.parametrize("q", ["sym_int4", "asym_int4", "nf4", "nf3", "fp4", "sym_int8", "sym_int5", "asym_int5",
