@@ -23,6 +23,20 @@ def test_cached_choice_is_shared_within_a_bucket():
         G._CHOICE.update(saved)
 
 
+def test_choice_does_not_follow_the_noise_of_a_timing(monkeypatch):
+    """two candidates as fast as each other: the same one whichever the clock puts first; a faster one is taken"""
+    monkeypatch.setattr(G, "_CHOICE", {})
+    monkeypatch.setattr(G, "_AUTOTUNE", True)
+    monkeypatch.setattr(G.torch.cuda, "is_current_stream_capturing", lambda: False)
+
+    def pick(*times, key=iter(range(100))):
+        monkeypatch.setattr(G, "_time_ms", lambda fns: list(times))
+        return G._pick((1024, next(key), 64, False, 0), *[lambda: None] * len(times))
+    assert pick(139.1, 140.0) == pick(141.0, 138.9) == "g8d"
+    assert pick(82.5, 62.2) == "lib" and pick(1480.4, 1401.9) == "lib" and pick(250.0, 265.0) == "g8d"
+    assert pick(100.0, 99.0, 90.0) == "lib1" and pick(100.0, 90.0, 89.0) == "lib"
+
+
 def test_table_formats_lose_no_bit():
     """nf4 / nf3 weights under bf16 activations: the finer table wherever the fused kernel's f16 one served them, and
     its own gate/up pairs"""
