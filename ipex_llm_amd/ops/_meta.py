@@ -163,7 +163,23 @@ def _(part, bias, q_out, k_cache, v_cache, pos, block_tables, tq, inv_freq, q_no
 
 
 @register_fake("ipex_llm_amd::gemv_accum")
-def _(x, blob, fmt, n, k, acc, ksplit, zero=None, rope_cs=None, rope_pos=None, rope_cols=0, rope_d=0):
+def _(x, blob, fmt, n, k, acc, ksplit, zero=None, rope_cs=None, rope_pos=None, rope_cols=0, rope_d=0, xss=None, xss_n=0,
+      xss_eps=0.0):
+    return None
+
+
+@register_fake("ipex_llm_amd::gemv_rope")
+def _(x, blob, fmt, n, k, bias, out, rope_cs, rope_pos, rope_cols, rope_d, xss=None, xss_n=0, xss_eps=0.0):
+    return None
+
+
+@register_fake("ipex_llm_amd::gemv_row_norm")
+def _(x, blob, fmt, n, k, residual, res_out, norm_w, unit_offset, xo, ss, zero=None):
+    return None
+
+
+@register_fake("ipex_llm_amd::decode_set_state")
+def _(ids, pos, off, ids_out, pos_out, off_out, block_tables, bs, slots, seq_lens):
     return None
 
 

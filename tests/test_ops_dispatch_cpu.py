@@ -146,3 +146,24 @@ def test_traced_slabs_of_unknown_rows():
         x = torch.empty(env.create_unbacked_symint(), 64, dtype=torch.bfloat16, device="cuda")
         y = torch.ops.ipex_llm_amd.gemm_rows_slabs(x, torch.empty(64, dtype=torch.uint8, device="cuda"), 0, 96, 64)
         assert isinstance(y.shape[0], torch.SymInt) and y.shape[2] == 96
+
+
+def test_traced_decode_launches_take_what_the_ops_take():
+    """the launches of a decode step that add or scale by parts of the rows' sums, and the step's state, under tracing"""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    import ipex_llm_amd.ops as ops
+    ops.require()
+    o, M, H, N = torch.ops.ipex_llm_amd, 3, 256, 512
+    with FakeTensorMode():
+        new = lambda *s, dtype=torch.bfloat16: torch.empty(s, dtype=dtype, device="cuda")      # noqa: E731
+        x, blob, parts = new(M, H), new(64, dtype=torch.uint8), new(M, H // 16, dtype=torch.float32)
+        tab, pos, acc = new(64, 64, 2, dtype=torch.float32), new(M, dtype=torch.long), new(M, N, dtype=torch.float32)
+        assert o.gemv_accum(x, blob, 0, N, H, acc, 0, None, tab, pos, N, 128, parts, H, 1e-5) is None
+        assert o.gemv_accum(x, blob, 0, N, H, acc, 0) is None
+        assert o.gemv_rope(x, blob, 0, N, H, None, acc, tab, pos, N, 128, parts, H, 1e-5) is None
+        assert o.gemv_row_norm(x, blob, 0, H, H, x, new(M, H), new(H), False, new(M, H), parts) is None
+        assert o.gemv_glu_ss(x, blob, 0, N, H, 0, parts, H, 1e-5).shape == (M, N // 2)
+        bt, lens = new(M, 4, dtype=torch.int32), new(M, dtype=torch.int32)
+        assert o.decode_set_state(pos, pos, None, *(new(M, dtype=torch.long) for _ in range(3)), bt, 64,
+                                  new(M, dtype=torch.long), lens) is None
