@@ -31,6 +31,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import reference as R
+from ..quantize import qtypes as Q
 from ..transformers.low_bit_linear import LowBitLinear, DenseLinear
 
 
@@ -206,6 +207,7 @@ ROW_NORM = __import__("os").environ.get("ILLM_ROW_NORM", "1") != "0"
 # 1871 2316, 500 tokens, 9 / 16 sequences, asym_int4 2199 2343 / 1795 1984, nf4 2785 3049 / 2544 2788, sym_int8 2655 2807 /
 # 2368 2570; Qwen2.5-7B fp8_e5m2 10 / 16 sequences 2514 2630 / 2245 2387
 ROW_NORM_MAX_M = int(__import__("os").environ.get("ILLM_ROW_NORM_MAX_M", "16"))
+_TABLE_FMTS = (Q.FMT_NF4, Q.FMT_NF3)            # their products are f16 also under bf16 activations
 # decode batches up to this size take the fused-RoPE attention (qkv accumulated
 # atomically into one slab read by the attention, re-zeroed by its combine).
 # Measured on MI355X (Llama-3-8B, L=1024): batch 1 1.960 -> 1.910 ms/token,
@@ -569,12 +571,16 @@ class NativeCausalLM(nn.Module):
 
     def _rows_ok(self, T: int, meta: "AttnMeta", cache) -> bool:
         """more sequences than the split-K launches serve, up to 16: every launch of the step finishes its rows (or is the
-        skinny gate/up, whose product of up to 4096 k has a kernel for every format)"""
+        skinny gate/up, whose product of up to 4096 k has a kernel for every format).  Not where a product takes its rows in
+        f16 -- f16 activations, tables --: these launches hand on norm weight * residual, scaled by 1 / rms behind the
+        product, which is past 65504 for a residual channel that the norm itself brings back into range"""
         s, ref = self.spec, self.layers[0].input_layernorm
         return (ACC_MAX_M < T <= ROW_NORM_MAX_M and DEFER_NORM and s.hidden_size <= 4096 and self._rope_in_ok(meta, cache)
                 and GEMV_ROPE and s.rot_dim == s.head_dim and not s.rope_interleaved and s.head_dim in (64, 128)
-                and self._norm_in_ok(ref, T, True) and self._qkv_native(ref)
-                and self._row_norm_ok() and self._row_rope_ok(T))
+                and ref.dtype == torch.bfloat16 and self._norm_in_ok(ref, T, True) and self._qkv_native(ref)
+                and self._row_norm_ok() and self._row_rope_ok(T)
+                and not any(m.fmt in _TABLE_FMTS for L in self.layers for m in (
+                    L.self_attn.qkv_proj, L.self_attn.o_proj, L.mlp.gate_up_proj, L.mlp.down_proj)))
 
     def _row_rope_ok(self, T: int) -> bool:
         """every layer's qkv projection in a launch that stores its rotated rows, its input in memory: that launch needs no

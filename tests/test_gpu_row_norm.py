@@ -247,6 +247,39 @@ def test_step_of_many_sequences(B, q, bias):
         assert ((out - ref).norm() / ref.norm()).item() < 3e-2      # 16-bit activations through three layers, as smoke()
 
 
+@pytest.mark.parametrize("B", [9, 16])
+@pytest.mark.parametrize("q,dtype", [("sym_int4", torch.float16), ("nf4", torch.bfloat16), ("sym_int4", torch.bfloat16)])
+def test_large_residual_channel(B, q, dtype):
+    """a channel of the residual stream of 3e4 under a norm weight of 4: past what f16 holds before the norm's scale,
+    ordinary behind it.  The final norm leaves that channel out, so the logits are the layers' work"""
+    from transformers import LlamaConfig
+    from ipex_llm_amd.engine.runner import Engine
+    from ipex_llm_amd.models.builder import random_native_model
+    import __graft_entry__ as G
+    dev = torch.device("cuda")
+    cfg = LlamaConfig(vocab_size=512, hidden_size=1024, intermediate_size=2560, num_hidden_layers=3, num_attention_heads=8,
+                      num_key_value_heads=2, max_position_embeddings=512)
+    m = random_native_model(cfg, q, dev, dtype, seed=3)
+    m.embed_tokens.data[:, 77] = 3e4
+    for L in m.layers:
+        L.input_layernorm.data[77] = L.post_attention_layernorm.data[77] = 4.0
+    m.norm.data[77] = 0.0
+    eng, n, steps = Engine(m), 20, 2
+    eng._ensure_cache(B, 64)
+    seqs = [eng.new_sequence(64) for _ in range(B)]
+    ids = torch.randint(0, 512, (B, n + steps), generator=torch.Generator().manual_seed(9))
+    eng.prefill_batch(seqs, ids[:, :n])
+    st = eng.decode_step_obj(seqs, 64, False, True)
+    st.set_state(ids[:, n].to(dev), torch.full((B,), n, device=dev))
+    for i in range(steps):
+        st.ids.copy_(ids[:, n + i])
+        st.step()
+        got = st.logits.float().cpu()
+        for b in {0, B - 1}:
+            ref = G._fp32_reference(m, ids[b, :n + i + 1])[-1]
+            assert ((got[b] - ref).norm() / ref.norm()).item() < 3e-2       # 16-bit activations, as above
+
+
 def _reference(m, ids, biases, G):
     """``__graft_entry__``'s f32 forward with the qkv bias"""
     if biases[0] is None:
