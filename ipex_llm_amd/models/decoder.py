@@ -21,9 +21,10 @@ captured once per (batch, max_len bucket) as a hipGraph (engine/graph.py).
 """
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass, field
-from typing import List, Optional
+from typing import List, NamedTuple, Optional
 
 import torch
 import torch.nn as nn
@@ -263,6 +264,17 @@ def _watched(mod: nn.Module) -> bool:
 
 def linear(x: torch.Tensor, mod: nn.Module) -> torch.Tensor:
     return mod(x)
+
+
+class _Layers(NamedTuple):
+    """what the fused launches of a step ask of all layers (``NativeCausalLM._look_at_layers``)"""
+    norm_in: bool                    # low-bit projections and a gated MLP that take the norm of their input
+    native: bool                     # low-bit qkv projections of this process alone
+    row_norm: bool                   # norm_in, and o and down can finish their rows
+    bias: set                        # dtypes of the qkv projections' biases
+    tables: bool                     # a projection is in a format with f16 tables
+    qkv: set                         # (rows, columns, format) of the qkv projections
+    down: set                        # (columns, format) of the down projections but the last layer's
 
 
 class NativeCausalLM(nn.Module):
@@ -556,20 +568,43 @@ class NativeCausalLM(nn.Module):
     def _defer_ok(self, ref: torch.Tensor, T: int, rows: bool = False) -> bool:
         return DEFER_NORM and (rows or T <= min(ACC_MAX_M, DEFER_MAX_M))
 
-    def _row_norm_ok(self) -> bool:
-        """o and down projections whose launch finishes its rows: 16-column tiles, sums of squares in whole fours"""
-        ok = self.__dict__.get("_row_norm_layers")
-        if ok is None:
-            ok = (ROW_NORM and not self._oproj_combine and not DEFER_MLP_ACC
-                  and self.spec.hidden_size % 64 == 0
-                  and all(m.mp_group is None and m.in_features % 8 == 0 and m.out_features == self.spec.hidden_size
-                          for L in self.layers for m in (L.self_attn.o_proj, L.mlp.down_proj))
-                  and all(w.dtype == self.dtype and w.is_contiguous()
-                          for L in self.layers for w in (L.input_layernorm, L.post_attention_layernorm)))
-            self.__dict__["_row_norm_layers"] = ok
-        return ok and self.tp_group is None
+    def _look_at_layers(self) -> "_Layers":
+        """One walk, anew for every forward that asks (a layer may have been replaced or converted since the last one): some
+        0.07 ms for 32 layers, nothing of it in a captured step.  By way of the modules' own tables, attribute lookups on
+        modules are five times that"""
+        H, norm_in, native, row_norm, bias, tables, qkv, down = self.spec.hidden_size, True, True, True, set(), False, set(), []
+        for L in self.layers:
+            attn, mlp = L._modules.get("self_attn"), L._modules.get("mlp")
+            q, o = attn._modules.get("qkv_proj"), attn._modules.get("o_proj")
+            native = native and isinstance(q, LowBitLinear) and q.mp_group is None
+            b = getattr(q, "bias", None)
+            if b is not None:
+                bias.add(b.dtype)
+            if not (norm_in and native):
+                norm_in = False
+                continue
+            gu, d = (mlp._modules.get("gate_up_proj"), mlp._modules.get("down_proj")) if isinstance(mlp, NativeMLP) else (None, None)
+            norm_in = (isinstance(gu, LowBitLinear) and isinstance(d, LowBitLinear) and isinstance(o, LowBitLinear)
+                       and gu.bias is None and d.bias is None and o.bias is None and gu.mp_group is None
+                       and (d.mp_group is None or d.mp_group is self.tp_group) and (o.mp_group is None or o.mp_group is self.tp_group)
+                       and L.post_feedforward_layernorm is None)
+            if not norm_in:
+                continue
+            w1, w2 = L._parameters.get("input_layernorm"), L._parameters.get("post_attention_layernorm")
+            row_norm = (row_norm and o.mp_group is None and d.mp_group is None and o.out_features == H and d.out_features == H
+                        and o.in_features % 8 == 0 and d.in_features % 8 == 0 and w1 is not None and w2 is not None
+                        and w1.dtype == w2.dtype == self.dtype and w1.is_contiguous() and w2.is_contiguous())
+            tables = tables or q.fmt in _TABLE_FMTS or o.fmt in _TABLE_FMTS or gu.fmt in _TABLE_FMTS or d.fmt in _TABLE_FMTS
+            qkv.add((q.out_features, q.in_features, q.fmt))
+            down.append((d.in_features, d.fmt))
+        return _Layers(norm_in, native, norm_in and row_norm, bias, tables, qkv, set(down[:-1]))
 
-    def _rows_ok(self, T: int, meta: "AttnMeta", cache) -> bool:
+    def _row_norm_ok(self, T: int, seen) -> bool:
+        """o and down projections whose launch finishes its rows: 16-column tiles, sums of squares in whole fours"""
+        return (ROW_NORM and T <= 16 and not self._oproj_combine and not DEFER_MLP_ACC and self.spec.hidden_size % 64 == 0
+                and self.tp_group is None and seen().row_norm)
+
+    def _rows_ok(self, T: int, meta: "AttnMeta", cache, seen) -> bool:
         """more sequences than the split-K launches serve, up to 16: every launch of the step finishes its rows (or is the
         skinny gate/up, whose product of up to 4096 k has a kernel for every format).  Not where a product takes its rows in
         f16 -- f16 activations, tables --: these launches hand on norm weight * residual, scaled by 1 / rms behind the
@@ -577,43 +612,21 @@ class NativeCausalLM(nn.Module):
         s, ref = self.spec, self.layers[0].input_layernorm
         return (ACC_MAX_M < T <= ROW_NORM_MAX_M and DEFER_NORM and s.hidden_size <= 4096 and self._rope_in_ok(meta, cache)
                 and GEMV_ROPE and s.rot_dim == s.head_dim and not s.rope_interleaved and s.head_dim in (64, 128)
-                and ref.dtype == torch.bfloat16 and self._norm_in_ok(ref, T, True) and self._qkv_native(ref)
-                and self._row_norm_ok() and self._row_rope_ok(T)
-                and not any(m.fmt in _TABLE_FMTS for L in self.layers for m in (
-                    L.self_attn.qkv_proj, L.self_attn.o_proj, L.mlp.gate_up_proj, L.mlp.down_proj)))
+                and ref.dtype == torch.bfloat16 and self._norm_in_ok(ref, T, seen, True) and self._qkv_native(ref, seen)
+                and self._row_norm_ok(T, seen) and self._row_rope_ok(T, seen) and not seen().tables)
 
-    def _row_rope_ok(self, T: int) -> bool:
+    def _row_rope_ok(self, T: int, seen) -> bool:
         """every layer's qkv projection in a launch that stores its rotated rows, its input in memory: that launch needs no
         sums pending, so every down projection but the last has to finish its rows"""
-        known = self.__dict__.setdefault("_row_rope_rows", {})
-        if T in known:
-            return known[T]
-        H, D = self.spec.hidden_size, self.spec.head_dim
-        t = torch.ops.ipex_llm_amd
-        known[T] = all(q.in_features % 8 == 0 and q.out_features % D == 0
-                   and t.row_rope_takes(T, q.out_features, q.in_features, q.fmt)
-                   and (i == 0 or t.row_norm_takes(T, H, d.in_features, d.fmt, True))
-                   for i, (q, d) in enumerate(zip((L.self_attn.qkv_proj for L in self.layers),
-                                                  [None] + [L.mlp.down_proj for L in self.layers])))
-        return known[T]
+        H, D, t = self.spec.hidden_size, self.spec.head_dim, torch.ops.ipex_llm_amd
+        return (all(k % 8 == 0 and n % D == 0 and t.row_rope_takes(T, n, k, fmt) for n, k, fmt in seen().qkv)
+                and all(t.row_norm_takes(T, H, k, fmt, True) for k, fmt in seen().down))
 
-    def _norm_in_ok(self, ref: torch.Tensor, T: int, rows: bool = False) -> bool:
+    def _norm_in_ok(self, ref: torch.Tensor, T: int, seen, rows: bool = False) -> bool:
         lim = max(NORM_IN_MAX_M, DEFER_MAX_M if self._defer_ok(ref, T) else 0)
-        if not (self._norm_in_env and (rows or T <= min(ACC_MAX_M, lim)) and ref.is_cuda
+        return (self._norm_in_env and (rows or T <= min(ACC_MAX_M, lim)) and ref.is_cuda
                 and not self.spec.sandwich_norm and not self._attn_fuse and not self._glu_in_enabled
-                and self.spec.hidden_size % 8 == 0 and ops.native_gpu(ref)):
-            return False
-        ok = self.__dict__.get("_norm_in_layers")
-        if ok is None:
-            def lowbit(m, bias_ok=False):
-                return isinstance(m, LowBitLinear) and self._tp_ok(m) and (bias_ok or m.bias is None)
-            ok = all(isinstance(L.mlp, NativeMLP) and lowbit(L.mlp.gate_up_proj) and lowbit(L.mlp.down_proj)
-                     and lowbit(L.self_attn.o_proj) and lowbit(L.self_attn.qkv_proj, True)
-                     and L.self_attn.qkv_proj.mp_group is None and L.mlp.gate_up_proj.mp_group is None
-                     and (L.self_attn.qkv_proj.bias is None or L.self_attn.qkv_proj.bias.dtype == ref.dtype)
-                     and L.post_feedforward_layernorm is None for L in self.layers)
-            self.__dict__["_norm_in_layers"] = ok
-        return ok
+                and self.spec.hidden_size % 8 == 0 and ops.native_gpu(ref) and seen().norm_in and seen().bias <= {ref.dtype})
 
     # decode (one new token per sequence) attention that applies RoPE to q/k
     # from the qkv accumulator and appends the new key/value itself: one
@@ -629,22 +642,9 @@ class NativeCausalLM(nn.Module):
                 and ((s.head_dim == 128 and group <= 16) or (s.head_dim == 256 and group <= 8))
                 and all(L.self_attn.q_norm is None and L.self_attn.k_norm is None for L in self.layers))
 
-    def _qkv_bias_free(self) -> bool:
-        ok = self.__dict__.get("_qkv_nobias")
-        if ok is None:
-            ok = all(getattr(L.self_attn.qkv_proj, "bias", None) is None for L in self.layers)
-            self.__dict__["_qkv_nobias"] = ok
-        return ok
-
-    def _qkv_native(self, ref: torch.Tensor) -> bool:
+    def _qkv_native(self, ref: torch.Tensor, seen) -> bool:
         """every layer's qkv projection runs the native atomic GEMV"""
-        ok = self.__dict__.get("_qkv_native_ok")
-        if ok is None:
-            ok = all(isinstance(L.self_attn.qkv_proj, LowBitLinear) and L.self_attn.qkv_proj.mp_group is None
-                     and (L.self_attn.qkv_proj.bias is None or L.self_attn.qkv_proj.bias.dtype == ref.dtype)
-                     for L in self.layers)
-            self.__dict__["_qkv_native_ok"] = ok
-        return ok and ref.is_cuda and ops.native_gpu(ref)
+        return ref.is_cuda and ops.native_gpu(ref) and seen().native and seen().bias <= {ref.dtype}
 
     def _fused_mlp_ok(self, x, layer, need_env: bool = True) -> bool:
         mlp = layer.mlp
@@ -715,11 +715,12 @@ class NativeCausalLM(nn.Module):
         s = self.spec
         T = ids.shape[0]
         ss_zeroed = None
-        rows = self._rows_ok(T, meta, cache)
+        seen = functools.cache(self._look_at_layers)
+        rows = self._rows_ok(T, meta, cache, seen)
         if hidden_in is None and self._embed_norm_ok(ids):
             # one launch: embedding gather (the residual stream), the first
             # layer's RMSNorm and the zeroing of the step's deferred-norm sums
-            defer0 = self._norm_in_ok(self.embed_tokens, T, rows) and self._defer_ok(self.embed_tokens, T, rows)
+            defer0 = self._norm_in_ok(self.embed_tokens, T, seen, rows) and self._defer_ok(self.embed_tokens, T, rows)
             ss_zeroed = self._acc(T, 2 * len(self.layers), ids.device, "SS") if defer0 else None
             residual, x = torch.ops.ipex_llm_amd.embed_rms_norm(ids.contiguous(), self.embed_tokens,
                                                                self.layers[0].input_layernorm, s.rms_eps,
@@ -738,7 +739,7 @@ class NativeCausalLM(nn.Module):
         # norm-in decode: the down projection's atomic accumulator stays pending
         # and the next layer's qkv GEMV adds + normalises it in its prologue;
         # the residual ping-pongs between two buffers (written by one workgroup)
-        norm_in = self._norm_in_ok(residual, T, rows)
+        norm_in = self._norm_in_ok(residual, T, seen, rows)
         pend = None                     # accumulator awaiting residual-add + norm
         consumed = None                 # accumulator read by the last launch: zeroed by the next GEMV
         res_pp = (residual, torch.empty_like(residual)) if norm_in else None
@@ -750,17 +751,18 @@ class NativeCausalLM(nn.Module):
             if ss_zeroed is not ss_all:
                 ss_all.zero_()
         ss_q = None                     # sums of squares of the current layer's qkv input (deferred)
-        row_norm = defer and self._row_norm_ok()        # o / down that finish their rows (ops.gemv_row_norm)
+        row_norm = defer and self._row_norm_ok(T, seen)  # o / down that finish their rows (ops.gemv_row_norm)
         x_ss = None                     # (sums of squares by 16 columns, n, eps) of x: a deferred-norm qkv input
         zero_gu = None                  # consumed gate/up accumulator (batch > DEFER_GLU_MAX_M), zeroed next
         # fused-RoPE decode attention (batch <= ROPE_IN_MAX_M, one token each): the qkv
         # GEMV accumulates into one atomic slab that the attention reads and the
         # combine launch re-zeroes
-        rope_ok = self._rope_in_ok(meta, cache) and self._qkv_native(residual)
+        rope_ok = ((rows or T <= max(ACC_MAX_M, ROPE_IN_MAX_M)) and self._rope_in_ok(meta, cache)
+                   and self._qkv_native(residual, seen))
         prerot = (GEMV_ROPE and rope_ok and (rows or T <= ACC_MAX_M) and s.rot_dim == s.head_dim and not s.rope_interleaved
                   and s.head_dim in (64, 128))
-        row_rope = prerot and row_norm and self._row_rope_ok(T)       # bias and rotation ahead of the store
-        prerot = row_rope or (prerot and self._qkv_bias_free())
+        row_rope = prerot and row_norm and self._row_rope_ok(T, seen)  # bias and rotation ahead of the store
+        prerot = row_rope or (prerot and not seen().bias)
         rope_in = rope_ok and (T <= ROPE_IN_MAX_M or prerot)
         qrope = (self.rope_cache, pos, (s.num_heads + s.num_kv_heads) * s.head_dim, s.head_dim) if prerot else None
         nxt_res = lambda r: res_pp[1] if r is res_pp[0] else res_pp[0]

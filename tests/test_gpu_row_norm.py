@@ -280,6 +280,58 @@ def test_large_residual_channel(B, q, dtype):
             assert ((got[b] - ref).norm() / ref.norm()).item() < 3e-2       # 16-bit activations, as above
 
 
+def _steps(m, B, first):
+    """logits of two eager steps behind the same prompts"""
+    from ipex_llm_amd.engine.runner import Engine
+    eng = Engine(m)
+    eng._ensure_cache(B, 64)
+    seqs = [eng.new_sequence(64) for _ in range(B)]
+    ids = torch.randint(0, 512, (B, 22), generator=torch.Generator().manual_seed(4))
+    eng.prefill_batch(seqs, ids[:, :20])
+    st = eng.decode_step_obj(seqs, 64, False, False)
+    st.set_state(ids[:, 20].cuda(), torch.full((B,), 20, device="cuda"))
+    out = []
+    for i in range(2):
+        st.ids.copy_(ids[:, 20 + i])
+        st.step()
+        out.append(st.logits.float().clone())
+        if i == 0:
+            first()
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("what", ["dense_o", "dense_qkv", "oproj_combine", "row_norm_off"])
+@pytest.mark.parametrize("B", [2, 9])
+def test_model_that_changes_between_steps(B, what, monkeypatch):
+    """a projection replaced or a launch switched after a step: the next step goes by what is there"""
+    import ipex_llm_amd.models.decoder as D
+    from transformers import LlamaConfig
+    from ipex_llm_amd.models.builder import random_native_model
+    cfg = LlamaConfig(vocab_size=512, hidden_size=1024, intermediate_size=2560, num_hidden_layers=3, num_attention_heads=8,
+                      num_key_value_heads=2, max_position_embeddings=512)
+    m = random_native_model(cfg, "sym_int4", torch.device("cuda"), torch.bfloat16, seed=0)
+    want = _steps(m, B, lambda: None)
+
+    def dense(mod):
+        lin = torch.nn.Linear(mod.in_features, mod.out_features, bias=False, device="meta")
+        lin.weight = torch.nn.Parameter(mod.dequantize(torch.float32).to("cuda", torch.bfloat16), False)
+        return lin
+
+    def change():
+        L = m.layers[1]
+        if what == "dense_o":
+            L.self_attn.o_proj = dense(L.self_attn.o_proj)
+        elif what == "dense_qkv":
+            L.self_attn.qkv_proj = dense(L.self_attn.qkv_proj)
+        elif what == "oproj_combine":
+            monkeypatch.setattr(D.NativeCausalLM, "_oproj_combine", True)
+        else:
+            monkeypatch.setattr(D, "ROW_NORM", False)
+    got = _steps(m, B, change)
+    for g, w in zip(got, want):
+        assert ((g - w).norm() / w.norm()).item() < 2e-2        # 16-bit activations, rounded at other places
+
+
 def _reference(m, ids, biases, G):
     """``__graft_entry__``'s f32 forward with the qkv bias"""
     if biases[0] is None:
