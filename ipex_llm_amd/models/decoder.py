@@ -612,7 +612,7 @@ class NativeCausalLM(nn.Module):
         s, ref = self.spec, self.layers[0].input_layernorm
         return (ACC_MAX_M < T <= ROW_NORM_MAX_M and DEFER_NORM and s.hidden_size <= 4096 and self._rope_in_ok(meta, cache)
                 and GEMV_ROPE and s.rot_dim == s.head_dim and not s.rope_interleaved and s.head_dim in (64, 128)
-                and ref.dtype == torch.bfloat16 and self._norm_in_ok(ref, T, seen, True) and self._qkv_native(ref, seen)
+                and ref.dtype == torch.bfloat16 and self._norm_in_ok(ref, T, True, seen) and self._qkv_native(ref, seen)
                 and self._row_norm_ok(T, seen) and self._row_rope_ok(T, seen) and not seen().tables)
 
     def _row_rope_ok(self, T: int, seen) -> bool:
@@ -622,7 +622,8 @@ class NativeCausalLM(nn.Module):
         return (all(k % 8 == 0 and n % D == 0 and t.row_rope_takes(T, n, k, fmt) for n, k, fmt in seen().qkv)
                 and all(t.row_norm_takes(T, H, k, fmt, True) for k, fmt in seen().down))
 
-    def _norm_in_ok(self, ref: torch.Tensor, T: int, seen, rows: bool = False) -> bool:
+    def _norm_in_ok(self, ref: torch.Tensor, T: int, rows: bool = False, seen=None) -> bool:
+        seen = seen or functools.cache(self._look_at_layers)
         lim = max(NORM_IN_MAX_M, DEFER_MAX_M if self._defer_ok(ref, T) else 0)
         return (self._norm_in_env and (rows or T <= min(ACC_MAX_M, lim)) and ref.is_cuda
                 and not self.spec.sandwich_norm and not self._attn_fuse and not self._glu_in_enabled
@@ -720,7 +721,7 @@ class NativeCausalLM(nn.Module):
         if hidden_in is None and self._embed_norm_ok(ids):
             # one launch: embedding gather (the residual stream), the first
             # layer's RMSNorm and the zeroing of the step's deferred-norm sums
-            defer0 = self._norm_in_ok(self.embed_tokens, T, seen, rows) and self._defer_ok(self.embed_tokens, T, rows)
+            defer0 = self._norm_in_ok(self.embed_tokens, T, rows, seen) and self._defer_ok(self.embed_tokens, T, rows)
             ss_zeroed = self._acc(T, 2 * len(self.layers), ids.device, "SS") if defer0 else None
             residual, x = torch.ops.ipex_llm_amd.embed_rms_norm(ids.contiguous(), self.embed_tokens,
                                                                self.layers[0].input_layernorm, s.rms_eps,
@@ -739,7 +740,7 @@ class NativeCausalLM(nn.Module):
         # norm-in decode: the down projection's atomic accumulator stays pending
         # and the next layer's qkv GEMV adds + normalises it in its prologue;
         # the residual ping-pongs between two buffers (written by one workgroup)
-        norm_in = self._norm_in_ok(residual, T, seen, rows)
+        norm_in = self._norm_in_ok(residual, T, rows, seen)
         pend = None                     # accumulator awaiting residual-add + norm
         consumed = None                 # accumulator read by the last launch: zeroed by the next GEMV
         res_pp = (residual, torch.empty_like(residual)) if norm_in else None
