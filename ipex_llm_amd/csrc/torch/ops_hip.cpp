@@ -1065,15 +1065,15 @@ bool glu_rows_takes(int64_t M, int64_t NT, int64_t k, int fmt) {
 
 // gate/up GLU GEMV over a deferred-norm input (gemv_accum_norm's xo): the row
 // scale rsqrt(ss[m] / ss_n + eps) is applied to gate and up before the activation
+// (parted: ss [M, parts] of gemv_row_norm, else M whole sums in any shape)
 Tensor gemv_glu_ss(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, int64_t act,
-                   const Tensor& ss, int64_t ss_n, double eps) {
+                   const Tensor& ss, int64_t ss_n, double eps, bool parted) {
   TORCH_CHECK(x.is_cuda() && blob.is_cuda() && x.size(-1) == k, "gemv_glu_ss: GPU x [M, k]");
   c10::DeviceGuard g(x.device());
   const bool bf16 = is_bf16(x);
   Tensor xc = rows16(x);
   const int64_t M = xc.numel() / k;
   TORCH_CHECK(M >= 1 && M <= 16 && n % 32 == 0, "gemv_glu_ss: 1..16 rows, n a multiple of 32");
-  const bool parted = ss.dim() == 2;                               // [M, parts] of gemv_row_norm
   TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && (parted || ss.numel() >= M), "gemv_glu_ss: ss f32 [>= M]");
   TORCH_CHECK(blob.numel() >= illm::dev_total_bytes((int)fmt, n, k), "gemv_glu_ss: weight blob too small");
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N;

@@ -886,7 +886,7 @@ class NativeCausalLM(nn.Module):
                 gu, dn = mlp.gate_up_proj, mlp.down_proj
                 if fin_o:
                     act = ops.gemv_glu_ss(xo, gu.weight, gu.fmt, gu.out_features, gu.in_features, s.act, sp,
-                                          s.hidden_size, s.rms_eps)
+                                          s.hidden_size, s.rms_eps, parts=True)
                     if fin_d:
                         r2 = nxt_res(residual)
                         x, sp = self._acc(H, T, x.device, "XD", self.dtype), self._acc((H + 15) // 16, T, x.device, "SPD")

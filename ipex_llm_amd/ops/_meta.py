@@ -189,7 +189,7 @@ def _(x, blob, fmt, n, k, acc, ctr, residual, res_out, norm_w, unit_offset, xo, 
 
 
 @register_fake("ipex_llm_amd::gemv_glu_ss")
-def _(x, blob, fmt, n, k, act, ss, ss_n, eps):
+def _(x, blob, fmt, n, k, act, ss, ss_n, eps, parts=False):
     return x.new_empty((x.numel() // k, n // 2))
 
 

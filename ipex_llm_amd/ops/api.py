@@ -225,10 +225,9 @@ def gemv_partials(x, blob, fmt, n, k, ksplit: int) -> torch.Tensor:
     return _ops().gemv(x, blob, fmt, n, k, None, 1, ksplit, 0)
 
 
-def _row_scale(ss: torch.Tensor, M: int, ss_n: int, eps: float) -> torch.Tensor:
-    """1 / rms [M, 1] of a deferred norm from its rows' sums of squares: [M] or, from ``gemv_row_norm``, parts [M, parts]"""
-    s = ss[:M].float()
-    return torch.rsqrt((s.sum(-1) if ss.dim() == 2 else s) / ss_n + eps)[:, None]
+def _row_scale(s: torch.Tensor, ss_n: int, eps: float) -> torch.Tensor:
+    """1 / rms [M, 1] of a deferred norm from its rows' sums of squares [M]"""
+    return torch.rsqrt(s / ss_n + eps)[:, None]
 
 
 def gemv_accum(x, blob, fmt, n, k, acc: torch.Tensor, ksplit: int = 0,
@@ -249,7 +248,7 @@ def gemv_accum(x, blob, fmt, n, k, acc: torch.Tensor, ksplit: int = 0,
         zero.zero_()
     y = lowbit_matmul(x, blob, fmt, n, k).float().view_as(acc)
     if xss is not None:
-        y = y * _row_scale(xss[0], y.shape[0], xss[1], xss[2])
+        y = y * _row_scale(xss[0].float().sum(-1), xss[1], xss[2])
     acc += _rope_cols(y, rope, x.dtype).view_as(acc)
     return acc
 
@@ -264,7 +263,7 @@ def gemv_rope(x, blob, fmt, n, k, bias: Optional[torch.Tensor], out: torch.Tenso
         return out
     y = lowbit_matmul(x, blob, fmt, n, k).float().view_as(out)
     if xss is not None:
-        y = y * _row_scale(xss[0], y.shape[0], xss[1], xss[2])
+        y = y * _row_scale(xss[0].float().sum(-1), xss[1], xss[2])
     if bias is not None:
         y = y + bias.float()
     out.copy_(_rope_cols(y, rope, x.dtype).view_as(out))
@@ -315,14 +314,15 @@ def gemv_accum_norm(x, blob, fmt, n, k, acc: torch.Tensor, ctr: torch.Tensor, re
     return xo
 
 
-def gemv_glu_ss(x, blob, fmt, n, k, act: int, ss: torch.Tensor, ss_n: int, eps: float) -> torch.Tensor:
+def gemv_glu_ss(x, blob, fmt, n, k, act: int, ss: torch.Tensor, ss_n: int, eps: float, parts: bool = False) -> torch.Tensor:
     """act(s x Wg^T) * (s x Wu^T) with s = rsqrt(ss / ss_n + eps) per row: the
-    gate/up GEMV over ``gemv_accum_norm``'s (ss [M]) or ``gemv_row_norm``'s (ss [M, parts]) deferred-norm input."""
+    gate/up GEMV over ``gemv_accum_norm``'s (M sums, in any shape) or, ``parts``, ``gemv_row_norm``'s (ss [M, parts])
+    deferred-norm input."""
     if _native(x):
-        return _ops().gemv_glu_ss(x, blob, fmt, n, k, act, ss, ss_n, eps)
+        return _ops().gemv_glu_ss(x, blob, fmt, n, k, act, ss, ss_n, eps, parts)
     from ..models.decoder import deinterleave_glu
     M = x.numel() // k
-    inv = _row_scale(ss, M, ss_n, eps)
+    inv = _row_scale(ss.float().sum(-1) if parts else ss.float().reshape(-1)[:M], ss_n, eps)
     g, u = deinterleave_glu(lowbit_matmul(x, blob, fmt, n, k).float())
     g, u = g * inv, u * inv
     return ((F.silu(g) if act == 0 else F.gelu(g, approximate="tanh")) * u).to(x.dtype).contiguous()

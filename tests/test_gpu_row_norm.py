@@ -110,7 +110,7 @@ def test_consumers_add_the_parts(q, n, k, M):
     fmt, blob, w, x, _, _ = make(q, n, k, M, torch.bfloat16, 1)
     parts = torch.rand(M, k // 16, device="cuda") * 16
     whole = parts.double().sum(-1)
-    a = ops.gemv_glu_ss(x, blob, fmt, n, k, 0, parts, k, 1e-5)
+    a = ops.gemv_glu_ss(x, blob, fmt, n, k, 0, parts, k, 1e-5, parts=True)
     b = ops.gemv_glu_ss(x, blob, fmt, n, k, 0, whole.float(), k, 1e-5)
     # both rounded to 16 bits, by half a step at most, from 32-bit sums in another order
     assert ((a.double() - b.double()).norm() / b.double().norm()).item() <= 2 * 2.0 ** -8 * 1.01
@@ -127,6 +127,17 @@ def test_consumers_add_the_parts(q, n, k, M):
     r = y[:, :cols].reshape(M, -1, D)
     y[:, :cols] = (r * c + torch.cat([-r[..., D // 2:], r[..., :D // 2]], -1) * s).reshape(M, cols)
     assert ((acc.double() - y).norm() / y.norm()).item() < (2e-3 if q == "nf4" else 1e-5)   # (an f16 table)
+
+
+@pytest.mark.parametrize("M", [1, 4, 9])
+def test_whole_sums_in_any_shape(M):
+    """sums of squares that are not called parts are one a row, whatever the shape that holds them"""
+    fmt, blob, _, x, _, _ = make("sym_int4", 256, 512, M, torch.bfloat16, 5)
+    whole = torch.rand(M, device="cuda") * 512
+    want = ops.gemv_glu_ss(x, blob, fmt, 256, 512, 0, whole, 512, 1e-5)
+    more = torch.cat([whole, torch.rand(3 * M, device="cuda")])
+    for ss in (whole[:, None], whole[None], more.view(M, 4), more.view(4, M)):
+        assert torch.equal(ops.gemv_glu_ss(x, blob, fmt, 256, 512, 0, ss, 512, 1e-5), want)
 
 
 def test_rule():
@@ -197,7 +208,7 @@ def test_gate_up_rows(q, n, k):
                           (9, torch.bfloat16, 0)):
         fmt, blob, w, x, _, _ = make(q, n, k, M, dtype, 3)
         parts = torch.rand(M, 8, device="cuda") * k / 4
-        got = ops.gemv_glu_ss(x, blob, fmt, n, k, act, parts, k, 1e-5)
+        got = ops.gemv_glu_ss(x, blob, fmt, n, k, act, parts, k, 1e-5, parts=True)
         y = (x.double() @ w.t()) * torch.rsqrt(parts.double().sum(-1) / k + 1e-5)[:, None]
         g, u = y.view(M, n // 32, 2, 16).unbind(2)
         f = torch.nn.functional.silu(g) if act == 0 else torch.nn.functional.gelu(g, approximate="tanh")

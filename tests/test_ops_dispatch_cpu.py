@@ -163,7 +163,7 @@ def test_traced_decode_launches_take_what_the_ops_take():
         assert o.gemv_accum(x, blob, 0, N, H, acc, 0) is None
         assert o.gemv_rope(x, blob, 0, N, H, None, acc, tab, pos, N, 128, parts, H, 1e-5) is None
         assert o.gemv_row_norm(x, blob, 0, H, H, x, new(M, H), new(H), False, new(M, H), parts) is None
-        assert o.gemv_glu_ss(x, blob, 0, N, H, 0, parts, H, 1e-5).shape == (M, N // 2)
+        assert o.gemv_glu_ss(x, blob, 0, N, H, 0, parts, H, 1e-5, True).shape == (M, N // 2)
         bt, lens = new(M, 4, dtype=torch.int32), new(M, dtype=torch.int32)
         assert o.decode_set_state(pos, pos, None, *(new(M, dtype=torch.long) for _ in range(3)), bt, 64,
                                   new(M, dtype=torch.long), lens) is None
