@@ -297,9 +297,10 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
     if (!fin) return;
     const float c = rnd(cs.x), sn = rnd(cs.y);                    // as the model casts its tables
     const float y0 = __builtin_fmaf(y[0], rs, bias[0]), y1 = __builtin_fmaf(y[NT - 1], rs, bias[NT - 1]);
+    const bool rot = on < a.rcols;                                // v: as it is (an infinity times a sine of 0 is no number)
     float* o = a.out32 + (size_t)om * a.N + on;
-    o[0] = __builtin_fmaf(-y1, sn, y0 * c);                       // (spelled out: one rounding in every instantiation)
-    o[ht * 16] = __builtin_fmaf(y0, sn, y1 * c);
+    o[0] = rot ? __builtin_fmaf(-y1, sn, y0 * c) : y0;            // (spelled out: one rounding in every instantiation)
+    o[ht * 16] = rot ? __builtin_fmaf(y0, sn, y1 * c) : y1;
   } else {
     const float gv = y[0] * rs, uv = y[NT - 1] * rs;
     const int n = blockIdx.x * 16 + r16;

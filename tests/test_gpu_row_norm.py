@@ -200,6 +200,23 @@ def test_rotated_rows(q, n, k, D, cols):
         assert torch.equal(a, out[-2:-1])
 
 
+@pytest.mark.parametrize("q", ["sym_int4", "fp8_e5m2"])
+def test_columns_that_are_not_rotated_stand_alone(q):
+    """an infinite value column says nothing of the column half a head away"""
+    n, k, D, cols, M = 384, 256, 128, 256, 3
+    fmt, blob, _, x, _, _ = make(q, n, k, M, torch.bfloat16, 6)
+    tab, pos = torch.randn(64, D // 2, 2, device="cuda"), torch.randint(0, 64, (M,), device="cuda")
+    bias = torch.zeros(n, device="cuda", dtype=torch.bfloat16)
+    want, got = torch.empty(M, n, device="cuda"), torch.empty(M, n, device="cuda")
+    ops.gemv_rope(x, blob, fmt, n, k, bias, want, (tab, pos, cols, D))
+    at = [cols + 5, cols + 70, cols + 127]
+    bias[at] = torch.tensor([float("inf"), -float("inf"), float("nan")], device="cuda").to(torch.bfloat16)
+    ops.gemv_rope(x, blob, fmt, n, k, bias, got, (tab, pos, cols, D))
+    assert (got[:, at[0]] == float("inf")).all() and (got[:, at[1]] == -float("inf")).all() and got[:, at[2]].isnan().all()
+    rest = [c for c in range(n) if c not in at]
+    assert torch.equal(got[:, rest], want[:, rest])
+
+
 # one chunk, chunks for some waves only, one piece a wave; M <= 8 on the product that finishes its rows, then the others
 @pytest.mark.parametrize("n,k", [(64, 128), (96, 576), (1024, 2048), (160, 4096), (64, 4160), (28672, 512)])
 @pytest.mark.parametrize("q", ["sym_int4", "asym_int4", "nf4", "fp4", "sym_int8", "asym_int5", "fp8_e4m3", "fp8_e5m2"])
