@@ -932,6 +932,11 @@ void gemv_accum_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n
 // atomics:
 //   * 8-bit codes: sym_int8 [4096, 14336] 4 / 8 / 16 rows 2326 2512 2915 / 2321 2489 2829; fp8_e5m2 [3584, 18944] 1 / 5 / 8
 //     / 16 rows 2081 2222 2285 2545 / 1995 2182 2240 2528; alone [8192, 28672] 5 rows 48 / 44;
+//     ... integers (whose offset is more work a workgroup) not where the last round of one workgroup per CU is less than half
+//     full: a step's layer with its o projection in rows, us, [5120, 13824], 320 tiles, sym_int8 1 / 3 / 5 / 8 rows 85.8 97.5
+//     125.2 138.9 / 88.7 102.1 131.5 144.7, asym_int5 5 / 8 rows 128.1 142.8 / 137.8 150.9; [6144, 16384], 384 tiles, sym_int8 3
+//     / 8 rows 105.7 124.7 / 102.6 120.0; [8192, 28672], 512 tiles, 3 / 5 / 8 rows 179.3 192.2 205.1 / 178.8 195.4 202.9;
+//     fp8_e5m2 [5120, 13824] 1 / 5 / 8 rows 90.2 123.0 137.4 / 89.2 122.5 136.2;
 //   * 4-bit codes, one workgroup per CU (alone [5120, 13824] 1 row 10.4 / 12.4, [8192, 28672] 3 rows 25.9 / 28.4): asym_int4
 //     [4096, 14336] 9 / 16 rows 2143 2432 / 2070 2338;
 //   * ... of few rows only where the next qkv launch adds slices too (not stored: it takes its input from the sums on its
@@ -945,13 +950,28 @@ bool row_norm_takes(int64_t M, int64_t n, int64_t k, int64_t fmt, bool stored) {
   TORCH_CHECK(M >= 1 && n >= 1 && k >= 1, "row_norm_takes: sizes");
   const int64_t NT = illm::pad_to(n, illm::TILE_N) / illm::TILE_N, KC = illm::pad_to(k, illm::CHUNK_K) / illm::CHUNK_K;
   if (M > 16) return false;
-  if (illm::fmt_bits((int)fmt) == 8) return true;
+  if (illm::fmt_bits((int)fmt) == 8) {
+    const int dk = illm::fmt_to_dk((int)fmt);
+    return (dk != illm::DK_INT8S && dk != illm::DK_INT8A) || NT <= 256 || NT % 256 == 0 || NT % 256 >= 128;
+  }
   if (NT > 256) return false;
   if (M <= 2 || stored) return true;
   if (illm::fmt_to_dk((int)fmt) == illm::DK_LUT4) return M > 12;
   if (fmt != illm::FMT_SYM_INT4 || M > 8) return true;
   const Plan5 p = plan5(M, NT, KC, true, 0, true, (int)fmt);
   return p.cpk > 7;
+}
+
+// An o projection that finishes its rows, instead of one in slices whose sums the gate/up launch (to 4 rows) or its last
+// workgroups (from 5) normalise: all but tables of 5 rows and more and over one workgroup per CU, us a step's layer, slices /
+// rows: nf4, hidden size 5120, 4 / 5 / 6 / 8 rows 108.2 115.7 120.3 131.6 / 105.4 119.1 123.1 135.7, 6144 3 / 5 / 8 rows 94.2
+// 99.5 107.6 / 90.6 101.5 109.2, 8192 4 / 5 / 8 rows 169.9 167.0 184.7 / 154.8 168.2 183.9, but 4096 5 / 8 rows 75.5 80.7 / 70.2
+// 72.2; sym_int4 5120 1 / 4 / 8 rows 65.5 88.2 111.5 / 63.8 86.1 110.2, 8192 116.2 129.2 130.8 / 112.3 113.8 128.0, asym_int4
+// 5120 74.8 101.9 123.2 / 69.4 92.7 117.3, fp4 5120 3 / 8 rows 76.0 108.0 / 72.0 107.4, sym_int8 8192 1 / 4 / 8 rows 185 196 212
+// / 180 181 203, fp8_e5m2 5120 93.5 119.6 143.1 / 87.0 108.9 135.3, 8192 190 193 210 / 177 173 190 (with gate/up on its parts).
+bool row_norm_o_takes(int64_t M, int64_t n, int64_t fmt) {
+  TORCH_CHECK(M >= 1 && n >= 1, "row_norm_o_takes: sizes");
+  return M <= 16 && !(illm::fmt_to_dk((int)fmt) == illm::DK_LUT4 && M > 4 && n > 256 * illm::TILE_N);
 }
 
 // lowbit_fullk.cuh: x W^T of 1..16 rows, the residual add, the deferred-norm input of the next product and the parts of
@@ -2138,6 +2158,7 @@ int* illm_kernel_err(const c10::Device& dev) { return kernel_err(dev); }
 TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("skinny_geometry(int M, int n, int k, int fmt, bool glu, int ksplit, bool fine=False) -> int[]", &skinny_geometry);
   m.def("row_norm_takes(int M, int n, int k, int fmt, bool stored=False) -> bool", &row_norm_takes);
+  m.def("row_norm_o_takes(int M, int n, int fmt) -> bool", &row_norm_o_takes);
   m.def("row_rope_takes(int M, int n, int k, int fmt) -> bool", &row_rope_takes);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
   m.def("attn_decode_groups(int batch, int kv_heads, int nsplit) -> int", [](int64_t b, int64_t h, int64_t n) -> int64_t {

@@ -199,7 +199,7 @@ DEFER_MLP_ACC = __import__("os").environ.get("ILLM_DEFER_MLP_ACC", "0") == "1"
 # add_rms_norm launch between attention and MLP (ILLM_ONORM=0 restores it)
 ONORM = __import__("os").environ.get("ILLM_ONORM", "1") != "0"
 ONORM_MIN_M = int(__import__("os").environ.get("ILLM_ONORM_MIN_M", "5"))
-# the o projection (and the down projection, where row_norm_takes in csrc/torch/ops_hip.cpp says so) in launches that
+# the o and down projections, where row_norm_o_takes and row_norm_takes in csrc/torch/ops_hip.cpp say so, in launches that
 # finish their rows: residual add, the deferred-norm input of the next launch and the parts of its sums of squares
 # (ops.gemv_row_norm), no atomics and no accumulator to clear.  ILLM_ROW_NORM=0: the split-K launches above
 ROW_NORM = __import__("os").environ.get("ILLM_ROW_NORM", "1") != "0"
@@ -273,6 +273,7 @@ class _Layers(NamedTuple):
     row_norm: bool                   # norm_in, and o and down can finish their rows
     bias: set                        # dtypes of the qkv projections' biases
     tables: bool                     # a projection is in a format with f16 tables
+    o: set                           # formats of the o projections
     qkv: set                         # (rows, columns, format) of the qkv projections
     down: set                        # (columns, format) of the down projections but the last layer's
 
@@ -572,7 +573,7 @@ class NativeCausalLM(nn.Module):
         """One walk, anew for every forward that asks (a layer may have been replaced or converted since the last one): some
         0.07 ms for 32 layers, nothing of it in a captured step.  By way of the modules' own tables, attribute lookups on
         modules are five times that"""
-        H, norm_in, native, row_norm, bias, tables, qkv, down = self.spec.hidden_size, True, True, True, set(), False, set(), []
+        H, norm_in, native, row_norm, bias, tables, fo, qkv, down = self.spec.hidden_size, True, True, True, set(), False, set(), set(), []
         for L in self.layers:
             attn, mlp = L._modules.get("self_attn"), L._modules.get("mlp")
             q, o = attn._modules.get("qkv_proj"), attn._modules.get("o_proj")
@@ -595,14 +596,17 @@ class NativeCausalLM(nn.Module):
                         and o.in_features % 8 == 0 and d.in_features % 8 == 0 and w1 is not None and w2 is not None
                         and w1.dtype == w2.dtype == self.dtype and w1.is_contiguous() and w2.is_contiguous())
             tables = tables or q.fmt in _TABLE_FMTS or o.fmt in _TABLE_FMTS or gu.fmt in _TABLE_FMTS or d.fmt in _TABLE_FMTS
+            fo.add(o.fmt)
             qkv.add((q.out_features, q.in_features, q.fmt))
             down.append((d.in_features, d.fmt))
-        return _Layers(norm_in, native, norm_in and row_norm, bias, tables, qkv, set(down[:-1]))
+        return _Layers(norm_in, native, norm_in and row_norm, bias, tables, fo, qkv, set(down[:-1]))
 
     def _row_norm_ok(self, T: int, seen) -> bool:
-        """o and down projections whose launch finishes its rows: 16-column tiles, sums of squares in whole fours"""
-        return (ROW_NORM and T <= 16 and not self._oproj_combine and not DEFER_MLP_ACC and self.spec.hidden_size % 64 == 0
-                and self.tp_group is None and seen().row_norm)
+        """o and down projections whose launch finishes its rows: 16-column tiles, sums of squares in whole fours, where
+        row_norm_o_takes in csrc/torch/ops_hip.cpp says so"""
+        H, t = self.spec.hidden_size, torch.ops.ipex_llm_amd
+        return (ROW_NORM and not self._oproj_combine and not DEFER_MLP_ACC and H % 64 == 0 and self.tp_group is None
+                and seen().row_norm and all(t.row_norm_o_takes(T, H, fmt) for fmt in seen().o))
 
     def _rows_ok(self, T: int, meta: "AttnMeta", cache, seen) -> bool:
         """more sequences than the split-K launches serve, up to 16: every launch of the step finishes its rows (or is the

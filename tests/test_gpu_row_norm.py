@@ -141,13 +141,22 @@ def test_whole_sums_in_any_shape(M):
 
 
 def test_rule():
-    """a down projection finishes its rows: 8 bits; 4 bits of at most one workgroup per CU but for what row_norm_takes names"""
+    """a down projection finishes its rows: 8 bits, integers in well-filled rounds; 4 bits of at most one workgroup per CU
+    but for what row_norm_takes names; an o projection but for wide tables"""
     ops.require()
     f = lambda M, n, k, q: torch.ops.ipex_llm_amd.row_norm_takes(M, n, k, fmt_of(q))      # noqa: E731
     assert [f(M, 4096, 14336, "sym_int4") for M in (1, 2, 3, 8, 9, 16, 17)] == [True, True, False, False, True, True, False]
     assert [f(M, 4096, 14336, "nf4") for M in (1, 2, 3, 12, 13)] == [True, True, False, False, True]
     assert f(8, 3584, 18944, "sym_int4") and f(8, 8192, 28672, "fp8_e5m2") and f(4, 4096, 14336, "asym_int4")
     assert not f(1, 5120, 13824, "sym_int4")
+    for q in ("sym_int8", "sym_int5", "asym_int5"):          # rounds of one workgroup per CU: the last at least half full
+        assert [f(5, 16 * t, 13824, q) for t in (256, 257, 320, 383, 384, 512, 513)] == [True, False, False, False, True, True,
+                                                                                          False]
+    assert all(f(5, 5120, 13824, q) for q in ("fp8_e4m3", "fp8_e5m2", "fp6"))
+    o = lambda M, n, q: torch.ops.ipex_llm_amd.row_norm_o_takes(M, n, fmt_of(q))          # noqa: E731
+    for q in ("nf4", "nf3"):
+        assert [o(M, 5120, q) for M in (1, 4, 5, 8)] == [True, True, False, False] and o(16, 4096, q) and not o(17, 4096, q)
+    assert o(8, 5120, "sym_int4") and o(8, 8192, "fp4") and o(8, 8192, "sym_int8") and not o(17, 4096, "sym_int4")
     g = lambda M, n, k, q: torch.ops.ipex_llm_amd.row_norm_takes(M, n, k, fmt_of(q), True)      # noqa: E731
     assert g(8, 4096, 14336, "sym_int4") and g(8, 4096, 14336, "nf4") and not g(8, 5120, 13824, "sym_int4")
     r = lambda M, n, k, q: torch.ops.ipex_llm_amd.row_rope_takes(M, n, k, fmt_of(q))            # noqa: E731
