@@ -220,10 +220,14 @@ def test_decode_onorm_matches_standalone_norm(cuda, monkeypatch):
                       num_attention_heads=8, num_key_value_heads=2, max_position_embeddings=1024)
     m = random_native_model(cfg, "sym_int4", cuda, torch.bfloat16, seed=5)
     prompts = [list(range(1 + i, 40 + 3 * i)) for i in range(8)]
-    outs = {}
+    outs, seen = {}, []
+    monkeypatch.setattr(D, "ROW_NORM", False)                 # (o finishes its rows otherwise, whatever ONORM says)
+    call = ops.gemv_accum_norm
+    monkeypatch.setattr(ops, "gemv_accum_norm", lambda *a, **k: (seen.append(1), call(*a, **k))[1])
     for flag in (False, True):
         monkeypatch.setattr(D, "ONORM", flag)
         outs[flag] = Engine(m).generate(prompts, max_new_tokens=8, use_graph=True)
+        assert bool(seen) == flag
     a, b = sum(outs[False], []), sum(outs[True], [])
     assert sum(x == y for x, y in zip(a, b)) >= 0.95 * len(a)
 
@@ -752,7 +756,7 @@ def test_dequantize_device_transposed(cuda, name, n, k):
         assert wt.shape == (k, n) and torch.equal(wt, w.t())
 
 
-def test_decode_oproj_combine_with_deferred_norm(cuda):
+def test_decode_oproj_combine_with_deferred_norm(cuda, monkeypatch):
     """attention partials merged in the o_proj GEMV prologue (opt-in) on top of
     the deferred norm and the GEMV-epilogue RoPE: same greedy tokens as the
     combine launch up to rare last-bit ties, graph == eager"""
@@ -760,15 +764,18 @@ def test_decode_oproj_combine_with_deferred_norm(cuda):
     from ipex_llm_amd.engine.runner import Engine
     from ipex_llm_amd.models.builder import random_native_model
     from ipex_llm_amd.models.decoder import NativeCausalLM
-    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024, num_hidden_layers=3,
+    cfg = LlamaConfig(vocab_size=512, hidden_size=1024, intermediate_size=1024, num_hidden_layers=3,
                       num_attention_heads=8, num_key_value_heads=2, max_position_embeddings=1024)
     m = random_native_model(cfg, "sym_int4", cuda, torch.bfloat16, seed=8)
     prompts = [list(range(1, 50)), list(range(7, 70))]
-    outs = {}
+    outs, seen = {}, []
+    call = ops.gemv_attn
+    monkeypatch.setattr(ops, "gemv_attn", lambda *a, **k: (seen.append(1), call(*a, **k))[1])
     try:
         for flag in (False, True):
             NativeCausalLM._oproj_combine = flag
             outs[flag] = Engine(m).generate(prompts, max_new_tokens=10, use_graph=True)
+            assert bool(seen) == flag                         # heads of 128: what the fused rotation has
         eager = Engine(m).generate(prompts, max_new_tokens=10, use_graph=False)
     finally:
         NativeCausalLM._oproj_combine = False
