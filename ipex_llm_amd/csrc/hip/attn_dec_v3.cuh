@@ -267,9 +267,10 @@ __global__ void __launch_bounds__(256) attn_combine_v3_kernel(const AttnDecodeAr
 // A wave's 32 K rows are requested in whole rows (a load is 4 rows of 256 bytes) and go to the fragments of the score
 // products by way of the LDS rows that its V takes afterwards: requested as fragments, a load is a piece of 16 rows for each
 // 16 lanes, which holds the address unit four times as long.  LDS operations of a wave are done in order: no wait and no
-// barrier, only the compiler has to keep the order of what other lanes wrote.  A decode step of Llama-3-8B, 1024 tokens, 1 /
-// 8 / 16 sequences: 1377 1770 2316 -> 1371 1762 2311 us, 20 of 2000 tokens 3001 -> 2940.  (The kernel with several tiles a
-// wave spills with it.)
+// barrier, only the compiler has to keep the order of what other lanes wrote.  Little at short contexts: a decode step of
+// Llama-3-8B, 1024 tokens, fragments / rows in turn on one card, twice, 1 sequence 1412 1414 / 1408 1404 us, 8 sequences 1780
+// 1789 / 1774 1780 (runs of one side 0.2 to 0.4 % apart), Qwen2.5-7B fp8_e5m2, 5 sequences, 1897 / 1896; 20 sequences of 2000
+// tokens 3001 / 2940.  (The kernel with several tiles a wave spills with it.)
 __device__ __forceinline__ void v3_lds_order() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_wave_barrier();

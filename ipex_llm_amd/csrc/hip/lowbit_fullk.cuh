@@ -6,9 +6,10 @@
 // A projection of 9 to 70 MB at few rows is bound by its chain of latencies, not by its bytes: launch, x from L2, weights,
 // sum over K, and -- where K is cut over workgroups -- f32 atomics, a ticket and the sums read back before the row can be
 // finished, 3 to 5 us of a 5 us product.  So K is not cut over workgroups:
-//   * a workgroup's 8 (16) waves take an eighth (a 16th) of K each and meet once, in LDS; every wave stages its own x (a piece = 4 chunks
-//     of 128 k; 2 from 9 rows on) in an LDS region of its own, so nothing waits for another wave before the end, and
-//     requests its weights before it needs x: all of them where K is one piece a wave (to K = 4096), two pieces ahead else.
+//   * a workgroup's 8 (16) waves take an eighth (a 16th) of K each and meet once, in LDS; every wave stages its own x (a
+//     piece = 4 chunks of 128 k; 2 from 9 rows on) in an LDS region of its own, so nothing waits for another wave before the
+//     end, and requests its weights before it needs x: all of them where K is one piece a wave (to K = 4096), two pieces
+//     ahead else.
 //     A request out of range is not free (its turn in the address unit, 1 us over the 24 of a wave of K = 4096 whose ring
 //     was 16 chunks deep), hence the exact ends;
 //   * x is the A operand, raw codes the B operand, and the offset a product of x with a constant (lowbit_skinny.cuh), shared
@@ -19,7 +20,8 @@
 // / this: sym_int4 [4096, 4096] 7.9 8.0 8.9 12.0 / 4.6 4.6 4.8 5.7, asym_int4 8.9 9.2 10.5 13.6 / 4.7 4.8 5.2 6.1, fp8_e5m2
 // [3584, 3584] 9.2 9.4 10.3 12.7 / 4.6 4.8 5.2 6.3 (the split-K product without its rows 6.6 6.8 7.3 8.3).  A long K is
 // bound by x, which every workgroup reads in full (sym_int4 [4096, 14336] 8.8 / 10.1 / 11.9 / 13.2, of 58 MB of x at 8 rows;
-// the rules row_norm_takes, row_rope_takes and glu_rows_takes of csrc/torch/ops_hip.cpp, with qkv's and gate/up's figures).
+// the rules row_norm_takes, row_norm_o_takes, row_rope_takes and glu_rows_takes of csrc/torch/ops_hip.cpp, with qkv's and
+// gate/up's figures).
 // 16 waves of a K that 8 hold in one piece, or pieces four ahead, were slower.  A decode step, us: Llama-3-8B sym_int4,
 // 1024 tokens, 1 / 4 / 8 rows 1572 1844 1981, with o and down here 1499 1635 1809, and qkv 1473 1599 1774, and gate/up 1379
 // 1551 1769; Qwen2.5-7B fp8_e5m2, 1 / 5 rows 2149 2372, 1995 2182, 1887 2014, 1704 1886.

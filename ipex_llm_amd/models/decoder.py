@@ -205,7 +205,7 @@ ONORM_MIN_M = int(__import__("os").environ.get("ILLM_ONORM_MIN_M", "5"))
 ROW_NORM = __import__("os").environ.get("ILLM_ROW_NORM", "1") != "0"
 # ... up to this many sequences where every launch of the step does so (hidden sizes up to 4096).  A step, us, 8 launches a
 # layer with slabs, rope and norm launches of their own / 5: Llama-3-8B sym_int4, 1024 tokens, 10 / 16 sequences 2260 2473 /
-# 1871 2316, 500 tokens, 9 / 16 sequences, asym_int4 2199 2343 / 1795 1984, nf4 2785 3049 / 2544 2788, sym_int8 2655 2807 /
+# 1871 2316, 500 tokens, 9 / 16 sequences, asym_int4 2199 2343 / 1795 1984, sym_int8 2655 2807 /
 # 2368 2570; Qwen2.5-7B fp8_e5m2 10 / 16 sequences 2514 2630 / 2245 2387
 ROW_NORM_MAX_M = int(__import__("os").environ.get("ILLM_ROW_NORM_MAX_M", "16"))
 _TABLE_FMTS = (Q.FMT_NF4, Q.FMT_NF3)            # their products are f16 also under bf16 activations
