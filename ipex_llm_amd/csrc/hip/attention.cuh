@@ -1162,6 +1162,7 @@ static void launch_v2(const AttnDecodeArgs& a0, hipStream_t st) {
 
 }  // namespace illm
 #include "attn_dec_v3.cuh"
+#include "attn_dec_v4.cuh"
 namespace illm {
 
 template <typename T, int D>
@@ -1170,8 +1171,9 @@ void launch_d(const AttnDecodeArgs& a, hipStream_t st) {
   if constexpr (D == 64 || D == 128) {
     if (v3_ok(a, D)) {
       if constexpr (D == 128) {
-        if (a.rq_part != nullptr)
-          return a.rq_prerot && a.rq_bias == nullptr ? launch_v3<T, D, 2>(a, st) : launch_v3<T, D, 1>(a, st);
+        const bool pre = a.rq_part != nullptr && a.rq_prerot && a.rq_bias == nullptr;
+        if (pre ? launch_v4<T, D, 2>(a, st) : a.rq_part == nullptr && launch_v4<T, D, 0>(a, st)) return;
+        if (a.rq_part != nullptr) return pre ? launch_v3<T, D, 2>(a, st) : launch_v3<T, D, 1>(a, st);
       }
       return launch_v3<T, D, 0>(a, st);
     }

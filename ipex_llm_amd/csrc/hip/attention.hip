@@ -38,5 +38,10 @@ int attn_decode_groups(int B, int Hkv, int nsplit) {
   a.nsplit = nsplit;
   return v3_long_grid(a, 0);
 }
+int attn_decode_plan(int B, int Hkv, int nsplit, int* groups) {
+  const V4Plan p = v4_plan(B, Hkv, nsplit);
+  *groups = p.groups;
+  return p.nw;
+}
 
 }  // namespace illm

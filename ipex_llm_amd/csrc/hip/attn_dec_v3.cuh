@@ -591,7 +591,7 @@ __global__ void __launch_bounds__(64 * NW, ILLM_V3_MINW(RQ)) attn_decode_v3_kern
   attn_v3_body<T, D, NW, RQ, FUSE>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, sm);
 }
 
-// ---- long contexts: several 32-key tiles per wave -------------------------
+// ---- long contexts: several 32-key tiles per wave (the rotation here, or head dim 64; else attn_dec_v4.cuh) --------
 // One tile per wave pays a workgroup's fixed chain (sequence length -> block
 // table -> K / V round trip -> max and sum over the waves -> partial) for every
 // 32 NW keys: 20 K keys x 3 sequences were 1896 workgroups in 7 rounds, 74 us

@@ -2161,6 +2161,12 @@ TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("row_norm_o_takes(int M, int n, int fmt) -> bool", &row_norm_o_takes);
   m.def("row_rope_takes(int M, int n, int k, int fmt) -> bool", &row_rope_takes);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
+  m.def("attn_decode_plan(int batch, int kv_heads, int nsplit) -> int[]", [](int64_t b, int64_t h, int64_t n) -> std::vector<int64_t> {
+    TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_plan: sizes");
+    int groups = 0;
+    const int nw = illm::attn_decode_plan((int)b, (int)h, (int)n, &groups);
+    return {nw, groups};
+  });
   m.def("attn_decode_groups(int batch, int kv_heads, int nsplit) -> int", [](int64_t b, int64_t h, int64_t n) -> int64_t {
     TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_groups: sizes");
     return illm::attn_decode_groups((int)b, (int)h, (int)n);
