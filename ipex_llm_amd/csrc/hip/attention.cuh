@@ -1168,6 +1168,9 @@ namespace illm {
 template <typename T, int D>
 void launch_d(const AttnDecodeArgs& a, hipStream_t st) {
   const int R = (a.Hq / a.Hkv) * a.Tq;
+  if constexpr (D == 128) {
+    if (a.rq_slabs > 0) return launch_v4_slabs<T>(a, st);         // (attn_slabs_takes)
+  }
   if constexpr (D == 64 || D == 128) {
     if (v3_ok(a, D)) {
       if constexpr (D == 128) {

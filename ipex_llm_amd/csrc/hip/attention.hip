@@ -43,5 +43,10 @@ int attn_decode_plan(int B, int Hkv, int nsplit, int* groups) {
   *groups = p.groups;
   return p.nw;
 }
+bool attn_slabs_takes(int B, int Hkv, int nsplit) {
+  AttnDecodeArgs a{};
+  a.Hq = a.Hkv = a.Tq = 1;
+  return v3_ok(a, 128) && v4_plan(B, Hkv, nsplit).groups == 1;
+}
 
 }  // namespace illm

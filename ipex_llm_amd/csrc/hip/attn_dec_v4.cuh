@@ -17,17 +17,108 @@
 // below by the chain: 2.1 us a tile and wave with 8 waves on the CU, 1.3 with four.
 #pragma once
 #include <algorithm>
+#include <climits>
 
 namespace illm {
+
+// RQ 3: the qkv product's f32 slabs [ks, B, ld], bias and rotation as in rope_kv.hip, the same bits.  An item is dims d, d + 1
+// and their partners D / 2 on of one head, for a thread; q goes to LDS for all waves, k and v there and to the cache.  Only
+// where one workgroup has a pair (launch_v4_slabs): with several, each would rotate the same rows.  The rope launch takes 5.2 us
+// for 0.5 us of bytes; this prologue, its loads ahead of the first tile's, 1.5 to 3: us a step, launch / this, Llama-3-8B 17 x 1024
+// tokens 2374 / 2305, 24 x 600 2342 / 2262, 33 x 300 2597 / 2508, 64 x 900 asym_int4 4071 / 3980, 64 x 128 3013 / 2900, Qwen2.5-7B
+// fp8_e5m2 40 x 500 2906 / 2868, 20 x 150 sym_int4 2082 / 1984, nf4 12 x 180 2680 / 2640.  (The block of the new key asked for behind
+// the tile's requests, so that its wait is also for them: 0.7 us a launch more.)
+template <typename T, int D>
+struct V4Slabs {
+  float2 f[4][2];                                                 // the first four slabs, in flight together
+  uint16_t bias[2][2];
+  float4 cs;
+  int64_t pos, off;
+  int hh, d, col, blk;
+  __device__ void load(const AttnDecodeArgs& a, int b, int kvh, int group, int item) {
+    const int it = min(item, (group + 2) * (D / 4) - 1);          // (past the last: not stored)
+    hh = it / (D / 4) - group;                                    // below 0: a query head, 0: k, 1: v
+    d = it % (D / 4) * 2;
+    col = (hh < 0 ? kvh * group + hh + group : a.Hq + hh * a.Hkv + kvh) * D + d;
+    pos = a.rq_pos[b];
+    off = a.rq_pos_offset ? a.rq_pos_offset[b] : 0;
+    const float* p = a.rq_part + (size_t)b * a.rq_ld + col;
+    const size_t slab = (size_t)a.B * a.rq_ld;
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) f[s][h] = *(const float2*)(p + min(s, a.rq_slabs - 1) * slab + h * (D / 2));
+    const uint16_t* bp = a.rq_bias ? a.rq_bias + col : (const uint16_t*)p;
+#pragma unroll
+    for (int h = 0; h < 2; h++) bias[h][0] = bp[h * (D / 2)], bias[h][1] = bp[h * (D / 2) + 1];
+  }
+  // what the position leads to: ahead of the keys' requests, a wait is for all that was asked before
+  __device__ void follow(const AttnDecodeArgs& a, int b) {
+    cs = *(const float4*)(a.rq_cos_sin + ((size_t)pos * (D / 2) + d) * 2);
+    const int64_t k = pos - off;
+    const bool in = k >= 0 && k < (int64_t)a.max_blocks * a.bs;
+    blk = a.block_tables[(size_t)b * a.max_blocks + (in ? (uint32_t)k / (uint32_t)a.bs : 0u)];
+    blk = in ? blk : INT_MAX;
+  }
+  __device__ int key(int len) const {                             // index of the new key, -1: not among the len of the call
+    const int64_t k = pos - off;
+    return __builtin_amdgcn_readfirstlane(k >= 0 && k < len ? (int)k : -1);
+  }
+  __device__ void finish(const AttnDecodeArgs& a, int b, int kvh, int item, uint16_t (*q)[D], uint16_t (*kv)[D]) const {
+    const int group = a.Hq / a.Hkv;
+    if (item >= (group + 2) * (D / 4)) return;
+    float v[2][2] = {};
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        v[h][0] = s < a.rq_slabs ? v[h][0] + f[s][h].x : v[h][0];
+        v[h][1] = s < a.rq_slabs ? v[h][1] + f[s][h].y : v[h][1];
+      }
+    for (int s = 4; s < a.rq_slabs; s++) {
+      const float* p = a.rq_part + ((size_t)s * a.B + b) * a.rq_ld + col;
+      for (int h = 0; h < 2; h++) v[h][0] += p[h * (D / 2)], v[h][1] += p[h * (D / 2) + 1];
+    }
+    auto rnd = [](float x) { return to_f32<T>(from_f32<T>(x)); };
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        if (a.rq_bias) v[h][e] += to_f32<T>(bias[h][e]);
+        v[h][e] = rnd(v[h][e]);
+      }
+    if (hh < 1) {                                                 // cos and sin in T, each product rounded to it
+      const float osc = hh < 0 ? a.rq_qscale : 1.f;
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        const float c = rnd(e ? cs.z : cs.x), sn = rnd(e ? cs.w : cs.y), x0 = v[0][e], x1 = v[1][e];
+        v[0][e] = (rnd(x0 * c) - rnd(x1 * sn)) * osc;
+        v[1][e] = (rnd(x1 * c) + rnd(x0 * sn)) * osc;
+      }
+    }
+    const uint32_t o[2] = {pack2<T>(v[0][0], v[0][1]), pack2<T>(v[1][0], v[1][1])};
+    uint16_t* l = hh < 0 ? q[hh + group] : kv[hh];
+#pragma unroll
+    for (int h = 0; h < 2; h++) *(uint32_t*)(l + d + h * (D / 2)) = o[h];
+    if (hh < 0) return;
+    const bool oob = blk >= a.num_blocks;
+    if (oob) kerr(a.err, ERR_SLOT);
+    if (blk < 0 || oob) return;                                   // a padding row
+    uint16_t* c = (uint16_t*)(hh == 0 ? a.k_cache : a.v_cache) + (((size_t)blk * a.Hkv + kvh) * a.bs + (uint32_t)(pos - off) % (uint32_t)a.bs) * D + d;
+#pragma unroll
+    for (int h = 0; h < 2; h++) *(uint32_t*)(c + h * (D / 2)) = o[h];
+  }
+};
 
 template <typename T, int D, int NW, int RQ, bool FUSE>
 __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDecodeArgs a) {
   constexpr int SK = V3_KPW * NW;                  // keys of a tile
   constexpr int KSTEP = D / 32, DT = D / 16, VU = D / 8, KPJ = 64 / VU, VJ = V3_KPW / KPJ;
   static_assert(D == 64 || D == 128, "v4: head_dim 64 / 128");
-  static_assert(RQ == 0 || (RQ == 2 && D == 128), "v4: q from memory, or pre-rotated with head_dim 128");
+  static_assert(RQ == 0 || ((RQ == 2 || RQ == 3) && D == 128), "v4: q from memory, pre-rotated or as slabs with head_dim 128");
   __shared__ __attribute__((aligned(16))) uint16_t vl[V3_KPW * NW * D];   // a wave's 32 K rows, then its V rows; the sums at the end
   __shared__ __attribute__((aligned(16))) uint16_t fresh[RQ != 0 ? 2 : 1][D];   // the new token's k and v rows
+  __shared__ __attribute__((aligned(16))) uint16_t qrot[RQ == 3 ? 16 : 1][D];
   __shared__ float smx[NW][16], sml[NW][16];
   __shared__ int s_last;
   const int split = blockIdx.x, S = gridDim.x, kvh = blockIdx.y, b = blockIdx.z;
@@ -49,10 +140,13 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
   int ent = entries(0);
   const int row = r16 < R ? r16 : 0;
   const int t = row / group, h = kvh * group + row % group;
-  const V3Rope<T, D, true> rp(a, b, g, RQ != 0);
+  const V3Rope<T, D, true> rp(a, b, g, RQ == 2);
   typename V3Rope<T, D, true>::Raw qraw;
   uint4 qf[KSTEP];
-  if constexpr (RQ != 0) {
+  V4Slabs<T, D> sl;
+  if constexpr (RQ == 3) {
+    sl.load(a, b, kvh, group, threadIdx.x);
+  } else if constexpr (RQ != 0) {
     if constexpr (D == 128) rp.load(h * D, qraw);
   } else {
     const uint16_t* qr = a.q + (((size_t)b * a.Tq + t) * a.Hq + h) * D;
@@ -102,6 +196,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     }
   };
 
+  if constexpr (RQ == 3) sl.follow(a, b);                        // (the position came with the length)
   uint4 kc[VJ], vc[VJ];
   auto request = [&](int j, uint4 (&k)[VJ], uint4 (&v)[VJ]) {
     int kw, blk;
@@ -113,8 +208,19 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
   if (nt > 0) request(0, kc, vc);
 
   // ---- the new token's rows (RQ): the wave whose last tile ends the sequence appends them and uses them from registers
-  const bool holds_new = RQ != 0 && nt > 0 && (len - 1) / SK % S == split && (len - 1) % SK / V3_KPW == wv;
-  if constexpr (RQ != 0) {
+  const int newest = RQ == 3 ? sl.key(len) : len - 1;             // (slabs: -1, not among the keys)
+  const bool holds_new = RQ != 0 && nt > 0 && newest >= 0 && newest / SK % S == split && newest % SK / V3_KPW == wv;
+  if constexpr (RQ == 3) {
+    for (int it = threadIdx.x;;) {
+      sl.finish(a, b, kvh, it, qrot, fresh);
+      if ((it += NW * 64) >= (group + 2) * (D / 4)) break;
+      sl.load(a, b, kvh, group, it);
+      sl.follow(a, b);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < KSTEP; s++) qf[s] = *(const uint4*)(qrot[row] + 32 * s + 8 * g);
+  } else if constexpr (RQ != 0) {
     const int d0 = 8 * (lane % VU);
     float4 k0, k1, v0, v1;
     uint4 nb;
@@ -162,7 +268,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     int kwc, blk;
     size_t base;
     const int nvis = tile_at(j, kwc, base, blk);
-    const int at = holds_new && j == nt - 1 && nvis > 0 ? nvis - 1 : -1;
+    const int at = holds_new && j == (RQ == 3 ? newest / SK : nt - 1) && nvis > 0 ? newest - kwc : -1;
     v3_lds_order();
     store(k, 0, at);
     v3_lds_order();
@@ -299,7 +405,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     }
   }
   if (S == 1) {
-    if constexpr (RQ != 0) {
+    if constexpr (RQ == 2) {
       // every wave has read its columns of the qkv sums: zero for the next layer's adds
       float* pr = (float*)a.rq_part + (size_t)b * a.rq_ld;
       for (int i = threadIdx.x * 4; i < (group + 2) * D; i += NW * 64 * 4) {
@@ -363,6 +469,14 @@ static void launch_v4_nw(const AttnDecodeArgs& a, int S, hipStream_t st) {
     hipLaunchKernelGGL((attn_decode_v4_kernel<T, D, NW, RQ, false>), grid, dim3(64 * NW), 0, st, a);
     hipLaunchKernelGGL((attn_combine_v3_kernel<T>), dim3(a.Hkv, a.B), dim3(256), 0, st, a, S);
   }
+}
+
+// q, k and v as slabs of the qkv product: one workgroup a pair (v4_plan), checked by the caller
+template <typename T>
+static void launch_v4_slabs(const AttnDecodeArgs& a, hipStream_t st) {
+  dim3 grid(1, a.Hkv, a.B);
+  if (v4_plan(a.B, a.Hkv, a.nsplit).nw == 8) hipLaunchKernelGGL((attn_decode_v4_kernel<T, 128, 8, 3, false>), grid, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((attn_decode_v4_kernel<T, 128, 4, 3, false>), grid, dim3(256), 0, st, a);
 }
 
 template <typename T, int D, int RQ>

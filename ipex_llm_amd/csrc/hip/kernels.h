@@ -208,12 +208,16 @@ struct AttnDecodeArgs {
   // v3 (attn_dec_v3.cuh): zeroed [B * Hkv] arrival counters for its in-kernel
   // combine (null: separate combine launch)
   int* v3_counters;
+  int rq_slabs;             // > 0: rq_part is that many unrotated slabs [rq_slabs, B, rq_ld] (attn_dec_v4.cuh), left as they are
+  const int64_t* rq_pos_offset;   // [B] or null: rq_pos less this is the new key's index (slabs only)
 };
 void launch_attn_decode(bool bf16, const AttnDecodeArgs& a, hipStream_t st);
 // workgroups per (sequence, kv head) of several tiles per wave, q from memory (0: one tile per wave)
 int attn_decode_groups(int B, int Hkv, int nsplit);
 // waves of a workgroup (returned) and workgroups per pair of the streaming kernel, head dim 128 (0, 0: not taken)
 int attn_decode_plan(int B, int Hkv, int nsplit, int* groups);
+// one workgroup a pair: it can take q, k and v as slabs of the qkv product (AttnDecodeArgs::rq_slabs)
+bool attn_slabs_takes(int B, int Hkv, int nsplit);
 
 // ---- prefill / long-query attention over the paged cache (attn_prefill.hip)
 struct AttnPrefillArgs {

@@ -1665,6 +1665,66 @@ static std::tuple<Tensor, Tensor, Tensor> attn_decode_rope_impl(
 }
 
 
+// decode attention (Tq == 1, head dim 128, full NeoX rotation) over the slabs [ks, B, ld] of the qkv product: their sum, bias,
+// rotation and the append at pos - pos_offset as in rope_kv_fused, without its launch.  Where attn_slabs_takes says so
+Tensor attn_decode_slabs(const Tensor& part, const c10::optional<Tensor>& bias, const Tensor& cos_sin, const Tensor& pos,
+                         const c10::optional<Tensor>& pos_offset, Tensor& k_cache, Tensor& v_cache, const Tensor& block_tables,
+                         const Tensor& seq_lens, int64_t nsplit, double scale, double softcap, int64_t window, int64_t Hq,
+                         at::ScalarType dt) {
+  c10::DeviceGuard g(part.device());
+  TORCH_CHECK(dt == at::kBFloat16 || dt == at::kHalf, "attn_decode_slabs: bf16/fp16 activations");
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.scalar_type() == dt && v_cache.scalar_type() == dt && k_cache.is_contiguous() &&
+                  v_cache.is_contiguous() && v_cache.sizes() == k_cache.sizes(), "attn_decode_slabs: contiguous 16-bit KV cache");
+  TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.scalar_type() == at::kFloat && part.is_contiguous() && part.size(0) >= 1,
+              "attn_decode_slabs: part must be contiguous f32 [ks, B, ld]");
+  const int64_t B = part.size(1), Hkv = k_cache.size(1), bs = k_cache.size(2);
+  TORCH_CHECK(k_cache.size(3) == 128 && Hq >= Hkv && Hq % Hkv == 0 && Hq / Hkv <= 16 && bs % 64 == 0, "attn_decode_slabs: geometry");
+  TORCH_CHECK(part.size(2) == (Hq + 2 * Hkv) * 128, "attn_decode_slabs: part width != (Hq + 2 Hkv) * 128");
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() && cos_sin.dim() == 3 && cos_sin.size(1) == 64 &&
+                  cos_sin.size(2) == 2, "attn_decode_slabs: f32 cos/sin table [max_pos, 64, 2]");
+  TORCH_CHECK((uintptr_t)part.data_ptr() % 16 == 0 && (uintptr_t)cos_sin.data_ptr() % 16 == 0, "attn_decode_slabs: alignment");
+  TORCH_CHECK(pos.scalar_type() == at::kLong && pos.is_contiguous() && pos.numel() >= B && block_tables.scalar_type() == at::kInt &&
+                  block_tables.is_contiguous() && block_tables.size(0) >= B && seq_lens.scalar_type() == at::kInt &&
+                  seq_lens.is_contiguous() && seq_lens.numel() >= B, "attn_decode_slabs: int64 positions, int32 tables of B rows");
+  TORCH_CHECK(nsplit >= 1 && nsplit <= kMaxDecodeSplits && !fused_combine_on() && illm::attn_slabs_takes((int)B, (int)Hkv, (int)nsplit),
+              "attn_decode_slabs: not taken");
+  illm::AttnDecodeArgs a{};
+  Tensor out = at::empty({B, 1, Hq, 128}, part.options().dtype(dt));
+  a.k_cache = (const uint8_t*)k_cache.data_ptr();
+  a.v_cache = (const uint8_t*)v_cache.data_ptr();
+  a.block_tables = block_tables.data_ptr<int32_t>();
+  a.seq_lens = seq_lens.data_ptr<int32_t>();
+  a.max_blocks = (int)block_tables.size(1);
+  a.num_blocks = (int)k_cache.size(0);
+  a.err = kernel_err(k_cache.device());
+  a.out = m16(out);
+  a.B = (int)B;
+  a.Tq = 1;
+  a.Hq = (int)Hq;
+  a.Hkv = (int)Hkv;
+  a.D = 128;
+  a.bs = (int)bs;
+  a.nsplit = (int)nsplit;
+  a.scale = (float)scale;
+  a.softcap = (float)softcap;
+  a.sliding_window = (int)window;
+  a.k_scale = a.v_scale = 1.f;
+  a.rq_part = part.data_ptr<float>();
+  a.rq_slabs = (int)part.size(0);
+  a.rq_bias = p16o(bias);
+  a.rq_cos_sin = cos_sin.data_ptr<float>();
+  a.rq_pos = pos.data_ptr<int64_t>();
+  if (pos_offset.has_value() && pos_offset->defined()) {
+    TORCH_CHECK(pos_offset->scalar_type() == at::kLong && pos_offset->is_contiguous() && pos_offset->numel() >= B, "attn_decode_slabs: int64 offsets");
+    a.rq_pos_offset = pos_offset->data_ptr<int64_t>();
+  }
+  a.rq_ld = (int)part.size(2);
+  a.rq_rot = 128;
+  a.rq_qscale = 1.f;
+  illm::launch_attn_decode(dt == at::kBFloat16, a, cur_stream());
+  return out;
+}
+
 Tensor attn_decode_rope(const Tensor& part, const c10::optional<Tensor>& bias, const Tensor& cos_sin,
                         const Tensor& pos, Tensor& k_cache, Tensor& v_cache, const Tensor& block_tables,
                         const Tensor& seq_lens, int64_t nsplit, double scale, double softcap, int64_t window,
@@ -2161,6 +2221,9 @@ TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("row_norm_o_takes(int M, int n, int fmt) -> bool", &row_norm_o_takes);
   m.def("row_rope_takes(int M, int n, int k, int fmt) -> bool", &row_rope_takes);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
+  m.def("attn_slabs_takes(int batch, int kv_heads, int nsplit) -> bool", [](int64_t b, int64_t h, int64_t n) {
+    return b >= 1 && b < (1 << 20) && n >= 1 && n <= kMaxDecodeSplits && !fused_combine_on() && illm::attn_slabs_takes((int)b, (int)h, (int)n);
+  });
   m.def("attn_decode_plan(int batch, int kv_heads, int nsplit) -> int[]", [](int64_t b, int64_t h, int64_t n) -> std::vector<int64_t> {
     TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_plan: sizes");
     int groups = 0;
@@ -2205,6 +2268,7 @@ TORCH_LIBRARY_IMPL(ipex_llm_amd, CUDA, m) {
   m.impl("rwkv_wkv5", &rwkv_wkv5);
   m.impl("attn_decode_rope", &attn_decode_rope);
   m.impl("attn_decode_rope_split", &attn_decode_rope_split);
+  m.impl("attn_decode_slabs", &attn_decode_slabs);
   m.impl("gemm", &gemm);
   m.impl("attn_decode_split", &attn_decode_split);
   m.impl("attn_prefill", &attn_prefill);

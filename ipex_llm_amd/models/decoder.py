@@ -769,6 +769,12 @@ class NativeCausalLM(nn.Module):
         row_rope = prerot and row_norm and self._row_rope_ok(T, seen)  # bias and rotation ahead of the store
         prerot = row_rope or (prerot and not seen().bias)
         rope_in = rope_ok and (T <= ROPE_IN_MAX_M or prerot)
+        # more sequences than that: qkv slabs, whose sum, rotation and append the attention does where a workgroup has a whole
+        # (sequence, kv head)
+        slabs_in = (T > ACC_MAX_M and not rope_in and self._rope_in_ok(meta, cache) and s.head_dim == s.rot_dim == 128
+                    and not s.rope_interleaved and self.alibi is None and not self._attn_fuse and x.is_cuda
+                    and cache.k[0].dtype == x.dtype and ops.native_gpu(x)
+                    and torch.ops.ipex_llm_amd.attn_slabs_takes(meta.B, s.num_kv_heads, meta.nsplit))
         qrope = (self.rope_cache, pos, (s.num_heads + s.num_kv_heads) * s.head_dim, s.head_dim) if prerot else None
         nxt_res = lambda r: res_pp[1] if r is res_pp[0] else res_pp[0]
         zero_next = None                # consumed atomic slab the next accumulating GEMV zeroes
@@ -791,6 +797,7 @@ class NativeCausalLM(nn.Module):
             qp = attn.qkv_proj
             ss_q = None
             q = torch.empty(T, s.num_heads, s.head_dim, dtype=x.dtype, device=x.device)
+            a_rope = None                   # attention output of a launch that takes q, k and v from the qkv sums
             if x.is_cuda and isinstance(qp, LowBitLinear) and qp.mp_group is None and T <= ops.GEMV_MAX_M \
                     and (qp.bias is None or qp.bias.dtype == x.dtype) and ops.native_gpu(x):
                 # split-K GEMV reduced (+bias) inside the RoPE/KV kernel, slots from the block table:
@@ -818,7 +825,11 @@ class NativeCausalLM(nn.Module):
                     part = part.unsqueeze(0)
                 else:
                     part = ops.gemv_partials(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, 0)
-                if not rope_in:
+                if slabs_in:
+                    a_rope = ops.attn_decode_slabs(part, qp.bias, self.rope_cache, pos, meta.pos_offset, cache.k[li], cache.v[li],
+                                                   meta.block_tables, meta.seq_lens, meta.nsplit, s.scale, s.attn_softcap,
+                                                   attn.sliding_window, s.num_heads, x.dtype).view(T, -1)
+                elif not rope_in:
                     ops.rope_kv_fused(part, qp.bias, q, cache.k[li], cache.v[li], pos, meta.block_tables, meta.Tq,
                                       rope, s.num_heads, s.num_kv_heads, s.head_dim, s.rot_dim, s.rope_interleaved,
                                       attn.q_norm, attn.k_norm, s.rms_eps, 1.0, cache.kv_fp8, cache.k_scale,
@@ -867,7 +878,7 @@ class NativeCausalLM(nn.Module):
                                   self._oproj_ks, x.dtype, zero=consumed, nw=self._oproj_nw)
                     zero_qkv = qkv_acc
                 else:
-                    a = a_rope if rope_in else self._attention(li, attn, q, meta, cache)
+                    a = a_rope if a_rope is not None else self._attention(li, attn, q, meta, cache)
                     if fin_o:
                         # o_proj + residual add + deferred-norm staging of the gate/up input
                         r2 = nxt_res(residual)
@@ -937,14 +948,14 @@ class NativeCausalLM(nn.Module):
                     x, _ = ops.add_rms_norm(None, residual, nxt, s.rms_eps, partials=accD.unsqueeze(0),
                                             unit_offset=s.norm_unit_offset, zero_partials=True)
                 continue
-            if not rope_in and self._attn_oproj_fuse_ok(attn, q, meta):
+            if a_rope is None and self._attn_oproj_fuse_ok(attn, q, meta):
                 x = self._attn_oproj_norm(li, attn, q, meta, cache, residual, layer.post_attention_layernorm)
             elif s.sandwich_norm:
-                a = a_rope if rope_in else self._attention(li, attn, q, meta, cache)
+                a = a_rope if a_rope is not None else self._attention(li, attn, q, meta, cache)
                 x = self._proj_residual_norm(a, attn.o_proj, residual, layer.pre_feedforward_layernorm,
                                              post_norm_w=layer.post_attention_layernorm)
             else:
-                a = a_rope if rope_in else self._attention(li, attn, q, meta, cache)
+                a = a_rope if a_rope is not None else self._attention(li, attn, q, meta, cache)
                 x = self._proj_residual_norm(a, attn.o_proj, residual, layer.post_attention_layernorm)
             if li + 1 < len(self.layers):
                 nxt = self.layers[li + 1].input_layernorm

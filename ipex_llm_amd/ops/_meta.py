@@ -241,6 +241,11 @@ def _(part, bias, cos_sin, pos, k_cache, v_cache, block_tables, seq_lens, nsplit
     return part.new_empty((part.shape[0], 1, Hq, k_cache.shape[3]), dtype=dtype)
 
 
+@register_fake("ipex_llm_amd::attn_decode_slabs")
+def _(part, bias, cos_sin, pos, pos_offset, k_cache, v_cache, block_tables, seq_lens, nsplit, scale, softcap, window, Hq, dtype):
+    return part.new_empty((part.shape[1], 1, Hq, 128), dtype=dtype)
+
+
 @register_fake("ipex_llm_amd::attn_decode_rope_split")
 def _(part, bias, cos_sin, pos, k_cache, v_cache, block_tables, seq_lens, nsplit, scale, softcap, window, Hq,
       rot_dim, interleaved, q_scale, dtype, pss=None, pss_n=0, pss_eps=0.0, prerot=False):

@@ -19,7 +19,7 @@ __all__ = [
     "gemv_partials", "gemv_glu", "add_rms_norm", "rms_norm", "layer_norm", "rope_kv",
     "attn_decode", "glu", "attn_softmax_", "moe_topk", "reduce_partials", "to_fp8_bytes", "GEMV_MAX_M", "gather_kv",
     "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_row_norm", "gemv_rope", "gemv_glu_ss",
-    "attn_decode_split", "gemv_attn", "gemv_norm_in", "attn_decode_rope", "attn_decode_rope_split", "attn_prefill", "moe_group_topk",
+    "attn_decode_split", "gemv_attn", "gemv_norm_in", "attn_decode_rope", "attn_decode_rope_split", "attn_decode_slabs", "attn_prefill", "moe_group_topk",
 ]
 
 
@@ -693,6 +693,14 @@ def attn_decode_rope(part, bias, cos_sin, pos, k_cache, v_cache, block_tables, s
     return _ops().attn_decode_rope(part, bias, cos_sin, pos, k_cache, v_cache, block_tables, seq_lens, nsplit,
                                    scale, softcap, window, Hq, rot_dim, interleaved, q_scale, dtype, pss, pss_n,
                                    pss_eps, prerot)
+
+
+def attn_decode_slabs(part, bias, cos_sin, pos, pos_offset, k_cache, v_cache, block_tables, seq_lens, nsplit, scale, softcap,
+                      window, Hq: int, dtype):
+    """rope_kv_fused and attn_decode of one new token per sequence in one launch: ``part`` [ks, B, (Hq + 2 Hkv) * 128] f32
+    slabs of the qkv product, full NeoX rotation, 16-bit cache, where ``attn_slabs_takes`` says so."""
+    return _ops().attn_decode_slabs(part, bias, cos_sin, pos, pos_offset, k_cache, v_cache, block_tables, seq_lens, nsplit,
+                                    scale, softcap, window, Hq, dtype)
 
 
 def attn_decode_split(q, k_cache, v_cache, block_tables, seq_lens, nsplit, scale, softcap=0.0, window=0,

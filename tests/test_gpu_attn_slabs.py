@@ -1,0 +1,128 @@
+"""Decode attention over the slabs of the qkv product (attn_decode_slabs): bit for bit rope_kv_fused and attn_decode, in the
+output and in the caches -- one to six slabs, items of one pass over the workgroup and of several, the new key at the edges of
+tiles, offsets of a compressed cache, padding rows, bad blocks -- and in a model's step, captured too."""
+import pytest
+import torch
+
+import ipex_llm_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+T = torch.ops.ipex_llm_amd
+
+
+def _both(dev, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset, tables=None):
+    torch.manual_seed(len(L) * cap + ks)
+    B, Hq, D, nb = len(L), Hkv * G, 128, -(-cap // bs)
+    kc, vc = (torch.randn(nb * B, Hkv, bs, D, device=dev).to(dtype) for _ in range(2))
+    bt = torch.randperm(nb * B, device=dev).int().view(B, nb).contiguous()
+    if tables is not None:
+        tables(bt)
+    sl, ns = torch.tensor(L, dtype=torch.int32, device=dev), -(-cap // 64)
+    off = torch.arange(B, device=dev) * 3 if offset else None
+    pos = (sl.long() - 1).clamp(min=0) + (off if offset else 0)
+    cs = torch.randn(cap + 3 * B, D // 2, 2, device=dev)
+    part = torch.randn(ks, B, (Hq + 2 * Hkv) * D, device=dev)
+    b = torch.randn((Hq + 2 * Hkv) * D, device=dev).to(dtype) if bias else None
+    k1, v1, q = kc.clone(), vc.clone(), torch.empty(B, Hq, D, dtype=dtype, device=dev)
+    ops.rope_kv_fused(part, b, q, k1, v1, pos, bt, 1, cs, Hq, Hkv, D, pos_offset=off)
+    want = ops.attn_decode(q.view(B, 1, Hq, D), k1, v1, bt, sl, ns, D ** -0.5, 0.0, window)
+    assert T.attn_slabs_takes(B, Hkv, ns)
+    keep = part.clone()
+    got = ops.attn_decode_slabs(part, b, cs, pos, off, kc, vc, bt, sl, ns, D ** -0.5, 0.0, window, Hq, dtype)
+    assert torch.equal(part, keep)
+    return want.view(B, -1), got.view(B, -1), (k1, v1), (kc, vc)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L,cap,Hkv,G,bs", [
+    ([1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 511, 512, 513, 640, 639, 2, 64], 640, 8, 4, 64),
+    ([1, 128, 129, 256, 257, 513, 640, 31, 32, 33] * 4, 640, 8, 7, 128),
+    ([1, 32, 129, 191, 192], 192, 8, 16, 192),
+    ([511, 33, 1], 512, 2, 1, 64),
+])
+@pytest.mark.parametrize("ks,bias,window,offset", [(1, True, 0, False), (2, False, 0, False), (4, True, 100, True), (6, False, 0, True)])
+def test_same_bits(cuda, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset):
+    want, got, old, new = _both(cuda, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset)
+    ops.check_kernel_errors(cuda)
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(old, new))
+
+
+def test_padding_rows_and_bad_blocks(cuda):
+    L = [0, 100, 64, 65, 7, 128] * 3
+
+    def padded(bt):
+        bt[0] = -1
+    want, got, old, new = _both(cuda, torch.bfloat16, L, 128, 8, 4, 64, 2, False, 0, False, padded)
+    ops.check_kernel_errors(cuda)
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(old, new))
+
+    def bad(bt):
+        bt[1, 1] = bt.numel() + 5
+    want, got, old, new = _both(cuda, torch.bfloat16, L, 128, 8, 4, 64, 2, False, 0, False, bad)
+    with pytest.raises(RuntimeError):
+        ops.check_kernel_errors(cuda)
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(old, new))
+
+
+def test_not_taken(cuda):
+    """several workgroups a pair, and widths that are not the heads'"""
+    assert not T.attn_slabs_takes(1, 8, 100)
+    x = torch.zeros(2, 1, 6144, device=cuda)
+    kc = torch.zeros(100, 8, 64, 128, dtype=torch.bfloat16, device=cuda)
+    i = torch.zeros(1, 100, dtype=torch.int32, device=cuda)
+    args = (None, torch.zeros(8, 64, 2, device=cuda), i[0, :1].long(), None, kc, kc.clone(), i, i[0, :1].contiguous())
+    with pytest.raises(RuntimeError):
+        ops.attn_decode_slabs(x, *args, 100, 0.1, 0.0, 0, 32, torch.bfloat16)
+    with pytest.raises(RuntimeError):
+        ops.attn_decode_slabs(x, *args, 1, 0.1, 0.0, 0, 16, torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind,qtype", [("llama", "sym_int4"), ("qwen2", "fp8_e5m2"), ("mistral", "nf4")])
+@pytest.mark.parametrize("B", [11, 17, 64])
+def test_model_step(cuda, kind, qtype, B, monkeypatch):
+    from transformers import LlamaConfig, MistralConfig, Qwen2Config
+    from ipex_llm_amd.engine.runner import nsplit_for
+    from ipex_llm_amd.models.builder import random_native_model
+    from ipex_llm_amd.models.decoder import AttnMeta
+    kw = dict(vocab_size=512, hidden_size=1024, intermediate_size=768, num_hidden_layers=2, num_attention_heads=8,
+              num_key_value_heads=2, max_position_embeddings=1024)
+    cfg = {"llama": lambda: LlamaConfig(**kw), "qwen2": lambda: Qwen2Config(**kw),
+           "mistral": lambda: MistralConfig(sliding_window=16, **kw)}[kind]()
+    model = random_native_model(cfg, qtype, cuda, torch.bfloat16, seed=1)
+    inner, calls = ops.attn_decode_slabs, []
+    monkeypatch.setattr(ops, "attn_decode_slabs", lambda *a: (calls.append(1), inner(*a))[1])
+
+    def step(on):
+        cache = model.make_cache(128, batch=B)
+        g = torch.Generator(device=cuda).manual_seed(B)
+        for t in (*cache.k, *cache.v):
+            t.normal_(generator=g)
+        ids = torch.randint(0, 512, (B,), generator=g, device=cuda)
+        pos = torch.arange(B, device=cuda) * 7 % 128
+        bt = torch.arange(B * 2, device=cuda, dtype=torch.int32).view(B, 2)
+        slots = bt.long()[torch.arange(B, device=cuda), pos // 64] * 64 + pos % 64
+        meta = AttnMeta(B, 1, bt, (pos + 1).int(), nsplit_for(128))
+        monkeypatch.setattr(type(model), "_rope_in_env", on)
+        with torch.no_grad():
+            out = model.forward_tokens(ids, pos, slots, meta, cache)
+            if not on:
+                return out, cache
+            model.forward_tokens(ids, pos, slots, meta, cache)
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                cap = model.forward_tokens(ids, pos, slots, meta, cache)
+            for _ in range(3):
+                cap.zero_()
+                graph.replay()
+                assert torch.equal(cap, out)
+                torch.cuda.synchronize()
+        return out, cache
+    want, c0 = step(False)
+    assert not calls
+    got, c1 = step(True)
+    # (up to 16 sequences whose launches finish their rows have their own)
+    rows = B <= 16 and qtype != "nf4"
+    assert len(calls) == (0 if rows else 2 * 3)
+    ops.check_kernel_errors(cuda)
+    if not rows:
+        assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip((*c0.k, *c0.v), (*c1.k, *c1.v)))
