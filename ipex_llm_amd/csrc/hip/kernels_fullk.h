@@ -8,7 +8,7 @@ namespace illm {
 // what a workgroup does with its 16 columns (FK_ROPE, FK_GLU: twice 16) of x W^T
 enum FullkEpi : int {
   FK_NORM = 0,  // h = rnd(rnd(y) + res) -> res_out, rnd(w * h) -> xo, sums of squares of h by 16 columns -> ss
-  FK_ROPE = 1,  // y * row scale (+ bias), columns below rcols rotated by the row's position -> out32
+  FK_ROPE = 1,  // y * row scale (+ bias), columns below rcols rotated by the row's position -> out32, or q16 and the cache
   FK_GLU = 2,   // act(gate) * up of tile-interleaved rows, both times the row scale -> xo [M, N / 2]
 };
 
@@ -37,6 +37,11 @@ struct FullkArgs {
   const float* rcs;
   const int64_t* rpos;
   int rcols, rD;
+  // ... instead of out32 (q16 not null): columns below qcols -> q16 [M, qcols], below rcols -> k_cache, then v_cache
+  // [num_blocks, kv heads, bs, rD], the row of key lens[m] - 1; each rounded once
+  uint16_t *q16, *k_cache, *v_cache;
+  const int32_t *tables, *lens;   // [M, max_blocks], [M]
+  int qcols, max_blocks, num_blocks, bs;
   uint32_t nib_mask, nib_magic;
 };
 

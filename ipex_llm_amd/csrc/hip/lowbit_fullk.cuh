@@ -22,6 +22,10 @@
 // bound by x, which every workgroup reads in full (sym_int4 [4096, 14336] 8.8 / 10.1 / 11.9 / 13.2, of 58 MB of x at 8 rows;
 // the rules row_norm_takes, row_norm_o_takes, row_rope_takes and glu_rows_takes of csrc/torch/ops_hip.cpp, with qkv's and
 // gate/up's figures).
+// qkv that hands q on as the attention takes it and stores k and v in the cache (gemv_rope_kv): f32 sums / this, [6144, 4096]
+// sym_int4 5.4 6.05 6.3 8.1 / 5.6 6.2 6.4 8.3 at 1 / 5 / 8 / 16 rows (with integer divisions for the addresses 6.1 7.0 7.1 8.4),
+// for 0.5 to 1.5 us less of the attention: a step of 1 / 8 rows Llama-3-8B 1.018x / 1.011x of the tree without it and the shifts,
+// 5 rows Qwen2.5-7B fp8_e5m2 1.013x.
 // 16 waves of a K that 8 hold in one piece, or pieces four ahead, were slower.  A decode step, us: Llama-3-8B sym_int4,
 // 1024 tokens, 1 / 4 / 8 rows 1572 1844 1981, with o and down here 1499 1635 1809, and qkv 1473 1599 1774, and gate/up 1379
 // 1551 1769; Qwen2.5-7B fp8_e5m2, 1 / 5 rows 2149 2372, 1995 2182, 1887 2014, 1704 1886.
@@ -67,8 +71,11 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
   float* red = (float*)(smem + (size_t)NW * MR * ROW);            // [NT][NW][MR][16]
   uint32_t* lut2 = (uint32_t*)(red + NT * NW * MR * 16);
 
-  const int KC = a.KC, ht = EPI == FK_ROPE ? a.rD / 32 : 1;       // FK_ROPE: tiles of a head's half
-  const int tile0 = EPI == FK_NORM ? blockIdx.x : EPI == FK_GLU ? 2 * blockIdx.x : blockIdx.x / ht * 2 * ht + blockIdx.x % ht;
+  // FK_ROPE: heads of 64 or 128 columns, shifts instead of divisions (an integer division is 0.1 us of the launch's chain
+  // wherever it stands); tiles of a head's half
+  const int dsh = EPI == FK_ROPE && a.rD == 128 ? 7 : 6, ht = EPI == FK_ROPE ? 1 << (dsh - 5) : 1;
+  const int KC = a.KC;
+  const int tile0 = EPI == FK_NORM ? blockIdx.x : EPI == FK_GLU ? 2 * blockIdx.x : (blockIdx.x >> (dsh - 5) << (dsh - 4)) + (blockIdx.x & (ht - 1));
   const int c0 = (int)((uint32_t)wave * KC / NW), c1 = (int)((uint32_t)(wave + 1) * KC / NW);
 
   // x: piece p of the wave is chunks c0 + PC p ..; rows past M and k past K or the wave's range: out of the descriptor, 0
@@ -130,16 +137,39 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
     }
   };
 
+  const int om = tid >> 4, on = tile0 * 16 + r16;                 // output of threads below 16 M; its (first) column
+  const bool fin = tid < a.M * 16 && on < a.N;
+  // FK_ROPE: the row's position and newest key ahead of all; what they lead to (cos / sin, the key's block) behind the weights'
+  // requests, which its round trip would hold back -- of 9 to 16 rows ahead of them (us of 16 rows, ahead / behind: sym_int4 [6144,
+  // 4096] 7.9 / 8.2, fp8_e5m2 [4608, 3584] 9.4 / 10.3; of 1 row 5.7 / 5.45)
+  constexpr bool LATE = MR <= 8;
+  const int mc = min(om, a.M - 1);                                // (in every thread: the counted waits of the loop stay exact)
+  int64_t pos = 0, key = -1;
+  if constexpr (EPI == FK_ROPE) {
+    pos = a.rpos[mc];
+    if (a.q16) key = (int64_t)a.lens[mc] - 1;
+  }
   constexpr int XV = MR <= 4 ? RG : 1;                            // pieces of x ahead
   uint4 xv[XV][XL];
 #pragma unroll
   for (int u = 0; u < XV; u++) load_x(xv[u], u);
   // what the last step reads: requested now
-  const int om = tid >> 4, on = tile0 * 16 + r16;                 // output of threads below 16 M; its (first) column
-  const bool fin = tid < a.M * 16 && on < a.N;
+  uint32_t blk = ~0u, in_blk = 0;                                 // block of the new key, offset in it (below 2^32: host)
   uint16_t res16 = 0, nw16 = 0;
   float2 cs = make_float2(1.f, 0.f);
   float bias[NT] = {};
+  auto lead = [&]() {
+    const int d = on & ((1 << dsh) - 1);                          // (below half a head)
+    cs = ((const float2*)a.rcs)[((size_t)pos << (dsh - 1)) + d];
+    // (a key beyond the table, a bad block: left out here, reported by the attention, which reads them)
+    if (on >= a.qcols && key >= 0 && key < (int64_t)a.max_blocks * a.bs) {
+      const int bsh = (a.bs & (a.bs - 1)) == 0 ? 31 - __builtin_clz(a.bs) : -1;   // (a power of two but for odd configurations)
+      const uint32_t bi = bsh >= 0 ? (uint32_t)key >> bsh : (uint32_t)key / (uint32_t)a.bs;
+      blk = (uint32_t)a.tables[(size_t)mc * a.max_blocks + bi];
+      const uint32_t head = (uint32_t)(on - (on < a.rcols ? a.qcols : a.rcols)) >> dsh;
+      in_blk = ((head * (uint32_t)a.bs + ((uint32_t)key - bi * (uint32_t)a.bs)) << dsh) + d;
+    }
+  };
   RowParts<NW> parts;
   __shared__ float rscale[EPI == FK_NORM ? 1 : 16];
   if constexpr (EPI == FK_NORM) {
@@ -151,8 +181,8 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
   } else {
     parts.request(a, wave, lane);
     if constexpr (EPI == FK_ROPE) {
+      if constexpr (!LATE) lead();
       if (fin) {
-        if (on < a.rcols) cs = ((const float2*)a.rcs)[(size_t)a.rpos[om] * (a.rD / 2) + on % a.rD];
         if (a.bias) {
 #pragma unroll
           for (int t = 0; t < NT; t++) bias[t] = to_f32<T>(a.bias[on + t * ht * 16]);
@@ -167,6 +197,11 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
     load_sc(ring[u], c0 + u * PC);
 #pragma unroll
     for (int i = 0; i < PC; i++) load_w1(ring[u], c0 + u * PC, i);
+  }
+  if constexpr (EPI == FK_ROPE) {
+    asm volatile("" ::: "memory");
+    if constexpr (LATE) lead();
+    asm volatile("" : "+v"(in_blk));                              // (here, not behind the sums)
   }
 
   if constexpr (DK == DK_LUT4) {
@@ -300,9 +335,21 @@ __global__ void __launch_bounds__(NW * 64) lowbit_fullk_kernel(const FullkArgs a
     const float c = rnd(cs.x), sn = rnd(cs.y);                    // as the model casts its tables
     const float y0 = __builtin_fmaf(y[0], rs, bias[0]), y1 = __builtin_fmaf(y[NT - 1], rs, bias[NT - 1]);
     const bool rot = on < a.rcols;                                // v: as it is (an infinity times a sine of 0 is no number)
-    float* o = a.out32 + (size_t)om * a.N + on;
-    o[0] = rot ? __builtin_fmaf(-y1, sn, y0 * c) : y0;            // (spelled out: one rounding in every instantiation)
-    o[ht * 16] = rot ? __builtin_fmaf(y0, sn, y1 * c) : y1;
+    const float o0 = rot ? __builtin_fmaf(-y1, sn, y0 * c) : y0;  // (spelled out: one rounding in every instantiation)
+    const float o1 = rot ? __builtin_fmaf(y0, sn, y1 * c) : y1;
+    if (a.q16 == nullptr) {
+      float* o = a.out32 + (size_t)om * a.N + on;
+      o[0] = o0;
+      o[ht * 16] = o1;
+      return;
+    }
+    uint16_t* o = a.q16 + (size_t)om * a.qcols + on;
+    if (on >= a.qcols) {
+      if (blk >= (uint32_t)a.num_blocks) return;
+      o = (rot ? a.k_cache : a.v_cache) + (size_t)blk * ((uint32_t)(a.rcols - a.qcols) * (uint32_t)a.bs) + in_blk;
+    }
+    o[0] = from_f32<T>(o0);
+    o[ht * 16] = from_f32<T>(o1);
   } else {
     const float gv = y[0] * rs, uv = y[NT - 1] * rs;
     const int n = blockIdx.x * 16 + r16;

@@ -171,6 +171,7 @@ TORCH_LIBRARY(ipex_llm_amd, m) {
   m.def("gemv_attn(Tensor po, Tensor pml, Tensor seq_lens, Tensor blob, int fmt, int n, int k, Tensor(a!)? acc, int ksplit, ScalarType dtype, Tensor(b!)? zero=None, int nw=0) -> Tensor");
   m.def("gemm(Tensor x, Tensor blob, int fmt, int n, int k, Tensor? bias) -> Tensor");
   m.def("gemv_accum(Tensor x, Tensor blob, int fmt, int n, int k, Tensor(a!) acc, int ksplit, Tensor(b!)? zero=None, Tensor? rope_cs=None, Tensor? rope_pos=None, int rope_cols=0, int rope_d=0, Tensor? xss=None, int xss_n=0, float xss_eps=0.0) -> ()");
+  m.def("gemv_rope_kv(Tensor x, Tensor blob, int fmt, int n, int k, Tensor? bias, Tensor rope_cs, Tensor rope_pos, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor block_tables, Tensor seq_lens, int Hq, Tensor? xss=None, int xss_n=0, float xss_eps=0.0) -> Tensor");
   m.def("gemv_rope(Tensor x, Tensor blob, int fmt, int n, int k, Tensor? bias, Tensor(a!) out, Tensor rope_cs, Tensor rope_pos, int rope_cols, int rope_d, Tensor? xss=None, int xss_n=0, float xss_eps=0.0) -> ()");
   m.def("gemv_row_norm(Tensor x, Tensor blob, int fmt, int n, int k, Tensor residual, Tensor(a!) res_out, Tensor norm_w, bool unit_offset, Tensor(b!) xo, Tensor(c!) ss, Tensor(d!)? zero=None) -> ()");
   m.def("gemv_accum_norm(Tensor x, Tensor blob, int fmt, int n, int k, Tensor(a!) acc, Tensor(b!) ctr, Tensor residual, Tensor(c!) res_out, Tensor norm_w, bool unit_offset, Tensor(d!) xo, Tensor(e!) ss, Tensor(f!)? zero=None) -> ()");

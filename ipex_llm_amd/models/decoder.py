@@ -802,7 +802,11 @@ class NativeCausalLM(nn.Module):
                     and (qp.bias is None or qp.bias.dtype == x.dtype) and ops.native_gpu(x):
                 # split-K GEMV reduced (+bias) inside the RoPE/KV kernel, slots from the block table:
                 # T <= 16 accumulates with atomics into one zeroed slab (re-zeroed by the kernel)
-                if T <= ACC_MAX_M or rope_in:
+                if row_rope:                    # (no sums pending: _row_rope_ok) q as the attention takes it, k and v in the cache
+                    q = ops.gemv_rope_kv(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, qp.bias, self.rope_cache, pos,
+                                         cache.k[li], cache.v[li], meta.block_tables, meta.seq_lens, s.num_heads, xss=x_ss)
+                    x_ss = None
+                elif T <= ACC_MAX_M or rope_in:
                     part = self._acc(qp.out_features, T, x.device)
                     ss_q = None
                     if pend is not None:
@@ -813,10 +817,6 @@ class NativeCausalLM(nn.Module):
                                          ss=ss_q, rope=qrope, zero=zero_gu)
                         zero_gu = None
                         residual, consumed, pend = r2, pend, None
-                    elif row_rope:
-                        ops.gemv_rope(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, qp.bias, part, qrope,
-                                      xss=x_ss)
-                        x_ss = None
                     else:
                         ops.gemv_accum(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, part,
                                        zero=zero_next, rope=qrope, xss=x_ss)
@@ -825,7 +825,10 @@ class NativeCausalLM(nn.Module):
                     part = part.unsqueeze(0)
                 else:
                     part = ops.gemv_partials(x, qp.weight, qp.fmt, qp.out_features, qp.in_features, 0)
-                if slabs_in:
+                if row_rope:
+                    a_rope = ops.attn_decode(q.view(meta.B, 1, s.num_heads, s.head_dim), cache.k[li], cache.v[li], meta.block_tables,
+                                             meta.seq_lens, meta.nsplit, s.scale, s.attn_softcap, attn.sliding_window).view(T, -1)
+                elif slabs_in:
                     a_rope = ops.attn_decode_slabs(part, qp.bias, self.rope_cache, pos, meta.pos_offset, cache.k[li], cache.v[li],
                                                    meta.block_tables, meta.seq_lens, meta.nsplit, s.scale, s.attn_softcap,
                                                    attn.sliding_window, s.num_heads, x.dtype).view(T, -1)
@@ -836,7 +839,7 @@ class NativeCausalLM(nn.Module):
                                       cache.v_scale, meta.pos_offset, zero_part=T <= ACC_MAX_M,
                                       pss=ss_q, pss_n=s.hidden_size, pss_eps=s.rms_eps)
                 elif not (norm_in and self._oproj_combine and attn.o_proj.bias is None):
-                    a_rope = ops.attn_decode_rope(qkv_acc, None if row_rope else qp.bias, self.rope_cache, pos, cache.k[li], cache.v[li],
+                    a_rope = ops.attn_decode_rope(qkv_acc, qp.bias, self.rope_cache, pos, cache.k[li], cache.v[li],
                                                   meta.block_tables, meta.seq_lens, meta.nsplit, s.scale,
                                                   s.attn_softcap, attn.sliding_window, s.num_heads, s.rot_dim,
                                                   s.rope_interleaved, 1.0, x.dtype, pss=ss_q,

@@ -173,6 +173,11 @@ def _(x, blob, fmt, n, k, bias, out, rope_cs, rope_pos, rope_cols, rope_d, xss=N
     return None
 
 
+@register_fake("ipex_llm_amd::gemv_rope_kv")
+def _(x, blob, fmt, n, k, bias, rope_cs, rope_pos, k_cache, v_cache, block_tables, seq_lens, Hq, xss=None, xss_n=0, xss_eps=0.0):
+    return x.new_empty((x.numel() // k, Hq, k_cache.shape[3]))
+
+
 @register_fake("ipex_llm_amd::gemv_row_norm")
 def _(x, blob, fmt, n, k, residual, res_out, norm_w, unit_offset, xo, ss, zero=None):
     return None

@@ -18,7 +18,7 @@ __all__ = [
     "fp8_quantize_weight", "dense_linear", "check_kernel_errors", "KernelError", "repack_to_device", "repack_from_device", "lowbit_matmul",
     "gemv_partials", "gemv_glu", "add_rms_norm", "rms_norm", "layer_norm", "rope_kv",
     "attn_decode", "glu", "attn_softmax_", "moe_topk", "reduce_partials", "to_fp8_bytes", "GEMV_MAX_M", "gather_kv",
-    "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_row_norm", "gemv_rope", "gemv_glu_ss",
+    "moe_align", "moe_gemm", "moe_gemv_glu", "moe_gemv_partials", "moe_combine", "moe_route", "moe_gemv_accum", "rope_kv_fused", "gemv_glu_in", "gemv_accum", "gemv_accum_norm", "gemv_row_norm", "gemv_rope", "gemv_rope_kv", "gemv_glu_ss",
     "attn_decode_split", "gemv_attn", "gemv_norm_in", "attn_decode_rope", "attn_decode_rope_split", "attn_decode_slabs", "attn_prefill", "moe_group_topk",
 ]
 
@@ -268,6 +268,25 @@ def gemv_rope(x, blob, fmt, n, k, bias: Optional[torch.Tensor], out: torch.Tenso
         y = y + bias.float()
     out.copy_(_rope_cols(y, rope, x.dtype).view_as(out))
     return out
+
+
+def gemv_rope_kv(x, blob, fmt, n, k, bias: Optional[torch.Tensor], cos_sin, pos, k_cache, v_cache, block_tables, seq_lens,
+                 Hq: int, xss=None) -> torch.Tensor:
+    """``gemv_rope`` of one new token per sequence: rotated q [M, Hq, D] in x's dtype, k and v stored in the paged cache at key
+    ``seq_lens`` - 1 (rows whose key lies beyond their table, or in a block that the cache does not have, are left out)."""
+    Hkv, bs, D = k_cache.shape[1:]
+    if _native(x):
+        ss, ss_n, eps = xss if xss is not None else (None, 0, 0.0)
+        return _ops().gemv_rope_kv(x, blob, fmt, n, k, bias, cos_sin, pos, k_cache, v_cache, block_tables, seq_lens, Hq, ss, ss_n,
+                                   eps)
+    M = x.numel() // k
+    out = gemv_rope(x, blob, fmt, n, k, bias, torch.empty(M, n, device=x.device), (cos_sin, pos, (Hq + Hkv) * D, D), xss=xss)
+    q, kn, vn = out.to(x.dtype).view(M, -1, D).split([Hq, Hkv, Hkv], 1)
+    for m, at in enumerate((seq_lens[:M].long() - 1).tolist()):
+        blk = int(block_tables[m, at // bs]) if 0 <= at < block_tables.shape[1] * bs else -1
+        if 0 <= blk < k_cache.shape[0]:
+            k_cache[blk, :, at % bs], v_cache[blk, :, at % bs] = kn[m], vn[m]
+    return q.contiguous()
 
 
 def gemv_row_norm(x, blob, fmt, n, k, residual: torch.Tensor, res_out: torch.Tensor, norm_w: torch.Tensor,
