@@ -437,9 +437,11 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
 //   * from 136 pairs on one workgroup each, 8 waves while they are one per CU, else 4 (two per CU): 18 x 1024 29.3 / 19.8, 20 x
 //     800 22.1 / 16.5, 24 x 1024 24.5 / 19.8, 32 x 600 21.6 / 16.9, 48 x 700 31.9 / 25.3 (8 waves 28.6), 64 x 256 19.0 / 14.5,
 //     100 x 600 52.4 / 43.1, 28 x 2100 45.9 / 40.5;
-//   * fewer pairs, so few keys that the merge is most of the time: 1 x 128 8.4 / 6.0 (4 waves), 8 x 400 10.8 / 10.1, 16 x 256
-//     12.2 / 9.1, 8 x 600 12.1 / 11.8, 16 x 800 (q pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9; 1 x 400 is even, 1 x 600
-//     8.9 / 9.2 and 6 x 600 11.3 / 11.6 are not taken;
+//   * fewer pairs of more than 8 sequences, so few keys that the merge is most of the time: 16 x 256 12.2 / 9.1, 16 x 800 (q
+//     pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9.  Up to 8 sequences not, though some are ahead (1 x 128 8.4 / 6.0, 8 x
+//     400 10.8 / 10.1, 8 x 600 12.1 / 11.8; 1 x 400 even, 1 x 600 8.9 / 9.2): there, steps that rotate in the attention keep
+//     attn_dec_v3.cuh, and p is rounded beside its wave's maximum here and its workgroup's there: 1.9e-3 between the two over 70
+//     keys, and the tokens of two ranks parted from those of one at a tie;
 //   * long ones, where one tile a wave takes rounds: 4 waves and as many workgroups as make 512, at most 16 (32) a pair: 1 x
 //     4200 14.8 / 11.8, 3 x 20000 45.7 / 42.0, 4 x 3000 19.3 / 16.2, 5 x 4200 23.5 / 20.2, 8 x 2400 31.0 / 20.5, 10 x 4200 35.0 /
 //     33.7, 16 x 2000 41.0 / 27.0; from 64, 80 and 112 pairs on at fewer keys: 8 x 1024 15.0 / 14.0, 10 x 1300 17.1 / 16.9, 12 x
@@ -453,8 +455,7 @@ inline V4Plan v4_plan(int B, int Hkv, int nsplit) {
   if (off) return {0, 0};                        // a forced form of attn_dec_v3.cuh (A/B runs)
   const long pairs = (long)B * Hkv, keys = (long)nsplit * SPLIT;
   if (pairs >= 136) return {pairs <= 256 ? 8 : 4, 1};
-  if (keys <= 192) return {4, 1};
-  if (keys <= (pairs >= 112 ? 896 : pairs >= 64 ? 704 : 512)) return {8, 1};
+  if (B > 8 && keys <= (pairs >= 112 ? 896 : pairs >= 64 ? 704 : 512)) return {keys <= 192 ? 4 : 8, 1};
   if (keys < (pairs >= 112 ? 0 : pairs >= 80 ? 1152 : pairs >= 64 ? 1024 : 1920)) return {0, 0};
   const long s = std::min({512 / pairs, pairs >= 16 || keys < 16384 ? 16L : 32L, keys / (4 * V3_KPW)});
   return {4, (int)s};

@@ -7,8 +7,8 @@ import ipex_llm_amd.ops as ops
 
 @pytest.mark.parametrize("batch,heads,keys,plan", [
     (17, 8, 64, [8, 1]), (32, 8, 1 << 20, [8, 1]), (33, 8, 64, [4, 1]), (100, 8, 640, [4, 1]),     # a workgroup a pair
-    (1, 8, 192, [4, 1]), (1, 8, 256, [8, 1]), (1, 8, 512, [8, 1]), (1, 8, 576, [0, 0]),
-    (8, 8, 704, [8, 1]), (8, 8, 768, [0, 0]), (14, 8, 896, [8, 1]), (14, 8, 960, [4, 4]), (16, 8, 1088, [4, 4]),
+    (1, 8, 64, [0, 0]), (8, 8, 192, [0, 0]), (9, 8, 192, [4, 1]), (9, 8, 256, [8, 1]), (9, 2, 512, [8, 1]), (9, 2, 576, [0, 0]),
+    (9, 8, 704, [8, 1]), (8, 8, 768, [0, 0]), (14, 8, 896, [8, 1]), (14, 8, 960, [4, 4]), (16, 8, 1088, [4, 4]),
     (8, 8, 960, [0, 0]), (8, 8, 1024, [4, 8]), (10, 8, 1088, [0, 0]), (10, 8, 1152, [4, 6]),
     (1, 8, 1856, [0, 0]), (1, 8, 1920, [4, 15]), (1, 8, 4096, [4, 16]), (1, 8, 16384, [4, 32]), (2, 8, 16384, [4, 16]),
     (3, 8, 20032, [4, 16]), (5, 8, 4224, [4, 12]), (1, 1, 1 << 20, [4, 32])])

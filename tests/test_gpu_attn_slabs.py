@@ -37,8 +37,8 @@ def _both(dev, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset, tables=None)
 @pytest.mark.parametrize("L,cap,Hkv,G,bs", [
     ([1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 511, 512, 513, 640, 639, 2, 64], 640, 8, 4, 64),
     ([1, 128, 129, 256, 257, 513, 640, 31, 32, 33] * 4, 640, 8, 7, 128),
-    ([1, 32, 129, 191, 192], 192, 8, 16, 192),
-    ([511, 33, 1], 512, 2, 1, 64),
+    ([1, 32, 129, 191, 192] * 2, 192, 8, 16, 192),
+    ([511, 33, 1] * 3, 512, 2, 1, 64),
 ])
 @pytest.mark.parametrize("ks,bias,window,offset", [(1, True, 0, False), (2, False, 0, False), (4, True, 100, True), (6, False, 0, True)])
 def test_same_bits(cuda, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset):

@@ -40,8 +40,8 @@ def _setup(dev, L, cap, Hkv, bs, dtype):
 CASES = [  # lengths, keys of the grid, kv heads, group, block, (waves, workgroups)
     ([EDGES[i % 13] for i in range(17)], 640, 8, 4, 64, [8, 1]),
     ([EDGES[i % 13] for i in range(40)], 640, 8, 1, 64, [4, 1]),
-    ([1, 32, 129, 191, 192], 192, 8, 4, 192, [4, 1]),
-    ([511, 33, 1], 512, 2, 16, 128, [8, 1]),
+    ([1, 32, 129, 191, 192] * 2, 192, 8, 4, 192, [4, 1]),
+    ([511, 33, 1] * 3, 512, 2, 16, 128, [8, 1]),
     ([1024, 895, 129, 127, 128, 1, 640, 960], 1088, 8, 7, 64, [4, 8]),
     ([4100, 2047, 33], 4224, 8, 4, 192, [4, 16]),
     ([17000, 16384, 1] + [65] * 14, 17024, 8, 2, 64, [8, 1]),      # 67 tiles a wave
