@@ -209,6 +209,24 @@ def apply_repetition_penalty(logits, seqs, penalty):
     return logits
 
 
+def _to_device(dev, parts: List[torch.Tensor]) -> List[torch.Tensor]:
+    """Host tensors as contiguous tensors on ``dev``, in one copy: each copy from pageable memory waits for the stream, and six of
+    them ahead of a short prompt left the GPU idle for as long as its first layers take.  (What is there already stays.)"""
+    if torch.device(dev).type == "cpu":
+        return [p.to(dev) for p in parts]
+    at, end = [], 0
+    for p in parts:
+        at.append(end)
+        end += 0 if p.device.type != "cpu" else -(-p.numel() * p.element_size() // 16) * 16
+    host = torch.empty(end, dtype=torch.uint8)
+    for p, o in zip(parts, at):
+        if p.device.type == "cpu":
+            host[o:o + p.numel() * p.element_size()].view(p.dtype).copy_(p.reshape(-1))
+    buf = host.to(dev)
+    return [buf[o:o + p.numel() * p.element_size()].view(p.dtype).view(p.shape) if p.device.type == "cpu" else p.to(dev)
+            for p, o in zip(parts, at)]
+
+
 class Engine:
     """Owns a model + KV cache; runs prefill and (graph) decode."""
 
@@ -253,13 +271,12 @@ class Engine:
         m, c = self.model, self.cache
         dev = m.device
         n = ids.numel()
-        pos = torch.arange(start, start + n, device=dev)
-        slots = slots_for(seq, start, n, c.bs).to(dev)
         L = start + n
-        bt = make_block_table([seq], len(seq.blocks), dev)
-        meta = AttnMeta(1, n, bt, torch.tensor([L], dtype=torch.int32, device=dev), nsplit_for(L), [L])
-        logits = m.forward_tokens(ids.to(dev), pos, slots, meta, c,
-                                  logits_idx=torch.tensor([n - 1], device=dev))
+        ids, pos, slots, last, bt, lens = _to_device(dev, [ids, torch.arange(start, L), slots_for(seq, start, n, c.bs),
+                                                           torch.tensor([n - 1]), make_block_table([seq], len(seq.blocks), "cpu"),
+                                                           torch.tensor([L], dtype=torch.int32)])
+        meta = AttnMeta(1, n, bt, lens, nsplit_for(L), [L])
+        logits = m.forward_tokens(ids, pos, slots, meta, c, logits_idx=last)
         seq.length = L
         return logits
 

@@ -6,6 +6,7 @@ and the torch references otherwise.
 """
 from __future__ import annotations
 
+import sys
 from typing import Optional, Tuple
 
 import torch
@@ -23,14 +24,18 @@ __all__ = [
 ]
 
 
+# The package, looked up once: an import statement in each of these two was 0.3 to 0.7 us of every call.  The host's share of a
+# prompt of 45 tokens, some 260 launches, fell from 2.75 to 2.45 ms with this and its inputs in one copy (engine/runner.py).
+# Its functions by name at each call: a program may replace them.
+_pkg = sys.modules[__package__]
+
+
 def _ops():
-    from . import require
-    return require()
+    return _pkg.require()
 
 
 def _native(t: torch.Tensor) -> bool:
-    from . import native_gpu
-    return native_gpu(t)
+    return _pkg.native_gpu(t)
 
 
 # ------------------------------------------------------------ quantization
