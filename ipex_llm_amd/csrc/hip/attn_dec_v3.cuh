@@ -199,13 +199,21 @@ struct V3Rope {
 // thread -> (row, 16-B quad of D); all of a row's (m, l) and o quads of a
 // 16-split chunk are requested before any is used (one memory round trip for
 // ns <= 16), later chunks rescale online.  SC1: handed over inside the launch.
-template <typename T, bool SC1>
+// D_: the head dim where the caller knows it, for one token without the integer
+// divisions between ticket and requests (some 0.1 us each; with those on the way
+// to a wave's first request, us: 1 x 128 keys 6.8 / 6.6, 1 x 1024 7.8 / 7.6, q
+// pre-rotated 8.2 / 7.7, 9.0 / 8.6, 28 / 4 heads 5 x 777 10.3 / 9.8).  Not from
+// attn_dec_v4.cuh, whose merge is 0.2 slower with it (8 x 1024 12.8 / 13.0, 28 /
+// 4 heads 16 x 1024 13.9 / 14.1).
+template <typename T, bool SC1, int D_ = 0>
 __device__ __forceinline__ void v3_combine(const AttnDecodeArgs& a, int b, int kvh, int ns, int tid, int nthr) {
   constexpr int CH = 16;
-  const int group = a.Hq / a.Hkv, R = group * a.Tq, Q = a.D / 4;
+  const int D = D_ > 0 ? D_ : a.D;
+  const int group = a.Hq / a.Hkv, R = group * a.Tq, Q = D / 4;
   for (int idx = tid; idx < R * Q; idx += nthr) {
     const int r = idx / Q, q = idx % Q;
-    const int t = r / group, h = kvh * group + r % group;
+    const bool one = D_ > 0 && a.Tq == 1;
+    const int t = one ? 0 : r / group, h = kvh * group + (one ? r : r % group);
     const size_t row0 = (((size_t)b * a.Hq + h) * a.Tq + t) * a.nsplit;
     float M = -INFINITY, L = 0.f;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -217,10 +225,10 @@ __device__ __forceinline__ void v3_combine(const AttnDecodeArgs& a, int b, int k
         const size_t s = row0 + min(s0 + j, ns - 1);
         if constexpr (SC1) {
           ml[j] = ld8_sc1(a.part_ml + s * 2);
-          pv[j] = ld16_sc1(a.part_o, s * a.D + 4 * q);
+          pv[j] = ld16_sc1(a.part_o, s * D + 4 * q);
         } else {
           ml[j] = *(const float2*)(a.part_ml + s * 2);
-          pv[j] = *(const float4*)(a.part_o + s * a.D + 4 * q);
+          pv[j] = *(const float4*)(a.part_o + s * D + 4 * q);
         }
       }
       float mc = -INFINITY;
@@ -243,14 +251,13 @@ __device__ __forceinline__ void v3_combine(const AttnDecodeArgs& a, int b, int k
       M = Mn;
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    uint16_t* out = a.out + (((size_t)b * a.Tq + t) * a.Hq + h) * a.D + 4 * q;
+    uint16_t* out = a.out + (((size_t)b * a.Tq + t) * a.Hq + h) * D + 4 * q;
     *(uint2*)out = make_uint2(pack2<T>(o.x * inv, o.y * inv), pack2<T>(o.z * inv, o.w * inv));
   }
   if (a.rq_part != nullptr) {
     // fused-RoPE decode: every split of (b, kvh) has read its q / k / v columns
     // of the qkv accumulator: re-zero them for the next layer's atomic GEMV
     float* prow = (float*)a.rq_part + (size_t)b * a.rq_ld;
-    const int D = a.D;
     for (int i = tid * 4; i < (group + 2) * D; i += nthr * 4) {
       const int hh = i / D, d = i % D;
       const int col = hh < group ? (kvh * group + hh) * D : (a.Hq + (hh - group) * a.Hkv + kvh) * D;
@@ -300,7 +307,7 @@ __device__ __forceinline__ void attn_v3_body(const AttnDecodeArgs& a, int split,
   static_assert(D == 64 || D == 128, "v3: head_dim 64 / 128");
   static_assert(RQ == 0 || D == 128, "v3: fused RoPE needs head_dim 128");
   const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
-  const int wv = threadIdx.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: the block and the tile's address in scalars
   const int group = a.Hq / a.Hkv;
   const int R = group * a.Tq;
   const int k0 = split * SK, kw0 = k0 + V3_KPW * wv;
@@ -313,7 +320,10 @@ __device__ __forceinline__ void attn_v3_body(const AttnDecodeArgs& a, int split,
   // ---- sequence length and this wave's block-table entry, in flight together
   // (fused RoPE: with the row's rms scale, position and the wave's q columns)
   int len = a.seq_lens[b];
-  const int blk = a.block_tables[(size_t)b * a.max_blocks + min(kw0 / a.bs, a.max_blocks - 1)];
+  // (blocks are a power of two tokens long but for odd configurations: no division on the way to the first request)
+  const int bsh = (a.bs & (a.bs - 1)) == 0 ? 31 - __clz(a.bs) : -1;
+  const int bi = bsh >= 0 ? kw0 >> bsh : kw0 / a.bs;
+  const int blk = a.block_tables[(size_t)b * a.max_blocks + min(bi, a.max_blocks - 1)];
   const int row = r16 < R ? r16 : 0;
   const int t = row / group, h = kvh * group + row % group;
   const V3Rope<T, D, RQ == 2> rp(a, b, g, RQ != 0);
@@ -344,7 +354,7 @@ __device__ __forceinline__ void attn_v3_body(const AttnDecodeArgs& a, int split,
     if (blk_bad && lane == 0) kerr(a.err, ERR_BLOCK_ID);
     const bool ld_on = nkw > 0 && !blk_bad;            // wave-uniform
     const int nvis = ld_on ? nkw : 0;
-    const size_t base = ld_on ? (((size_t)blk * a.Hkv + kvh) * a.bs + (kw0 % a.bs)) * D : 0;
+    const size_t base = ld_on ? (((size_t)blk * a.Hkv + kvh) * a.bs + (kw0 - bi * a.bs)) * D : 0;
     const uint16_t* kb = (const uint16_t*)a.k_cache + base;
     const uint16_t* vb = (const uint16_t*)a.v_cache + base;
 
@@ -581,7 +591,7 @@ __device__ __forceinline__ void attn_v3_body(const AttnDecodeArgs& a, int split,
     }
     __syncthreads();
     if (!sm.s_last) return;
-    v3_combine<T, true>(a, b, kvh, nsg, threadIdx.x, NW * 64);
+    v3_combine<T, true, D>(a, b, kvh, nsg, threadIdx.x, NW * 64);
   }
 }
 
@@ -881,7 +891,7 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
     }
     __syncthreads();
     if (!sm.s_last) return;
-    v3_combine<T, true>(a, b, kvh, gridDim.x, threadIdx.x, NW * 64);
+    v3_combine<T, true, D>(a, b, kvh, gridDim.x, threadIdx.x, NW * 64);
   }
 }
 
