@@ -1169,7 +1169,10 @@ template <typename T, int D>
 void launch_d(const AttnDecodeArgs& a, hipStream_t st) {
   const int R = (a.Hq / a.Hkv) * a.Tq;
   if constexpr (D == 128) {
-    if (a.rq_slabs > 0) return launch_v4_slabs<T>(a, st);         // (attn_slabs_takes)
+    if (a.rq_slabs > 0) {                                          // (attn_slabs_takes)
+      launch_v4<T, D, 3>(a, st);
+      return;
+    }
   }
   if constexpr (D == 64 || D == 128) {
     if (v3_ok(a, D)) {

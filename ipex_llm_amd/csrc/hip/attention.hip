@@ -46,7 +46,8 @@ int attn_decode_plan(int B, int Hkv, int nsplit, int* groups) {
 bool attn_slabs_takes(int B, int Hkv, int nsplit) {
   AttnDecodeArgs a{};
   a.Hq = a.Hkv = a.Tq = 1;
-  return v3_ok(a, 128) && v4_plan(B, Hkv, nsplit).groups == 1;
+  const V4Plan p = v4_plan(B, Hkv, nsplit);
+  return v3_ok(a, 128) && (p.groups == 1 || p.row > 0);
 }
 
 }  // namespace illm

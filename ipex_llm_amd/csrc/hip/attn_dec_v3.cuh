@@ -254,7 +254,7 @@ __device__ __forceinline__ void v3_combine(const AttnDecodeArgs& a, int b, int k
     uint16_t* out = a.out + (((size_t)b * a.Tq + t) * a.Hq + h) * D + 4 * q;
     *(uint2*)out = make_uint2(pack2<T>(o.x * inv, o.y * inv), pack2<T>(o.z * inv, o.w * inv));
   }
-  if (a.rq_part != nullptr) {
+  if (a.rq_part != nullptr && a.rq_slabs == 0) {
     // fused-RoPE decode: every split of (b, kvh) has read its q / k / v columns
     // of the qkv accumulator: re-zero them for the next layer's atomic GEMV
     float* prow = (float*)a.rq_part + (size_t)b * a.rq_ld;

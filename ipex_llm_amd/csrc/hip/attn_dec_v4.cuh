@@ -5,8 +5,9 @@
 // many pairs the workgroups come in rounds that each pay that chain again, and the merge -- partials to memory, a ticket, the
 // partials read back -- costs 2 to 3 us for sums that one workgroup could have kept.  Its variant of several tiles per wave
 // asks for K as fragments (16 rows of 64 bytes a load: four times the address unit's time), for want of registers.  Here:
-//   * NW = 8 (4) waves take the 32 NW-key tiles of the pair in turn (workgroup s of S: tiles s, s + S, ...); the waves meet
-//     once, at the end.  S = 1: the workgroup writes the result itself, no partials, no ticket, no second launch;
+//   * NW = 8 (4) waves take the 32 NW-key tiles of the pair in turn (workgroup s of S: tiles s, s + S, ..., or 1 << v4_row
+//     keys in a row, and those past the sequence's end leave at once); the waves meet once, at the end.  One workgroup: it
+//     writes the result itself, no partials, no ticket, no second launch;
 //   * a tile's 32 rows of K and of V are 8 KB in a row each: 16 loads of 1 KB through a buffer descriptor whose range ends
 //     with the tile's keys (rows past them are zeros), the next tile's requested as soon as this one's are in the wave's LDS
 //     rows, so 16 KB a wave and 128 KB a CU are in flight beside the products; 201 registers, 8 waves a CU.  Two tiles
@@ -22,8 +23,9 @@
 namespace illm {
 
 // RQ 3: the qkv product's f32 slabs [ks, B, ld], bias and rotation as in rope_kv.hip, the same bits.  An item is dims d, d + 1
-// and their partners D / 2 on of one head, for a thread; q goes to LDS for all waves, k and v there and to the cache.  Only
-// where one workgroup has a pair (launch_v4_slabs): with several, each would rotate the same rows.  The rope launch takes 5.2 us
+// and their partners D / 2 on of one head, for a thread; q goes to LDS for all waves, k and v there and, from the workgroup
+// that has the new key's tile, to the cache.  Only where a workgroup's tiles are in a row (attn_slabs_takes), so that all but
+// the longest sequences have one: each of a pair rotates the same rows.  The rope launch takes 5.2 us
 // for 0.5 us of bytes; this prologue, its loads ahead of the first tile's, 1.5 to 3: us a step, launch / this, Llama-3-8B 17 x 1024
 // tokens 2374 / 2305, 24 x 600 2342 / 2262, 33 x 300 2597 / 2508, 64 x 900 asym_int4 4071 / 3980, 64 x 128 3013 / 2900, Qwen2.5-7B
 // fp8_e5m2 40 x 500 2906 / 2868, 20 x 150 sym_int4 2082 / 1984, nf4 12 x 180 2680 / 2640.  (The block of the new key asked for behind
@@ -64,7 +66,7 @@ struct V4Slabs {
     const int64_t k = pos - off;
     return __builtin_amdgcn_readfirstlane(k >= 0 && k < len ? (int)k : -1);
   }
-  __device__ void finish(const AttnDecodeArgs& a, int b, int kvh, int item, uint16_t (*q)[D], uint16_t (*kv)[D]) const {
+  __device__ void finish(const AttnDecodeArgs& a, int b, int kvh, int item, bool append, uint16_t (*q)[D], uint16_t (*kv)[D]) const {
     const int group = a.Hq / a.Hkv;
     if (item >= (group + 2) * (D / 4)) return;
     float v[2][2] = {};
@@ -100,7 +102,7 @@ struct V4Slabs {
     uint16_t* l = hh < 0 ? q[hh + group] : kv[hh];
 #pragma unroll
     for (int h = 0; h < 2; h++) *(uint32_t*)(l + d + h * (D / 2)) = o[h];
-    if (hh < 0) return;
+    if (hh < 0 || !append) return;
     const bool oob = blk >= a.num_blocks;
     if (oob) kerr(a.err, ERR_SLOT);
     if (blk < 0 || oob) return;                                   // a padding row
@@ -110,7 +112,8 @@ struct V4Slabs {
   }
 };
 
-template <typename T, int D, int NW, int RQ, bool FUSE>
+// ROW: a workgroup has 1 << v4_row keys in a row.  A kernel of its own: with both in one, tiles in turn took 0.2 to 0.6 us more
+template <typename T, int D, int NW, int RQ, bool FUSE, bool ROW>
 __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDecodeArgs a) {
   constexpr int SK = V3_KPW * NW;                  // keys of a tile
   constexpr int KSTEP = D / 32, DT = D / 16, VU = D / 8, KPJ = 64 / VU, VJ = V3_KPW / KPJ;
@@ -121,11 +124,14 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
   __shared__ __attribute__((aligned(16))) uint16_t qrot[RQ == 3 ? 16 : 1][D];
   __shared__ float smx[NW][16], sml[NW][16];
   __shared__ int s_last;
-  const int split = blockIdx.x, S = gridDim.x, kvh = blockIdx.y, b = blockIdx.z;
+  // (ROW: the workgroups of a pair far apart.  Beside each other, all first ones, the only ones of most sequences, fall to the
+  // same XCDs: 31 x 500 and 1 x 16000 tokens 110 us instead of 52)
+  const int split = ROW ? blockIdx.z : blockIdx.x, S = ROW ? gridDim.z : gridDim.x;
+  const int kvh = ROW ? blockIdx.x : blockIdx.y, b = ROW ? blockIdx.y : blockIdx.z;
   const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int group = a.Hq / a.Hkv, R = group * a.Tq;
-  const int kw0 = split * SK + V3_KPW * wv, step = S * SK;
+  const int kfirst = ROW ? split << a.v4_row : split * SK, kw0 = kfirst + V3_KPW * wv, step = ROW ? SK : S * SK;
 
   // blocks are a power of two tokens long but for odd configurations: no division on the way to an address
   const int bsh = (a.bs & (a.bs - 1)) == 0 ? 31 - __clz(a.bs) : -1;
@@ -137,7 +143,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     const uint32_t k = min((uint32_t)kw0 + (uint32_t)(j + lane) * (uint32_t)step, (uint32_t)a.max_blocks * (uint32_t)a.bs - 1u);
     return a.block_tables[(size_t)b * a.max_blocks + block_of(k)];
   };
-  int ent = entries(0);
+  int ent = entries(0);                          // (of tiles j & ~63 ..)
   const int row = r16 < R ? r16 : 0;
   const int t = row / group, h = kvh * group + row % group;
   const V3Rope<T, D, true> rp(a, b, g, RQ == 2);
@@ -158,9 +164,14 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     len = min(min(len, a.max_blocks * a.bs), a.nsplit * SPLIT);
   }
   len = __builtin_amdgcn_readfirstlane(len);
+  const int nsg = FUSE && ROW ? max(1, min(S, (len + (1 << a.v4_row) - 1) >> a.v4_row)) : S;
+  if (split >= nsg) return;                      // (all of the workgroup; it is not among those that the ticket counts)
   const size_t prow = (((size_t)b * a.Hq + h) * a.Tq + t) * a.nsplit + split;
   const int win0 = a.sliding_window > 0 ? len - a.Tq - a.sliding_window : -1;   // keys up to here: no row sees them
-  const int nt = kw0 < len ? (len - kw0 + step - 1) / step : 0;
+  const int kend = ROW ? min(len, kfirst + (1 << a.v4_row)) : len, nt = kw0 < kend ? (kend - kw0 + step - 1) / step : 0;
+  // (a window: the wave's first tile with a key in it)
+  const int j0 = ROW && win0 - (V3_KPW - 1) >= kw0 ? min(nt, (win0 - (V3_KPW - 1) - kw0) / step + 1) : 0;
+  if (j0 >= 64) ent = entries(j0 & ~63);
 
   // ---- tile j of the wave: keys that can be seen (0: none, a bad block, past the window) and where they start
   auto tile_at = [&](int j, int& kw, size_t& base, int& blk) {
@@ -205,14 +216,15 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     load(a.k_cache, base, n, k);
     load(a.v_cache, base, n, v);
   };
-  if (nt > 0) request(0, kc, vc);
+  if (j0 < nt) request(j0, kc, vc);
 
-  // ---- the new token's rows (RQ): the wave whose last tile ends the sequence appends them and uses them from registers
+  // ---- the new token's rows (RQ): the wave whose last tile ends the sequence appends them and uses them from LDS
   const int newest = RQ == 3 ? sl.key(len) : len - 1;             // (slabs: -1, not among the keys)
-  const bool holds_new = RQ != 0 && nt > 0 && newest >= 0 && newest / SK % S == split && newest % SK / V3_KPW == wv;
+  const bool mine = ROW ? max(newest, 0) >> a.v4_row == split : newest / SK % S == split;   // this workgroup's
+  const bool holds_new = RQ != 0 && nt > 0 && newest >= 0 && mine && newest % SK / V3_KPW == wv;
   if constexpr (RQ == 3) {
     for (int it = threadIdx.x;;) {
-      sl.finish(a, b, kvh, it, qrot, fresh);
+      sl.finish(a, b, kvh, it, !ROW || mine, qrot, fresh);
       if ((it += NW * 64) >= (group + 2) * (D / 4)) break;
       sl.load(a, b, kvh, group, it);
       sl.follow(a, b);
@@ -268,7 +280,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     int kwc, blk;
     size_t base;
     const int nvis = tile_at(j, kwc, base, blk);
-    const int at = holds_new && j == (RQ == 3 ? newest / SK : nt - 1) && nvis > 0 ? newest - kwc : -1;
+    const int at = holds_new && j == (RQ == 3 ? (newest - (ROW ? kfirst : 0)) / SK : nt - 1) && nvis > 0 ? newest - kwc : -1;
     v3_lds_order();
     store(k, 0, at);
     v3_lds_order();
@@ -357,7 +369,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
       o[d] = mfma16<T>(make_uint4(v0.x, v0.y, v1.x, v1.y), pb, o[d]);
     }
   };
-  for (int j = 0; j < nt; j++) tile(j, kc, vc);
+  for (int j = j0; j < nt; j++) tile(j, kc, vc);
 
   // ---- merge the waves: one common maximum, every wave's sums scaled to it
   l += __shfl_xor(l, 16, 64);
@@ -390,7 +402,7 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
         const float4 u = *(const float4*)(ob + ((size_t)(w * DT + d) * 64 + lane) * 4);
         s4.x += u.x; s4.y += u.y; s4.z += u.z; s4.w += u.w;
       }
-      if (S == 1) {
+      if (nsg == 1) {
         uint16_t* out = a.out + (((size_t)b * a.Tq + t) * a.Hq + h) * D + 16 * d + 4 * g;
         *(uint2*)out = make_uint2(pack2<T>(s4.x * inv, s4.y * inv), pack2<T>(s4.z * inv, s4.w * inv));
       } else if constexpr (FUSE) {
@@ -399,12 +411,12 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
         *(float4*)(po + 16 * d) = s4;
       }
     }
-    if (S > 1 && wv == 0 && g == 0) {
+    if (nsg > 1 && wv == 0 && g == 0) {
       if constexpr (FUSE) st8_sc1(a.part_ml + prow * 2, M, L);
       else *(float2*)(a.part_ml + prow * 2) = make_float2(M, L);
     }
   }
-  if (S == 1) {
+  if (nsg == 1) {
     if constexpr (RQ == 2) {
       // every wave has read its columns of the qkv sums: zero for the next layer's adds
       float* pr = (float*)a.rq_part + (size_t)b * a.rq_ld;
@@ -422,12 +434,12 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
     if (threadIdx.x == 0) {
       int* ctr = a.v3_counters + (size_t)b * a.Hkv + kvh;
       const int prev = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      s_last = prev == S - 1;
+      s_last = prev == nsg - 1;
       if (s_last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     if (!s_last) return;
-    v3_combine<T, true>(a, b, kvh, S, threadIdx.x, NW * 64);
+    v3_combine<T, true>(a, b, kvh, nsg, threadIdx.x, NW * 64);
   }
 }
 
@@ -436,7 +448,16 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
 // keys, 32 / 8 heads, us, the kernels of attn_dec_v3.cuh / this:
 //   * from 136 pairs on one workgroup each, 8 waves while they are one per CU, else 4 (two per CU): 18 x 1024 29.3 / 19.8, 20 x
 //     800 22.1 / 16.5, 24 x 1024 24.5 / 19.8, 32 x 600 21.6 / 16.9, 48 x 700 31.9 / 25.3 (8 waves 28.6), 64 x 256 19.0 / 14.5,
-//     100 x 600 52.4 / 43.1, 28 x 2100 45.9 / 40.5;
+//     100 x 600 52.4 / 43.1, 28 x 2100 45.9 / 40.5 -- while the longest sequence that the grid is made for is no more than 10
+//     tiles a wave (2560, 1280 keys).  Beyond, 1024 keys in a row each, 2048 .. where that makes more than 8192 workgroups or 32
+//     a pair: with one long sequence among short ones a single workgroup streamed it while the others were done.  us with the rope
+//     launch or the slabs here, attn_dec_v3.cuh / one workgroup / this: 31 x 500 and 1 x 16000 84 / 151 / 56, 39 and one 116 / 213 / 61,
+//     56 x 300 and 8 x 8000 117 / 115 / 76, 16 x 500 and 1 x 16000 88 / 148 / 37, 63 x 200 and 1 x 30000 353 / 383 / 87, 47 x 300 and 1 x
+//     4000 47 / 63 / 38, 39 x 300 and 1 x 2000 34 / 38 / 29, 28 / 4 heads 39 x 500 and 1 x 16000 105 / 148 / 49, a window of 4096 in
+//     32 x 16000 295 / 145 / 126.  Up to 10 tiles one workgroup is no later than attn_dec_v3.cuh with those, either (17 x 300 and 1 x
+//     2000 36 / 27, 31 and one 30 / 28), and ahead where the lengths are alike: 28 x 2100 48 / 42 / 45, 50 x 1200 55 / 45 / 47.  Above,
+//     what rows of keys cost there: 20 x 3000 53 / 45 / 47, 17 x 3500 48 / 47 / 45, 24 x 4000 78 / 64 / 68, 40 x 1500 51 / 47 / 45, 33 x
+//     2500 71 / 69 / 57, 64 x 2000 91 / 81 / 86, 32 x 8000 170 / 161 / 166, 28 / 4 heads 40 x 3000 51 / 45 / 47, 64 x 3000 76 / 64 / 73;
 //   * fewer pairs of more than 8 sequences, so few keys that the merge is most of the time: 16 x 256 12.2 / 9.1, 16 x 800 (q
 //     pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9.  Up to 8 sequences not, though some are ahead (1 x 128 8.4 / 6.0, 8 x
 //     400 10.8 / 10.1, 8 x 600 12.1 / 11.8; 1 x 400 even, 1 x 600 8.9 / 9.2): there, steps that rotate in the attention keep
@@ -448,44 +469,48 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
 //     1300 23.2 / 17.8, 14 x 1024 22.8 / 17.9, 16 x 1024 24.2 / 18.7.  Between, one tile a wave has the shorter chain: 1 x 1100
 //     9.1 / 9.3, 4 x 1500 12.7 / 12.8, 6 x 1300 13.8 / 13.8, 8 x 700 12.6 / 12.9, 12 x 1024 16.5 / 17.1.
 struct V4Plan {
-  int nw, groups;
+  int nw, groups, row;                           // row > 0: 1 << row keys in a row for each of the groups (4 waves)
 };
 inline V4Plan v4_plan(int B, int Hkv, int nsplit) {
   static const bool off = getenv("ILLM_ATTN_V3_NW") || getenv("ILLM_ATTN_V3_TILES") || (getenv("ILLM_ATTN_V4") && atoi(getenv("ILLM_ATTN_V4")) == 0);
   if (off) return {0, 0};                        // a forced form of attn_dec_v3.cuh (A/B runs)
   const long pairs = (long)B * Hkv, keys = (long)nsplit * SPLIT;
-  if (pairs >= 136) return {pairs <= 256 ? 8 : 4, 1};
+  if (pairs >= 136) {
+    const int nw = pairs <= 256 ? 8 : 4;
+    if (keys <= 10 * V3_KPW * nw) return {nw, 1, 0};
+    const long most = std::max(8L, std::min(32L, 8192 / pairs));
+    int row = 10;
+    while (keys > most << row) row++;
+    return {4, (int)((keys + (1L << row) - 1) >> row), row};
+  }
   if (B > 8 && keys <= (pairs >= 112 ? 896 : pairs >= 64 ? 704 : 512)) return {keys <= 192 ? 4 : 8, 1};
   if (keys < (pairs >= 112 ? 0 : pairs >= 80 ? 1152 : pairs >= 64 ? 1024 : 1920)) return {0, 0};
   const long s = std::min({512 / pairs, pairs >= 16 || keys < 16384 ? 16L : 32L, keys / (4 * V3_KPW)});
   return {4, (int)s};
 }
 
-template <typename T, int D, int NW, int RQ>
+template <typename T, int D, int NW, int RQ, bool ROW>
 static void launch_v4_nw(const AttnDecodeArgs& a, int S, hipStream_t st) {
-  dim3 grid(S, a.Hkv, a.B);
-  if (S == 1 || a.v3_counters != nullptr) {
-    hipLaunchKernelGGL((attn_decode_v4_kernel<T, D, NW, RQ, true>), grid, dim3(64 * NW), 0, st, a);
+  const dim3 grid = ROW ? dim3(a.Hkv, a.B, S) : dim3(S, a.Hkv, a.B);
+  if (RQ == 3 ? ROW : S == 1 || a.v3_counters != nullptr) {
+    if constexpr (RQ != 3 || ROW) hipLaunchKernelGGL((attn_decode_v4_kernel<T, D, NW, RQ, true, ROW>), grid, dim3(64 * NW), 0, st, a);
+  } else if constexpr (RQ == 3) {
+    if constexpr (!ROW) hipLaunchKernelGGL((attn_decode_v4_kernel<T, D, NW, RQ, false, ROW>), grid, dim3(64 * NW), 0, st, a);
   } else {
-    hipLaunchKernelGGL((attn_decode_v4_kernel<T, D, NW, RQ, false>), grid, dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((attn_decode_v4_kernel<T, D, NW, RQ, false, ROW>), grid, dim3(64 * NW), 0, st, a);
     hipLaunchKernelGGL((attn_combine_v3_kernel<T>), dim3(a.Hkv, a.B), dim3(256), 0, st, a, S);
   }
 }
 
-// q, k and v as slabs of the qkv product: one workgroup a pair (v4_plan), checked by the caller
-template <typename T>
-static void launch_v4_slabs(const AttnDecodeArgs& a, hipStream_t st) {
-  dim3 grid(1, a.Hkv, a.B);
-  if (v4_plan(a.B, a.Hkv, a.nsplit).nw == 8) hipLaunchKernelGGL((attn_decode_v4_kernel<T, 128, 8, 3, false>), grid, dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((attn_decode_v4_kernel<T, 128, 4, 3, false>), grid, dim3(256), 0, st, a);
-}
-
 template <typename T, int D, int RQ>
-static bool launch_v4(const AttnDecodeArgs& a, hipStream_t st) {
-  const V4Plan p = v4_plan(a.B, a.Hkv, a.nsplit);
+static bool launch_v4(const AttnDecodeArgs& a0, hipStream_t st) {
+  const V4Plan p = v4_plan(a0.B, a0.Hkv, a0.nsplit);
   if (p.groups == 0) return false;
-  if (p.nw == 8) launch_v4_nw<T, D, 8, RQ>(a, p.groups, st);
-  else launch_v4_nw<T, D, 4, RQ>(a, p.groups, st);
+  AttnDecodeArgs a = a0;
+  a.v4_row = p.row;
+  if (p.row > 0) launch_v4_nw<T, D, 4, RQ, true>(a, p.groups, st);
+  else if (p.nw == 8) launch_v4_nw<T, D, 8, RQ, false>(a, p.groups, st);
+  else launch_v4_nw<T, D, 4, RQ, false>(a, p.groups, st);
   return true;
 }
 

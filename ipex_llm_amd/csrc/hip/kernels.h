@@ -209,6 +209,7 @@ struct AttnDecodeArgs {
   // combine (null: separate combine launch)
   int* v3_counters;
   int rq_slabs;             // > 0: rq_part is that many unrotated slabs [rq_slabs, B, rq_ld] (attn_dec_v4.cuh), left as they are
+  int v4_row;               // > 0: a workgroup of attn_dec_v4.cuh has 1 << v4_row keys in a row (0: tiles in turn)
   const int64_t* rq_pos_offset;   // [B] or null: rq_pos less this is the new key's index (slabs only)
 };
 void launch_attn_decode(bool bf16, const AttnDecodeArgs& a, hipStream_t st);
@@ -216,7 +217,7 @@ void launch_attn_decode(bool bf16, const AttnDecodeArgs& a, hipStream_t st);
 int attn_decode_groups(int B, int Hkv, int nsplit);
 // waves of a workgroup (returned) and workgroups per pair of the streaming kernel, head dim 128 (0, 0: not taken)
 int attn_decode_plan(int B, int Hkv, int nsplit, int* groups);
-// one workgroup a pair: it can take q, k and v as slabs of the qkv product (AttnDecodeArgs::rq_slabs)
+// a workgroup's keys are in a row: it can take q, k and v as slabs of the qkv product (AttnDecodeArgs::rq_slabs)
 bool attn_slabs_takes(int B, int Hkv, int nsplit);
 
 // ---- prefill / long-query attention over the paged cache (attn_prefill.hip)

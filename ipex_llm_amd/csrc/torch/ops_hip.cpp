@@ -1494,10 +1494,11 @@ static bool v3_fuse_on() {
   return on;
 }
 int* attn_counters(const c10::Device& dev, int64_t n);
+constexpr int64_t kV3Counters = 1 << 16;
 static int* v3_counters(const c10::Device& dev, int64_t n) {
   static std::vector<Tensor> bufs(64);
   const int idx = dev.index() < 0 ? 0 : dev.index();
-  constexpr int64_t kCap = 1 << 16;
+  constexpr int64_t kCap = kV3Counters;
   if (n > kCap) return nullptr;
   if (!bufs[idx].defined()) bufs[idx] = at::zeros({kCap}, at::TensorOptions().device(dev).dtype(at::kInt));
   return bufs[idx].data_ptr<int>();
@@ -1705,6 +1706,14 @@ static std::tuple<Tensor, Tensor, Tensor> attn_decode_rope_impl(
 }
 
 
+// where attn_decode_slabs is a launch: a workgroup's keys are in a row, and what several of a pair need is there
+static bool attn_slabs_takes(int64_t B, int64_t Hkv, int64_t nsplit) {
+  if (B < 1 || B >= (1 << 20) || Hkv < 1 || nsplit < 1 || nsplit > kMaxDecodeSplits || fused_combine_on()) return false;
+  int groups = 0;
+  illm::attn_decode_plan((int)B, (int)Hkv, (int)nsplit, &groups);
+  return illm::attn_slabs_takes((int)B, (int)Hkv, (int)nsplit) && (groups == 1 || (v3_fuse_on() && B * Hkv <= kV3Counters));
+}
+
 // decode attention (Tq == 1, head dim 128, full NeoX rotation) over the slabs [ks, B, ld] of the qkv product: their sum, bias,
 // rotation and the append at pos - pos_offset as in rope_kv_fused, without its launch.  Where attn_slabs_takes says so
 Tensor attn_decode_slabs(const Tensor& part, const c10::optional<Tensor>& bias, const Tensor& cos_sin, const Tensor& pos,
@@ -1726,9 +1735,18 @@ Tensor attn_decode_slabs(const Tensor& part, const c10::optional<Tensor>& bias, 
   TORCH_CHECK(pos.scalar_type() == at::kLong && pos.is_contiguous() && pos.numel() >= B && block_tables.scalar_type() == at::kInt &&
                   block_tables.is_contiguous() && block_tables.size(0) >= B && seq_lens.scalar_type() == at::kInt &&
                   seq_lens.is_contiguous() && seq_lens.numel() >= B, "attn_decode_slabs: int64 positions, int32 tables of B rows");
-  TORCH_CHECK(nsplit >= 1 && nsplit <= kMaxDecodeSplits && !fused_combine_on() && illm::attn_slabs_takes((int)B, (int)Hkv, (int)nsplit),
-              "attn_decode_slabs: not taken");
+  TORCH_CHECK(attn_slabs_takes(B, Hkv, nsplit), "attn_decode_slabs: not taken");
   illm::AttnDecodeArgs a{};
+  int groups = 0;                                // several: partials, merged by the last of a pair to arrive
+  illm::attn_decode_plan((int)B, (int)Hkv, (int)nsplit, &groups);
+  Tensor po, pml;
+  if (groups > 1) {
+    po = at::empty({B, Hq, nsplit, 128}, part.options());
+    pml = at::empty({B, Hq, nsplit, 2}, part.options());
+    a.part_o = po.data_ptr<float>();
+    a.part_ml = pml.data_ptr<float>();
+    a.v3_counters = v3_counters(part.device(), B * Hkv);
+  }
   Tensor out = at::empty({B, 1, Hq, 128}, part.options().dtype(dt));
   a.k_cache = (const uint8_t*)k_cache.data_ptr();
   a.v_cache = (const uint8_t*)v_cache.data_ptr();
@@ -2261,9 +2279,7 @@ TORCH_LIBRARY_FRAGMENT(ipex_llm_amd, m) {
   m.def("row_norm_o_takes(int M, int n, int fmt) -> bool", &row_norm_o_takes);
   m.def("row_rope_takes(int M, int n, int k, int fmt) -> bool", &row_rope_takes);
   m.def("skinny_takes(int M, int n, int k, int fmt, bool glu, bool bf16, int ksplit=0) -> bool", &skinny_takes);
-  m.def("attn_slabs_takes(int batch, int kv_heads, int nsplit) -> bool", [](int64_t b, int64_t h, int64_t n) {
-    return b >= 1 && b < (1 << 20) && n >= 1 && n <= kMaxDecodeSplits && !fused_combine_on() && illm::attn_slabs_takes((int)b, (int)h, (int)n);
-  });
+  m.def("attn_slabs_takes(int batch, int kv_heads, int nsplit) -> bool", &attn_slabs_takes);
   m.def("attn_decode_plan(int batch, int kv_heads, int nsplit) -> int[]", [](int64_t b, int64_t h, int64_t n) -> std::vector<int64_t> {
     TORCH_CHECK(b >= 1 && h >= 1 && n >= 1 && b < (1 << 20) && h < 4096 && n < (1 << 24), "attn_decode_plan: sizes");
     int groups = 0;

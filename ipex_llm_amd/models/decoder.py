@@ -769,8 +769,8 @@ class NativeCausalLM(nn.Module):
         row_rope = prerot and row_norm and self._row_rope_ok(T, seen)  # bias and rotation ahead of the store
         prerot = row_rope or (prerot and not seen().bias)
         rope_in = rope_ok and (T <= ROPE_IN_MAX_M or prerot)
-        # more sequences than that: qkv slabs, whose sum, rotation and append the attention does where a workgroup has a whole
-        # (sequence, kv head)
+        # more sequences than that: qkv slabs, whose sum, rotation and append the attention does where a workgroup's keys
+        # are in a row
         slabs_in = (T > ACC_MAX_M and not rope_in and self._rope_in_ok(meta, cache) and s.head_dim == s.rot_dim == 128
                     and not s.rope_interleaved and self.alibi is None and not self._attn_fuse and x.is_cuda
                     and cache.k[0].dtype == x.dtype and ops.native_gpu(x)

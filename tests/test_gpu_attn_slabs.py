@@ -1,6 +1,6 @@
 """Decode attention over the slabs of the qkv product (attn_decode_slabs): bit for bit rope_kv_fused and attn_decode, in the
 output and in the caches -- one to six slabs, items of one pass over the workgroup and of several, the new key at the edges of
-tiles, offsets of a compressed cache, padding rows, bad blocks -- and in a model's step, captured too."""
+tiles and of a workgroup's, offsets of a compressed cache, padding rows, bad blocks -- and in a model's step, captured too."""
 import pytest
 import torch
 
@@ -39,6 +39,8 @@ def _both(dev, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset, tables=None)
     ([1, 128, 129, 256, 257, 513, 640, 31, 32, 33] * 4, 640, 8, 7, 128),
     ([1, 32, 129, 191, 192] * 2, 192, 8, 16, 192),
     ([511, 33, 1] * 3, 512, 2, 1, 64),
+    ([3072, 1, 1024, 1025, 2048, 2049, 33, 3000, 1023] * 2, 3072, 8, 4, 64),   # several workgroups a pair
+    ([1345, 1, 1024, 1025] * 10, 1408, 8, 7, 128),
 ])
 @pytest.mark.parametrize("ks,bias,window,offset", [(1, True, 0, False), (2, False, 0, False), (4, True, 100, True), (6, False, 0, True)])
 def test_same_bits(cuda, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset):
@@ -47,25 +49,26 @@ def test_same_bits(cuda, dtype, L, cap, Hkv, G, bs, ks, bias, window, offset):
     assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(old, new))
 
 
-def test_padding_rows_and_bad_blocks(cuda):
-    L = [0, 100, 64, 65, 7, 128] * 3
+@pytest.mark.parametrize("cap", [128, 3072])                       # one workgroup a pair, three
+def test_padding_rows_and_bad_blocks(cuda, cap):
+    L = [0, 100, 64, 65, 7, cap] * 3
 
     def padded(bt):
         bt[0] = -1
-    want, got, old, new = _both(cuda, torch.bfloat16, L, 128, 8, 4, 64, 2, False, 0, False, padded)
+    want, got, old, new = _both(cuda, torch.bfloat16, L, cap, 8, 4, 64, 2, False, 0, False, padded)
     ops.check_kernel_errors(cuda)
     assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(old, new))
 
     def bad(bt):
-        bt[1, 1] = bt.numel() + 5
-    want, got, old, new = _both(cuda, torch.bfloat16, L, 128, 8, 4, 64, 2, False, 0, False, bad)
+        bt[1, 1] = bt[5, -1] = bt.numel() + 5
+    want, got, old, new = _both(cuda, torch.bfloat16, L, cap, 8, 4, 64, 2, False, 0, False, bad)
     with pytest.raises(RuntimeError):
         ops.check_kernel_errors(cuda)
     assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(old, new))
 
 
 def test_not_taken(cuda):
-    """several workgroups a pair, and widths that are not the heads'"""
+    """several workgroups a pair in turn, and widths that are not the heads'"""
     assert not T.attn_slabs_takes(1, 8, 100)
     x = torch.zeros(2, 1, 6144, device=cuda)
     kc = torch.zeros(100, 8, 64, 128, dtype=torch.bfloat16, device=cuda)

@@ -44,7 +44,10 @@ CASES = [  # lengths, keys of the grid, kv heads, group, block, (waves, workgrou
     ([511, 33, 1] * 3, 512, 2, 16, 128, [8, 1]),
     ([1024, 895, 129, 127, 128, 1, 640, 960], 1088, 8, 7, 64, [4, 8]),
     ([4100, 2047, 33], 4224, 8, 4, 192, [4, 16]),
-    ([17000, 16384, 1] + [65] * 14, 17024, 8, 2, 64, [8, 1]),      # 67 tiles a wave
+    ([17000, 16384, 1] + [65] * 14, 17024, 8, 2, 64, [4, 17]),     # 8 tiles in a row a workgroup, most without keys
+    ([1344, 1025, 1024, 1023, 129, 1, 33, 64] * 5, 1344, 8, 4, 64, [4, 2]),
+    ([2624, 2048, 2049, 1] + [200] * 14, 2688, 8, 7, 192, [4, 3]),
+    ([25600, 1, 33, 128, 129], 25600, 27, 1, 64, [4, 3]),          # 67 tiles a wave
 ]
 
 
