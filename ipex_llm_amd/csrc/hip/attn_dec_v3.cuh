@@ -29,7 +29,7 @@
 // Row r of the P V MFMA depends only on row r of P, and each split's
 // reductions run in a fixed key order: a multi-row verify (speculative decoding)
 // reduces every row exactly like one-token decoding with the same NW, as long as
-// both take q from memory; the kernel with several tiles per wave, too (v3_long_grid: which batches run it).
+// both take q from memory; the kernel with several tiles per wave, too (v3_long_grid: which batches of head dim 64).
 #pragma once
 
 namespace illm {
@@ -601,7 +601,7 @@ __global__ void __launch_bounds__(64 * NW, ILLM_V3_MINW(RQ)) attn_decode_v3_kern
   attn_v3_body<T, D, NW, RQ, FUSE>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, sm);
 }
 
-// ---- long contexts: several 32-key tiles per wave (the rotation here, or head dim 64; else attn_dec_v4.cuh) --------
+// ---- long contexts: several 32-key tiles per wave (head dim 128: the rotation here; head dim 64: q from memory) ------
 // One tile per wave pays a workgroup's fixed chain (sequence length -> block
 // table -> K / V round trip -> max and sum over the waves -> partial) for every
 // 32 NW keys: 20 K keys x 3 sequences were 1896 workgroups in 7 rounds, 74 us
@@ -621,8 +621,7 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
   constexpr int NW = V3L_NW;
   constexpr int KSTEP = D / 32, DT = D / 16, VU = D / 8, KPJ = 64 / VU, VJ = V3_KPW / KPJ;
   constexpr int SK = V3_KPW * NW;
-  static_assert(D == 64 || D == 128, "v3: head_dim 64 / 128");
-  static_assert(RQ == 0 || D == 128, "v3: fused RoPE needs head_dim 128");
+  static_assert(D == 64 ? RQ == 0 : D == 128 && RQ == 1, "v3l: the other modes of head dim 128 run attn_dec_v4.cuh");
   __shared__ V3Smem<D, NW, RQ> sm;
   const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
   const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
@@ -681,11 +680,11 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
 
     // tiles of this wave that hold keys (the first one runs in any case: fully masked if it holds none)
     const int nt = max(1, (len - kw + step - 1) / step);
-    // the first tile is requested before q, whose columns are then a round trip beside it, not ahead of it; not where
-    // the new token's rows are appended to it first, nor beside the registers of the rotation
+    // the first tile is requested before q, whose columns are then a round trip beside it, not ahead of it; not beside
+    // the registers of the rotation, nor where the new token's rows are appended to it first
     const bool appends = RQ != 0 && (len - 1) / SK % (int)gridDim.x == split && (len - 1) % SK / V3_KPW == wv;
-    const bool early = RQ != 1 && !(appends && nt == 1);          // wave-uniform
-    if (early) {
+    constexpr bool early = RQ == 0;
+    if constexpr (early) {
       tile_at(blk_next);
       load_k();
       load_v();
@@ -694,9 +693,9 @@ __global__ void __launch_bounds__(64 * V3L_NW, 3) attn_decode_v3l_kernel(const A
     // ---- q fragments (lane: row r16, dims 32 s + 8 g .. + 8)
     uint4 qf[KSTEP];
     if constexpr (RQ != 0) {
-      const V3Rope<T, D, RQ == 2> rp(a, b, g, true);
-      typename V3Rope<T, D, RQ == 2>::Raw raw;
-      typename V3Rope<T, D, RQ == 2>::CS cs;
+      const V3Rope<T, D, false> rp(a, b, g, true);
+      typename V3Rope<T, D, false>::Raw raw;
+      typename V3Rope<T, D, false>::CS cs;
       rp.load(h * D, raw);
       rp.load_cs(cs);
       float v[KSTEP][8];
@@ -933,30 +932,24 @@ static void launch_v3_nw(const AttnDecodeArgs& a, hipStream_t st) {
 
 // workgroups per (sequence, kv head) of the kernel with several tiles per wave (0: one tile per wave, the kernel above).
 //
-// q from memory (a batch past the fused RoPE, dense projections, a multi-row verify: one rule by batch, kv heads and
-// split grid, so a one-token step and a verify of the same batch keep one kernel and one order of reduction): from 256
-// pairs of sequence and kv head on as many as make 768, which are resident at once (three per CU), where the kernel
-// above needs rounds.  Sequences of half to all of the keys, 32 / 8 heads, one tile per wave / this, us: 48 x 700 32.2 /
-// 30.8, 48 x 400 23.9 / 21.2, 48 x 1200 48.0 / 47.1, 64 x 300 26.7 / 20.8, 56 x 800 47.6 / 39.4, 64 x 900 54.6 / 46.1,
-// 128 x 200 44.0 / 30.5, 36 x 300 19.8 / 16.2, 32 x 768 30.0 / 25.0, 32 x 1800 53.9 / 45.7, but 40 x 1500 48.2 / 48.8 (two
-// and a half per CU); 28 / 4 heads 96 x 300 22.6 / 19.1, 32 / 32 heads 64 x 500 98.6 / 90.5.  Not below: 24 x 512 15.5 /
-// 16.5, 24 x 1024 25.5 / 25.8, 28 / 4 heads 48 x 700 20.0 / 20.7; nor where a workgroup has one tile or the grid two: 64 x
-// 128 13.5 / 14.2, 32 x 100 10.4 / 11.9, 28 / 4 heads 64 x 300 14.7 / 15.6; nor where 8-wave groups of one tile per wave are
-// one round themselves (32 x 400 16.4 / 17.3, 28 / 4 heads 64 x 400 16.8 / 18.7), nor with 9 to 12 tiles a pair where two
-// workgroups a pair leave many CUs two of their three (33 x 1500 42.8 / 46.6, 28 / 4 heads 72 x 1200 37.1 / 41.0, 80 x 1200
-// 41.7 / 44.2; longer ones are even, 40 x 2500 78.2 / 76.0).  Some 4 % behind it is at 33 x 2500 and 28 / 4 heads 96 x 1200 in
-// one run of two.  Lengths that differ more: 31 of 500 tokens and one of 16000 137 / 78, 95 and one 424 / 209, 39 of 500 and
-// one of 16000 170 / 110, 56 of 300 and 8 of 8000 160 / 107 (most groups of a grid made for the longest find no keys; more
-// workgroups for these is open: 12 tiles each measured 60, 90, 69 and 75, 8 tiles 76, 193, 73 and 94).
+// Head dim 64, q from memory (one rule by batch, kv heads and split grid, so a one-token step and a verify of the same
+// batch keep one kernel and one order of reduction): from 256 pairs of sequence and kv head on as many as make 768, which
+// are resident at once (three per CU), where the kernel above needs rounds.  Sequences of half to all of the keys, 32 / 8
+// heads, one tile per wave / this, us: 32 x 768 16.3 / 14.3, 32 x 1800 28.4 / 24.2, 36 x 300 14.0 / 11.4, 48 x 400 16.2 / 13.9,
+// 48 x 700 20.8 / 18.2, 48 x 1200 27.6 / 23.6, 64 x 300 17.8 / 12.9, 64 x 900 33.7 / 23.0, 40 x 2500 45.4 / 38.4, 100 x 700 35.2 /
+// 30.4, 14 / 2 heads 200 x 500 19.4 / 15.6, 31 of 500 tokens and one of 16000 114 / 49, 56 of 300 and 8 of 8000 262 / 71.  Not below
+// 256 pairs, nor where a workgroup has one tile or the grid two, nor where 8-wave groups of one tile per wave are one round
+// themselves, nor with 9 to 12 tiles a pair where two workgroups a pair leave many CUs two of their three: the lines were
+// drawn with head dim 128, which attn_dec_v4.cuh has now (24 x 1024 25.5 / 25.8, 64 x 128 13.5 / 14.2, 32 x 400 16.4 / 17.3, 33 x 1500
+// 42.8 / 46.6).
 //
-// Fused-RoPE decode, 48 splits and more, for sequences of the grid's full length: the CU with the most workgroups has
-// n = ceil(workgroups / 256) of them, each t tiles and about 0.7 tiles' time to start and merge, and where the lengths
-// differ the longest workgroup ends the launch (0.2 t); t from 2 to 8 with the least n (t + 0.7) + 0.2 t.  Attention of
-// 32 / 8 heads, sequences of half to all of these keys, one tile per wave / t 2 .. 8 (us), the chosen one marked:
-// 4 x 4000 24.6 / 19.0 21.2 [19.9] 20.8 21.2 22.7 24.4; 8 x 6000 48.3 / 39.8 39.1 35.8 37.1 [34.9] 36.6 39.1; 16 x 3500
-// 47.8 / 41.5 40.4 40.1 38.1 41.3 [38.7] 38.9; 1 x 16000 30.9 / 22.0 19.8 [17.9] 17.7 18.5 19.8 18.2; 3 x 20000 72.5 /
-// 52.7 46.6 45.4 [41.0] 41.9 45.4 41.1.  Not below 48 splits (8 x 2000: layer 69.8 -> 70.8), nor for few workgroups just
-// above (4 x 3200 19.2 / 20.8).  (ILLM_ATTN_V3_TILES=t forces t; a function of batch, kv heads and split grid only.)
+// Head dim 128, the rotation here, 48 splits and more, for sequences of the grid's full length: the CU with the most
+// workgroups has n = ceil(workgroups / 256) of them, each t tiles and about 0.7 tiles' time to start and merge, and where
+// the lengths differ the longest workgroup ends the launch (0.2 t); t from 2 to 8 with the least n (t + 0.7) + 0.2 t.
+// Sequences of half to all of these keys, 32 / 8 heads, one tile per wave / this, us: 4 x 4000 30.1 / 25.7, 8 x 6000 76.2 / 47.5, 1 x
+// 16000 30.4 / 23.1, 3 x 20000 74.8 / 47.5; 4 x 3200 23.7 / 24.2 and below one tile is as fast or faster.  (The t were fitted with q
+// rotated ahead: 8 x 6000 39.8 39.1 35.8 37.1 [34.9] 36.6 39.1 for t 2 .. 8, one tile 48.3.)
+// (ILLM_ATTN_V3_TILES=t forces t; a function of batch, kv heads and split grid only.)
 inline int v3_long_grid(const AttnDecodeArgs& a, int rq) {
   static const int env = getenv("ILLM_ATTN_V3_TILES") ? atoi(getenv("ILLM_ATTN_V3_TILES")) : -1;
   const long all = (a.nsplit * SPLIT + V3_KPW * V3L_NW - 1) / (V3_KPW * V3L_NW);
@@ -980,15 +973,17 @@ inline int v3_long_grid(const AttnDecodeArgs& a, int rq) {
 
 template <typename T, int D, int RQ>
 static void launch_v3(const AttnDecodeArgs& a, hipStream_t st) {
-  if (const int ns = v3_long_grid(a, RQ)) {
-    dim3 grid(ns, a.Hkv, a.B);
-    if (a.v3_counters != nullptr) {
-      hipLaunchKernelGGL((attn_decode_v3l_kernel<T, D, RQ, true>), grid, dim3(64 * V3L_NW), 0, st, a);
-    } else {
-      hipLaunchKernelGGL((attn_decode_v3l_kernel<T, D, RQ, false>), grid, dim3(64 * V3L_NW), 0, st, a);
-      hipLaunchKernelGGL((attn_combine_v3_kernel<T>), dim3(a.Hkv, a.B), dim3(256), 0, st, a, ns);
+  if constexpr (D == 64 || RQ == 1) {            // (else attn_dec_v4.cuh's, or one tile per wave)
+    if (const int ns = v3_long_grid(a, RQ)) {
+      dim3 grid(ns, a.Hkv, a.B);
+      if (a.v3_counters != nullptr) {
+        hipLaunchKernelGGL((attn_decode_v3l_kernel<T, D, RQ, true>), grid, dim3(64 * V3L_NW), 0, st, a);
+      } else {
+        hipLaunchKernelGGL((attn_decode_v3l_kernel<T, D, RQ, false>), grid, dim3(64 * V3L_NW), 0, st, a);
+        hipLaunchKernelGGL((attn_combine_v3_kernel<T>), dim3(a.Hkv, a.B), dim3(256), 0, st, a, ns);
+      }
+      return;
     }
-    return;
   }
   switch (v3_pick_nw(a)) {
     case 1: return launch_v3_nw<T, D, 1, RQ>(a, st);

@@ -213,7 +213,7 @@ struct AttnDecodeArgs {
   const int64_t* rq_pos_offset;   // [B] or null: rq_pos less this is the new key's index (slabs only)
 };
 void launch_attn_decode(bool bf16, const AttnDecodeArgs& a, hipStream_t st);
-// workgroups per (sequence, kv head) of several tiles per wave, q from memory (0: one tile per wave)
+// workgroups per (sequence, kv head) of several tiles per wave, head dim 64 (0: one tile per wave)
 int attn_decode_groups(int B, int Hkv, int nsplit);
 // waves of a workgroup (returned) and workgroups per pair of the streaming kernel, head dim 128 (0, 0: not taken)
 int attn_decode_plan(int B, int Hkv, int nsplit, int* groups);

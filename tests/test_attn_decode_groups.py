@@ -1,4 +1,4 @@
-"""Decode attention with q from memory: where a wave takes several tiles (v3_long_grid in attn_dec_v3.cuh)."""
+"""Decode attention of head dim 64: where a wave takes several tiles (v3_long_grid in attn_dec_v3.cuh)."""
 import pytest
 
 import ipex_llm_amd.ops as ops

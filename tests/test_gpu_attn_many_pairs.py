@@ -1,5 +1,6 @@
-"""Decode attention of many sequences with q from memory: several tiles per wave from 256 pairs of sequence and kv head
-on (attn_dec_v3.cuh, v3_long_grid), vs float64; one-token steps and rows of a verify alike."""
+"""Decode attention of many sequences with q from memory, vs float64; one-token steps and rows of a verify alike.  Head dim
+64: several tiles per wave from 256 pairs of sequence and kv head on (attn_dec_v3.cuh, v3_long_grid), one to three workgroups
+a pair; head dim 128: streamed (attn_dec_v4.cuh)."""
 import pytest
 import torch
 
@@ -39,23 +40,34 @@ def _check(got, L, kc, vc, bt, q, scale, softcap, window, alibi):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,Hkv,G,D,softcap,window,slopes", [
-    (31, 8, 4, 128, 0.0, 0, False),       # 248 pairs: one tile per wave
-    (32, 8, 4, 128, 0.0, 0, False),       # 256: three workgroups a pair
-    (48, 8, 4, 128, 30.0, 0, False),      # two
-    (64, 4, 7, 128, 0.0, 100, False),     # 256, groups of 7, a window
-    (130, 4, 8, 64, 0.0, 0, True),        # one, head dim 64, ALiBi
-    (100, 8, 1, 128, 0.0, 0, False)])     # 800: one
+    (31, 8, 4, 128, 0.0, 0, False),
+    (32, 8, 4, 128, 0.0, 0, False),
+    (48, 8, 4, 128, 30.0, 0, False),
+    (64, 4, 7, 128, 0.0, 100, False),     # groups of 7, a window
+    (100, 8, 1, 128, 0.0, 0, False),
+    (31, 8, 4, 64, 0.0, 0, False),        # 248 pairs: one tile per wave
+    (32, 8, 4, 64, 0.0, 0, False),        # 256: three workgroups a pair
+    (48, 8, 4, 64, 30.0, 0, False),       # two
+    (64, 4, 7, 64, 0.0, 100, False),      # three, groups of 7, a window
+    (130, 4, 8, 64, 0.0, 0, True),        # two, ALiBi
+    (100, 8, 1, 64, 0.0, 0, False)])      # 800: one
 @pytest.mark.parametrize("cap", [768, 192])   # 6 tiles; 2: one tile per wave
 def test_decode(cuda, B, Hkv, G, D, softcap, window, slopes, cap, dtype):
     L, kc, vc, bt, q, sl, ns = _case(cuda, B, Hkv, G, D, dtype, cap=cap)
     alibi = torch.linspace(0.01, 0.5, Hkv * G, device=cuda) if slopes else None
+    if D == 64:
+        groups = 0 if cap < 256 or B * Hkv < 256 else min(3, max(1, 768 // (B * Hkv)))
+        assert torch.ops.ipex_llm_amd.attn_decode_groups(B, Hkv, ns) == groups
+    else:
+        assert torch.ops.ipex_llm_amd.attn_decode_plan(B, Hkv, ns)[1] == 1
     got = ops.attn_decode(q, kc, vc, bt, sl, ns, D ** -0.5, softcap, window, alibi=alibi)
     _check(got.view_as(q), L, kc, vc, bt, q, D ** -0.5, softcap, window, alibi)
     ops.check_kernel_errors(cuda)
 
 
-def test_verify_rows_equal_one_token_steps(cuda):
-    L, kc, vc, bt, q, sl, ns = _case(cuda, 40, 8, 4, 128, torch.bfloat16, Tq=3)
+@pytest.mark.parametrize("D", [64, 128])
+def test_verify_rows_equal_one_token_steps(cuda, D):
+    L, kc, vc, bt, q, sl, ns = _case(cuda, 40, 8, 4, D, torch.bfloat16, Tq=3)
     got = ops.attn_decode(q, kc, vc, bt, sl, ns, 0.1, 0.0, 0).view_as(q)
     _check(got, L, kc, vc, bt, q, 0.1, 0.0, 0, None)
     for t in range(3):
