@@ -459,10 +459,11 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
 //     what rows of keys cost there: 20 x 3000 53 / 45 / 47, 17 x 3500 48 / 47 / 45, 24 x 4000 78 / 64 / 68, 40 x 1500 51 / 47 / 45, 33 x
 //     2500 71 / 69 / 57, 64 x 2000 91 / 81 / 86, 32 x 8000 170 / 161 / 166, 28 / 4 heads 40 x 3000 51 / 45 / 47, 64 x 3000 76 / 64 / 73;
 //   * fewer pairs of more than 8 sequences, so few keys that the merge is most of the time: 16 x 256 12.2 / 9.1, 16 x 800 (q
-//     pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9.  Up to 8 sequences not, though some are ahead (1 x 128 8.4 / 6.0, 8 x
-//     400 10.8 / 10.1, 8 x 600 12.1 / 11.8; 1 x 400 even, 1 x 600 8.9 / 9.2): there, steps that rotate in the attention keep
-//     attn_dec_v3.cuh, and p is rounded beside its wave's maximum here and its workgroup's there: 1.9e-3 between the two over 70
-//     keys, and the tokens of two ranks parted from those of one at a tie;
+//     pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9.  Up to 8 sequences not, however many kv heads, though most are ahead (1 x 128 8.4 / 6.0, 8 x
+//     400 10.8 / 10.1, 8 x 600 12.1 / 11.8, 32 kv heads 4 x 100 8.4 / 6.3, 5 x 250 10.3 / 8.4, 8 x 436 16.6 / 15.4; 1 x 400 even, 1 x 600
+//     8.9 / 9.2, 32 kv heads 4 x 250 9.5 / 10.2, 4 x 1000 16.7 / 17.2): there, steps that rotate in the attention keep attn_dec_v3.cuh,
+//     and p is rounded beside its wave's maximum here and its workgroup's there: 1.9e-3 between the two over 70 keys, and the
+//     tokens of two ranks parted from those of one at a tie.  From `few` keys on the two do part (32 kv heads 5 x 950 22.5 / 18.4);
 //   * long ones, where one tile a wave takes rounds: 4 waves and as many workgroups as make 512, at most 16 (32) a pair: 1 x
 //     4200 14.8 / 11.8, 3 x 20000 45.7 / 42.0, 4 x 3000 19.3 / 16.2, 5 x 4200 23.5 / 20.2, 8 x 2400 31.0 / 20.5, 10 x 4200 35.0 /
 //     33.7, 16 x 2000 41.0 / 27.0; from 64, 80 and 112 pairs on at fewer keys: 8 x 1024 15.0 / 14.0, 10 x 1300 17.1 / 16.9, 12 x
@@ -475,6 +476,8 @@ inline V4Plan v4_plan(int B, int Hkv, int nsplit) {
   static const bool off = getenv("ILLM_ATTN_V3_NW") || getenv("ILLM_ATTN_V3_TILES") || (getenv("ILLM_ATTN_V4") && atoi(getenv("ILLM_ATTN_V4")) == 0);
   if (off) return {0, 0};                        // a forced form of attn_dec_v3.cuh (A/B runs)
   const long pairs = (long)B * Hkv, keys = (long)nsplit * SPLIT;
+  const long few = pairs >= 136 ? 576 : pairs >= 112 ? 960 : pairs >= 80 ? 1152 : pairs >= 64 ? 1024 : 1920;
+  if (B <= 8 && keys < few) return {0, 0};
   if (pairs >= 136) {
     const int nw = pairs <= 256 ? 8 : 4;
     if (keys <= 10 * V3_KPW * nw) return {nw, 1, 0};
@@ -484,7 +487,7 @@ inline V4Plan v4_plan(int B, int Hkv, int nsplit) {
     return {4, (int)((keys + (1L << row) - 1) >> row), row};
   }
   if (B > 8 && keys <= (pairs >= 112 ? 896 : pairs >= 64 ? 704 : 512)) return {keys <= 192 ? 4 : 8, 1};
-  if (keys < (pairs >= 112 ? 0 : pairs >= 80 ? 1152 : pairs >= 64 ? 1024 : 1920)) return {0, 0};
+  if (keys < few) return {0, 0};
   const long s = std::min({512 / pairs, pairs >= 16 || keys < 16384 ? 16L : 32L, keys / (4 * V3_KPW)});
   return {4, (int)s};
 }

@@ -10,6 +10,8 @@ import ipex_llm_amd.ops as ops
     # longer grids: 8 tiles in a row a workgroup, more past 32 workgroups a pair or 8192, so that one long sequence is not one's
     (32, 8, 2624, [4, 3]), (33, 8, 1344, [4, 2]), (32, 8, 16000, [4, 16]), (17, 8, 1 << 20, [4, 32]), (32, 8, 1 << 20, [4, 32]),
     (64, 8, 16384, [4, 16]), (64, 8, 32768, [4, 16]), (200, 8, 32768, [4, 8]), (100, 4, 3008, [4, 3]),
+    (4, 32, 64, [0, 0]), (4, 32, 128, [0, 0]), (4, 32, 896, [0, 0]), (4, 32, 960, [4, 4]),         # up to 8 sequences, few keys
+    (5, 32, 128, [0, 0]), (8, 32, 512, [0, 0]), (8, 32, 576, [8, 1]), (8, 40, 512, [0, 0]), (8, 40, 576, [4, 1]), (9, 32, 64, [4, 1]),
     (1, 8, 64, [0, 0]), (8, 8, 192, [0, 0]), (9, 8, 192, [4, 1]), (9, 8, 256, [8, 1]), (9, 2, 512, [8, 1]), (9, 2, 576, [0, 0]),
     (9, 8, 704, [8, 1]), (8, 8, 768, [0, 0]), (14, 8, 896, [8, 1]), (14, 8, 960, [4, 4]), (16, 8, 1088, [4, 4]),
     (8, 8, 960, [0, 0]), (8, 8, 1024, [4, 8]), (10, 8, 1088, [0, 0]), (10, 8, 1152, [4, 6]),

@@ -93,6 +93,27 @@ def test_pre_rotated(cuda, L, cap, Hkv, G, bs, plan, window, dtype):
     ops.check_kernel_errors(cuda)
 
 
+@pytest.mark.parametrize("L,Hkv", [([70, 131, 1, 64], 32), ([896, 70, 300, 512], 32), ([70, 131, 200, 33, 512], 32),
+                                   ([70, 512] * 4, 32), ([70, 512] * 4, 40), ([960, 70] * 4, 8)])
+def test_few_keys_of_up_to_8_sequences_keep_one_kernel(cuda, L, Hkv):
+    """q rotated ahead of the attention and in it: p is rounded beside the same maximum"""
+    kc, vc, bt, sl, ns = _setup(cuda, L, max(L), Hkv, 64, torch.bfloat16)
+    B, D = len(L), 128
+    assert torch.ops.ipex_llm_amd.attn_decode_plan(B, Hkv, ns) == [0, 0]
+    part = torch.randn(B, 3 * Hkv * D, device=cuda)
+    bias = torch.randn(3 * Hkv * D, device=cuda).bfloat16()
+    cs = torch.randn(max(L), D // 2, 2, device=cuda)
+    q, k1, v1 = torch.empty(B, Hkv, D, dtype=torch.bfloat16, device=cuda), kc.clone(), vc.clone()
+    ops.rope_kv_fused(part[None].clone(), bias, q, k1, v1, (sl - 1).long(), bt, 1, cs, Hkv, Hkv, D)
+    want = ops.attn_decode(q.view(B, 1, Hkv, D), k1, v1, bt, sl, ns, D ** -0.5)
+    got = ops.attn_decode_rope(part, bias, cs, (sl - 1).long(), kc, vc, bt, sl, ns, D ** -0.5, 0.0, 0, Hkv, D, False, 1.0,
+                               torch.bfloat16)
+    assert torch.equal(k1, kc) and torch.equal(v1, vc)
+    # the same sums but for the merge's order: far below the 2 ** -9 that p rounded beside another maximum is off
+    assert ((got.float() - want.float().view_as(got)).norm() / want.float().norm()).item() < 1e-3
+    ops.check_kernel_errors(cuda)
+
+
 def test_bad_block_and_length_are_reported(cuda):
     kc, vc, bt, sl, ns = _setup(cuda, [100] * 17, 128, 8, 64, torch.bfloat16)
     q = torch.randn(17, 1, 32, 128, device=cuda).bfloat16()
