@@ -444,7 +444,8 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
 }
 
 // waves of a workgroup and workgroups of a (sequence, kv head); groups 0: attn_dec_v3.cuh.  A function of batch, kv heads
-// and split grid only, so a one-token step and a verify of the same batch reduce alike.  Sequences of half to all of these
+// and split grid only, so a verify reduces as a one-token step of the same batch does -- one whose q lies in memory, rotated
+// ahead or as slabs; steps that rotate in the attention stay on attn_dec_v3.cuh.  Sequences of half to all of these
 // keys, 32 / 8 heads, us, the kernels of attn_dec_v3.cuh / this:
 //   * from 136 pairs on one workgroup each, 8 waves while they are one per CU, else 4 (two per CU): 18 x 1024 29.3 / 19.8, 20 x
 //     800 22.1 / 16.5, 24 x 1024 24.5 / 19.8, 32 x 600 21.6 / 16.9, 48 x 700 31.9 / 25.3 (8 waves 28.6), 64 x 256 19.0 / 14.5,

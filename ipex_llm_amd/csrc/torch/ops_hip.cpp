@@ -1722,6 +1722,9 @@ Tensor attn_decode_slabs(const Tensor& part, const c10::optional<Tensor>& bias, 
                          at::ScalarType dt) {
   c10::DeviceGuard g(part.device());
   TORCH_CHECK(dt == at::kBFloat16 || dt == at::kHalf, "attn_decode_slabs: bf16/fp16 activations");
+  auto here = [&](const Tensor& t) { return t.device() == part.device(); };
+  TORCH_CHECK(here(cos_sin) && here(pos) && here(k_cache) && here(v_cache) && here(block_tables) && here(seq_lens),
+              "attn_decode_slabs: tensors on part's device");
   TORCH_CHECK(k_cache.dim() == 4 && k_cache.scalar_type() == dt && v_cache.scalar_type() == dt && k_cache.is_contiguous() &&
                   v_cache.is_contiguous() && v_cache.sizes() == k_cache.sizes(), "attn_decode_slabs: contiguous 16-bit KV cache");
   TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.scalar_type() == at::kFloat && part.is_contiguous() && part.size(0) >= 1,
@@ -1733,8 +1736,11 @@ Tensor attn_decode_slabs(const Tensor& part, const c10::optional<Tensor>& bias, 
                   cos_sin.size(2) == 2, "attn_decode_slabs: f32 cos/sin table [max_pos, 64, 2]");
   TORCH_CHECK((uintptr_t)part.data_ptr() % 16 == 0 && (uintptr_t)cos_sin.data_ptr() % 16 == 0, "attn_decode_slabs: alignment");
   TORCH_CHECK(pos.scalar_type() == at::kLong && pos.is_contiguous() && pos.numel() >= B && block_tables.scalar_type() == at::kInt &&
-                  block_tables.is_contiguous() && block_tables.size(0) >= B && seq_lens.scalar_type() == at::kInt &&
-                  seq_lens.is_contiguous() && seq_lens.numel() >= B, "attn_decode_slabs: int64 positions, int32 tables of B rows");
+                  block_tables.dim() == 2 && block_tables.is_contiguous() && block_tables.size(0) >= B && block_tables.size(1) >= 1 &&
+                  seq_lens.scalar_type() == at::kInt && seq_lens.is_contiguous() && seq_lens.numel() >= B,
+              "attn_decode_slabs: int64 positions, int32 tables of B rows");
+  TORCH_CHECK(!bias.has_value() || !bias->defined() || (here(*bias) && bias->scalar_type() == dt && bias->is_contiguous() &&
+              bias->numel() == part.size(2)), "attn_decode_slabs: bias [(Hq + 2 Hkv) * 128] in the activations' dtype");
   TORCH_CHECK(attn_slabs_takes(B, Hkv, nsplit), "attn_decode_slabs: not taken");
   illm::AttnDecodeArgs a{};
   int groups = 0;                                // several: partials, merged by the last of a pair to arrive
@@ -1773,7 +1779,8 @@ Tensor attn_decode_slabs(const Tensor& part, const c10::optional<Tensor>& bias, 
   a.rq_cos_sin = cos_sin.data_ptr<float>();
   a.rq_pos = pos.data_ptr<int64_t>();
   if (pos_offset.has_value() && pos_offset->defined()) {
-    TORCH_CHECK(pos_offset->scalar_type() == at::kLong && pos_offset->is_contiguous() && pos_offset->numel() >= B, "attn_decode_slabs: int64 offsets");
+    TORCH_CHECK(here(*pos_offset) && pos_offset->scalar_type() == at::kLong && pos_offset->is_contiguous() && pos_offset->numel() >= B,
+                "attn_decode_slabs: int64 offsets");
     a.rq_pos_offset = pos_offset->data_ptr<int64_t>();
   }
   a.rq_ld = (int)part.size(2);

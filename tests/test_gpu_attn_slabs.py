@@ -80,6 +80,27 @@ def test_not_taken(cuda):
         ops.attn_decode_slabs(x, *args, 1, 0.1, 0.0, 0, 16, torch.bfloat16)
 
 
+def test_arguments_that_do_not_fit_are_refused(cuda):
+    """what the launch would read as another type, past its end or on another device"""
+    B, Hkv, Hq, bf = 17, 8, 32, torch.bfloat16
+    part, cs = torch.zeros(2, B, 6144, device=cuda), torch.zeros(64, 64, 2, device=cuda)
+    kc = torch.zeros(B, Hkv, 64, 128, dtype=bf, device=cuda)
+    bt, sl = torch.arange(B, dtype=torch.int32, device=cuda).view(B, 1), torch.ones(B, dtype=torch.int32, device=cuda)
+    good = dict(part=part, bias=torch.zeros(6144, dtype=bf, device=cuda), cos_sin=cs, pos=torch.zeros(B, dtype=torch.long, device=cuda),
+                pos_offset=torch.zeros(B, dtype=torch.long, device=cuda), k_cache=kc, v_cache=kc.clone(), block_tables=bt, seq_lens=sl)
+    rest = (1, 0.1, 0.0, 0, Hq, bf)
+    ops.attn_decode_slabs(*good.values(), *rest)
+    bad = [("bias", good["bias"].float()), ("bias", good["bias"].half()), ("bias", good["bias"][:6143].clone()), ("bias", good["bias"][:0]),
+           ("bias", torch.zeros(12288, dtype=bf, device=cuda)[::2]), ("block_tables", bt[:, :0]), ("block_tables", bt[:16].contiguous()),
+           ("block_tables", bt.flatten()), ("block_tables", bt.long()), ("seq_lens", sl[:16]), ("pos", good["pos"].int()),
+           ("pos_offset", good["pos_offset"][:16])]
+    bad += [(k, v.cpu()) for k, v in good.items() if k != "part"]
+    for name, value in bad:
+        with pytest.raises(RuntimeError):
+            ops.attn_decode_slabs(*{**good, name: value}.values(), *rest)
+    ops.check_kernel_errors(cuda)
+
+
 @pytest.mark.parametrize("kind,qtype", [("llama", "sym_int4"), ("qwen2", "fp8_e5m2"), ("mistral", "nf4")])
 @pytest.mark.parametrize("B", [11, 17, 64])
 def test_model_step(cuda, kind, qtype, B, monkeypatch):
