@@ -994,7 +994,8 @@ static void launch_v3(const AttnDecodeArgs& a, hipStream_t st) {
 }
 
 // v3 serves the 16-bit-KV, combined (not split-only) decode of head dim 64 /
-// 128 with <= 16 rows per kv head; ILLM_ATTN_V3=0 keeps v2 everywhere
+// 128 with <= 16 rows per kv head; ILLM_ATTN_V3=0 keeps v2 everywhere (attn_dec_v4.cuh is asked for behind this, and
+// attn_slabs_takes asks it)
 inline bool v3_ok(const AttnDecodeArgs& a, int D) {
   static const bool on = !(getenv("ILLM_ATTN_V3") && atoi(getenv("ILLM_ATTN_V3")) == 0);
   const int R = (a.Hq / a.Hkv) * a.Tq;

@@ -460,8 +460,8 @@ __global__ void __launch_bounds__(64 * NW, 2) attn_decode_v4_kernel(const AttnDe
 //     what rows of keys cost there: 20 x 3000 53 / 45 / 47, 17 x 3500 48 / 47 / 45, 24 x 4000 78 / 64 / 68, 40 x 1500 51 / 47 / 45, 33 x
 //     2500 71 / 69 / 57, 64 x 2000 91 / 81 / 86, 32 x 8000 170 / 161 / 166, 28 / 4 heads 40 x 3000 51 / 45 / 47, 64 x 3000 76 / 64 / 73;
 //   * fewer pairs of more than 8 sequences, so few keys that the merge is most of the time: 16 x 256 12.2 / 9.1, 16 x 800 (q
-//     pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9.  Up to 8 sequences not, however many kv heads, though most are ahead (1 x 128 8.4 / 6.0, 8 x
-//     400 10.8 / 10.1, 8 x 600 12.1 / 11.8, 32 kv heads 4 x 100 8.4 / 6.3, 5 x 250 10.3 / 8.4, 8 x 436 16.6 / 15.4; 1 x 400 even, 1 x 600
+//     pre-rotated) 22.8 / 16.1, (from memory) 16.1 / 14.9.  Up to 8 sequences not, however many kv heads, though most are ahead (q pre-rotated 1 x 128 8.4 /
+//     6.0, 8 x 400 10.8 / 10.1, 8 x 600 12.1 / 11.8, from memory 1 x 128 6.6 / 4.9, 32 kv heads 4 x 100 8.4 / 6.3, 5 x 250 10.3 / 8.4, 8 x 436 16.6 / 15.4; 1 x 400 even, 1 x 600
 //     8.9 / 9.2, 32 kv heads 4 x 250 9.5 / 10.2, 4 x 1000 16.7 / 17.2): there, steps that rotate in the attention keep attn_dec_v3.cuh,
 //     and p is rounded beside its wave's maximum here and its workgroup's there: 1.9e-3 between the two over 70 keys, and the
 //     tokens of two ranks parted from those of one at a tie.  From `few` keys on the two do part (32 kv heads 5 x 950 22.5 / 18.4);

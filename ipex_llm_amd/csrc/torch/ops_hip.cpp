@@ -1017,7 +1017,7 @@ void gemv_row_norm(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, 
   ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, illm::FK_NORM, a, st));
 }
 
-// A decode step's qkv projection that stores its rotated rows (gemv_rope) instead of adding slices of K: all, but few rows
+// A decode step's qkv projection that stores its rotated rows (gemv_rope_kv) instead of adding slices of K: all, but few rows
 // of a K past one piece a wave at 4 bits, where x is not all requested at once.  Alone, weights that no cache holds, slices
 // (their input in memory) / this, us at 1 / 4 / 8 / 16 rows: sym_int4 [6144, 4096] 6.5 7.1 8.4 11.1 / 5.6 5.9 6.4 7.9, [4608,
 // 3584] 5.0 5.3 6.7 8.6 / 4.9 5.1 5.8 7.3, [3072, 2048] 4.4 4.7 5.9 8.0 / 4.0 4.2 4.7 4.9, nf4 [6144, 4096] 9.5 10.4 11.9 14.9 /
@@ -1062,6 +1062,7 @@ static void gemv_rope_launch(const Tensor& x, const Tensor& blob, int64_t fmt, i
   ILLM_DK_SWITCH((int)fmt, illm::launch_fullk_dk<DKV>(bf16, illm::FK_ROPE, a, st));
 }
 
+// the f32 sums themselves.  No step of the models takes this form: it is what gemv_rope_kv is compared with, bit for bit
 void gemv_rope(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, const c10::optional<Tensor>& bias,
                Tensor& out, const Tensor& rope_cs, const Tensor& rope_pos, int64_t rope_cols, int64_t rope_d,
                const c10::optional<Tensor>& xss, int64_t xss_n, double xss_eps) {
@@ -1076,8 +1077,8 @@ void gemv_rope(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int6
 
 // gemv_rope of a decode step (one new token per row) that hands its columns on as the attention takes them: q [M, Hq, D]
 // rounded, the token's k and v in the paged cache at key seq_lens - 1.  The attention then has nothing to round, append or clear
-// ahead of and behind its keys: us of the attention, q, k and v as f32 sums / this, Llama-3-8B 1 x 1024 tokens 9.1 / 7.8, 4 x 1024
-// 12.3 / 10.7, 8 x 1024 13.7 / 12.8, 8 x 512 11.6 / 10.1, 1 x 128 5.9 / 4.9, Qwen2.5-7B 5 x 777 10.2 / 8.5
+// ahead of and behind its keys: us of the attention, q, k and v as f32 sums / this, Llama-3-8B 1 x 1024 tokens 9.1 / 8.0, 4 x 1024
+// 11.4 / 10.3, 8 x 1024 14.9 / 14.1, 8 x 512 11.1 / 10.1, 1 x 128 8.3 / 7.0, Qwen2.5-7B 5 sequences of up to 777 10.1 / 8.8
 Tensor gemv_rope_kv(const Tensor& x, const Tensor& blob, int64_t fmt, int64_t n, int64_t k, const c10::optional<Tensor>& bias,
                     const Tensor& rope_cs, const Tensor& rope_pos, Tensor& k_cache, Tensor& v_cache, const Tensor& block_tables,
                     const Tensor& seq_lens, int64_t Hq, const c10::optional<Tensor>& xss, int64_t xss_n, double xss_eps) {

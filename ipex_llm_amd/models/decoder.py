@@ -376,9 +376,9 @@ class NativeCausalLM(nn.Module):
             # time, the later tokens' keys cut off by a shorter length, so
             # every query row is reduced exactly as in one-token decoding
             # (greedy speculative output == plain greedy output; the fused step
-            # of a low-bit model sums q, k and v in no fixed order, and from
-            # some 3 K keys, or its verify from 256 pairs of sequence and kv
-            # head on, runs another kernel, v3_long_grid)
+            # of a low-bit model sums q, k and v in no fixed order, or where
+            # it rotates in the attention is on another kernel than its
+            # verify: head dim 128, where v4_plan takes the batch)
             c = 16 // group
             qv = q.view(meta.B, meta.Tq, s.num_heads, s.head_dim)
             outs = []
