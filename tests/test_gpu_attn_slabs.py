@@ -101,6 +101,30 @@ def test_arguments_that_do_not_fit_are_refused(cuda):
     ops.check_kernel_errors(cuda)
 
 
+def test_replays_of_a_long_grid(cuda):
+    """several workgroups a pair, captured: the tickets are left as they were, whichever sequences are long in a replay"""
+    torch.manual_seed(7)
+    B, Hkv, Hq, D, cap, bf = 18, 8, 32, 128, 3072, torch.bfloat16
+    kc, vc = (torch.randn(B * 48, Hkv, 64, D, device=cuda).to(bf) for _ in range(2))
+    bt, cs = torch.arange(B * 48, dtype=torch.int32, device=cuda).view(B, 48), torch.randn(cap, D // 2, 2, device=cuda)
+    part, sl, pos = torch.randn(2, B, 6144, device=cuda), torch.ones(B, dtype=torch.int32, device=cuda), torch.zeros(B, dtype=torch.long, device=cuda)
+    k1, v1, q = kc.clone(), vc.clone(), torch.empty(B, Hq, D, dtype=bf, device=cuda)
+    run = lambda: ops.attn_decode_slabs(part, None, cs, pos, None, kc, vc, bt, sl, 48, 0.1, 0.0, 0, Hq, bf)  # noqa: E731
+    run()
+    k1.copy_(kc), v1.copy_(vc)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for step in range(6):
+        L = torch.tensor([[1, 3072, 1024, 1025, 200, 2049][(b + step) % 6] for b in range(B)])
+        sl.copy_(L), pos.copy_(L - 1), part.normal_()
+        graph.replay()
+        ops.rope_kv_fused(part, None, q, k1, v1, pos, bt, 1, cs, Hq, Hkv, D)
+        want = ops.attn_decode(q.view(B, 1, Hq, D), k1, v1, bt, sl, 48, 0.1)
+        assert torch.equal(out.view(B, -1), want.view(B, -1)) and torch.equal(k1, kc) and torch.equal(v1, vc)
+    ops.check_kernel_errors(cuda)
+
+
 @pytest.mark.parametrize("kind,qtype", [("llama", "sym_int4"), ("qwen2", "fp8_e5m2"), ("mistral", "nf4")])
 @pytest.mark.parametrize("B", [11, 17, 64])
 def test_model_step(cuda, kind, qtype, B, monkeypatch):
